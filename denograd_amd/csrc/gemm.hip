@@ -1,404 +1,18 @@
-// Several-row linear layers on the gfx950 matrix cores: y[M][N] = x[M][K] . W[N][K]^T for M > 1 rows of fp16
-// activations (batched prefill and batched decode), fp32 accumulate, fp16 out.
+// Several-row linear layers, few rows: y[M][N] = x[M][K] . W[N][K]^T for 1 to 32 rows of fp16 activations (batched decode), fp32
+// accumulate, fp16 out, and the entry points for any number of rows (more rows: gemm_tile.hip).
 //
 // What the reference computes (/root/reference/jsgrad/tensor.ts:2593-2605 `dot`, :3800 `linear`; Int8Linear.call
 // /root/reference/jsgrad/models/llama3.ts:35; NF4Linear.call :91-97): with more than one input row the weight operand is
 // expanded over the rows, so a quantised weight is first realised in fp16, W = RN16(code * scale), and the products of
-// two fp16 values are then summed in float.  The dequantised fp16 tile written to LDS here is exactly that realised
-// matrix; v_pk_mul_f16 of the exact fp16 code by the fp16 scale is the single rounding RN16(code * scale).
-//
-// Tiling: 256 threads = 4 wavefronts laid out WGM x WGN; a wavefront owns TM x TN tiles of 32x32 outputs and walks K in
-// steps of 16 with v_mfma_f32_32x32x16_f16.  Both operands are K-contiguous in memory (x rows, W rows), so a lane's
-// 8-element operand fragment is one 128-bit LDS read.  LDS rows are padded by 8 halves (144-byte stride), which
-// spreads the 32 rows of a fragment read over all banks.  The weight fragment is the first MFMA operand, so a lane ends up
-// with four neighbouring output columns of one output row per accumulator quad: 8-byte stores in the epilogue.
-//
-// Two loop shapes.  One LDS buffer (two barriers per K tile, the next tile prefetched into registers) with two or three
-// blocks per CU, whose wavefronts cover each other's barriers and conversions.  Two LDS buffers with one 256x256 block
-// per CU (one wavefront per SIMD): one barrier per K tile, and the instruction order of a K tile is spelled out so that
-// fragment reads, conversion, LDS writes and the requests of the tile after next sit between the matrix instructions.
-// Tile ids are remapped so that the blocks resident on one XCD (round-robin by block id) share operand tiles in that
-// XCD's L2.
+// two fp16 values are then summed in float.  v_pk_mul_f16 of the exact fp16 code by the fp16 scale is that single rounding.
 #include <stdlib.h>
 #include <string.h>
 
 #include <type_traits>
 
-#include "common.h"
+#include "gemm.h"
 
 namespace jsg {
-
-typedef float f16_t __attribute__((ext_vector_type(16)));
-typedef _Float16 h4_t __attribute__((ext_vector_type(4)));
-
-enum { GEPI_STORE = 0, GEPI_ROPE_KV = 1, GEPI_SWIGLU = 2 };
-
-constexpr int GEMM_BK = 64;           // K elements per LDS tile
-constexpr int GEMM_LDS_STRIDE = 72;   // halves per LDS row (64 + 8 padding)
-constexpr int GEMM_THREADS = 256;
-
-struct GemmArgs {
-  const void *w0, *w1, *w2;           // up to three weight matrices stacked along N (wq|wk|wv, or w1|w3)
-  const _Float16 *s0, *s1, *s2;       // their scales (int8: per row; nf4: per 64 elements)
-  int n0, n1, n2;                     // their row counts
-  int M, N, K;                        // N = columns of the output this launch produces
-  const _Float16 *x;                  // [M][K]
-  _Float16 *y;                        // [M][N]  (ROPE_KV: q rows [M][n0])
-  const _Float16 *residual;           // [M][N] or null
-  // ROPE_KV
-  const _Float16 *rope_table;         // [2*max_context][hd/2][2]
-  _Float16 *cache_k, *cache_v;        // [B][max_context][n1]
-  int seq_len, start_pos, head_dim, max_context;
-};
-
-__device__ __forceinline__ uint32_t pk_mul_h2(uint32_t a, h2_t s) {
-  h2_t r = as_h2(a) * s;
-  return __builtin_bit_cast(uint32_t, r);
-}
-
-// 4 int8 codes (one dword) -> 4 exact fp16 values: byte | 0x6400 is 1024 + (code ^ 0x80), minus 1152 leaves the code
-__device__ __forceinline__ void i8x4_to_h2x2(uint32_t q, uint32_t &lo, uint32_t &hi) {
-  const uint32_t u = q ^ 0x80808080u;
-  const h2_t bias = {(_Float16)1152.0f, (_Float16)1152.0f};
-  h2_t a = as_h2(__builtin_amdgcn_perm(0x64646464u, u, 0x04010400u)) - bias;   // bytes 0,1
-  h2_t b = as_h2(__builtin_amdgcn_perm(0x64646464u, u, 0x04030402u)) - bias;   // bytes 2,3
-  lo = __builtin_bit_cast(uint32_t, a);
-  hi = __builtin_bit_cast(uint32_t, b);
-}
-
-template <int KIND, int EPI, int WGM, int WGN, int TM, int TN, bool DB = false>
-__global__ __launch_bounds__(GEMM_THREADS, (TM * TN > 8 ? 1 : (TM * TN > 4 ? 2 : 3))) void gemm_kernel(GemmArgs a) {
-  static_assert(WGM * WGN == 4, "four wavefronts");
-  static_assert(EPI != GEPI_SWIGLU || TN % 2 == 0, "a wavefront holds the w1 and the w3 tile of the same columns");
-  constexpr int BM = WGM * TM * 32, BN = WGN * TN * 32, LS = GEMM_LDS_STRIDE;
-  constexpr int A_LOADS = BM / 32;                                                    // 16-byte loads per thread per K tile
-  constexpr int B_ROWS_PER_PASS = KIND == JSGRAD_W_F16 ? 32 : KIND == JSGRAD_W_I8 ? 64 : 128;
-  constexpr int B_CHUNKS = GEMM_THREADS / B_ROWS_PER_PASS;                             // 16-byte chunks per row of the K tile
-  constexpr int B_LOADS = BN / B_ROWS_PER_PASS;
-  static_assert(B_LOADS >= 1, "tile too narrow for this weight format");
-  constexpr int BUF = (BM + BN) * LS;                     // halves per LDS buffer
-  extern __shared__ __align__(16) _Float16 gemm_lds[];   // one or two buffers of [BM + BN rows][LS], then 32 spare bytes and the 256-entry NF4 table
-  _Float16 *As = gemm_lds, *Bs = gemm_lds + BM * LS, *lut = gemm_lds + (DB ? 2 : 1) * BUF;
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave / WGN, wn = wave % WGN;
-  const int l32 = lane & 31, lg = lane >> 5;
-
-  // NF4: one table entry per BYTE, the two code values of its nibbles as a packed pair (element 2j is the high nibble,
-  // llama3.ts:92-94), so a byte costs one LDS read and one packed multiplication by the block scale
-  uint32_t *pairs = (uint32_t *)(lut + 16);
-  if constexpr (KIND == JSGRAD_W_NF4) {
-    pairs[tid] = nf4_code_bits(tid >> 4) | (nf4_code_bits(tid & 15) << 16);   // from literals: no memory round trip at the head of the launch
-  }
-
-  // ---- tile id: XCD-contiguous, then grouped so that neighbouring ids share an x tile column-block
-  const int tiles_m = (a.M + BM - 1) / BM, tiles_n = a.N / (EPI == GEPI_SWIGLU ? BN / 2 : BN);
-  const int nblocks = tiles_m * tiles_n;
-  int bid = blockIdx.x;
-  {
-    const int per = nblocks / 8;
-    if (bid < per * 8) bid = (bid & 7) * per + (bid >> 3);
-  }
-  constexpr int GROUP = KIND == JSGRAD_W_F16 ? 8 : 4;   // quantised weight tiles are half or a quarter of the bytes of an x tile: fewer x tiles, more weight tiles per XCD
-  const int in_group = GROUP * tiles_n;
-  const int first_m = (bid / in_group) * GROUP;
-  const int gsz = min(tiles_m - first_m, GROUP);
-  const int tm_ = first_m + (bid % in_group) % gsz, tn_ = (bid % in_group) / gsz;
-  const int m0 = tm_ * BM;
-  const int n0_out = tn_ * (EPI == GEPI_SWIGLU ? BN / 2 : BN);   // first output column of this tile
-
-  // ---- B source of every row this thread loads: (matrix, row) is fixed over the K loop
-  const unsigned char *bsrc[B_LOADS];
-  h2_t bscale[B_LOADS];
-  const _Float16 *bscale_ptr[B_LOADS];
-  const int brow_t = tid / B_CHUNKS, bchunk = tid % B_CHUNKS;
-#pragma unroll
-  for (int i = 0; i < B_LOADS; i++) {
-    const int r = brow_t + i * B_ROWS_PER_PASS;      // row inside the B tile
-    const void *w; const _Float16 *s; int row;
-    if constexpr (EPI == GEPI_SWIGLU) {
-      const bool up = r >= BN / 2;
-      w = up ? a.w1 : a.w0; s = up ? a.s1 : a.s0; row = n0_out + (up ? r - BN / 2 : r);
-    } else if constexpr (EPI == GEPI_ROPE_KV) {
-      const int n = n0_out + r;
-      if (n < a.n0) { w = a.w0; s = a.s0; row = n; }
-      else if (n < a.n0 + a.n1) { w = a.w1; s = a.s1; row = n - a.n0; }
-      else { w = a.w2; s = a.s2; row = n - a.n0 - a.n1; }
-    } else { w = a.w0; s = a.s0; row = n0_out + r; }
-    const size_t e = (size_t)row * a.K;              // element offset of the row
-    if constexpr (KIND == JSGRAD_W_F16) bsrc[i] = (const unsigned char *)w + e * 2 + bchunk * 16;
-    else if constexpr (KIND == JSGRAD_W_I8) { bsrc[i] = (const unsigned char *)w + e + bchunk * 16; const _Float16 sv = s[row]; bscale[i] = h2_t{sv, sv}; }
-    else { bsrc[i] = (const unsigned char *)w + e / 2 + bchunk * 16; bscale_ptr[i] = s + e / 64; }
-  }
-  const unsigned char *asrc[A_LOADS];
-  const int arow_t = tid / 8, achunk = tid % 8;
-#pragma unroll
-  for (int i = 0; i < A_LOADS; i++) {
-    int m = m0 + arow_t + i * 32;
-    if (m >= a.M) m = a.M - 1;                        // rows past the end are computed and never stored
-    asrc[i] = (const unsigned char *)(a.x + (size_t)m * a.K) + achunk * 16;
-  }
-
-  f16_t acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; i++)
-#pragma unroll
-    for (int j = 0; j < TN; j++)
-#pragma unroll
-      for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
-
-  u4_t ga[A_LOADS], gb[B_LOADS];
-  _Float16 gs[B_LOADS];
-  auto issue_a = [&](int kt) {
-    const size_t ko = (size_t)kt * GEMM_BK;
-#pragma unroll
-    for (int i = 0; i < A_LOADS; i++) ga[i] = *(const u4_t *)(asrc[i] + ko * 2);
-  };
-  auto issue_b = [&](int kt, int lo = 0, int hi = 1 << 30) {
-    const size_t ko = (size_t)kt * GEMM_BK;
-#pragma unroll
-    for (int i = 0; i < B_LOADS; i++) {
-      if (i < lo || i >= hi) continue;
-      if constexpr (KIND == JSGRAD_W_F16) gb[i] = *(const u4_t *)(bsrc[i] + ko * 2);
-      else if constexpr (KIND == JSGRAD_W_I8) gb[i] = *(const u4_t *)(bsrc[i] + ko);
-      else { gb[i] = *(const u4_t *)(bsrc[i] + ko / 2); gs[i] = bscale_ptr[i][kt]; }
-    }
-  };
-  auto issue = [&](int kt) { issue_a(kt); issue_b(kt); };
-  auto commit_a = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < A_LOADS; i++) *(u4_t *)&As[buf * BUF + (arow_t + i * 32) * LS + achunk * 8] = ga[i];
-  };
-  auto commit_b = [&](int buf, int lo = 0, int hi = 1 << 30) {
-#pragma unroll
-    for (int i = 0; i < B_LOADS; i++) {
-      if (i < lo || i >= hi) continue;
-      _Float16 *dst = &Bs[buf * BUF + (brow_t + i * B_ROWS_PER_PASS) * LS];
-      if constexpr (KIND == JSGRAD_W_F16) *(u4_t *)(dst + bchunk * 8) = gb[i];
-      else if constexpr (KIND == JSGRAD_W_I8) {
-        u4_t o0, o1;
-        uint32_t lo, hi;
-        i8x4_to_h2x2(gb[i].x, lo, hi); o0.x = pk_mul_h2(lo, bscale[i]); o0.y = pk_mul_h2(hi, bscale[i]);
-        i8x4_to_h2x2(gb[i].y, lo, hi); o0.z = pk_mul_h2(lo, bscale[i]); o0.w = pk_mul_h2(hi, bscale[i]);
-        i8x4_to_h2x2(gb[i].z, lo, hi); o1.x = pk_mul_h2(lo, bscale[i]); o1.y = pk_mul_h2(hi, bscale[i]);
-        i8x4_to_h2x2(gb[i].w, lo, hi); o1.z = pk_mul_h2(lo, bscale[i]); o1.w = pk_mul_h2(hi, bscale[i]);
-        *(u4_t *)(dst + bchunk * 16) = o0;
-        *(u4_t *)(dst + bchunk * 16 + 8) = o1;
-      } else {
-        // 16 bytes = 32 elements; the high nibble of a byte is the even element (llama3.ts:92-94)
-        const h2_t sv = {gs[i], gs[i]};
-        uint32_t wds[4] = {gb[i].x, gb[i].y, gb[i].z, gb[i].w};
-#pragma unroll
-        for (int d = 0; d < 4; d++) {
-          u4_t o;
-          uint32_t outw[4];
-#pragma unroll
-          for (int b = 0; b < 4; b++) {
-            const uint32_t byte = (wds[d] >> (8 * b)) & 0xffu;
-            outw[b] = pk_mul_h2(pairs[byte], sv);
-          }
-          o.x = outw[0]; o.y = outw[1]; o.z = outw[2]; o.w = outw[3];
-          *(u4_t *)(dst + bchunk * 32 + d * 8) = o;
-        }
-      }
-    }
-  };
-  auto commit = [&](int buf = 0) { commit_a(buf); commit_b(buf); };
-
-  auto frags = [&](int buf, int kk, h8_t *af, h8_t *bf) {
-#pragma unroll
-    for (int i = 0; i < TM; i++) af[i] = *(const h8_t *)&As[buf * BUF + ((wm * TM + i) * 32 + l32) * LS + kk * 16 + lg * 8];
-#pragma unroll
-    for (int j = 0; j < TN; j++) {
-      int rbase;
-      if constexpr (EPI == GEPI_SWIGLU) rbase = j < TN / 2 ? (wn * (TN / 2) + j) * 32 : BN / 2 + (wn * (TN / 2) + j - TN / 2) * 32;
-      else rbase = (wn * TN + j) * 32;
-      bf[j] = *(const h8_t *)&Bs[buf * BUF + (rbase + l32) * LS + kk * 16 + lg * 8];
-    }
-  };
-  auto mfmas = [&](const h8_t *af, const h8_t *bf) {
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-      for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(bf[j], af[i], acc[i][j], 0, 0, 0);   // D = W tile . x tile^T
-  };
-
-  const int nk = a.K / GEMM_BK;
-  issue(0);
-  if constexpr (KIND == JSGRAD_W_NF4) __syncthreads();   // the code table is in LDS
-  if constexpr (DB) {
-    // Two LDS buffers, one barrier per K tile: while the matrix cores work on tile kt out of one buffer, the same
-    // wavefront turns the registers of tile kt+1 into the other buffer and requests tile kt+2 into the registers just
-    // freed: the x half in K step 0, the weight half in K steps 1 and 2 (half of its loads each, which also spreads the
-    // conversion of quantised weights), so every request has a whole tile's time to arrive and the requests of a CU
-    // (64 KiB per tile through a 64 B/clock L1) are spread over the tile.
-    // The barrier sits between K steps 2 and 3.  By then every wavefront has written its share of tile kt+1 and has
-    // read all fragments of tile kt (those of step 3 are read during step 2), so during step 3 the fragments of the
-    // first step of tile kt+1 are read and the matrix instructions run on across the end of the tile.  The buffer
-    // written during tile kt is the one read during tile kt-1, whose last reads precede the barrier of kt-1.  The
-    // barrier waits for LDS traffic only, so the requests stay in flight across it.
-    commit(0);
-    if (nk > 1) issue(1);
-    lds_barrier();
-    h8_t af[2][TM], bf[2][TN];
-    frags(0, 0, af[0], bf[0]);
-    for (int kt = 0; kt < nk; kt++) {
-      const int cur = kt & 1;
-      const int after_next = min(kt + 2, nk - 1);   // past the last tile the same steps run on the last tile again, into
-                                                    // the buffer nobody computes from any more: a straight-line loop body
-      __builtin_amdgcn_sched_barrier(0);
-      auto k_step = [&](auto KK) {
-        constexpr int kk = decltype(KK)::value;
-        constexpr int LAST = GEMM_BK / 16 - 1;
-        if (kk == LAST) lds_barrier();
-        if (kk < LAST) frags(cur, kk + 1, af[(kk + 1) & 1], bf[(kk + 1) & 1]);
-        else frags(cur ^ 1, 0, af[0], bf[0]);
-        if (kk == 0) { commit_a(cur ^ 1); issue_a(after_next); }
-        constexpr int HB = B_LOADS > 1 ? B_LOADS / 2 : 1;   // weight loads of K step 1; the rest in step 2
-        if (kk == 1) { commit_b(cur ^ 1, 0, HB); issue_b(after_next, 0, HB); }
-        if (kk == 2) { commit_b(cur ^ 1, HB, B_LOADS); issue_b(after_next, HB, B_LOADS); }
-        mfmas(af[kk & 1], bf[kk & 1]);
-        // The order inside this K step, spelled out for the instruction scheduler: every matrix instruction is followed by
-        // a share of the other work of the step (fragment reads of the next step, conversion and LDS writes of the next
-        // tile, then the requests of the tile after it), so that work runs while the matrix core is busy.  Left alone the
-        // scheduler puts each fragment read directly before its first use and waits out the LDS latency every time.
-        constexpr int NMF = TM * TN;
-        constexpr int BL = kk == 1 ? HB : B_LOADS - HB;
-        constexpr int LOADS = kk == 0 ? A_LOADS : BL;
-        constexpr int WRITES = kk == 0 ? A_LOADS : (KIND == JSGRAD_W_F16 ? BL : (KIND == JSGRAD_W_I8 ? 2 * BL : 4 * BL));
-        constexpr int WSTEPS = NMF - (LOADS < NMF / 2 ? LOADS : NMF / 2);     // matrix instructions that carry the writes
-#pragma unroll
-        for (int i = 0; i < NMF; i++) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                          // one MFMA
-          if (i < TM + TN) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);          // one LDS read
-          if (kk < LAST && LOADS > 0) {
-            if (i < WSTEPS) {
-              if (kk > 0 && KIND != JSGRAD_W_F16) __builtin_amdgcn_sched_group_barrier(0x002, KIND == JSGRAD_W_I8 ? 6 : 10, 0);
-              if constexpr (kk > 0 && KIND == JSGRAD_W_NF4) __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);   // table look-ups
-              __builtin_amdgcn_sched_group_barrier(0x200, (WRITES + WSTEPS - 1) / WSTEPS, 0);
-            } else {
-              __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
-              __builtin_amdgcn_sched_group_barrier(0x020, (LOADS + NMF - WSTEPS - 1) / (NMF - WSTEPS), 0);
-            }
-          }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      };
-      static_assert(GEMM_BK / 16 == 4, "four K steps per tile");
-      k_step(std::integral_constant<int, 0>{});
-      k_step(std::integral_constant<int, 1>{});
-      k_step(std::integral_constant<int, 2>{});
-      k_step(std::integral_constant<int, 3>{});
-    }
-  } else {
-    for (int kt = 0; kt < nk; kt++) {
-      commit();
-      __syncthreads();
-      if (kt + 1 < nk) issue(kt + 1);
-#pragma unroll
-      for (int kk = 0; kk < GEMM_BK / 16; kk++) {
-        h8_t af[TM], bf[TN];
-        frags(0, kk, af, bf);
-        mfmas(af, bf);
-      }
-      __syncthreads();
-    }
-  }
-
-  // ---- epilogue.  The weight fragment is the first MFMA operand, so the 32x32 result tile is held transposed: a lane has
-  // output row m = lane % 32 and, in accumulators 4g .. 4g+3, the four neighbouring output columns 8g + 4 * (lane / 32) + 0..3.
-  // Stored from there, one instruction would touch 32 output rows with 8 bytes each.  Instead every wavefront turns 32 rows
-  // x its CW columns at a time through its own piece of LDS (free after the K loop; rows padded by 8 bytes, which spreads
-  // the 8-byte writes of 16 rows over all banks) and reads them back as 16-byte pieces along the rows: a store instruction
-  // then covers whole cache lines, and so do the loads of the residual and of the rope table.
-  constexpr int TNE = EPI == GEPI_SWIGLU ? TN / 2 : TN;   // 32-column tiles of output per wavefront and row tile
-  constexpr int CW = TNE * 32, RS = CW + 4;               // columns per wavefront; halves per LDS row
-  constexpr int CPR = CW / 8;                             // 16-byte pieces per row
-  static_assert((size_t)4 * 32 * RS <= (size_t)(BM + BN) * LS, "the transposing pieces fit the K-loop buffer");
-  _Float16 *ep = gemm_lds + wave * 32 * RS;
-  const int ncol0 = n0_out + wn * CW;                     // first output column of this wavefront
-  // the residual of the whole wavefront tile is requested at once (the registers of the K loop are free): one trip to
-  // memory instead of one per 32 rows
-  h8_t res[EPI == GEPI_STORE ? TM : 1][EPI == GEPI_STORE ? 2 * TNE : 1];
-  if constexpr (EPI == GEPI_STORE) {
-    if (a.residual) {
-#pragma unroll
-      for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int p = 0; p < 2 * TNE; p++) {
-          const int q = p * 64 + lane, row = q / CPR, piece = q % CPR;
-          int m = m0 + (wm * TM + i) * 32 + row;
-          if (m >= a.M) m = a.M - 1;
-          res[i][p] = *(const h8_t *)&a.residual[(size_t)m * a.N + ncol0 + piece * 8];
-        }
-    }
-  }
-  __syncthreads();                                        // every wavefront is done with the K-loop buffers
-#pragma unroll
-  for (int i = 0; i < TM; i++) {
-#pragma unroll
-    for (int j = 0; j < TNE; j++) {
-#pragma unroll
-      for (int g = 0; g < 4; g++) {
-        h4_t o;
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-          if constexpr (EPI == GEPI_SWIGLU) {
-            // silu(w1 x) * (w3 x), each GEMM output and the product stored as fp16 (llama.ts:108-110)
-            const float gt = rn16(acc[i][j][4 * g + c]), up = rn16(acc[i][j + TN / 2][4 * g + c]);
-            o[c] = (_Float16)(silu_act<_Float16>(gt) * up);
-          } else {
-            o[c] = (_Float16)acc[i][j][4 * g + c];
-          }
-        }
-        *(h4_t *)&ep[l32 * RS + j * 32 + 8 * g + 4 * lg] = o;
-      }
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the wavefront's own writes, before its own reads
-    const int mrow0 = m0 + (wm * TM + i) * 32;
-#pragma unroll
-    for (int p = 0; p < 2 * TNE; p++) {
-      const int q = p * 64 + lane, row = q / CPR, piece = q % CPR;
-      const int m = mrow0 + row, n = ncol0 + piece * 8;
-      const h8_t v = *(const h8_t *)&ep[row * RS + piece * 8];
-      if (m >= a.M) continue;
-      if constexpr (EPI == GEPI_SWIGLU) {
-        *(h8_t *)&a.y[(size_t)m * a.N + n] = v;
-      } else if constexpr (EPI == GEPI_STORE) {
-        h8_t o = v;
-        if (a.residual) {
-#pragma unroll
-          for (int c = 0; c < 8; c++) o[c] = (_Float16)((float)res[i][p][c] + (float)v[c]);
-        }
-        *(h8_t *)&a.y[(size_t)m * a.N + n] = o;
-      } else {
-        // wq | wk | wv columns; q and k get the interleaved-pair rotation (llama.ts:17-32), k and v go to the cache rows.
-        // Eight neighbouring columns are four pairs of one head of one matrix (every boundary is a multiple of 8).
-        const int b = m / a.seq_len, pos = a.start_pos + m % a.seq_len;
-        const int which = n < a.n0 ? 0 : (n < a.n0 + a.n1 ? 1 : 2);
-        const int nl = which == 0 ? n : (which == 1 ? n - a.n0 : n - a.n0 - a.n1);
-        h8_t o = v;
-        if (which < 2) {
-          const int pair = (nl % a.head_dim) >> 1;
-          const h8_t cs = *(const h8_t *)(a.rope_table + ((size_t)pos * (a.head_dim / 2) + pair) * 2);   // cos, sin of four pairs
-#pragma unroll
-          for (int h = 0; h < 4; h++) {
-            const float ev = (float)v[2 * h], od = (float)v[2 * h + 1];
-            const float c = (float)cs[2 * h], d = (float)cs[2 * h + 1];
-            o[2 * h] = (_Float16)(ev * c - od * d);
-            o[2 * h + 1] = (_Float16)(ev * d + od * c);
-          }
-        }
-        if (which == 0) *(h8_t *)&a.y[(size_t)m * a.n0 + nl] = o;
-        else {
-          _Float16 *cache = which == 1 ? a.cache_k : a.cache_v;
-          *(h8_t *)&cache[((size_t)b * a.max_context + pos) * a.n1 + nl] = o;
-        }
-      }
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the reads, before the next row tile overwrites the piece
-  }
-}
 
 // ---- at most 32 rows (batched decode): the weights are streamed once, straight from memory into the B operand ------------
 //
@@ -1041,38 +655,7 @@ template <int KIND, int EPI> static int dispatch_skinny(const GemmArgs &a, int p
   return two ? launch_skinny<KIND, EPI, 2, 2>(a, prof_kind) : launch_skinny<KIND, EPI, 2, 1>(a, prof_kind);
 }
 
-template <int KIND, int EPI, int WGM, int WGN, int TM, int TN, bool DB = false> static int launch_gemm(const GemmArgs &a, int prof_kind) {
-  constexpr int BM = WGM * TM * 32, BN = WGN * TN * 32;
-  const int out_per_tile = EPI == GEPI_SWIGLU ? BN / 2 : BN;
-  const int tiles = ((a.M + BM - 1) / BM) * (a.N / out_per_tile);
-  constexpr size_t lds = (size_t)(DB ? 2 : 1) * (BM + BN) * GEMM_LDS_STRIDE * sizeof(_Float16) + 32 + (KIND == JSGRAD_W_NF4 ? 1024 : 0);
-  static_assert(lds <= 160 * 1024, "LDS of one compute unit");
-  if constexpr (lds > 64 * 1024) {
-    static bool raised = false;   // one process, one device, one thread: set once per instantiation
-    if (!raised) {
-      JSG_HIP(hipFuncSetAttribute((const void *)gemm_kernel<KIND, EPI, WGM, WGN, TM, TN, DB>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-      raised = true;
-    }
-  }
-  JSG_LAUNCH(prof_kind, (gemm_kernel<KIND, EPI, WGM, WGN, TM, TN, DB>), dim3(tiles), dim3(GEMM_THREADS), lds, a);
-  return 0;
-}
-
 template <int EPI> static int dispatch_gemm(int kind, const GemmArgs &a, int prof_kind) {
-  // tall inputs: 256x256 block tiles out of two LDS buffers when the output is wide enough, else 256x128 out of one; short
-  // ones (batched decode): 32 rows x 128 columns per block.
-  // JSG_GEMM_TILE pins a shape for tests and measurements: "db", "wide" (256x256, one buffer), "tall" (256x128), "small".
-  const bool tall = a.M > 64;
-  const int n_out = EPI == GEPI_SWIGLU ? 2 * a.N : a.N;
-  const char *pin = getenv("JSG_GEMM_TILE");
-  const bool can256 = tall && n_out % 256 == 0;
-  // unpinned: the largest block shape that still gives (nearly) every CU a block; a prompt of a few hundred rows is better off with
-  // 128x128 blocks on all CUs than with 256x256 blocks on a quarter of them
-  const int cus = state().cu_count;
-  auto blocks_of = [&](int bm, int bn) { return ((a.M + bm - 1) / bm) * (n_out / bn); };
-  const bool piped = can256 && (pin ? !strcmp(pin, "db") : 4 * blocks_of(256, 256) >= 3 * cus);
-  const bool wide = can256 && pin && !strcmp(pin, "wide");
-  const bool small = tall && (pin ? !strcmp(pin, "small") : (!piped && blocks_of(256, 128) < cus));
   bool taken = false;
   if (kind == JSGRAD_W_F16) { const int rc = dispatch_skinny<JSGRAD_W_F16, EPI>(a, prof_kind, &taken); if (taken) return rc; }
   // int8, at most 16 rows: the LDS-streamed kernel, except for matrices so small that its K parts cost more than they bring
@@ -1082,30 +665,26 @@ template <int EPI> static int dispatch_gemm(int kind, const GemmArgs &a, int pro
   if (kind == JSGRAD_W_I8 && !small_matrix) { const int rc = dispatch_stream<EPI>(a, prof_kind, &taken); if (taken || rc) return rc; }
   if (kind == JSGRAD_W_I8) { const int rc = dispatch_skinny<JSGRAD_W_I8, EPI>(a, prof_kind, &taken); if (taken) return rc; }
   if (kind == JSGRAD_W_NF4) { const int rc = dispatch_skinny<JSGRAD_W_NF4, EPI>(a, prof_kind, &taken); if (taken) return rc; }
-#define JSG_CASE(K)                                                                                                    \
-  case K:                                                                                                              \
-    if (piped) return launch_gemm<K, EPI, 2, 2, 4, 4, true>(a, prof_kind);                                            \
-    if (wide) return launch_gemm<K, EPI, 2, 2, 4, 4>(a, prof_kind);                                                   \
-    if (small) return launch_gemm<K, EPI, 2, 2, 2, 2>(a, prof_kind);                                                  \
-    return tall ? launch_gemm<K, EPI, 2, 2, 4, 2>(a, prof_kind) : launch_gemm<K, EPI, 1, 4, 1, EPI == GEPI_SWIGLU ? 2 : 1>(a, prof_kind);
-  switch (kind) {
-    JSG_CASE(JSGRAD_W_F16)
-    JSG_CASE(JSGRAD_W_I8)
-    JSG_CASE(JSGRAD_W_NF4)
-  }
-#undef JSG_CASE
-  return fail("jsgrad_hip_gemm: weight kind %d is not built for several rows (fp16, int8 and nf4 are)", kind);
+  return gemm_tiled(EPI, kind, a, prof_kind);
+}
+int gemm_scratch(void **host_out, size_t *host_out_bytes) {
+  static void *p = nullptr;
+  if (!p) JSG_HIP(hipGetSymbolAddress(&p, HIP_SYMBOL(sg_scratch)));
+  *host_out = p;
+  *host_out_bytes = SG_WS_BYTES;
+  return 0;
 }
 
 // largest column tile any configuration uses: output widths must be multiples of it
 constexpr int GEMM_N_ALIGN = 128;
+constexpr int GEMM_K_ALIGN = 64;   // a K tile
 
 static bool aligned16(const void *p) { return ((uintptr_t)p & 15) == 0; }
 
 static int check_gemm(const char *who, int kind, int rows, int in_f) {
   JSG_REQUIRE(kind == JSGRAD_W_F16 || kind == JSGRAD_W_I8 || kind == JSGRAD_W_NF4, "%s: weight kind %d is not built for several rows (fp16, int8 and nf4 are)", who, kind);
   JSG_REQUIRE(rows > 0, "%s: %d rows", who, rows);
-  JSG_REQUIRE(in_f > 0 && in_f % GEMM_BK == 0, "%s: in_features %d must be a positive multiple of %d", who, in_f, GEMM_BK);
+  JSG_REQUIRE(in_f > 0 && in_f % GEMM_K_ALIGN == 0, "%s: in_features %d must be a positive multiple of %d", who, in_f, GEMM_K_ALIGN);
   return 0;
 }
 

@@ -1,0 +1,667 @@
+// Several-row linear layers with more rows than the weight-streaming kernels take (gemm.hip): y[M][N] = x[M][K] . W[N][K]^T on
+// the gfx950 matrix cores, fp16 operands, float accumulation, fp16 out.
+//
+// What the reference computes (/root/reference/jsgrad/tensor.ts:2593-2605 `dot`, :3800 `linear`; Int8Linear.call
+// /root/reference/jsgrad/models/llama3.ts:35; NF4Linear.call :91-97): with more than one input row the weight operand is
+// expanded over the rows, so a quantised weight is first realised in fp16, W = RN16(code * scale), and the products of
+// two fp16 values are then summed in float.  So it is here: `realise_kernel` writes that matrix once per call (int8 8B w1|w3:
+// 117 MB in, 235 MB out, ~70 us, where the product takes 5.4 ms at 32768 rows) and one fp16 kernel serves the three formats.
+// Dequantising inside the product was the alternative: it needs the weight tile to pass through registers, and that
+// kernel stopped at 1.05-1.1 PFLOP/s.
+//
+// Both operands are K-contiguous in memory (x rows, W rows), so an operand fragment of v_mfma_f32_16x16x32_f16 (8 K elements
+// of one row per lane) is one 16-byte LDS read.  The 16x16 instruction is used because the chip is power-limited under this
+// load: registers only, random data, it sustains 1.87 PFLOP/s at 1.90 GHz, the 32x32 one 1.62 at 1.68 GHz.
+// K tiles of 64: a row of a tile is one 128-byte line.  Tiles come by direct global-to-LDS loads: a wavefront's load fills
+// 1 KiB of LDS in lane order, i.e. eight rows, and the lanes pick their 16-byte piece of the row so that piece p of row r
+// lands at position p ^ (r & 7): fragment reads of 16 rows then hit different banks without padding, which such a load
+// could not produce.  The loads are written as assembly, because the compiler, which sees LDS written, would drain them
+// before every LDS read.
+//
+// Eight wavefronts, two per SIMD, as two groups that take turns (half a phase apart, a barrier per turn): while one group's
+// matrix instructions run, the other reads its next fragments and asks for tiles further on.
+#include <stdlib.h>
+#include <string.h>
+
+#include "gemm.h"
+
+namespace jsg {
+
+constexpr int TILE_BK = 64;
+constexpr int TILE_THREADS = 512;
+
+// One launch of a tiled kernel: columns [col0, col0 + ncols) of the output.
+struct TileArgs {
+  GemmArgs g;                          // output side: y, residual, rope, cache, M, N, K
+  const _Float16 *b[3];                // fp16 weight rows of those columns, up to three matrices on top of each other
+  int b_end[2];                        // ends of the first two (SWIGLU: b[0] is w1, b[1] is w3, row for row)
+  int col0, ncols;
+  int split;                           // K parts
+  float *ws;                           // split > 1: [tile][part][BM * BN] floats
+  int *counters;                       // split > 1: one per tile, zero, and zero again afterwards
+};
+
+typedef int i4_t __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ i4_t tile_rsrc(const void *p) {
+  const uint64_t v = (uint64_t)p;
+  i4_t r;
+  r.x = __builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+  r.y = __builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+  r.z = -1;                            // offsets are in bounds by construction (rows past M are clamped)
+  r.w = 0x00020000;
+  return r;
+}
+// 64 lanes x 16 bytes from rs + voff(lane) + soff to LDS bytes [lds, lds + 1024) in lane order.  M0 holds the LDS address; one
+// wait state between writing it and the load that reads it.
+__device__ __forceinline__ void dma16(i4_t rs, uint32_t voff, uint32_t soff, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rs), "s"(soff) : "memory");
+}
+template <int N> __device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+__device__ __forceinline__ void turn_barrier() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_barrier" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+// ... after this wavefront's LDS reads have arrived
+__device__ __forceinline__ void turn_barrier_lds() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// Block id -> tile (and K part): blocks are dealt to the eight XCDs round-robin, so ids are first made contiguous per XCD; K
+// parts of a tile are neighbours, then GROUP row tiles share each column tile, so that the blocks resident on one XCD share
+// operand tiles in its L2.  (GROUP 2 / 4 / 8 / 16 at 32768 x 4096 x 14336: 1453 / 1451 / 1413 / 1334 TFLOP/s, at
+// 32768 x 28672 x 4096: 1392 / 1422 / 1440 / 1318.)
+struct TileId { int tile, part, m0, col; };
+template <int BM, int CW> __device__ __forceinline__ TileId tile_id(const TileArgs &t) {
+  constexpr int GROUP = 4;
+  const int tiles_m = (t.g.M + BM - 1) / BM, tiles_n = t.ncols / CW, nblocks = tiles_m * tiles_n * t.split;
+  int bid = blockIdx.x;
+  const int per = nblocks / 8;
+  if (bid < per * 8) bid = (bid & 7) * per + (bid >> 3);
+  TileId r;
+  r.part = bid % t.split;
+  r.tile = bid / t.split;
+  const int in_group = GROUP * tiles_n, first_m = (r.tile / in_group) * GROUP, gsz = min(tiles_m - first_m, GROUP);
+  r.m0 = (first_m + (r.tile % in_group) % gsz) * BM;
+  r.col = ((r.tile % in_group) / gsz) * CW;
+  return r;
+}
+
+// Where row r (a multiple of 8; eight rows never straddle two matrices) of the weight tile of BN rows lies.
+template <int EPI, int BN> __device__ __forceinline__ const _Float16 *weight_row(const TileArgs &t, int col, int r) {
+  if constexpr (EPI == GEPI_SWIGLU) return (r < BN / 2 ? t.b[0] : t.b[1]) + (size_t)(col + (r < BN / 2 ? r : r - BN / 2)) * t.g.K;
+  else {
+    const int n = col + r;
+    if (n < t.b_end[0]) return t.b[0] + (size_t)n * t.g.K;
+    if (n < t.b_end[1]) return t.b[1] + (size_t)(n - t.b_end[0]) * t.g.K;
+    return t.b[2] + (size_t)(n - t.b_end[1]) * t.g.K;
+  }
+}
+
+// ---- epilogue of one wavefront: R16 x C16 tiles of 16x16 outputs.  The weight fragment is the first MFMA operand, so a lane
+// holds output row lane % 16 and the four neighbouring columns 4 * (lane / 16) + 0..3 of a tile.  Stored from there an
+// instruction would touch 16 rows with 32 bytes each (4 % on a K = 4096 product); the wavefront turns RB row tiles at a time through
+// its own piece of LDS and reads them back as 16-byte pieces along the rows, so stores, residual and rope table move whole
+// lines.  val(i, j, c): accumulator c of row tile i, column tile j as a float.
+template <int EPI, int R16, int C16, int RB, typename F>
+__device__ __forceinline__ void tile_epilogue(const GemmArgs &a, _Float16 *ep, int mrow, int ncol, const F &val) {
+  constexpr int CW = C16 * 16, RS = CW + 8, CPR = CW / 8, PASS = RB * 16 * CPR / 64;
+  static_assert(R16 % RB == 0 && PASS >= 1 && 64 % CPR == 0, "whole passes of 64 lanes");
+  const int lane = threadIdx.x & 63, l16 = lane & 15, lq = lane >> 4;
+#pragma unroll
+  for (int i0 = 0; i0 < R16; i0 += RB) {
+    // the residual of these rows is requested before they are turned
+    h8_t res[EPI == GEPI_STORE ? PASS : 1];
+    if constexpr (EPI == GEPI_STORE) {
+      if (a.residual) {
+#pragma unroll
+        for (int p = 0; p < PASS; p++) {
+          const int q = p * 64 + lane, m = min(mrow + i0 * 16 + q / CPR, a.M - 1);
+          res[p] = *(const h8_t *)&a.residual[(size_t)m * a.N + ncol + (q % CPR) * 8];
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < RB; i++)
+#pragma unroll
+      for (int j = 0; j < C16; j++) {
+        h4_t o;
+#pragma unroll
+        for (int c = 0; c < 4; c++) o[c] = (_Float16)val(i0 + i, j, c);
+        *(h4_t *)&ep[(i * 16 + l16) * RS + j * 16 + lq * 4] = o;
+      }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the wavefront's own writes, before its own reads
+#pragma unroll
+    for (int p = 0; p < PASS; p++) {
+      const int q = p * 64 + lane, row = q / CPR, piece = q % CPR;
+      const int m = mrow + i0 * 16 + row, n = ncol + piece * 8;
+      const h8_t v = *(const h8_t *)&ep[row * RS + piece * 8];
+      if (m >= a.M) continue;
+      if constexpr (EPI == GEPI_SWIGLU) {
+        *(h8_t *)&a.y[(size_t)m * a.N + n] = v;
+      } else if constexpr (EPI == GEPI_STORE) {
+        h8_t o = v;
+        if (a.residual) {
+#pragma unroll
+          for (int c = 0; c < 8; c++) o[c] = (_Float16)((float)res[p][c] + (float)v[c]);
+        }
+        *(h8_t *)&a.y[(size_t)m * a.N + n] = o;
+      } else {
+        // wq | wk | wv columns; q and k get the interleaved-pair rotation (llama.ts:17-32), k and v go to the cache rows.
+        // Eight neighbouring columns are four pairs of one head of one matrix (every boundary is a multiple of 8).
+        const int b = m / a.seq_len, pos = a.start_pos + m % a.seq_len;
+        const int which = n < a.n0 ? 0 : (n < a.n0 + a.n1 ? 1 : 2);
+        const int nl = which == 0 ? n : (which == 1 ? n - a.n0 : n - a.n0 - a.n1);
+        h8_t o = v;
+        if (which < 2) {
+          const int pair = (nl % a.head_dim) >> 1;
+          const h8_t cs = *(const h8_t *)(a.rope_table + ((size_t)pos * (a.head_dim / 2) + pair) * 2);   // cos, sin of four pairs
+#pragma unroll
+          for (int h = 0; h < 4; h++) {
+            const float ev = (float)v[2 * h], od = (float)v[2 * h + 1];
+            const float c = (float)cs[2 * h], d = (float)cs[2 * h + 1];
+            o[2 * h] = (_Float16)(ev * c - od * d);
+            o[2 * h + 1] = (_Float16)(ev * d + od * c);
+          }
+        }
+        if (which == 0) *(h8_t *)&a.y[(size_t)m * a.n0 + nl] = o;
+        else {
+          _Float16 *cache = which == 1 ? a.cache_k : a.cache_v;
+          *(h8_t *)&cache[((size_t)b * a.max_context + pos) * a.n1 + nl] = o;
+        }
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the reads, before the next rows overwrite the piece
+  }
+}
+// silu(w1 x) * (w3 x), each GEMM output and the product stored as fp16 (llama.ts:108-110)
+__device__ __forceinline__ float swiglu(float gate, float up) { return silu_act<_Float16>(rn16(gate)) * rn16(up); }
+
+// ---------------------------------------------------------------- 256 x 256
+//
+// Wavefront (g, wn) owns rows 128 g .. +127 and columns 64 wn .. +63 as four quadrants of 64 x 32; a phase of a K tile is one
+// quadrant (16 matrix instructions, ~270 cycles): A0 B0 | A0 B1 | A1 B1 | A1 B0, so a tile costs 24 fragment reads and
+// fits 210 registers.  Time runs in slots separated by barriers; group 0 reads in slot 2p and computes in slot 2p + 1 of
+// phase p, group 1 one slot later.  Two LDS buffers of 64 KiB: the part of a buffer that both groups have read is refilled
+// at once with the tile after next (A0 read in slots 0 and 1, refilled in slots 2 and 3; B0 in 4 and 5; B1, read in 2 and
+// 3, in 6 and 7; A1, read in 4 and 5, in 8 and 9), so every load has 11 slots (3000 cycles) to arrive and five pairs of a
+// wavefront's loads may be outstanding when a phase needs the sixth.
+// Measured (fp16): 32768 x 28672 x 4096 1420, 32768 x 4096 x 14336 1430-1450, 4096^3 1410 TFLOP/s (1050-1110 for the kernel
+// with 32x32 instructions and tiles through registers it replaces; the same loop without its epilogue 1500).
+constexpr int T256_OPERAND = 256 * 128;                       // bytes of one operand tile
+template <int EPI> __global__ __launch_bounds__(TILE_THREADS, 2) void tile256_kernel(TileArgs t) {
+  const GemmArgs &a = t.g;
+  extern __shared__ __align__(16) unsigned char tile_lds[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, lq = lane >> 4;
+  const int g = wave >> 2, wn = wave & 3;
+  constexpr int CW = EPI == GEPI_SWIGLU ? 128 : 256;
+  const TileId id = tile_id<256, CW>(t);
+  const int m0 = id.m0;
+
+  // Loads: half h of an operand is 128 rows = 16 loads of eight rows, two per wavefront.  The tile's rows are ordered by
+  // who reads them: LDS row = 128 g + 64 h + .. for x, 64 wn + 32 h + .. for the weights.
+  const uint32_t row_bytes = (uint32_t)a.K * 2;
+  const i4_t ra = tile_rsrc(a.x + (size_t)m0 * a.K);
+  const int lr = lane >> 3, lp = lane & 7;
+  const uint32_t piece = (uint32_t)(lp ^ lr) * 16;            // rows of a load start at a multiple of 8
+  uint32_t va[2][2], la[2][2], lb[2][2];
+  i4_t rb[2][2];
+#pragma unroll
+  for (int h = 0; h < 2; h++)
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      const int idx = 2 * wave + i;
+      const int ar = (idx >> 3) * 128 + h * 64 + (idx & 7) * 8, br = (idx >> 2) * 64 + h * 32 + (idx & 3) * 8;
+      va[h][i] = (uint32_t)min(ar + lr, a.M - 1 - m0) * row_bytes + piece;   // rows past the end are computed and never stored
+      const int src = EPI == GEPI_SWIGLU ? h * 128 + (idx >> 2) * 32 + (idx & 3) * 8 : br;   // half 0: w1 rows, half 1: w3 rows
+      rb[h][i] = tile_rsrc(weight_row<EPI, 256>(t, id.col, src));
+      la[h][i] = ar * 128;
+      lb[h][i] = T256_OPERAND + br * 128;
+    }
+  const uint32_t vb = (uint32_t)lr * row_bytes + piece;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)tile_lds;
+  const int nk = a.K / TILE_BK;
+  // past the last tile the last one is asked for again, into a buffer nobody computes from any more
+  auto load_a = [&](int kt, int h) {
+    const uint32_t so = (uint32_t)min(kt, nk - 1) * 128, base = lds0 + (kt & 1) * 2 * T256_OPERAND;
+    dma16(ra, va[h][0], so, base + la[h][0]);
+    dma16(ra, va[h][1], so, base + la[h][1]);
+  };
+  auto load_b = [&](int kt, int h) {
+    const uint32_t so = (uint32_t)min(kt, nk - 1) * 128, base = lds0 + (kt & 1) * 2 * T256_OPERAND;
+    dma16(rb[h][0], vb, so, base + lb[h][0]);
+    dma16(rb[h][1], vb, so, base + lb[h][1]);
+  };
+
+  f4_t acc[2][4][2][2];                                       // [x half][row tile][weight half][column tile]
+#pragma unroll
+  for (int p = 0; p < 2; p++)
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+      for (int q = 0; q < 2; q++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) acc[p][i][q][j] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  h8_t af[4][2], bf[2][2][2];
+  const uint32_t sw0 = (uint32_t)(lq ^ (l16 & 7)) * 16, sw1 = sw0 ^ 64;   // position of K pieces lq and lq + 4 in rows congruent to l16
+  auto read_a = [&](int cur, int h) {
+    const unsigned char *p = tile_lds + cur * 2 * T256_OPERAND + (g * 128 + h * 64 + l16) * 128;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      af[i][0] = *(const h8_t *)(p + i * 2048 + sw0);
+      af[i][1] = *(const h8_t *)(p + i * 2048 + sw1);
+    }
+  };
+  auto read_b = [&](int cur, int h) {
+    const unsigned char *p = tile_lds + cur * 2 * T256_OPERAND + T256_OPERAND + (wn * 64 + h * 32 + l16) * 128;
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      bf[h][j][0] = *(const h8_t *)(p + j * 2048 + sw0);
+      bf[h][j][1] = *(const h8_t *)(p + j * 2048 + sw1);
+    }
+  };
+  auto compute = [&](int ah, int bh) {
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int k = 0; k < 2; k++)
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) acc[ah][i][bh][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bf[bh][j][k], af[i][k], acc[ah][i][bh][j], 0, 0, 0);
+    __builtin_amdgcn_s_setprio(0);
+  };
+
+  load_a(0, 0); load_b(0, 0); load_b(0, 1); load_a(0, 1);
+  load_a(1, 0); load_b(1, 0); load_b(1, 1);
+  wait_loads<10>();
+  turn_barrier();                                             // A0 and B0 of tile 0 are there
+  if (g == 1) turn_barrier();                                 // group 1 is a slot behind
+  for (int kt = 0; kt < nk; kt++) {
+    const int cur = kt & 1;
+    read_a(cur, 0); read_b(cur, 0); load_a(kt + 1, 1);
+    wait_loads<10>(); turn_barrier_lds();                     // B1 of this tile has landed
+    compute(0, 0); turn_barrier();
+    read_b(cur, 1); load_a(kt + 2, 0);
+    wait_loads<10>(); turn_barrier_lds();                     // A1 of this tile
+    compute(0, 1); turn_barrier();
+    read_a(cur, 1); load_b(kt + 2, 0);
+    turn_barrier_lds();
+    compute(1, 1); turn_barrier();
+    load_b(kt + 2, 1);
+    wait_loads<10>(); turn_barrier();                         // A0 and B0 of the next tile
+    compute(1, 0); turn_barrier();
+  }
+  if (g == 0) turn_barrier();
+  wait_loads<0>();
+  turn_barrier();                                             // nobody reads or fills the tiles any more
+
+  constexpr int C16 = EPI == GEPI_SWIGLU ? 2 : 4;
+  _Float16 *ep = (_Float16 *)tile_lds + wave * 64 * (C16 * 16 + 8);
+  tile_epilogue<EPI, 8, C16, 4>(a, ep, m0 + g * 128, t.col0 + id.col + wn * C16 * 16, [&](int i, int j, int c) {
+    if constexpr (EPI == GEPI_SWIGLU) return swiglu(acc[i >> 2][i & 3][0][j][c], acc[i >> 2][i & 3][1][j][c]);
+    else return acc[i >> 2][i & 3][j >> 1][j & 1][c];
+  });
+}
+
+// ---------------------------------------------------------------- smaller tiles, K parts
+//
+// The same eight wavefronts as 2 x 4 over a BM x BN tile, a phase per K tile (two groups half a phase apart as above), ST tiles
+// in LDS, of which ST - 1 are on their way or being read.  For inputs of some dozens to some hundred rows, where 256 x 256
+// tiles would leave most of the chip idle.  What bounds it, from builds with parts of the loop left out (128 x 128, 64 K
+// tiles, us): nothing but barriers 3, matrix instructions 15, direct loads 18 (the 64 bytes a clock of a CU's L1), fragment
+// reads 21 (each group reads alone and waits), all of it 30.
+// K parts: a part leaves its float sums in the workspace and the last of a tile's parts to arrive adds them in K order, so
+// the result does not depend on who is last.
+template <int EPI, int BM, int BN, int ST> constexpr size_t tile_lds_bytes() { return (size_t)(BM + BN) * 128 * ST; }
+template <int EPI, int BM, int BN, int ST> __global__ __launch_bounds__(TILE_THREADS, 2) void tile_kernel(TileArgs t) {
+  const GemmArgs &a = t.g;
+  extern __shared__ __align__(16) unsigned char tile_lds[];
+  constexpr int TM = BM / 32, TN = BN / 64, NLD = (BM + BN) / 64, BUF = (BM + BN) * 128;
+  static_assert(EPI != GEPI_SWIGLU || TN % 2 == 0, "a wavefront holds the w1 and the w3 tile of the same columns");
+  constexpr int CW = EPI == GEPI_SWIGLU ? BN / 2 : BN;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, lq = lane >> 4;
+  const int g = wave >> 2, wn = wave & 3;
+  const TileId id = tile_id<BM, CW>(t);
+  const int m0 = id.m0;
+
+  const uint32_t row_bytes = (uint32_t)a.K * 2;
+  const i4_t ra = tile_rsrc(a.x + (size_t)m0 * a.K);
+  const int lr = lane >> 3, lp = lane & 7;
+  const uint32_t piece = (uint32_t)(lp ^ lr) * 16;
+  constexpr int NA = BM / 64, NB = BN / 64;                   // a wavefront's loads per tile: eight rows each, 64 rows apart
+  uint32_t va[NA];
+  i4_t rb[NB];
+#pragma unroll
+  for (int i = 0; i < NA; i++) va[i] = (uint32_t)min(wave * 8 + i * 64 + lr, a.M - 1 - m0) * row_bytes + piece;
+#pragma unroll
+  for (int i = 0; i < NB; i++) rb[i] = tile_rsrc(weight_row<EPI, BN>(t, id.col, wave * 8 + i * 64));
+  const uint32_t vb = (uint32_t)lr * row_bytes + piece;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)tile_lds + wave * 1024;
+  const int nkt = a.K / TILE_BK, k0 = (int)((long long)id.part * nkt / t.split), nk = (int)((long long)(id.part + 1) * nkt / t.split) - k0;
+  auto load = [&](int kt, int buf) {
+    const uint32_t so = (uint32_t)(k0 + min(kt, nk - 1)) * 128, base = lds0 + buf * BUF;
+#pragma unroll
+    for (int i = 0; i < NA; i++) dma16(ra, va[i], so, base + i * 8192);
+#pragma unroll
+    for (int i = 0; i < NB; i++) dma16(rb[i], vb, so, base + BM * 128 + i * 8192);
+  };
+
+  f4_t acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; i++)
+#pragma unroll
+    for (int j = 0; j < TN; j++) acc[i][j] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  h8_t af[2][TM], bf[2][TN];
+  const uint32_t sw0 = (uint32_t)(lq ^ (l16 & 7)) * 16, sw1 = sw0 ^ 64;
+  auto read = [&](int buf) {
+    const unsigned char *pa = tile_lds + buf * BUF + (g * TM * 16 + l16) * 128, *pb = tile_lds + buf * BUF + BM * 128 + l16 * 128;
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+      const uint32_t sw = k ? sw1 : sw0;
+#pragma unroll
+      for (int i = 0; i < TM; i++) af[k][i] = *(const h8_t *)(pa + i * 2048 + sw);
+#pragma unroll
+      for (int j = 0; j < TN; j++) {
+        const int row = EPI == GEPI_SWIGLU ? (j < TN / 2 ? 0 : BN / 2) + (wn * (TN / 2) + j % (TN / 2 > 0 ? TN / 2 : 1)) * 16 : (wn * TN + j) * 16;
+        bf[k][j] = *(const h8_t *)(pb + row * 128 + sw);
+      }
+    }
+  };
+
+#pragma unroll
+  for (int i = 0; i < ST - 1; i++) load(i, i);
+  wait_loads<(ST - 2) * NLD>();
+  turn_barrier();
+  if (g == 1) turn_barrier();
+  int buf = 0, into = ST - 1;
+  for (int kt = 0; kt < nk; kt++) {
+    read(buf);
+    load(kt + ST - 1, into);                                  // the buffer of tile kt - 1, which both groups have read
+    wait_loads<(ST - 2) * NLD>();                             // tile kt + 1 has landed
+    turn_barrier_lds();
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int k = 0; k < 2; k++)
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bf[k][j], af[k][i], acc[i][j], 0, 0, 0);
+    __builtin_amdgcn_s_setprio(0);
+    turn_barrier();
+    buf = buf + 1 == ST ? 0 : buf + 1;
+    into = into + 1 == ST ? 0 : into + 1;
+  }
+  if (g == 0) turn_barrier();
+  wait_loads<0>();
+  turn_barrier();
+
+  if (t.split > 1) {
+    // Parts run on different XCDs: stores and loads that go to the point all of them share (cache policy 16: device scope),
+    // and the count goes up once the block's stores are acknowledged.  The part is in the vector offset: behind a 16-byte store
+    // with its offset in a scalar register the compiler overwrites the first data register too early (sums came out
+    // with every fourth value zero).
+    __shared__ int last;
+    const __amdgpu_buffer_rsrc_t rw = wave_buffer(t.ws + (size_t)id.tile * t.split * BM * BN, (uint32_t)t.split * BM * BN * 4u);
+    const uint32_t o0 = ((uint32_t)wave * TM * TN * 64 + lane) * 16;
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+      for (int j = 0; j < TN; j++)
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4_t, acc[i][j]), rw, o0 + (uint32_t)id.part * BM * BN * 4u + (i * TN + j) * 1024, 0, 16);
+    wait_loads<0>();
+    turn_barrier();
+    if (tid == 0) {
+      const int old = __hip_atomic_fetch_add(&t.counters[id.tile], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      last = old == t.split - 1;
+      if (last) __hip_atomic_store(&t.counters[id.tile], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // for the next launch
+    }
+    __syncthreads();
+    if (!last) return;
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+      for (int j = 0; j < TN; j++) acc[i][j] = __builtin_bit_cast(f4_t, __builtin_amdgcn_raw_buffer_load_b128(rw, o0 + (i * TN + j) * 1024, 0, 16));
+    for (int p = 1; p < t.split; p++) {
+      f4_t u[TM][TN];
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+          u[i][j] = __builtin_bit_cast(f4_t, __builtin_amdgcn_raw_buffer_load_b128(rw, o0 + (uint32_t)p * BM * BN * 4u + (i * TN + j) * 1024, 0, 16));
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i][j] += u[i][j];
+    }
+  }
+
+  constexpr int C16 = EPI == GEPI_SWIGLU ? TN / 2 : TN, RB = TM < 4 ? TM : 4;
+  _Float16 *ep = (_Float16 *)tile_lds + wave * RB * 16 * (C16 * 16 + 8);
+  static_assert((size_t)8 * RB * 16 * (C16 * 16 + 8) * 2 <= tile_lds_bytes<EPI, BM, BN, ST>(), "the turning pieces fit the tiles' LDS");
+  tile_epilogue<EPI, TM, C16, RB>(a, ep, m0 + g * TM * 16, t.col0 + id.col + wn * C16 * 16, [&](int i, int j, int c) {
+    if constexpr (EPI == GEPI_SWIGLU) return swiglu(acc[i][j][c], acc[i][j + TN / 2][c]);
+    else return acc[i][j][c];
+  });
+}
+
+// ---------------------------------------------------------------- quantised weights, realised in fp16
+//
+// Rows [row0, row0 + rows) of one matrix to out[rows][K].  A thread takes 16 bytes of codes and stores 32 (int8) or 64 (nf4)
+// bytes; bound by memory (4.5-5 TB/s of codes in and halves out).
+template <int KIND> __global__ __launch_bounds__(256) void realise_kernel(const unsigned char *w, const _Float16 *scale, _Float16 *out, int row0, size_t pieces, int ppr) {
+  // nf4: one table entry per BYTE, the two code values of its nibbles as a packed pair (element 2j is the high nibble,
+  // llama3.ts:92-94)
+  __shared__ uint32_t pairs[KIND == JSGRAD_W_NF4 ? 256 : 1];
+  if constexpr (KIND == JSGRAD_W_NF4) {
+    pairs[threadIdx.x] = nf4_code_bits(threadIdx.x >> 4) | (nf4_code_bits(threadIdx.x & 15) << 16);
+    __syncthreads();
+  }
+  const size_t first = (size_t)row0 * ppr;
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < pieces; i += (size_t)gridDim.x * 256) {
+    const u4_t q = ldg_stream16(w + (first + i) * 16);
+    const uint32_t wds[4] = {q.x, q.y, q.z, q.w};
+    if constexpr (KIND == JSGRAD_W_I8) {
+      const _Float16 s1 = scale[row0 + (int)(i / (unsigned)ppr)];
+      const h2_t s = {s1, s1};
+      u4_t o[2];
+#pragma unroll
+      for (int d = 0; d < 4; d++) {
+        uint32_t lo, hi;
+        i8x4_to_h2x2(wds[d], lo, hi);
+        o[d / 2][(d % 2) * 2] = pk_mul_h2(lo, s);
+        o[d / 2][(d % 2) * 2 + 1] = pk_mul_h2(hi, s);
+      }
+      u4_t *dst = (u4_t *)(out + i * 16);
+      dst[0] = o[0];
+      dst[1] = o[1];
+    } else {
+      const _Float16 s1 = scale[(first + i) >> 1];            // 32 codes: half a scale block
+      const h2_t s = {s1, s1};
+      u4_t *dst = (u4_t *)(out + i * 32);
+#pragma unroll
+      for (int d = 0; d < 4; d++) {
+        u4_t o;
+#pragma unroll
+        for (int b = 0; b < 4; b++) o[b] = pk_mul_h2(pairs[(wds[d] >> (8 * b)) & 0xffu], s);
+        dst[d] = o;
+      }
+    }
+  }
+}
+
+static int realise(int kind, const void *w, const _Float16 *scale, int row0, int rows, int K, _Float16 *out, int prof_kind) {
+  const int ppr = kind == JSGRAD_W_I8 ? K / 16 : K / 32;      // pieces per row
+  const size_t pieces = (size_t)rows * ppr;
+  const size_t want = (pieces + 255) / 256;
+  const int grid = (int)(want < (size_t)16 * state().cu_count ? want : (size_t)16 * state().cu_count);
+  if (kind == JSGRAD_W_I8) JSG_LAUNCH(prof_kind, realise_kernel<JSGRAD_W_I8>, dim3(grid), dim3(256), 0, (const unsigned char *)w, scale, out, row0, pieces, ppr);
+  else JSG_LAUNCH(prof_kind, realise_kernel<JSGRAD_W_NF4>, dim3(grid), dim3(256), 0, (const unsigned char *)w, scale, out, row0, pieces, ppr);
+  return 0;
+}
+
+// ---------------------------------------------------------------- host side
+
+constexpr int TILE_COUNTERS = 4096;
+static __device__ int tile_counters[TILE_COUNTERS];
+
+// A block of the allocator's pool for the length of one call.  Handing it back right behind the launches is safe: one
+// in-order stream serves every launch, so whoever gets the block next writes it after these launches have read it.  The pool
+// is bounded and gives memory back (runtime.hip).  During a graph capture nothing can be allocated: p stays null.
+struct PoolBlock {
+  void *p = nullptr;
+  int get(size_t nbytes) { return state().capturing ? 0 : jsgrad_hip_malloc(nbytes, &p); }
+  ~PoolBlock() { if (p) jsgrad_hip_free(p); }
+};
+
+template <int EPI> static int launch_tile256(const TileArgs &t, int prof_kind) {
+  constexpr int lds = 4 * T256_OPERAND;
+  static bool raised = false;   // one process, one device, one thread: set once per instantiation
+  if (!raised) {
+    JSG_HIP(hipFuncSetAttribute((const void *)tile256_kernel<EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    raised = true;
+  }
+  const int tiles = ((t.g.M + 255) / 256) * (t.ncols / (EPI == GEPI_SWIGLU ? 128 : 256));
+  JSG_LAUNCH(prof_kind, (tile256_kernel<EPI>), dim3(tiles), dim3(TILE_THREADS), lds, t);
+  return 0;
+}
+template <int EPI, int BM, int BN, int ST> static int launch_tile(const TileArgs &t, int prof_kind) {
+  constexpr int lds = (int)tile_lds_bytes<EPI, BM, BN, ST>();
+  static_assert(lds + 64 <= 160 * 1024, "LDS of one compute unit");
+  static bool raised = false;
+  if (!raised) {
+    JSG_HIP(hipFuncSetAttribute((const void *)tile_kernel<EPI, BM, BN, ST>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    raised = true;
+  }
+  const int tiles = ((t.g.M + BM - 1) / BM) * (t.ncols / (EPI == GEPI_SWIGLU ? BN / 2 : BN));
+  JSG_LAUNCH(prof_kind, (tile_kernel<EPI, BM, BN, ST>), dim3(tiles * t.split), dim3(TILE_THREADS), lds, t);
+  return 0;
+}
+
+// The shapes, with what a block takes for one K tile and how many blocks share a CU.  us per K tile, fitted to launches of
+// 57 to 1500 rows over matrices of 2048 to 28672 columns and 2048 to 14336 rows.
+struct TileShape { int bm, bn; float us; int per_cu; const char *pin; };
+static const TileShape TILE_SHAPES[] = {
+  {64, 64, 0.20f, 2, "small"},      // not for w1|w3 (its tiles come in pairs)
+  {64, 128, 0.33f, 1, "small"},
+  {128, 64, 0.33f, 1, nullptr},     // not for w1|w3
+  {128, 128, 0.47f, 1, "tall"},
+  {256, 128, 0.85f, 1, "wide"},
+  {256, 256, 1.43f, 1, "db"},
+};
+constexpr int N_SHAPES = sizeof(TILE_SHAPES) / sizeof(TILE_SHAPES[0]);
+
+// Which shape and how many K parts: the least of an estimate of the launch's time (rounds of blocks over the CUs times
+// K tiles per block, a fixed 5 us for start and first tiles, for K parts 3 us and the last arriver's reading of all sums at
+// a CU's 64 bytes a clock).  Examples, us, this choice | the neighbours: 371 x 2048 x 8192 128x128 in 4 parts 29.5 | in 2 parts
+// 41, 64x64 36, 256x128 in 8 parts 52; 371 x 2048 x 2048 64x64 10.4 | 128x64 15.6, 64x64 in 2 parts 11.9; 700 x 28672 x 4096
+// 256x128 178 | 128x128 227; 4096 x 4096 x 4096 256x256 98 | 256x128 116.
+static void choose_tile(int epi, int M, int weight_rows, int K, size_t ws_limit, int *shape, int *split) {
+  const int cus = state().cu_count, nk = K / TILE_BK;
+  const char *pin = getenv("JSG_GEMM_TILE");                  // tests and measurements: "db", "wide", "tall" or "small", no K parts
+  float best = 0.0f;
+  *shape = -1;
+  for (int s = 0; s < N_SHAPES; s++) {
+    const TileShape &c = TILE_SHAPES[s];
+    if (weight_rows % c.bn || (epi == GEPI_SWIGLU && c.bn < 128)) continue;
+    const int tiles = ((M + c.bm - 1) / c.bm) * (weight_rows / c.bn);
+    for (int d = 1; d <= 16; d++) {
+      if (d > 1 && (pin || c.bm * c.bn == 65536 || nk / d < 4 || tiles > TILE_COUNTERS || tiles * d > 2 * cus || (size_t)tiles * d * c.bm * c.bn * 4 > ws_limit)) break;
+      const int blocks = tiles * d, rounds = (blocks + cus * c.per_cu - 1) / (cus * c.per_cu);
+      const float shared = c.per_cu > 1 && blocks > cus ? 1.7f : 1.0f;   // two blocks of a CU share its L1 and matrix cores
+      float us = 5.0f + rounds * shared * c.us * ((nk + d - 1) / d);
+      if (d > 1) us += 3.0f + (float)d * c.bm * c.bn * 4 / 120e3f;
+      if (pin && c.pin && !strcmp(pin, c.pin)) us = 0.0f;      // taken
+      if (*shape < 0 || us < best) { best = us; *shape = s; *split = d; }
+    }
+  }
+}
+
+template <int EPI> static int launch_shape(int s, const TileArgs &t, int prof_kind) {
+  switch (s) {
+    case 0: if constexpr (EPI != GEPI_SWIGLU) return launch_tile<EPI, 64, 64, 4>(t, prof_kind); else break;
+    case 1: return launch_tile<EPI, 64, 128, 4>(t, prof_kind);
+    case 2: if constexpr (EPI != GEPI_SWIGLU) return launch_tile<EPI, 128, 64, 4>(t, prof_kind); else break;
+    case 3: return launch_tile<EPI, 128, 128, 4>(t, prof_kind);
+    case 4: return launch_tile<EPI, 256, 128, 3>(t, prof_kind);
+    case 5: return launch_tile256<EPI>(t, prof_kind);
+  }
+  return fail("jsgrad_hip_gemm: no tile shape");
+}
+
+template <int EPI> static int gemm_tiled_epi(int kind, const GemmArgs &a, int prof_kind) {
+  constexpr int NMAT = EPI == GEPI_SWIGLU ? 2 : 1;            // weight rows per output column
+  TileArgs t = {};
+  t.g = a;
+  static int *counters = nullptr;
+  if (!counters) JSG_HIP(hipGetSymbolAddress((void **)&counters, HIP_SYMBOL(tile_counters)));
+  t.counters = counters;
+
+  // fp16 weights are read where they are; quantised ones are realised into a block of the pool, all columns at once, or,
+  // while a graph is being captured, into the library's own scratch memory, as many columns at a time as fit
+  int step = a.N;
+  PoolBlock realised;
+  void *scratch = nullptr;
+  size_t scratch_bytes = 0;
+  const size_t row = (size_t)a.K * 2;
+  if (kind != JSGRAD_W_F16) {
+    if (int rc = realised.get((size_t)a.N * NMAT * row)) return rc;
+    if (!realised.p) {
+      if (int rc = gemm_scratch(&scratch, &scratch_bytes)) return rc;
+      step = (int)(scratch_bytes / (NMAT * row)) / 128 * 128;
+      JSG_REQUIRE(step > 0, "jsgrad_hip_gemm: in_features %d is too long for quantised weights during a graph capture", a.K);
+    }
+  }
+  _Float16 *const out = (_Float16 *)(realised.p ? realised.p : scratch);
+  const bool in_pool = kind == JSGRAD_W_F16 ? !state().capturing : realised.p != nullptr;
+
+  for (int c0 = 0; c0 < a.N; c0 += step) {
+    const int nc = a.N - c0 < step ? a.N - c0 : step;
+    t.col0 = c0;
+    t.ncols = nc;
+    if (kind == JSGRAD_W_F16) {
+      t.b[0] = (const _Float16 *)a.w0; t.b[1] = (const _Float16 *)a.w1; t.b[2] = (const _Float16 *)a.w2;
+      t.b_end[0] = EPI == GEPI_ROPE_KV ? a.n0 : a.N;
+      t.b_end[1] = EPI == GEPI_ROPE_KV ? a.n0 + a.n1 : a.N;
+    } else {
+      t.b[0] = out;
+      t.b[1] = t.b[2] = out + (size_t)nc * a.K;
+      t.b_end[0] = t.b_end[1] = nc;
+      if constexpr (EPI == GEPI_SWIGLU) {
+        if (int rc = realise(kind, a.w0, a.s0, c0, nc, a.K, out, prof_kind)) return rc;
+        if (int rc = realise(kind, a.w1, a.s1, c0, nc, a.K, out + (size_t)nc * a.K, prof_kind)) return rc;
+      } else {
+        const void *w[3] = {a.w0, a.w1, a.w2};
+        const _Float16 *s[3] = {a.s0, a.s1, a.s2};
+        const int n[3] = {EPI == GEPI_ROPE_KV ? a.n0 : a.N, EPI == GEPI_ROPE_KV ? a.n1 : 0, EPI == GEPI_ROPE_KV ? a.n2 : 0};
+        for (int q = 0, base = 0; q < 3; base += n[q++]) {
+          const int lo = c0 > base ? c0 : base, hi = c0 + nc < base + n[q] ? c0 + nc : base + n[q];
+          if (lo < hi)
+            if (int rc = realise(kind, w[q], s[q], lo - base, hi - lo, a.K, out + (size_t)(lo - c0) * a.K, prof_kind)) return rc;
+        }
+      }
+    }
+    int shape, split;
+    choose_tile(EPI, a.M, nc * NMAT, a.K, in_pool ? (size_t)256 << 20 : 0, &shape, &split);
+    JSG_REQUIRE(shape >= 0, "jsgrad_hip_gemm: no tile shape for %d columns", nc);
+    t.split = split;
+    PoolBlock sums;
+    if (split > 1) {
+      const int bm = TILE_SHAPES[shape].bm, bn = TILE_SHAPES[shape].bn;
+      if (int rc = sums.get((size_t)((a.M + bm - 1) / bm) * (nc * NMAT / bn) * split * bm * bn * 4)) return rc;
+      t.ws = (float *)sums.p;
+    }
+    if (int rc = launch_shape<EPI>(shape, t, prof_kind)) return rc;
+  }
+  return 0;
+}
+
+int gemm_tiled(int epi, int kind, const GemmArgs &a, int prof_kind) {
+  if (epi == GEPI_STORE) return gemm_tiled_epi<GEPI_STORE>(kind, a, prof_kind);
+  if (epi == GEPI_ROPE_KV) return gemm_tiled_epi<GEPI_ROPE_KV>(kind, a, prof_kind);
+  return gemm_tiled_epi<GEPI_SWIGLU>(kind, a, prof_kind);
+}
+
+}  // namespace jsg

@@ -1,0 +1,67 @@
+"""The tiled several-row kernels where they can go wrong: edges of the row tiles, output widths that only some shapes
+divide, one K tile, K parts, and quantised weights realised piece by piece while a graph is captured.
+
+Tolerance: products and sums are those of the oracle's several-row Linear in another order (assert_close, an fp16 unit of the
+result or of the operands of the residual sum)."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import oracle as orc
+from denograd_amd import ffi
+from denograd_amd.ffi import check
+from denograd_amd.tensor import Tensor
+from tests.helpers import assert_close
+from tests.test_gpu_rows import KINDS, dev, make_weight, sp
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("kind", ["float16", "int8", "nf4"])
+@pytest.mark.parametrize("rows,out_f,in_f", [(33, 128, 64), (64, 640, 128), (65, 384, 8192), (129, 256, 4096), (257, 768, 1088), (520, 128, 2048)])
+def test_tiled_gemm_at_the_edges(hip, kind, rows, out_f, in_f):
+    rng = np.random.default_rng(rows)
+    w, s = make_weight(kind, out_f, in_f)
+    x = rng.standard_normal((rows, in_f)).astype(np.float16)
+    res = rng.standard_normal((rows, out_f)).astype(np.float16)
+    tw, ts = dev(w, s)
+    tx, tr = Tensor(x), Tensor(res)
+    lin = orc.linear(w, s, x, out_f, in_f, True)
+    ref = (res.astype(np.float32) + lin).astype(np.float16).astype(np.float32)
+    runs = []
+    for _ in range(3):
+        y = Tensor.full((rows + 1, out_f), 7.0, "float16")
+        check(hip.jsgrad_hip_gemm(KINDS[kind], tw.ptr, sp(ts), out_f, in_f, tx.ptr, rows, y.ptr, tr.ptr))
+        runs.append(y.numpy())
+    assert np.all(runs[0][rows] == 7.0)                                       # nothing behind the last row
+    assert all(np.array_equal(runs[0].view(np.uint16), r.view(np.uint16)) for r in runs)   # parts are added in K order, whoever is last
+    assert_close(runs[0][:rows].astype(np.float32), ref, True, f"{kind} {rows}x{out_f}x{in_f}", ulp_at=lin)
+
+
+@pytest.mark.parametrize("kind", ["float16", "int8", "nf4"])
+def test_tiled_gemm_captured_in_a_graph(hip, kind):
+    """A call that is captured cannot allocate: quantised weights are realised a few columns at a time in scratch memory.
+    K is long enough for several such pieces; every replay equals the oracle, with eager work in between."""
+    rows, out_f, in_f = 40, 512, 14336
+    rng = np.random.default_rng(5)
+    w, s = make_weight(kind, out_f, in_f)
+    x = rng.standard_normal((rows, in_f)).astype(np.float16)
+    tw, ts = dev(w, s)
+    tx, y, other = Tensor(x), Tensor.empty((rows, out_f), "float16"), Tensor.empty((rows, out_f), "float16")
+    ref = orc.linear(w, s, x, out_f, in_f, True)
+    check(hip.jsgrad_hip_gemm(KINDS[kind], tw.ptr, sp(ts), out_f, in_f, tx.ptr, rows, other.ptr, None))
+    graph = C.c_void_p()
+    check(hip.jsgrad_hip_graph_begin())
+    try:
+        status = hip.jsgrad_hip_gemm(KINDS[kind], tw.ptr, sp(ts), out_f, in_f, tx.ptr, rows, y.ptr, None)
+    finally:
+        check(hip.jsgrad_hip_graph_end(C.byref(graph)))
+    check(status)
+    for _ in range(4):
+        check(hip.jsgrad_hip_memset(y.ptr, 0, y.nbytes))
+        check(hip.jsgrad_hip_graph_launch(graph))
+        assert_close(y.numpy().astype(np.float32), ref, True, f"captured {kind}")
+        check(hip.jsgrad_hip_gemm(KINDS[kind], tw.ptr, sp(ts), out_f, in_f, tx.ptr, rows, other.ptr, None))
+        assert_close(other.numpy().astype(np.float32), ref, True, f"eager {kind}")
+    check(hip.jsgrad_hip_graph_destroy(graph))
