@@ -4,10 +4,10 @@
 // What the reference computes (/root/reference/jsgrad/tensor.ts:2593-2605 `dot`, :3800 `linear`; Int8Linear.call
 // /root/reference/jsgrad/models/llama3.ts:35; NF4Linear.call :91-97): with more than one input row the weight operand is
 // expanded over the rows, so a quantised weight is first realised in fp16, W = RN16(code * scale), and the products of
-// two fp16 values are then summed in float.  So it is here: `realise_kernel` writes that matrix once per call (int8 8B w1|w3:
-// 117 MB in, 235 MB out, ~70 us, where the product takes 5.4 ms at 32768 rows) and one fp16 kernel serves the three formats.
-// Dequantising inside the product was the alternative: it needs the weight tile to pass through registers, and that
-// kernel stopped at 1.05-1.1 PFLOP/s.
+// two fp16 values are then summed in float.  So it is here.  With many rows `realise_kernel` writes that matrix once per call
+// (int8 8B w1|w3: 117 MB in, 235 MB out, ~75 us, where the product takes 5.4 ms at 32768 rows) and the fp16 kernels serve the
+// three formats.  With some hundred rows or fewer the writing and reading of the realised matrix would be most of the
+// time; `qtile_kernel` keeps the codes in LDS and dequantises a fragment as it is read.
 //
 // Both operands are K-contiguous in memory (x rows, W rows), so an operand fragment of v_mfma_f32_16x16x32_f16 (8 K elements
 // of one row per lane) is one 16-byte LDS read.  The 16x16 instruction is used because the chip is power-limited under this
@@ -33,7 +33,8 @@ constexpr int TILE_THREADS = 512;
 // One launch of a tiled kernel: columns [col0, col0 + ncols) of the output.
 struct TileArgs {
   GemmArgs g;                          // output side: y, residual, rope, cache, M, N, K
-  const _Float16 *b[3];                // fp16 weight rows of those columns, up to three matrices on top of each other
+  const void *b[3];                    // weight rows of those columns (fp16, or codes), up to three matrices on top of each other
+  const _Float16 *s[3];                // codes: their scales
   int b_end[2];                        // ends of the first two (SWIGLU: b[0] is w1, b[1] is w3, row for row)
   int col0, ncols;
   int split;                           // K parts
@@ -56,6 +57,10 @@ __device__ __forceinline__ i4_t tile_rsrc(const void *p) {
 // wait state between writing it and the load that reads it.
 __device__ __forceinline__ void dma16(i4_t rs, uint32_t voff, uint32_t soff, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rs), "s"(soff) : "memory");
+}
+// the same with four bytes per lane
+__device__ __forceinline__ void dma4(i4_t rs, uint32_t voff, uint32_t soff, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rs), "s"(soff) : "memory");
 }
 template <int N> __device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 __device__ __forceinline__ void turn_barrier() {
@@ -90,15 +95,22 @@ template <int BM, int CW> __device__ __forceinline__ TileId tile_id(const TileAr
   return r;
 }
 
-// Where row r (a multiple of 8; eight rows never straddle two matrices) of the weight tile of BN rows lies.
-template <int EPI, int BN> __device__ __forceinline__ const _Float16 *weight_row(const TileArgs &t, int col, int r) {
-  if constexpr (EPI == GEPI_SWIGLU) return (r < BN / 2 ? t.b[0] : t.b[1]) + (size_t)(col + (r < BN / 2 ? r : r - BN / 2)) * t.g.K;
+// Where row r of a weight tile of BN rows lies: the matrix and its row.  Boundaries are multiples of 64, so the 8 or 16 rows of a
+// load, or of a fragment, never straddle two matrices.
+struct WeightRow { int mat, row; };
+template <int EPI, int BN> __device__ __forceinline__ WeightRow weight_row(const TileArgs &t, int col, int r) {
+  if constexpr (EPI == GEPI_SWIGLU) return r < BN / 2 ? WeightRow{0, col + r} : WeightRow{1, col + r - BN / 2};
   else {
     const int n = col + r;
-    if (n < t.b_end[0]) return t.b[0] + (size_t)n * t.g.K;
-    if (n < t.b_end[1]) return t.b[1] + (size_t)(n - t.b_end[0]) * t.g.K;
-    return t.b[2] + (size_t)(n - t.b_end[1]) * t.g.K;
+    if (n < t.b_end[0]) return {0, n};
+    if (n < t.b_end[1]) return {1, n - t.b_end[0]};
+    return {2, n - t.b_end[1]};
   }
+}
+template <typename T> __device__ __forceinline__ const T *pick(const T *const (&p)[3], int i) { return i == 0 ? p[0] : (i == 1 ? p[1] : p[2]); }
+template <int EPI, int BN> __device__ __forceinline__ const unsigned char *weight_ptr(const TileArgs &t, int col, int r, size_t row_bytes) {
+  const WeightRow w = weight_row<EPI, BN>(t, col, r);
+  return (const unsigned char *)pick(t.b, w.mat) + (size_t)w.row * row_bytes;
 }
 
 // ---- epilogue of one wavefront: R16 x C16 tiles of 16x16 outputs.  The weight fragment is the first MFMA operand, so a lane
@@ -180,6 +192,49 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs &a, _Float16 *ep, i
 // silu(w1 x) * (w3 x), each GEMM output and the product stored as fp16 (llama.ts:108-110)
 __device__ __forceinline__ float swiglu(float gate, float up) { return silu_act<_Float16>(rn16(gate)) * rn16(up); }
 
+// ---- K parts: every part leaves its sums in the workspace, the last of a tile's parts to arrive adds them in K order, so the
+// result does not depend on who is last.  False: this block was not the last.
+// Parts run on different XCDs: stores and loads go to the point all of them share (cache policy 16: device scope), and the
+// count goes up once the block's stores are acknowledged.  The part is in the vector offset: behind a 16-byte store with its
+// offset in a scalar register the compiler overwrites the first data register too early (sums came out with every fourth
+// value zero).
+template <int TM, int TN, int SUMS> __device__ __forceinline__ bool sum_parts(const TileArgs &t, const TileId &id, int wave, f4_t (&acc)[TM][TN]) {
+  __shared__ int last;
+  const __amdgpu_buffer_rsrc_t rw = wave_buffer(t.ws + (size_t)id.tile * t.split * SUMS, (uint32_t)t.split * SUMS * 4u);
+  const uint32_t o0 = ((uint32_t)wave * TM * TN * 64 + (threadIdx.x & 63)) * 16;
+#pragma unroll
+  for (int i = 0; i < TM; i++)
+#pragma unroll
+    for (int j = 0; j < TN; j++)
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4_t, acc[i][j]), rw, o0 + (uint32_t)id.part * SUMS * 4u + (i * TN + j) * 1024, 0, 16);
+  wait_loads<0>();
+  turn_barrier();
+  if (threadIdx.x == 0) {
+    const int old = __hip_atomic_fetch_add(&t.counters[id.tile], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    last = old == t.split - 1;
+    if (last) __hip_atomic_store(&t.counters[id.tile], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // for the next launch
+  }
+  __syncthreads();
+  if (!last) return false;
+#pragma unroll
+  for (int i = 0; i < TM; i++)
+#pragma unroll
+    for (int j = 0; j < TN; j++) acc[i][j] = __builtin_bit_cast(f4_t, __builtin_amdgcn_raw_buffer_load_b128(rw, o0 + (i * TN + j) * 1024, 0, 16));
+  for (int p = 1; p < t.split; p++) {
+    f4_t u[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+      for (int j = 0; j < TN; j++)
+        u[i][j] = __builtin_bit_cast(f4_t, __builtin_amdgcn_raw_buffer_load_b128(rw, o0 + (uint32_t)p * SUMS * 4u + (i * TN + j) * 1024, 0, 16));
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+      for (int j = 0; j < TN; j++) acc[i][j] += u[i][j];
+  }
+  return true;
+}
+
 // ---------------------------------------------------------------- 256 x 256
 //
 // Wavefront (g, wn) owns rows 128 g .. +127 and columns 64 wn .. +63 as four quadrants of 64 x 32; a phase of a K tile is one
@@ -217,7 +272,7 @@ template <int EPI> __global__ __launch_bounds__(TILE_THREADS, 2) void tile256_ke
       const int ar = (idx >> 3) * 128 + h * 64 + (idx & 7) * 8, br = (idx >> 2) * 64 + h * 32 + (idx & 3) * 8;
       va[h][i] = (uint32_t)min(ar + lr, a.M - 1 - m0) * row_bytes + piece;   // rows past the end are computed and never stored
       const int src = EPI == GEPI_SWIGLU ? h * 128 + (idx >> 2) * 32 + (idx & 3) * 8 : br;   // half 0: w1 rows, half 1: w3 rows
-      rb[h][i] = tile_rsrc(weight_row<EPI, 256>(t, id.col, src));
+      rb[h][i] = tile_rsrc(weight_ptr<EPI, 256>(t, id.col, src, row_bytes));
       la[h][i] = ar * 128;
       lb[h][i] = T256_OPERAND + br * 128;
     }
@@ -313,8 +368,6 @@ template <int EPI> __global__ __launch_bounds__(TILE_THREADS, 2) void tile256_ke
 // tiles would leave most of the chip idle.  What bounds it, from builds with parts of the loop left out (128 x 128, 64 K
 // tiles, us): nothing but barriers 3, matrix instructions 15, direct loads 18 (the 64 bytes a clock of a CU's L1), fragment
 // reads 21 (each group reads alone and waits), all of it 30.
-// K parts: a part leaves its float sums in the workspace and the last of a tile's parts to arrive adds them in K order, so
-// the result does not depend on who is last.
 template <int EPI, int BM, int BN, int ST> constexpr size_t tile_lds_bytes() { return (size_t)(BM + BN) * 128 * ST; }
 template <int EPI, int BM, int BN, int ST> __global__ __launch_bounds__(TILE_THREADS, 2) void tile_kernel(TileArgs t) {
   const GemmArgs &a = t.g;
@@ -337,7 +390,7 @@ template <int EPI, int BM, int BN, int ST> __global__ __launch_bounds__(TILE_THR
 #pragma unroll
   for (int i = 0; i < NA; i++) va[i] = (uint32_t)min(wave * 8 + i * 64 + lr, a.M - 1 - m0) * row_bytes + piece;
 #pragma unroll
-  for (int i = 0; i < NB; i++) rb[i] = tile_rsrc(weight_row<EPI, BN>(t, id.col, wave * 8 + i * 64));
+  for (int i = 0; i < NB; i++) rb[i] = tile_rsrc(weight_ptr<EPI, BN>(t, id.col, wave * 8 + i * 64, row_bytes));
   const uint32_t vb = (uint32_t)lr * row_bytes + piece;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)tile_lds + wave * 1024;
   const int nkt = a.K / TILE_BK, k0 = (int)((long long)id.part * nkt / t.split), nk = (int)((long long)(id.part + 1) * nkt / t.split) - k0;
@@ -398,45 +451,7 @@ template <int EPI, int BM, int BN, int ST> __global__ __launch_bounds__(TILE_THR
   wait_loads<0>();
   turn_barrier();
 
-  if (t.split > 1) {
-    // Parts run on different XCDs: stores and loads that go to the point all of them share (cache policy 16: device scope),
-    // and the count goes up once the block's stores are acknowledged.  The part is in the vector offset: behind a 16-byte store
-    // with its offset in a scalar register the compiler overwrites the first data register too early (sums came out
-    // with every fourth value zero).
-    __shared__ int last;
-    const __amdgpu_buffer_rsrc_t rw = wave_buffer(t.ws + (size_t)id.tile * t.split * BM * BN, (uint32_t)t.split * BM * BN * 4u);
-    const uint32_t o0 = ((uint32_t)wave * TM * TN * 64 + lane) * 16;
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-      for (int j = 0; j < TN; j++)
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4_t, acc[i][j]), rw, o0 + (uint32_t)id.part * BM * BN * 4u + (i * TN + j) * 1024, 0, 16);
-    wait_loads<0>();
-    turn_barrier();
-    if (tid == 0) {
-      const int old = __hip_atomic_fetch_add(&t.counters[id.tile], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      last = old == t.split - 1;
-      if (last) __hip_atomic_store(&t.counters[id.tile], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // for the next launch
-    }
-    __syncthreads();
-    if (!last) return;
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-      for (int j = 0; j < TN; j++) acc[i][j] = __builtin_bit_cast(f4_t, __builtin_amdgcn_raw_buffer_load_b128(rw, o0 + (i * TN + j) * 1024, 0, 16));
-    for (int p = 1; p < t.split; p++) {
-      f4_t u[TM][TN];
-#pragma unroll
-      for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++)
-          u[i][j] = __builtin_bit_cast(f4_t, __builtin_amdgcn_raw_buffer_load_b128(rw, o0 + (uint32_t)p * BM * BN * 4u + (i * TN + j) * 1024, 0, 16));
-#pragma unroll
-      for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++) acc[i][j] += u[i][j];
-    }
-  }
+  if (t.split > 1 && !sum_parts<TM, TN, BM * BN>(t, id, wave, acc)) return;
 
   constexpr int C16 = EPI == GEPI_SWIGLU ? TN / 2 : TN, RB = TM < 4 ? TM : 4;
   _Float16 *ep = (_Float16 *)tile_lds + wave * RB * 16 * (C16 * 16 + 8);
@@ -447,55 +462,215 @@ template <int EPI, int BM, int BN, int ST> __global__ __launch_bounds__(TILE_THR
   });
 }
 
+// ---------------------------------------------------------------- quantised weights, dequantised as they are read
+//
+// Four wavefronts side by side over a BM x BN tile, each with all BM rows of its BN / 4 columns, so that a weight is dequantised
+// once per block: RN16(code * scale) of the eight codes of a fragment, then BM / 16 matrix instructions that use it.  x tiles as
+// above; of the weights the codes go to LDS (a stage is 64 K elements of int8, 128 of nf4: 64 bytes of a row, four rows per 256
+// bytes, piece p of row r at position p ^ (r / 4 & 3)), for nf4 with the two block scales of every row behind them.
+// Fragments are read one step ahead of the matrix instructions; two or three blocks share a CU.
+// Against realising first (us, int8, that | this): 57 x 5120 x 3072 15.7 + 11.3 | 11.4, 57 x 16384 x 3072 42 + 22 | 18.7,
+// 371 x 16384 x 2048 27 + 34 | 40, 700 x 28672 x 4096 78 + 178 | 222, 1500 x 4096 x 4096 14 + 55 | 75.
+template <int KIND> struct QFmt {
+  static constexpr int KS = KIND == JSGRAD_W_I8 ? 64 : 128;   // K elements per stage: 64 bytes of codes per row
+  static constexpr int SCALES = KIND == JSGRAD_W_NF4 ? 16 : 0;   // LDS bytes of scales per weight row and stage (a load brings 16 rows four times)
+};
+constexpr int QT_THREADS = 256;
+template <int KIND, int BM, int BN> constexpr int qtile_stage() { return BM * QFmt<KIND>::KS * 2 + BN * (64 + QFmt<KIND>::SCALES); }
+template <int KIND, int EPI, int BM, int BN, int ST> __global__ __launch_bounds__(QT_THREADS, 2) void qtile_kernel(TileArgs t) {
+  const GemmArgs &a = t.g;
+  extern __shared__ __align__(16) unsigned char tile_lds[];
+  __shared__ uint32_t pairs[KIND == JSGRAD_W_NF4 ? 256 : 1];  // nf4: the two code values of a byte (element 2j is the high nibble, llama3.ts:92-94)
+  constexpr int KS = QFmt<KIND>::KS, KF = KS / 32, SLABS = KS / 64;
+  constexpr int TM = BM / 16, TN = BN / 64, NA = BM / 32 * SLABS, NB = BN / 64, NLD = NA + NB + (KIND == JSGRAD_W_NF4 ? TN : 0), BUF = qtile_stage<KIND, BM, BN>();
+  static_assert(EPI != GEPI_SWIGLU || TN == 2, "a wavefront holds the w1 and the w3 tile of the same columns");
+  constexpr int CW = EPI == GEPI_SWIGLU ? BN / 2 : BN;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, lq = lane >> 4;
+  const TileId id = tile_id<BM, CW>(t);
+  const int m0 = id.m0;
+  if constexpr (KIND == JSGRAD_W_NF4) pairs[tid] = nf4_code_bits(tid >> 4) | (nf4_code_bits(tid & 15) << 16);   // read after the barrier below
+
+  const uint32_t x_bytes = (uint32_t)a.K * 2, w_bytes = KIND == JSGRAD_W_I8 ? a.K : a.K / 2;
+  const i4_t ra = tile_rsrc(a.x + (size_t)m0 * a.K);
+  const uint32_t piece = (uint32_t)((lane & 7) ^ (lane >> 3)) * 16;
+  constexpr int NA1 = NA / SLABS;
+  uint32_t va[NA1];
+#pragma unroll
+  for (int i = 0; i < NA1; i++) va[i] = (uint32_t)min((wave * NA1 + i) * 8 + (lane >> 3), a.M - 1 - m0) * x_bytes + piece;
+  i4_t rb[NB];
+#pragma unroll
+  for (int i = 0; i < NB; i++) rb[i] = tile_rsrc(weight_ptr<EPI, BN>(t, id.col, (wave * NB + i) * 16, w_bytes));
+  const uint32_t vb = (uint32_t)(lane >> 2) * w_bytes + (uint32_t)((lane & 3) ^ (lane >> 4)) * 16;   // rows of a load start at a multiple of 16
+  // the tile's weight row of fragment row l16 of this wavefront's column tile j
+  auto frag_row = [&](int j) { return EPI == GEPI_SWIGLU ? j * (BN / 2) + wave * 16 : (wave * TN + j) * 16; };
+  i4_t rs[TN];                                                // scales.  nf4: one per block of 64, a dword has those of a stage
+  const uint32_t vs = (uint32_t)l16 * (a.K / 32);
+#pragma unroll
+  for (int j = 0; j < TN; j++) {
+    const WeightRow w = weight_row<EPI, BN>(t, id.col, frag_row(j));
+    rs[j] = tile_rsrc(pick(t.s, w.mat) + (size_t)w.row * (KIND == JSGRAD_W_I8 ? 1 : a.K / 64));
+  }
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)tile_lds;
+  const int nst = a.K / KS, k0 = (int)((long long)id.part * nst / t.split), nk = (int)((long long)(id.part + 1) * nst / t.split) - k0;
+  auto load = [&](int kt, int buf) {
+    const uint32_t k = (uint32_t)(k0 + min(kt, nk - 1)), base = lds0 + buf * BUF;
+#pragma unroll
+    for (int sl = 0; sl < SLABS; sl++)
+#pragma unroll
+      for (int i = 0; i < NA1; i++) dma16(ra, va[i], k * (KS * 2) + sl * 128, base + sl * BM * 128 + (wave * NA1 + i) * 1024);
+#pragma unroll
+    for (int i = 0; i < NB; i++) dma16(rb[i], vb, k * 64, base + BM * KS * 2 + (wave * NB + i) * 1024);
+    if constexpr (KIND == JSGRAD_W_NF4)
+#pragma unroll
+      for (int j = 0; j < TN; j++) dma4(rs[j], vs, k * 4, base + BM * KS * 2 + BN * 64 + (wave * TN + j) * 256);
+  };
+
+  f4_t acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; i++)
+#pragma unroll
+    for (int j = 0; j < TN; j++) acc[i][j] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  h8_t af[2][TM];
+  uint2 bq[2][TN];                                            // eight codes (nf4: in the first word)
+  h2_t bs[2][TN];                                             // nf4: the scales of the stage's two blocks
+  auto read = [&](int buf, int f) {
+    const unsigned char *pa = tile_lds + buf * BUF + (f / 2) * BM * 128 + l16 * 128, *pb = tile_lds + buf * BUF + BM * KS * 2;
+    const uint32_t sw = (uint32_t)(((f & 1) * 4 + lq) ^ (l16 & 7)) * 16;
+#pragma unroll
+    for (int i = 0; i < TM; i++) af[f & 1][i] = *(const h8_t *)(pa + i * 2048 + sw);
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+      const unsigned char *pr = pb + (frag_row(j) + l16) * 64;
+      if constexpr (KIND == JSGRAD_W_I8) bq[f & 1][j] = *(const uint2 *)(pr + (uint32_t)((f * 2 + (lq >> 1)) ^ (l16 >> 2)) * 16 + (lq & 1) * 8);
+      else {
+        bq[f & 1][j].x = *(const uint32_t *)(pr + (uint32_t)(f ^ (l16 >> 2)) * 16 + lq * 4);
+        bs[f & 1][j] = *(const h2_t *)(pb + BN * 64 + (wave * TN + j) * 256 + l16 * 4);
+      }
+    }
+  };
+  // int8: one scale per row.  They come through LDS as well, in front of everything: a load to a register would be waited for
+  // with all later loads, which the compiler does not count.
+  h2_t scale[TN];
+  if constexpr (KIND == JSGRAD_W_I8)
+#pragma unroll
+    for (int j = 0; j < TN; j++) dma4(rs[j], (uint32_t)(lane & 7) * 4, 0, lds0 + ST * BUF + (wave * TN + j) * 256);
+#pragma unroll
+  for (int i = 0; i < ST; i++) load(i, i);
+  wait_loads<(ST - 1) * NLD>();
+  turn_barrier_lds();
+  if constexpr (KIND == JSGRAD_W_I8)
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+      const _Float16 v = *(const _Float16 *)(tile_lds + ST * BUF + (wave * TN + j) * 256 + l16 * 2);
+      scale[j] = h2_t{v, v};
+    }
+  auto compute = [&](int f) {
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+      u4_t o;
+      if constexpr (KIND == JSGRAD_W_I8) {
+        uint32_t lo, hi;
+        i8x4_to_h2x2(bq[f & 1][j].x, lo, hi); o.x = pk_mul_h2(lo, scale[j]); o.y = pk_mul_h2(hi, scale[j]);
+        i8x4_to_h2x2(bq[f & 1][j].y, lo, hi); o.z = pk_mul_h2(lo, scale[j]); o.w = pk_mul_h2(hi, scale[j]);
+      } else {
+        const _Float16 s1 = f / 2 ? bs[f & 1][j].y : bs[f & 1][j].x;
+        const h2_t s = {s1, s1};
+        const uint32_t c = bq[f & 1][j].x;
+        o.x = pk_mul_h2(pairs[c & 0xffu], s);
+        o.y = pk_mul_h2(pairs[(c >> 8) & 0xffu], s);
+        o.z = pk_mul_h2(pairs[(c >> 16) & 0xffu], s);
+        o.w = pk_mul_h2(pairs[c >> 24], s);
+      }
+      const h8_t b = __builtin_bit_cast(h8_t, o);
+#pragma unroll
+      for (int i = 0; i < TM; i++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b, af[f & 1][i], acc[i][j], 0, 0, 0);
+    }
+  };
+
+  read(0, 0);
+  int buf = 0;
+  for (int kt = 0; kt < nk; kt++) {
+#pragma unroll
+    for (int f = 0; f < KF; f++) {
+      if (f < KF - 1) read(buf, f + 1);
+      else {
+        // every fragment of this stage is in registers: its buffer is refilled, the next stage has landed
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        wait_loads<(ST - 2) * NLD>();
+        turn_barrier();
+        load(kt + ST, buf);
+        buf = buf + 1 == ST ? 0 : buf + 1;
+        read(buf, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      compute(f);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  wait_loads<0>();
+  turn_barrier();
+  if (t.split > 1 && !sum_parts<TM, TN, BM * BN>(t, id, wave, acc)) return;
+
+  constexpr int C16 = EPI == GEPI_SWIGLU ? 1 : TN, RB = 4;
+  _Float16 *ep = (_Float16 *)tile_lds + wave * RB * 16 * (C16 * 16 + 8);
+  static_assert((size_t)4 * RB * 16 * (C16 * 16 + 8) * 2 <= (size_t)ST * BUF, "the turning pieces fit the stages' LDS");
+  tile_epilogue<EPI, TM, C16, RB>(a, ep, m0, t.col0 + id.col + wave * C16 * 16, [&](int i, int j, int c) {
+    if constexpr (EPI == GEPI_SWIGLU) return swiglu(acc[i][0][c], acc[i][1][c]);
+    else return acc[i][j][c];
+  });
+}
+
 // ---------------------------------------------------------------- quantised weights, realised in fp16
 //
-// Rows [row0, row0 + rows) of one matrix to out[rows][K].  A thread takes 16 bytes of codes and stores 32 (int8) or 64 (nf4)
-// bytes; bound by memory (4.5-5 TB/s of codes in and halves out).
+// Rows [row0, row0 + rows) of one matrix to out[rows][K].  A thread makes eight elements at a time, so a wavefront's store is 1 KiB
+// without gaps (nf4 with 64 bytes per thread: 3.0 TB/s of codes in and halves out), and has four such pieces in flight.
 template <int KIND> __global__ __launch_bounds__(256) void realise_kernel(const unsigned char *w, const _Float16 *scale, _Float16 *out, int row0, size_t pieces, int ppr) {
-  // nf4: one table entry per BYTE, the two code values of its nibbles as a packed pair (element 2j is the high nibble,
-  // llama3.ts:92-94)
   __shared__ uint32_t pairs[KIND == JSGRAD_W_NF4 ? 256 : 1];
   if constexpr (KIND == JSGRAD_W_NF4) {
     pairs[threadIdx.x] = nf4_code_bits(threadIdx.x >> 4) | (nf4_code_bits(threadIdx.x & 15) << 16);
     __syncthreads();
   }
+  constexpr int U = 4;
   const size_t first = (size_t)row0 * ppr;
-  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < pieces; i += (size_t)gridDim.x * 256) {
-    const u4_t q = ldg_stream16(w + (first + i) * 16);
-    const uint32_t wds[4] = {q.x, q.y, q.z, q.w};
-    if constexpr (KIND == JSGRAD_W_I8) {
-      const _Float16 s1 = scale[row0 + (int)(i / (unsigned)ppr)];
-      const h2_t s = {s1, s1};
-      u4_t o[2];
+  for (size_t i0 = (size_t)blockIdx.x * (256 * U) + threadIdx.x; i0 < pieces; i0 += (size_t)gridDim.x * (256 * U)) {
+    uint2 q[U];
+    _Float16 s1[U];
 #pragma unroll
-      for (int d = 0; d < 4; d++) {
+    for (int u = 0; u < U; u++) {
+      const size_t i = i0 + u * 256 < pieces ? i0 + u * 256 : pieces - 1;
+      if constexpr (KIND == JSGRAD_W_I8) {
+        q[u] = *(const uint2 *)(w + (first + i) * 8);
+        s1[u] = scale[row0 + (int)((uint32_t)i / (uint32_t)ppr)];
+      } else {
+        q[u].x = *(const uint32_t *)(w + (first + i) * 4);
+        s1[u] = scale[(first + i) >> 3];                      // a block of 64 is eight pieces
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const size_t i = i0 + u * 256;
+      if (i >= pieces) break;
+      const h2_t s = {s1[u], s1[u]};
+      u4_t o;
+      if constexpr (KIND == JSGRAD_W_I8) {
         uint32_t lo, hi;
-        i8x4_to_h2x2(wds[d], lo, hi);
-        o[d / 2][(d % 2) * 2] = pk_mul_h2(lo, s);
-        o[d / 2][(d % 2) * 2 + 1] = pk_mul_h2(hi, s);
-      }
-      u4_t *dst = (u4_t *)(out + i * 16);
-      dst[0] = o[0];
-      dst[1] = o[1];
-    } else {
-      const _Float16 s1 = scale[(first + i) >> 1];            // 32 codes: half a scale block
-      const h2_t s = {s1, s1};
-      u4_t *dst = (u4_t *)(out + i * 32);
+        i8x4_to_h2x2(q[u].x, lo, hi); o.x = pk_mul_h2(lo, s); o.y = pk_mul_h2(hi, s);
+        i8x4_to_h2x2(q[u].y, lo, hi); o.z = pk_mul_h2(lo, s); o.w = pk_mul_h2(hi, s);
+      } else {
 #pragma unroll
-      for (int d = 0; d < 4; d++) {
-        u4_t o;
-#pragma unroll
-        for (int b = 0; b < 4; b++) o[b] = pk_mul_h2(pairs[(wds[d] >> (8 * b)) & 0xffu], s);
-        dst[d] = o;
+        for (int b = 0; b < 4; b++) o[b] = pk_mul_h2(pairs[(q[u].x >> (8 * b)) & 0xffu], s);
       }
+      *(u4_t *)(out + i * 8) = o;
     }
   }
 }
 
 static int realise(int kind, const void *w, const _Float16 *scale, int row0, int rows, int K, _Float16 *out, int prof_kind) {
-  const int ppr = kind == JSGRAD_W_I8 ? K / 16 : K / 32;      // pieces per row
+  const int ppr = K / 8;                                      // pieces per row
   const size_t pieces = (size_t)rows * ppr;
-  const size_t want = (pieces + 255) / 256;
+  JSG_REQUIRE(pieces < (size_t)1 << 32, "jsgrad_hip_gemm: a matrix of %d x %d is too large", rows, K);
+  const size_t want = (pieces + 1023) / 1024;
   const int grid = (int)(want < (size_t)16 * state().cu_count ? want : (size_t)16 * state().cu_count);
   if (kind == JSGRAD_W_I8) JSG_LAUNCH(prof_kind, realise_kernel<JSGRAD_W_I8>, dim3(grid), dim3(256), 0, (const unsigned char *)w, scale, out, row0, pieces, ppr);
   else JSG_LAUNCH(prof_kind, realise_kernel<JSGRAD_W_NF4>, dim3(grid), dim3(256), 0, (const unsigned char *)w, scale, out, row0, pieces, ppr);
@@ -540,45 +715,69 @@ template <int EPI, int BM, int BN, int ST> static int launch_tile(const TileArgs
   return 0;
 }
 
-// The shapes, with what a block takes for one K tile and how many blocks share a CU.  us per K tile, fitted to launches of
-// 57 to 1500 rows over matrices of 2048 to 28672 columns and 2048 to 14336 rows.
-struct TileShape { int bm, bn; float us; int per_cu; const char *pin; };
+template <int KIND, int EPI, int BM, int BN, int ST> static int launch_qtile(const TileArgs &t, int prof_kind) {
+  constexpr int lds = qtile_stage<KIND, BM, BN>() * ST + (KIND == JSGRAD_W_I8 ? BN * 16 : 0);
+  static_assert(lds + 1100 <= 160 * 1024, "LDS of one compute unit");
+  static bool raised = false;
+  if (!raised) {
+    JSG_HIP(hipFuncSetAttribute((const void *)qtile_kernel<KIND, EPI, BM, BN, ST>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    raised = true;
+  }
+  const int tiles = ((t.g.M + BM - 1) / BM) * (t.ncols / (EPI == GEPI_SWIGLU ? BN / 2 : BN));
+  JSG_LAUNCH(prof_kind, (qtile_kernel<KIND, EPI, BM, BN, ST>), dim3(tiles * t.split), dim3(QT_THREADS), lds, t);
+  return 0;
+}
+
+// The shapes, with the K elements of a step, what a block takes for one, and how many blocks share a CU before they slow each
+// other down.  us per step, fitted to launches of 40 to 1500 rows over matrices of 2048 to 28672 columns and 2048 to 14336 rows.
+struct TileShape { int bm, bn, bk; float us; int per_cu; const char *pin; };
 static const TileShape TILE_SHAPES[] = {
-  {64, 64, 0.20f, 2, "small"},      // not for w1|w3 (its tiles come in pairs)
-  {64, 128, 0.33f, 1, "small"},
-  {128, 64, 0.33f, 1, nullptr},     // not for w1|w3
-  {128, 128, 0.47f, 1, "tall"},
-  {256, 128, 0.85f, 1, "wide"},
-  {256, 256, 1.43f, 1, "db"},
+  {64, 64, 64, 0.20f, 2, "small"},     // not for w1|w3 (its tiles come in pairs)
+  {64, 128, 64, 0.33f, 1, "small"},
+  {128, 64, 64, 0.33f, 1, nullptr},    // not for w1|w3
+  {128, 128, 64, 0.47f, 1, "tall"},
+  {256, 128, 64, 0.85f, 1, "wide"},
+  {256, 256, 64, 1.43f, 1, "db"},
 };
-constexpr int N_SHAPES = sizeof(TILE_SHAPES) / sizeof(TILE_SHAPES[0]);
+static const TileShape QTILE_SHAPES_I8[] = {{64, 64, 64, 0.28f, 1, nullptr}, {64, 128, 64, 0.44f, 1, nullptr}, {128, 128, 64, 0.58f, 1, nullptr}};
+static const TileShape QTILE_SHAPES_NF4[] = {{64, 64, 128, 0.60f, 1, nullptr}, {64, 128, 128, 0.95f, 1, nullptr}, {128, 128, 128, 1.50f, 1, nullptr}};
+constexpr int N_SHAPES = sizeof(TILE_SHAPES) / sizeof(TILE_SHAPES[0]), N_QSHAPES = sizeof(QTILE_SHAPES_I8) / sizeof(QTILE_SHAPES_I8[0]);
 
 // Which shape and how many K parts: the least of an estimate of the launch's time (rounds of blocks over the CUs times
-// K tiles per block, a fixed 5 us for start and first tiles, for K parts 3 us and the last arriver's reading of all sums at
+// steps per block, a fixed 5 us for start and first tiles, for K parts 3 us and the last arriver's reading of all sums at
 // a CU's 64 bytes a clock).  Examples, us, this choice | the neighbours: 371 x 2048 x 8192 128x128 in 4 parts 29.5 | in 2 parts
 // 41, 64x64 36, 256x128 in 8 parts 52; 371 x 2048 x 2048 64x64 10.4 | 128x64 15.6, 64x64 in 2 parts 11.9; 700 x 28672 x 4096
 // 256x128 178 | 128x128 227; 4096 x 4096 x 4096 256x256 98 | 256x128 116.
-static void choose_tile(int epi, int M, int weight_rows, int K, size_t ws_limit, int *shape, int *split) {
-  const int cus = state().cu_count, nk = K / TILE_BK;
-  const char *pin = getenv("JSG_GEMM_TILE");                  // tests and measurements: "db", "wide", "tall" or "small", no K parts
-  float best = 0.0f;
-  *shape = -1;
-  for (int s = 0; s < N_SHAPES; s++) {
-    const TileShape &c = TILE_SHAPES[s];
-    if (weight_rows % c.bn || (epi == GEPI_SWIGLU && c.bn < 128)) continue;
-    const int tiles = ((M + c.bm - 1) / c.bm) * (weight_rows / c.bn);
+struct Choice { float us; int shape, split; };
+static Choice choose_tile(const TileShape *shapes, int n_shapes, int epi, int M, int weight_rows, int K, size_t ws_limit, const char *pin) {
+  const int cus = state().cu_count;
+  Choice best = {0.0f, -1, 1};
+  for (int s = 0; s < n_shapes; s++) {
+    const TileShape &c = shapes[s];
+    if (weight_rows % c.bn || K % c.bk || (epi == GEPI_SWIGLU && c.bn < 128)) continue;
+    const int tiles = ((M + c.bm - 1) / c.bm) * (weight_rows / c.bn), nk = K / c.bk;
     for (int d = 1; d <= 16; d++) {
-      if (d > 1 && (pin || c.bm * c.bn == 65536 || nk / d < 4 || tiles > TILE_COUNTERS || tiles * d > 2 * cus || (size_t)tiles * d * c.bm * c.bn * 4 > ws_limit)) break;
+      if (d > 1 && (pin || c.bm * c.bn == 65536 || nk / d * c.bk < 256 || tiles > TILE_COUNTERS || tiles * d > 2 * cus || (size_t)tiles * d * c.bm * c.bn * 4 > ws_limit)) break;
       const int blocks = tiles * d, rounds = (blocks + cus * c.per_cu - 1) / (cus * c.per_cu);
       const float shared = c.per_cu > 1 && blocks > cus ? 1.7f : 1.0f;   // two blocks of a CU share its L1 and matrix cores
       float us = 5.0f + rounds * shared * c.us * ((nk + d - 1) / d);
       if (d > 1) us += 3.0f + (float)d * c.bm * c.bn * 4 / 120e3f;
       if (pin && c.pin && !strcmp(pin, c.pin)) us = 0.0f;      // taken
-      if (*shape < 0 || us < best) { best = us; *shape = s; *split = d; }
+      if (best.shape < 0 || us < best.us) best = {us, s, d};
     }
   }
+  return best;
 }
 
+template <int KIND, int EPI> static int launch_qshape(int s, const TileArgs &t, int prof_kind) {
+  constexpr bool I8 = KIND == JSGRAD_W_I8;
+  switch (s) {
+    case 0: if constexpr (EPI != GEPI_SWIGLU) return launch_qtile<KIND, EPI, 64, 64, I8 ? 4 : 3>(t, prof_kind); else break;
+    case 1: return launch_qtile<KIND, EPI, 64, 128, I8 ? 4 : 3>(t, prof_kind);
+    case 2: return launch_qtile<KIND, EPI, 128, 128, I8 ? 3 : 2>(t, prof_kind);
+  }
+  return fail("jsgrad_hip_gemm: no tile shape");
+}
 template <int EPI> static int launch_shape(int s, const TileArgs &t, int prof_kind) {
   switch (s) {
     case 0: if constexpr (EPI != GEPI_SWIGLU) return launch_tile<EPI, 64, 64, 4>(t, prof_kind); else break;
@@ -593,67 +792,78 @@ template <int EPI> static int launch_shape(int s, const TileArgs &t, int prof_ki
 
 template <int EPI> static int gemm_tiled_epi(int kind, const GemmArgs &a, int prof_kind) {
   constexpr int NMAT = EPI == GEPI_SWIGLU ? 2 : 1;            // weight rows per output column
+  const void *const w[3] = {a.w0, a.w1, a.w2};
+  const _Float16 *const sc[3] = {a.s0, a.s1, a.s2};
+  const int n[3] = {EPI == GEPI_ROPE_KV ? a.n0 : a.N, EPI == GEPI_ROPE_KV ? a.n1 : 0, EPI == GEPI_ROPE_KV ? a.n2 : 0};   // rows on top of each other
   TileArgs t = {};
   t.g = a;
   static int *counters = nullptr;
   if (!counters) JSG_HIP(hipGetSymbolAddress((void **)&counters, HIP_SYMBOL(tile_counters)));
   t.counters = counters;
+  t.ncols = a.N;
+  for (int q = 0; q < 3; q++) { t.b[q] = w[q]; t.s[q] = sc[q]; }
+  t.b_end[0] = n[0];
+  t.b_end[1] = n[0] + n[1];
 
-  // fp16 weights are read where they are; quantised ones are realised into a block of the pool, all columns at once, or,
-  // while a graph is being captured, into the library's own scratch memory, as many columns at a time as fit
-  int step = a.N;
-  PoolBlock realised;
-  void *scratch = nullptr;
-  size_t scratch_bytes = 0;
-  const size_t row = (size_t)a.K * 2;
-  if (kind != JSGRAD_W_F16) {
-    if (int rc = realised.get((size_t)a.N * NMAT * row)) return rc;
-    if (!realised.p) {
-      if (int rc = gemm_scratch(&scratch, &scratch_bytes)) return rc;
-      step = (int)(scratch_bytes / (NMAT * row)) / 128 * 128;
-      JSG_REQUIRE(step > 0, "jsgrad_hip_gemm: in_features %d is too long for quantised weights during a graph capture", a.K);
+  const char *pin = getenv("JSG_GEMM_TILE");                  // tests and measurements: "db", "wide", "tall" or "small" of the fp16 shapes, no K parts
+  const size_t ws_limit = state().capturing ? 0 : (size_t)256 << 20;
+  auto run = [&](const TileShape *shapes, const Choice &c, int nmat_cols, auto launch) -> int {
+    JSG_REQUIRE(c.shape >= 0, "jsgrad_hip_gemm: no tile shape for %d columns", t.ncols);
+    PoolBlock sums;
+    t.split = c.split;
+    if (c.split > 1) {
+      const int bm = shapes[c.shape].bm, bn = shapes[c.shape].bn;
+      if (int rc = sums.get((size_t)((a.M + bm - 1) / bm) * (nmat_cols / bn) * c.split * bm * bn * 4)) return rc;
+      t.ws = (float *)sums.p;
     }
-  }
-  _Float16 *const out = (_Float16 *)(realised.p ? realised.p : scratch);
-  const bool in_pool = kind == JSGRAD_W_F16 ? !state().capturing : realised.p != nullptr;
+    return launch(c.shape, t, prof_kind);
+  };
 
+  Choice f = choose_tile(TILE_SHAPES, N_SHAPES, EPI, a.M, a.N * NMAT, a.K, ws_limit, pin);
+  if (kind == JSGRAD_W_F16) return run(TILE_SHAPES, f, a.N * NMAT, launch_shape<EPI>);
+
+  // Quantised: dequantised as read, or realised first (memory at 4.5 TB/s, and 2 us a launch), whichever is estimated to be
+  // done first: on the 8B shapes the line lies near a thousand rows.  During a capture nothing can be allocated for the
+  // realised matrix, so the codes are read in place whenever a shape takes them.
+  const double elems = (double)a.N * NMAT * a.K;
+  const float realise_us = (float)(elems * (kind == JSGRAD_W_I8 ? 3.0 : 2.5) / 4.5e6) + 2.0f * (EPI == GEPI_STORE ? 1 : NMAT + 1);
+  const TileShape *qs = kind == JSGRAD_W_I8 ? QTILE_SHAPES_I8 : QTILE_SHAPES_NF4;
+  const Choice q = choose_tile(qs, N_QSHAPES, EPI, a.M, a.N * NMAT, a.K, ws_limit, nullptr);
+  if (!pin && q.shape >= 0 && (state().capturing || q.us < f.us + realise_us))
+    return kind == JSGRAD_W_I8 ? run(qs, q, a.N * NMAT, launch_qshape<JSGRAD_W_I8, EPI>) : run(qs, q, a.N * NMAT, launch_qshape<JSGRAD_W_NF4, EPI>);
+
+  // Realised into a block of the pool, all columns at once, or, during a capture, into the library's own scratch memory, as many
+  // columns at a time as fit.
+  int step = a.N;
+  PoolBlock block;
+  const size_t row = (size_t)a.K * 2;
+  if (int rc = block.get((size_t)a.N * NMAT * row)) return rc;
+  _Float16 *out = (_Float16 *)block.p;
+  if (!out) {
+    size_t bytes = 0;
+    if (int rc = gemm_scratch((void **)&out, &bytes)) return rc;
+    step = (int)(bytes / (NMAT * row)) / 128 * 128;
+    JSG_REQUIRE(step > 0, "jsgrad_hip_gemm: in_features %d is too long for these weights during a graph capture", a.K);
+  }
   for (int c0 = 0; c0 < a.N; c0 += step) {
     const int nc = a.N - c0 < step ? a.N - c0 : step;
     t.col0 = c0;
     t.ncols = nc;
-    if (kind == JSGRAD_W_F16) {
-      t.b[0] = (const _Float16 *)a.w0; t.b[1] = (const _Float16 *)a.w1; t.b[2] = (const _Float16 *)a.w2;
-      t.b_end[0] = EPI == GEPI_ROPE_KV ? a.n0 : a.N;
-      t.b_end[1] = EPI == GEPI_ROPE_KV ? a.n0 + a.n1 : a.N;
+    t.b[0] = out;
+    t.b[1] = t.b[2] = out + (size_t)nc * a.K;
+    t.b_end[0] = t.b_end[1] = nc;
+    if constexpr (EPI == GEPI_SWIGLU) {
+      for (int m = 0; m < 2; m++)
+        if (int rc = realise(kind, w[m], sc[m], c0, nc, a.K, out + (size_t)m * nc * a.K, prof_kind)) return rc;
     } else {
-      t.b[0] = out;
-      t.b[1] = t.b[2] = out + (size_t)nc * a.K;
-      t.b_end[0] = t.b_end[1] = nc;
-      if constexpr (EPI == GEPI_SWIGLU) {
-        if (int rc = realise(kind, a.w0, a.s0, c0, nc, a.K, out, prof_kind)) return rc;
-        if (int rc = realise(kind, a.w1, a.s1, c0, nc, a.K, out + (size_t)nc * a.K, prof_kind)) return rc;
-      } else {
-        const void *w[3] = {a.w0, a.w1, a.w2};
-        const _Float16 *s[3] = {a.s0, a.s1, a.s2};
-        const int n[3] = {EPI == GEPI_ROPE_KV ? a.n0 : a.N, EPI == GEPI_ROPE_KV ? a.n1 : 0, EPI == GEPI_ROPE_KV ? a.n2 : 0};
-        for (int q = 0, base = 0; q < 3; base += n[q++]) {
-          const int lo = c0 > base ? c0 : base, hi = c0 + nc < base + n[q] ? c0 + nc : base + n[q];
-          if (lo < hi)
-            if (int rc = realise(kind, w[q], s[q], lo - base, hi - lo, a.K, out + (size_t)(lo - c0) * a.K, prof_kind)) return rc;
-        }
+      for (int m = 0, base = 0; m < 3; base += n[m++]) {
+        const int lo = c0 > base ? c0 : base, hi = c0 + nc < base + n[m] ? c0 + nc : base + n[m];
+        if (lo < hi)
+          if (int rc = realise(kind, w[m], sc[m], lo - base, hi - lo, a.K, out + (size_t)(lo - c0) * a.K, prof_kind)) return rc;
       }
     }
-    int shape, split;
-    choose_tile(EPI, a.M, nc * NMAT, a.K, in_pool ? (size_t)256 << 20 : 0, &shape, &split);
-    JSG_REQUIRE(shape >= 0, "jsgrad_hip_gemm: no tile shape for %d columns", nc);
-    t.split = split;
-    PoolBlock sums;
-    if (split > 1) {
-      const int bm = TILE_SHAPES[shape].bm, bn = TILE_SHAPES[shape].bn;
-      if (int rc = sums.get((size_t)((a.M + bm - 1) / bm) * (nc * NMAT / bn) * split * bm * bn * 4)) return rc;
-      t.ws = (float *)sums.p;
-    }
-    if (int rc = launch_shape<EPI>(shape, t, prof_kind)) return rc;
+    if (nc != a.N) f = choose_tile(TILE_SHAPES, N_SHAPES, EPI, a.M, nc * NMAT, a.K, ws_limit, pin);
+    if (int rc = run(TILE_SHAPES, f, nc * NMAT, launch_shape<EPI>)) return rc;
   }
   return 0;
 }
