@@ -1,4 +1,4 @@
-// Arguments and entry points that the several-row kernels share (gemm.hip: few rows, gemm_tile.hip: more than that).
+// What the several-row kernels share: gemm.hip (few rows), gemm_tile.hip (more than that), prefill.hip (causal attention).
 #pragma once
 #include "common.h"
 
@@ -36,6 +36,37 @@ __device__ __forceinline__ void i8x4_to_h2x2(uint32_t q, uint32_t &lo, uint32_t 
   lo = __builtin_bit_cast(uint32_t, a);
   hi = __builtin_bit_cast(uint32_t, b);
 }
+
+// ---- direct global-to-LDS loads
+typedef int i4_t __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ i4_t dma_rsrc(const void *p) {
+  const uint64_t v = (uint64_t)p;
+  i4_t r;
+  r.x = __builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+  r.y = __builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
+  r.z = -1;                            // callers keep their offsets in bounds
+  r.w = 0x00020000;
+  return r;
+}
+// 64 lanes x 16 bytes from rs + voff(lane) + soff to LDS bytes [lds, lds + 1024) in lane order.  M0 holds the LDS address; one
+// wait state between writing it and the load that reads it.
+__device__ __forceinline__ void dma16(i4_t rs, uint32_t voff, uint32_t soff, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rs), "s"(soff) : "memory");
+}
+// the same with four bytes per lane
+__device__ __forceinline__ void dma4(i4_t rs, uint32_t voff, uint32_t soff, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rs), "s"(soff) : "memory");
+}
+
+// A block of the allocator's pool for the length of one call.  Handing it back right behind the launches is safe: one
+// in-order stream serves every launch, so whoever gets the block next writes it after these launches have read it.  The pool
+// is bounded and gives memory back (runtime.hip).  During a graph capture nothing can be allocated: p stays null.
+struct PoolBlock {
+  void *p = nullptr;
+  int get(size_t nbytes) { return state().capturing ? 0 : jsgrad_hip_malloc(nbytes, &p); }
+  ~PoolBlock() { if (p) jsgrad_hip_free(p); }
+};
 
 // gemm_tile.hip: the tiled kernels, any number of rows; epi: GEPI_*
 int gemm_tiled(int epi, int kind, const GemmArgs &a, int prof_kind);

@@ -42,26 +42,6 @@ struct TileArgs {
   int *counters;                       // split > 1: one per tile, zero, and zero again afterwards
 };
 
-typedef int i4_t __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ i4_t tile_rsrc(const void *p) {
-  const uint64_t v = (uint64_t)p;
-  i4_t r;
-  r.x = __builtin_amdgcn_readfirstlane((int)(uint32_t)v);
-  r.y = __builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
-  r.z = -1;                            // offsets are in bounds by construction (rows past M are clamped)
-  r.w = 0x00020000;
-  return r;
-}
-// 64 lanes x 16 bytes from rs + voff(lane) + soff to LDS bytes [lds, lds + 1024) in lane order.  M0 holds the LDS address; one
-// wait state between writing it and the load that reads it.
-__device__ __forceinline__ void dma16(i4_t rs, uint32_t voff, uint32_t soff, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rs), "s"(soff) : "memory");
-}
-// the same with four bytes per lane
-__device__ __forceinline__ void dma4(i4_t rs, uint32_t voff, uint32_t soff, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rs), "s"(soff) : "memory");
-}
 template <int N> __device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 __device__ __forceinline__ void turn_barrier() {
   __builtin_amdgcn_sched_barrier(0);
@@ -259,7 +239,7 @@ template <int EPI> __global__ __launch_bounds__(TILE_THREADS, 2) void tile256_ke
   // Loads: half h of an operand is 128 rows = 16 loads of eight rows, two per wavefront.  The tile's rows are ordered by
   // who reads them: LDS row = 128 g + 64 h + .. for x, 64 wn + 32 h + .. for the weights.
   const uint32_t row_bytes = (uint32_t)a.K * 2;
-  const i4_t ra = tile_rsrc(a.x + (size_t)m0 * a.K);
+  const i4_t ra = dma_rsrc(a.x + (size_t)m0 * a.K);
   const int lr = lane >> 3, lp = lane & 7;
   const uint32_t piece = (uint32_t)(lp ^ lr) * 16;            // rows of a load start at a multiple of 8
   uint32_t va[2][2], la[2][2], lb[2][2];
@@ -272,7 +252,7 @@ template <int EPI> __global__ __launch_bounds__(TILE_THREADS, 2) void tile256_ke
       const int ar = (idx >> 3) * 128 + h * 64 + (idx & 7) * 8, br = (idx >> 2) * 64 + h * 32 + (idx & 3) * 8;
       va[h][i] = (uint32_t)min(ar + lr, a.M - 1 - m0) * row_bytes + piece;   // rows past the end are computed and never stored
       const int src = EPI == GEPI_SWIGLU ? h * 128 + (idx >> 2) * 32 + (idx & 3) * 8 : br;   // half 0: w1 rows, half 1: w3 rows
-      rb[h][i] = tile_rsrc(weight_ptr<EPI, 256>(t, id.col, src, row_bytes));
+      rb[h][i] = dma_rsrc(weight_ptr<EPI, 256>(t, id.col, src, row_bytes));
       la[h][i] = ar * 128;
       lb[h][i] = T256_OPERAND + br * 128;
     }
@@ -381,7 +361,7 @@ template <int EPI, int BM, int BN, int ST> __global__ __launch_bounds__(TILE_THR
   const int m0 = id.m0;
 
   const uint32_t row_bytes = (uint32_t)a.K * 2;
-  const i4_t ra = tile_rsrc(a.x + (size_t)m0 * a.K);
+  const i4_t ra = dma_rsrc(a.x + (size_t)m0 * a.K);
   const int lr = lane >> 3, lp = lane & 7;
   const uint32_t piece = (uint32_t)(lp ^ lr) * 16;
   constexpr int NA = BM / 64, NB = BN / 64;                   // a wavefront's loads per tile: eight rows each, 64 rows apart
@@ -390,7 +370,7 @@ template <int EPI, int BM, int BN, int ST> __global__ __launch_bounds__(TILE_THR
 #pragma unroll
   for (int i = 0; i < NA; i++) va[i] = (uint32_t)min(wave * 8 + i * 64 + lr, a.M - 1 - m0) * row_bytes + piece;
 #pragma unroll
-  for (int i = 0; i < NB; i++) rb[i] = tile_rsrc(weight_ptr<EPI, BN>(t, id.col, wave * 8 + i * 64, row_bytes));
+  for (int i = 0; i < NB; i++) rb[i] = dma_rsrc(weight_ptr<EPI, BN>(t, id.col, wave * 8 + i * 64, row_bytes));
   const uint32_t vb = (uint32_t)lr * row_bytes + piece;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)tile_lds + wave * 1024;
   const int nkt = a.K / TILE_BK, k0 = (int)((long long)id.part * nkt / t.split), nk = (int)((long long)(id.part + 1) * nkt / t.split) - k0;
@@ -491,7 +471,7 @@ template <int KIND, int EPI, int BM, int BN, int ST> __global__ __launch_bounds_
   if constexpr (KIND == JSGRAD_W_NF4) pairs[tid] = nf4_code_bits(tid >> 4) | (nf4_code_bits(tid & 15) << 16);   // read after the barrier below
 
   const uint32_t x_bytes = (uint32_t)a.K * 2, w_bytes = KIND == JSGRAD_W_I8 ? a.K : a.K / 2;
-  const i4_t ra = tile_rsrc(a.x + (size_t)m0 * a.K);
+  const i4_t ra = dma_rsrc(a.x + (size_t)m0 * a.K);
   const uint32_t piece = (uint32_t)((lane & 7) ^ (lane >> 3)) * 16;
   constexpr int NA1 = NA / SLABS;
   uint32_t va[NA1];
@@ -499,7 +479,7 @@ template <int KIND, int EPI, int BM, int BN, int ST> __global__ __launch_bounds_
   for (int i = 0; i < NA1; i++) va[i] = (uint32_t)min((wave * NA1 + i) * 8 + (lane >> 3), a.M - 1 - m0) * x_bytes + piece;
   i4_t rb[NB];
 #pragma unroll
-  for (int i = 0; i < NB; i++) rb[i] = tile_rsrc(weight_ptr<EPI, BN>(t, id.col, (wave * NB + i) * 16, w_bytes));
+  for (int i = 0; i < NB; i++) rb[i] = dma_rsrc(weight_ptr<EPI, BN>(t, id.col, (wave * NB + i) * 16, w_bytes));
   const uint32_t vb = (uint32_t)(lane >> 2) * w_bytes + (uint32_t)((lane & 3) ^ (lane >> 4)) * 16;   // rows of a load start at a multiple of 16
   // the tile's weight row of fragment row l16 of this wavefront's column tile j
   auto frag_row = [&](int j) { return EPI == GEPI_SWIGLU ? j * (BN / 2) + wave * 16 : (wave * TN + j) * 16; };
@@ -508,7 +488,7 @@ template <int KIND, int EPI, int BM, int BN, int ST> __global__ __launch_bounds_
 #pragma unroll
   for (int j = 0; j < TN; j++) {
     const WeightRow w = weight_row<EPI, BN>(t, id.col, frag_row(j));
-    rs[j] = tile_rsrc(pick(t.s, w.mat) + (size_t)w.row * (KIND == JSGRAD_W_I8 ? 1 : a.K / 64));
+    rs[j] = dma_rsrc(pick(t.s, w.mat) + (size_t)w.row * (KIND == JSGRAD_W_I8 ? 1 : a.K / 64));
   }
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)tile_lds;
   const int nst = a.K / KS, k0 = (int)((long long)id.part * nst / t.split), nk = (int)((long long)(id.part + 1) * nst / t.split) - k0;
@@ -681,15 +661,6 @@ static int realise(int kind, const void *w, const _Float16 *scale, int row0, int
 
 constexpr int TILE_COUNTERS = 4096;
 static __device__ int tile_counters[TILE_COUNTERS];
-
-// A block of the allocator's pool for the length of one call.  Handing it back right behind the launches is safe: one
-// in-order stream serves every launch, so whoever gets the block next writes it after these launches have read it.  The pool
-// is bounded and gives memory back (runtime.hip).  During a graph capture nothing can be allocated: p stays null.
-struct PoolBlock {
-  void *p = nullptr;
-  int get(size_t nbytes) { return state().capturing ? 0 : jsgrad_hip_malloc(nbytes, &p); }
-  ~PoolBlock() { if (p) jsgrad_hip_free(p); }
-};
 
 template <int EPI> static int launch_tile256(const TileArgs &t, int prof_kind) {
   constexpr int lds = 4 * T256_OPERAND;

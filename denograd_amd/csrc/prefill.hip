@@ -5,120 +5,125 @@
 // Reference semantics: Attention.call with a mask (/root/reference/jsgrad/models/llama.ts:61-97, mask :208 =
 // triu(start_pos + 1) of -inf), repeat_kv :34-39, scaled_dot_product_attention /root/reference/jsgrad/tensor.ts:3920-3934
 // (float32 scores and softmax, probabilities cast to fp16, float32 P.V sum, fp16 out).
-#include "common.h"
+#include "gemm.h"
 
 namespace jsg {
 
 typedef float f16_t __attribute__((ext_vector_type(16)));
-typedef _Float16 h4_t __attribute__((ext_vector_type(4)));
+typedef short s4_t __attribute__((ext_vector_type(4)));
 
 // ---------------------------------------------------------------- causal attention, S new positions
 //
-// Block = 4 wavefronts = 128 query rows of one head of one sequence; a wavefront owns 32 rows.  Keys are walked in tiles
-// of 64.  Scores are computed TRANSPOSED, S^T = K . Q^T (A operand = K rows from LDS, B operand = the lane's query row
-// held in registers), so that a lane holds 32 scores of ONE query row per tile: the online-softmax statistics are
-// lane-local (plus one exchange between the two lane halves), and the fp16 probabilities are already laid out as the
-// B operand of O^T = V^T . P^T.  The k-slot order of an MFMA operand is free as long as both operands agree; V^T
-// fragments are read from a transposed LDS tile in the order the score accumulators come out.
-// Two blocks per CU: at head_dim 128 the kernel wants a few registers more than half of a SIMD's file, and a second block
-// that computes while this one waits at its barriers is worth more than those registers.
+// Block = 4 wavefronts = 128 query rows of one kv head of one sequence: its n_rep query heads side by side, row = position *
+// n_rep + head, so that a wavefront's 32 rows are a few positions (little is computed above the diagonal) and a short prompt
+// still fills its rows.  Keys are walked in tiles of 64.  Scores are computed TRANSPOSED, S^T = K . Q^T (A operand = K rows from
+// LDS, B operand = the lane's query row held in registers), so that a lane holds 32 scores of ONE query row per tile: the
+// online-softmax statistics are lane-local (plus one exchange between the two lane halves), and the fp16 probabilities are
+// already laid out as the B operand of O^T = V^T . P^T.  The k-slot order of an MFMA operand is free as long as both
+// operands agree.
+// K and V tiles come by direct global-to-LDS loads into one of two buffers, rows as they are in the cache, the 16-byte pieces
+// of a row exchanged by row number so that fragment reads hit different banks.  V^T fragments come out of the row-major tile
+// by transposing LDS reads: within 16 lanes, lane i gets element i of four rows, row j being what lanes 4j .. 4j+3 address.
+// One barrier per tile: tile t + 1 is asked for behind the barrier of tile t, into the buffer of tile t - 1.
+// What bounds it: per tile a wavefront has 32 matrix instructions (1100 cycles) and ~1000 cycles of vector work (a
+// quarter-rate exponential per score); two blocks per CU, so that one wavefront of a SIMD computes under the other's softmax.
+// Measured (TFLOP/s of visible scores, head_dim 128, 32 heads, 8 kv heads): 16 x 2048 positions 678, 1 x 4096 824 (437 and 463 for
+// the kernel with tiles through registers, V transposed on the way into LDS and one query head per block).
+// A grid that does not fill the chip is split along the keys: every part leaves its running sums in a workspace and the last
+// of a wavefront's parts to arrive folds them in order.
 constexpr int PF_THREADS = 256, PF_QROWS = 128, PF_KEYS = 64;
+constexpr int PF_COUNTERS = 4096;
+static __device__ int pf_counters[PF_COUNTERS];
 
 struct PrefillAttnArgs {
   const _Float16 *q;                 // [B*S][H*HD]
   const _Float16 *cache_k, *cache_v; // [B][max_context][KV][HD]
   _Float16 *out;                     // [B*S][H*HD]
-  int S, start_pos, n_heads, n_kv_heads, max_context;
+  int S, start_pos, n_rep, n_kv_heads, max_context;
+  int tiles, pairs;                  // query tiles per (sequence, kv head); sequences x kv heads
+  int parts;                         // key parts
+  float *ws;                         // parts > 1: [block][part][wavefront][HD / 2 + 2 values][64 lanes]
+  int *counters;                     // parts > 1: one per (block, wavefront), zero, and zero again afterwards
   float scale_log2;                  // float(1/sqrt(HD)) * log2(e)
 };
 
 template <int HD> __global__ __launch_bounds__(PF_THREADS, 2) void attn_prefill_kernel(PrefillAttnArgs a) {
-  constexpr int KS = HD + 8;          // K tile row stride in halves
-  constexpr int VS = PF_KEYS + 8;     // V^T tile row stride in halves
-  constexpr int KC = HD / 8;          // 16-byte chunks per cache row
-  constexpr int K_LOADS = PF_KEYS * KC / PF_THREADS;
-  constexpr int V_PASSES = KC / 8;    // a pass covers 8 chunks x 32 key pairs
-  __shared__ __align__(16) _Float16 Ks[PF_KEYS * KS];
-  __shared__ __align__(16) _Float16 Vt[HD * VS];
+  constexpr int ROWB = HD * 2, PPR = HD / 8;                 // bytes and 16-byte pieces of a cache row of one head
+  constexpr int TILE = PF_KEYS * ROWB, BUF = 2 * TILE;       // K tile, then V tile
+  constexpr int LOADS = TILE / 1024 / 4;                     // a wavefront's loads per tile of K, and of V
+  constexpr int RPL = 64 / PPR;                              // rows per load
+  constexpr int NT = HD / 32;                                // 32-feature tiles of the output
+  __shared__ __align__(16) unsigned char lds[2 * BUF];
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, lg = lane >> 5;
-  // the block with the most keys (the last query tile) is scheduled first
-  const int qt = gridDim.x - 1 - blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-  const int g = h / (a.n_heads / a.n_kv_heads);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l32 = lane & 31, lg = lane >> 5;
+  // Blocks are dealt to the eight XCDs round-robin: ids are made contiguous per XCD, so that the query tiles of a (sequence,
+  // kv head) run on one XCD and share its K and V in that L2; within one the tiles with the most keys come first.
+  const int nblocks = a.tiles * a.pairs * a.parts;
+  int bid = blockIdx.x;
+  const int per = nblocks / 8;
+  if (bid < per * 8) bid = (bid & 7) * per + (bid >> 3);
+  const int part = bid % a.parts, blk = bid / a.parts;
+  const int pair = blk / a.tiles, qt = a.tiles - 1 - blk % a.tiles;
+  const int b = pair / a.n_kv_heads, g = pair % a.n_kv_heads;
+  const int rows = a.S * a.n_rep;
   const int q0 = qt * PF_QROWS, qw0 = q0 + wave * 32;
-  const int row_hi = min(q0 + PF_QROWS, a.S) - 1;            // last valid query row of the block
-  const int n_tiles = (a.start_pos + row_hi) / PF_KEYS + 1;
-  int qrow = qw0 + l32;
-  const bool q_valid = qrow < a.S;
-  if (!q_valid) qrow = a.S - 1;
-  const int qpos = a.start_pos + qrow;                       // keys <= qpos are visible
+  const int n_tiles = (a.start_pos + (min(q0 + PF_QROWS, rows) - 1) / a.n_rep) / PF_KEYS + 1;
+  const int t_lo = part * n_tiles / a.parts, t_hi = (part + 1) * n_tiles / a.parts;
+  // this wavefront's first and last position; rows past the end repeat the last one and are never stored
+  const int pos_lo = a.start_pos + min(qw0, rows - 1) / a.n_rep, pos_hi = a.start_pos + min(qw0 + 31, rows - 1) / a.n_rep;
+  const bool q_valid = qw0 + l32 < rows;
+  const int qrow = min(qw0 + l32, rows - 1), qs = qrow / a.n_rep, qpos = a.start_pos + qs;   // keys <= qpos are visible
+  const size_t q_off = ((size_t)b * a.S + qs) * (a.n_kv_heads * a.n_rep) * HD + (size_t)(g * a.n_rep + qrow % a.n_rep) * HD;
 
+  const uint32_t row_stride = (uint32_t)a.n_kv_heads * ROWB;
+  const size_t base = (size_t)b * a.max_context * row_stride + (size_t)g * ROWB;
+  const i4_t rk = dma_rsrc((const unsigned char *)a.cache_k + base), rv = dma_rsrc((const unsigned char *)a.cache_v + base);
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)lds + wave * LOADS * 1024;
+  const int lrow = lane / PPR, lp = lane % PPR, last_row = a.max_context - 1;
+  // where piece p of row r of a tile is kept: K by all pieces of a row, V by pairs of pieces (a transposing read takes 32 bytes of
+  // eight rows)
+  auto k_at = [](int r, int p) { return HD == 128 ? p ^ (r & 15) : p ^ (r & 7); };
+  auto v_at = [](int r, int p) { return HD == 128 ? p ^ ((r & 7) << 1) : p ^ (((r >> 1) & 3) << 1); };
+  auto issue = [&](int t, int buf) {
+    const uint32_t to = lds0 + buf * BUF;
+#pragma unroll
+    for (int i = 0; i < LOADS; i++) {
+      const int r = (wave * LOADS + i) * RPL + lrow;          // row of the tile this lane brings a piece of
+      const uint32_t key = (uint32_t)min(t * PF_KEYS + r, last_row) * row_stride;   // behind the cache's end: masked, any row will do
+      dma16(rk, key + k_at(r, lp) * 16, 0, to + i * 1024);
+      dma16(rv, key + v_at(r, lp) * 16, 0, to + TILE + i * 1024);
+    }
+  };
+
+  if (t_lo < t_hi) issue(t_lo, 0);
   // query row fragments: chunk c covers features [16c, 16c+16), the lane half picks 8 of them
   h8_t qf[HD / 16];
   {
-    const _Float16 *qp = a.q + ((size_t)b * a.S + qrow) * a.n_heads * HD + (size_t)h * HD + lg * 8;
+    const _Float16 *qp = a.q + q_off + lg * 8;
 #pragma unroll
     for (int c = 0; c < HD / 16; c++) qf[c] = *(const h8_t *)(qp + c * 16);
   }
+#pragma unroll
+  for (int c = 0; c < HD / 16; c++) asm volatile("" : "+v"(qf[c]));   // waited for here, in front of the loop
 
-  const size_t row_stride = (size_t)a.n_kv_heads * HD;
-  const _Float16 *kbase = a.cache_k + (size_t)b * a.max_context * row_stride + (size_t)g * HD;
-  const _Float16 *vbase = a.cache_v + (size_t)b * a.max_context * row_stride + (size_t)g * HD;
-  const int last_row = a.max_context - 1;
-
-  u4_t gk[K_LOADS], gv[V_PASSES][2];
-  auto issue = [&](int t) {
-    const int k0 = t * PF_KEYS;
+  f16_t o_acc[NT];
 #pragma unroll
-    for (int i = 0; i < K_LOADS; i++) {
-      const int idx = tid + i * PF_THREADS, key = min(k0 + idx / KC, last_row), c = idx % KC;
-      gk[i] = *(const u4_t *)(kbase + (size_t)key * row_stride + c * 8);
-    }
-    const int kp = tid & 31;
-#pragma unroll
-    for (int p = 0; p < V_PASSES; p++) {
-      const int c = (tid >> 5) + p * 8;
-      gv[p][0] = *(const u4_t *)(vbase + (size_t)min(k0 + 2 * kp, last_row) * row_stride + c * 8);
-      gv[p][1] = *(const u4_t *)(vbase + (size_t)min(k0 + 2 * kp + 1, last_row) * row_stride + c * 8);
-    }
-  };
-  auto commit = [&]() {
-#pragma unroll
-    for (int i = 0; i < K_LOADS; i++) {
-      const int idx = tid + i * PF_THREADS;
-      *(u4_t *)&Ks[(idx / KC) * KS + (idx % KC) * 8] = gk[i];
-    }
-    const int kp = tid & 31;
-#pragma unroll
-    for (int p = 0; p < V_PASSES; p++) {
-      const int c = (tid >> 5) + p * 8;
-      const uint32_t e[4] = {gv[p][0].x, gv[p][0].y, gv[p][0].z, gv[p][0].w}, o[4] = {gv[p][1].x, gv[p][1].y, gv[p][1].z, gv[p][1].w};
-#pragma unroll
-      for (int w = 0; w < 4; w++) {
-        // features 2w, 2w+1 of the chunk for the even key (e) and the odd key (o): pack (even key, odd key) per feature
-        const uint32_t f0 = __builtin_amdgcn_perm(o[w], e[w], 0x05040100u);   // {e.lo16, o.lo16}
-        const uint32_t f1 = __builtin_amdgcn_perm(o[w], e[w], 0x07060302u);   // {e.hi16, o.hi16}
-        *(uint32_t *)&Vt[(c * 8 + 2 * w) * VS + 2 * kp] = f0;
-        *(uint32_t *)&Vt[(c * 8 + 2 * w + 1) * VS + 2 * kp] = f1;
-      }
-    }
-  };
-
-  f16_t o_acc[HD / 32];
-#pragma unroll
-  for (int t = 0; t < HD / 32; t++)
+  for (int t = 0; t < NT; t++)
 #pragma unroll
     for (int r = 0; r < 16; r++) o_acc[t][r] = 0.0f;
-  float m_run = -INFINITY, l_run = 0.0f;
+  // the maximum starts finite: a part of the keys may hold none that a row sees, and -inf minus -inf is not a number
+  float m_run = -1e30f, l_run = 0.0f;
 
-  issue(0);
-  for (int t = 0; t < n_tiles; t++) {
-    __syncthreads();           // everyone is done with the previous tile
-    commit();
-    __syncthreads();
-    if (t + 1 < n_tiles) issue(t + 1);
+  // K fragment of key l32 (+ 32): chunk 2c + lg of its row; V: lane -> row (lane / 4 % 4) of its half's four keys, 8 bytes
+  const unsigned char *const kp = lds + l32 * ROWB;
+  const int vrow = 4 * lg + ((lane >> 2) & 3), vcol = ((lane >> 4) & 1) * 32 + (lane & 3) * 8;   // byte column inside 64 (32 features)
+
+  for (int t = t_lo, buf = 0; t < t_hi; t++, buf ^= 1) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    lds_barrier();                                            // tile t is there, everyone is done with tile t - 1
+    if (t + 1 < t_hi) issue(t + 1, buf ^ 1);
     const int k0 = t * PF_KEYS;
-    if (k0 > a.start_pos + min(qw0 + 31, a.S - 1)) continue;   // every key of the tile is masked for this wavefront (uniform)
+    if (k0 > pos_hi) continue;                                // every key of the tile is masked for this wavefront (uniform)
 
     // S^T tile: 64 keys x 32 query rows
     f16_t s[2];
@@ -128,14 +133,14 @@ template <int HD> __global__ __launch_bounds__(PF_THREADS, 2) void attn_prefill_
       for (int r = 0; r < 16; r++) s[tk][r] = 0.0f;
 #pragma unroll
       for (int c = 0; c < HD / 16; c++) {
-        const h8_t kf = *(const h8_t *)&Ks[(tk * 32 + l32) * KS + c * 16 + lg * 8];
+        const h8_t kf = *(const h8_t *)(kp + buf * BUF + tk * 32 * ROWB + k_at(l32, 2 * c + lg) * 16);
         s[tk] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, qf[c], s[tk], 0, 0, 0);
       }
     }
     // accumulator r of s[tk] is key k0 + tk*32 + 8*(r/4) + 4*lg + r%4 for query row l32.  Only a tile that reaches past
     // the first query row of the wavefront has masked keys (uniform test); the scale is positive, so the maximum is
     // taken over the raw scores and the scale folded into the exponent: exp2(s * scale - max * scale).
-    if (k0 + PF_KEYS - 1 > a.start_pos + qw0) {
+    if (k0 + PF_KEYS - 1 > pos_lo) {
 #pragma unroll
       for (int tk = 0; tk < 2; tk++)
 #pragma unroll
@@ -148,51 +153,108 @@ template <int HD> __global__ __launch_bounds__(PF_THREADS, 2) void attn_prefill_
 #pragma unroll
     for (int tk = 0; tk < 2; tk++)
 #pragma unroll
-      for (int r = 0; r < 16; r++) mx = fmaxf(mx, s[tk][r]);
-    mx = fmaxf(mx, __shfl_xor(mx, 32));
-    const float alpha = __builtin_amdgcn_exp2f((m_run - mx) * a.scale_log2);   // first visible tile: exp2(-inf) = 0
-    m_run = mx;
-    const float mxs = mx * a.scale_log2;
-    float psum = 0.0f;
+      for (int r = 0; r < 16; r += 2) mx = fmaxf(fmaxf(mx, s[tk][r]), s[tk][r + 1]);
+    mx = max_xor32(mx);
+    // The sums are rescaled only when some row's maximum has grown by more than a factor of 2^8 since they last were (uniform
+    // branch; a probability is then at most 256, its fp16 rounding relative as ever).  With a rescale whenever a maximum of
+    // the 32 rows moves two tiles in three have one: 64 multiplications.
+    if (__builtin_amdgcn_ballot_w64((mx - m_run) * a.scale_log2 > 8.0f)) {
+      const float alpha = __builtin_amdgcn_exp2f((m_run - mx) * a.scale_log2);   // first visible tile: 0
+      m_run = mx;
+      l_run *= alpha;
+#pragma unroll
+      for (int td = 0; td < NT; td++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) o_acc[td][r] *= alpha;
+    }
+    const float mxs = m_run * a.scale_log2;
+    float psum[2] = {0.0f, 0.0f};
     h8_t pf[2][2];
 #pragma unroll
     for (int tk = 0; tk < 2; tk++)
 #pragma unroll
       for (int r = 0; r < 16; r++) {
         const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[tk][r], a.scale_log2, -mxs));
-        psum += p;
+        psum[tk] += p;
         pf[tk][r / 8][r % 8] = (_Float16)p;
       }
-    l_run = l_run * alpha + psum;
-    if (__builtin_amdgcn_ballot_w64(alpha != 1.0f)) {   // the running maximum of some row moved (uniform branch)
-#pragma unroll
-      for (int td = 0; td < HD / 32; td++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) o_acc[td][r] *= alpha;
-    }
+    l_run += psum[0] + psum[1];
 
     // O^T += V^T . P^T : k-slot s' of lane half lg in step (tk, hs) is key tk*32 + hs*16 + 8*(s'/4) + 4*lg + s'%4
+    const unsigned char *const vt = lds + buf * BUF + TILE;
 #pragma unroll
     for (int tk = 0; tk < 2; tk++)
 #pragma unroll
-      for (int hs = 0; hs < 2; hs++) {
-        const int kb = tk * 32 + hs * 16 + 4 * lg;
+      for (int hs = 0; hs < 2; hs++)
 #pragma unroll
-        for (int td = 0; td < HD / 32; td++) {
-          const _Float16 *vp = &Vt[(td * 32 + l32) * VS + kb];
-          const h4_t v0 = *(const h4_t *)vp, v1 = *(const h4_t *)(vp + 8);
-          const h8_t vf = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+        for (int td = 0; td < NT; td++) {
+          s4_t v[2];
+#pragma unroll
+          for (int e = 0; e < 2; e++) {
+            const int r = tk * 32 + hs * 16 + 8 * e + vrow, c = td * 64 + vcol;
+            v[e] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4_t *)(vt + r * ROWB + v_at(r, c >> 4) * 16 + (c & 15)));
+          }
+          const h8_t vf = __builtin_bit_cast(h8_t, __builtin_shufflevector(v[0], v[1], 0, 1, 2, 3, 4, 5, 6, 7));
           o_acc[td] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, pf[tk][hs], o_acc[td], 0, 0, 0);
         }
-      }
   }
 
-  const float l_tot = l_run + __shfl_xor(l_run, 32);
-  const float inv = 1.0f / l_tot;
-  if (q_valid) {
-    _Float16 *op = a.out + ((size_t)b * a.S + qrow) * a.n_heads * HD + (size_t)h * HD;
+  if (a.parts > 1) {
+    // Sums cross compute units on different XCDs: device-scope stores and loads (cache policy 16), counted once they are
+    // acknowledged (the offset in the vector register, see sum_parts in gemm_tile.hip).
+    constexpr int VALS = (HD / 2 + 4) * 64;                   // floats of one wavefront: O^T, then (m, l)
+    const uint32_t slot = (uint32_t)VALS * 4;
+    const __amdgpu_buffer_rsrc_t rw = wave_buffer(a.ws + ((size_t)blk * a.parts * 4 + wave) * VALS, (a.parts - 1) * 4u * slot + slot);
+    const uint32_t mine = (uint32_t)part * 4 * slot + lane * 16;
 #pragma unroll
-    for (int td = 0; td < HD / 32; td++)
+    for (int td = 0; td < NT; td++)
+#pragma unroll
+      for (int r4 = 0; r4 < 4; r4++) {
+        const f4_t v = {o_acc[td][r4 * 4], o_acc[td][r4 * 4 + 1], o_acc[td][r4 * 4 + 2], o_acc[td][r4 * 4 + 3]};
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4_t, v), rw, mine + (td * 4 + r4) * 1024, 0, 16);
+      }
+    const f4_t ml = {m_run, l_run, 0.0f, 0.0f};
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4_t, ml), rw, mine + NT * 4 * 1024, 0, 16);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    int old = 0;
+    if (lane == 0) old = __hip_atomic_fetch_add(&a.counters[blk * 4 + wave], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    old = __builtin_amdgcn_readfirstlane(old);
+    if (old != a.parts - 1) return;
+    if (lane == 0) __hip_atomic_store(&a.counters[blk * 4 + wave], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // for the next launch
+    // two parts per round trip; past the last part the last one again, with weight zero
+    m_run = -1e30f;
+    l_run = 0.0f;
+#pragma unroll
+    for (int td = 0; td < NT; td++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) o_acc[td][r] = 0.0f;
+    for (int p0 = 0; p0 < a.parts; p0 += 2) {
+      f4_t w[2], v[2][NT * 4];
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        const uint32_t from = (uint32_t)min(p0 + u, a.parts - 1) * 4 * slot + lane * 16;
+        w[u] = __builtin_bit_cast(f4_t, __builtin_amdgcn_raw_buffer_load_b128(rw, from + NT * 4 * 1024, 0, 16));
+#pragma unroll
+        for (int i = 0; i < NT * 4; i++) v[u][i] = __builtin_bit_cast(f4_t, __builtin_amdgcn_raw_buffer_load_b128(rw, from + i * 1024, 0, 16));
+      }
+      const float m = fmaxf(m_run, fmaxf(w[0][0], w[1][0]));
+      const float f = __builtin_amdgcn_exp2f((m_run - m) * a.scale_log2);
+      const float f0 = __builtin_amdgcn_exp2f((w[0][0] - m) * a.scale_log2);   // a part without a visible key: 0
+      const float f1 = p0 + 1 < a.parts ? __builtin_amdgcn_exp2f((w[1][0] - m) * a.scale_log2) : 0.0f;
+      m_run = m;
+      l_run = l_run * f + (w[0][1] * f0 + w[1][1] * f1);
+#pragma unroll
+      for (int i = 0; i < NT * 4; i++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) o_acc[i / 4][(i % 4) * 4 + e] = o_acc[i / 4][(i % 4) * 4 + e] * f + (v[0][i][e] * f0 + v[1][i][e] * f1);
+    }
+  }
+
+  const float inv = 1.0f / add_xor32(l_run);
+  if (q_valid) {
+    _Float16 *op = a.out + q_off;
+#pragma unroll
+    for (int td = 0; td < NT; td++)
 #pragma unroll
       for (int r4 = 0; r4 < 4; r4++) {
         h4_t v;
@@ -304,11 +366,34 @@ int jsgrad_hip_attn_prefill(const void *q, const void *cache_k, const void *cach
   JSG_REQUIRE(head_dim == 64 || head_dim == 128, "jsgrad_hip_attn_prefill: head_dim %d (64 and 128 are built)", head_dim);
   JSG_REQUIRE(start_pos >= 0 && start_pos + seq_len <= max_context, "jsgrad_hip_attn_prefill: positions [%d, %d) outside the cache of %d", start_pos,
               start_pos + seq_len, max_context);
-  PrefillAttnArgs a;
+  PrefillAttnArgs a = {};
   a.q = (const _Float16 *)q; a.cache_k = (const _Float16 *)cache_k; a.cache_v = (const _Float16 *)cache_v; a.out = (_Float16 *)out;
-  a.S = seq_len; a.start_pos = start_pos; a.n_heads = n_heads; a.n_kv_heads = n_kv_heads; a.max_context = max_context;
+  a.S = seq_len; a.start_pos = start_pos; a.n_rep = n_heads / n_kv_heads; a.n_kv_heads = n_kv_heads; a.max_context = max_context;
+  JSG_REQUIRE((size_t)max_context * n_kv_heads * head_dim * 2 < (size_t)BUF_END, "jsgrad_hip_attn_prefill: a cache of %d positions is too long for 32-bit offsets", max_context);
+  JSG_REQUIRE((size_t)seq_len * a.n_rep < (size_t)1 << 30, "jsgrad_hip_attn_prefill: seq_len %d", seq_len);
   a.scale_log2 = (float)(1.0 / sqrt((double)head_dim)) * 1.4426950408889634f;
-  dim3 grid((seq_len + PF_QROWS - 1) / PF_QROWS, n_heads, batch), block(PF_THREADS);
+  a.tiles = (seq_len * a.n_rep + PF_QROWS - 1) / PF_QROWS;
+  a.pairs = batch * n_kv_heads;
+  a.parts = 1;
+  // Fewer blocks than half of what the chip holds (two per CU): the keys are cut into parts.  Not during a graph capture,
+  // where nothing can be allocated.
+  const size_t blocks = (size_t)a.tiles * a.pairs;
+  PoolBlock sums;
+  if (!state().capturing && blocks * 2 <= (size_t)2 * state().cu_count && blocks * 4 <= PF_COUNTERS) {
+    // A tile takes 0.7-0.9 us and folding a part about as long, one after the other: least at about sqrt(tiles) parts, and nothing
+    // to gain below eight.  (57 positions behind 1024, 24 heads of 128: 24.6 / 18.6 / 15.5 / 17.1 us in 1 / 2 / 4 / 8 parts;
+    // 371 positions of 32 heads of 64: 9.3 / 9.1 / 12.2 in 1 / 2 / 4.)
+    const int fill = (int)((size_t)2 * state().cu_count / blocks), mean_tiles = (start_pos + seq_len / 2) / PF_KEYS + 1;
+    if (mean_tiles >= 8) a.parts = fill < (int)sqrtf((float)mean_tiles) ? fill : (int)sqrtf((float)mean_tiles);
+  }
+  if (a.parts > 1) {
+    static int *counters = nullptr;
+    if (!counters) JSG_HIP(hipGetSymbolAddress((void **)&counters, HIP_SYMBOL(pf_counters)));
+    if (int rc = sums.get(blocks * a.parts * 4 * (head_dim / 2 + 4) * 64 * sizeof(float))) return rc;
+    a.ws = (float *)sums.p;
+    a.counters = counters;
+  }
+  const dim3 grid((unsigned)(blocks * a.parts)), block(PF_THREADS);
   if (head_dim == 64) JSG_LAUNCH(PROF_ATTN_PREFILL, attn_prefill_kernel<64>, grid, block, 0, a);
   else JSG_LAUNCH(PROF_ATTN_PREFILL, attn_prefill_kernel<128>, grid, block, 0, a);
   return 0;
