@@ -61,10 +61,11 @@ __device__ __forceinline__ void dma4(i4_t rs, uint32_t voff, uint32_t soff, uint
 
 // A block of the allocator's pool for the length of one call.  Handing it back right behind the launches is safe: one
 // in-order stream serves every launch, so whoever gets the block next writes it after these launches have read it.  The pool
-// is bounded and gives memory back (runtime.hip).  During a graph capture nothing can be allocated: p stays null.
+// is bounded and gives memory back (runtime.hip).  False, and p stays null, during a graph capture, where nothing can be
+// allocated, and on a device without that much memory left: the caller has a way that needs none.
 struct PoolBlock {
   void *p = nullptr;
-  int get(size_t nbytes) { return state().capturing ? 0 : jsgrad_hip_malloc(nbytes, &p); }
+  bool get(size_t nbytes) { return !state().capturing && jsgrad_hip_malloc(nbytes, &p) == 0; }
   ~PoolBlock() { if (p) jsgrad_hip_free(p); }
 };
 

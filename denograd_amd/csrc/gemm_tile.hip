@@ -778,44 +778,46 @@ template <int EPI> static int gemm_tiled_epi(int kind, const GemmArgs &a, int pr
 
   const char *pin = getenv("JSG_GEMM_TILE");                  // tests and measurements: "db", "wide", "tall" or "small" of the fp16 shapes, no K parts
   const size_t ws_limit = state().capturing ? 0 : (size_t)256 << 20;
-  auto run = [&](const TileShape *shapes, const Choice &c, int nmat_cols, auto launch) -> int {
-    JSG_REQUIRE(c.shape >= 0, "jsgrad_hip_gemm: no tile shape for %d columns", t.ncols);
+  auto run = [&](const TileShape *shapes, int n_shapes, Choice c, int nmat_cols, auto launch) -> int {
     PoolBlock sums;
-    t.split = c.split;
     if (c.split > 1) {
       const int bm = shapes[c.shape].bm, bn = shapes[c.shape].bn;
-      if (int rc = sums.get((size_t)((a.M + bm - 1) / bm) * (nmat_cols / bn) * c.split * bm * bn * 4)) return rc;
-      t.ws = (float *)sums.p;
+      if (!sums.get((size_t)((a.M + bm - 1) / bm) * (nmat_cols / bn) * c.split * bm * bn * 4)) c = choose_tile(shapes, n_shapes, EPI, a.M, nmat_cols, a.K, 0, pin);
     }
+    JSG_REQUIRE(c.shape >= 0, "jsgrad_hip_gemm: no tile shape for %d columns", t.ncols);
+    t.split = c.split;
+    t.ws = (float *)sums.p;
     return launch(c.shape, t, prof_kind);
   };
 
   Choice f = choose_tile(TILE_SHAPES, N_SHAPES, EPI, a.M, a.N * NMAT, a.K, ws_limit, pin);
-  if (kind == JSGRAD_W_F16) return run(TILE_SHAPES, f, a.N * NMAT, launch_shape<EPI>);
+  if (kind == JSGRAD_W_F16) return run(TILE_SHAPES, N_SHAPES, f, a.N * NMAT, launch_shape<EPI>);
 
   // Quantised: dequantised as read, or realised first (memory at 4.5 TB/s, and 2 us a launch), whichever is estimated to be
-  // done first: on the 8B shapes the line lies near a thousand rows.  During a capture nothing can be allocated for the
-  // realised matrix, so the codes are read in place whenever a shape takes them.
+  // done first: on the 8B shapes the line lies near a thousand rows.  Where there is no memory for the realised matrix (a
+  // capture, a full device) the codes are read in place whenever a shape takes them.
   const double elems = (double)a.N * NMAT * a.K;
   const float realise_us = (float)(elems * (kind == JSGRAD_W_I8 ? 3.0 : 2.5) / 4.5e6) + 2.0f * (EPI == GEPI_STORE ? 1 : NMAT + 1);
   const TileShape *qs = kind == JSGRAD_W_I8 ? QTILE_SHAPES_I8 : QTILE_SHAPES_NF4;
   const Choice q = choose_tile(qs, N_QSHAPES, EPI, a.M, a.N * NMAT, a.K, ws_limit, nullptr);
-  if (!pin && q.shape >= 0 && (state().capturing || q.us < f.us + realise_us))
-    return kind == JSGRAD_W_I8 ? run(qs, q, a.N * NMAT, launch_qshape<JSGRAD_W_I8, EPI>) : run(qs, q, a.N * NMAT, launch_qshape<JSGRAD_W_NF4, EPI>);
-
-  // Realised into a block of the pool, all columns at once, or, during a capture, into the library's own scratch memory, as many
-  // columns at a time as fit.
-  int step = a.N;
-  PoolBlock block;
   const size_t row = (size_t)a.K * 2;
-  if (int rc = block.get((size_t)a.N * NMAT * row)) return rc;
+  bool in_place = !pin && q.shape >= 0 && q.us < f.us + realise_us;
+  PoolBlock block;
+  if (!in_place) in_place = !block.get((size_t)a.N * NMAT * row) && !pin && q.shape >= 0;
+  if (in_place)
+    return kind == JSGRAD_W_I8 ? run(qs, N_QSHAPES, q, a.N * NMAT, launch_qshape<JSGRAD_W_I8, EPI>) : run(qs, N_QSHAPES, q, a.N * NMAT, launch_qshape<JSGRAD_W_NF4, EPI>);
+
+  // Realised into a block of the pool, all columns at once (as many as the realising kernel counts in 32 bits), or into the
+  // library's own scratch memory, as many columns at a time as fit.
+  size_t fit = ((size_t)1 << 32) / (a.K / 8) - 1;
   _Float16 *out = (_Float16 *)block.p;
   if (!out) {
     size_t bytes = 0;
     if (int rc = gemm_scratch((void **)&out, &bytes)) return rc;
-    step = (int)(bytes / (NMAT * row)) / 128 * 128;
-    JSG_REQUIRE(step > 0, "jsgrad_hip_gemm: in_features %d is too long for these weights during a graph capture", a.K);
+    fit = bytes / (NMAT * row);
   }
+  const int step = fit >= (size_t)a.N ? a.N : (int)(fit >= 128 ? fit / 128 * 128 : fit / 64 * 64);   // 64: the narrowest tile
+  JSG_REQUIRE(step > 0, "jsgrad_hip_gemm: in_features %d is too long for these weights without memory to realise them in", a.K);
   for (int c0 = 0; c0 < a.N; c0 += step) {
     const int nc = a.N - c0 < step ? a.N - c0 : step;
     t.col0 = c0;
@@ -834,7 +836,7 @@ template <int EPI> static int gemm_tiled_epi(int kind, const GemmArgs &a, int pr
       }
     }
     if (nc != a.N) f = choose_tile(TILE_SHAPES, N_SHAPES, EPI, a.M, nc * NMAT, a.K, ws_limit, pin);
-    if (int rc = run(TILE_SHAPES, f, nc * NMAT, launch_shape<EPI>)) return rc;
+    if (int rc = run(TILE_SHAPES, N_SHAPES, f, nc * NMAT, launch_shape<EPI>)) return rc;
   }
   return 0;
 }

@@ -77,7 +77,6 @@ template <int HD> __global__ __launch_bounds__(PF_THREADS, 2) void attn_prefill_
 
   const uint32_t row_stride = (uint32_t)a.n_kv_heads * ROWB;
   const size_t base = (size_t)b * a.max_context * row_stride + (size_t)g * ROWB;
-  const i4_t rk = dma_rsrc((const unsigned char *)a.cache_k + base), rv = dma_rsrc((const unsigned char *)a.cache_v + base);
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)lds + wave * LOADS * 1024;
   const int lrow = lane / PPR, lp = lane % PPR, last_row = a.max_context - 1;
   // where piece p of row r of a tile is kept: K by all pieces of a row, V by pairs of pieces (a transposing read takes 32 bytes of
@@ -86,10 +85,13 @@ template <int HD> __global__ __launch_bounds__(PF_THREADS, 2) void attn_prefill_
   auto v_at = [](int r, int p) { return HD == 128 ? p ^ ((r & 7) << 1) : p ^ (((r >> 1) & 3) << 1); };
   auto issue = [&](int t, int buf) {
     const uint32_t to = lds0 + buf * BUF;
+    // the tile's first row is in the descriptors: a sequence's cache may be longer than 32-bit offsets reach
+    const size_t tile = base + (size_t)t * PF_KEYS * row_stride;
+    const i4_t rk = dma_rsrc((const unsigned char *)a.cache_k + tile), rv = dma_rsrc((const unsigned char *)a.cache_v + tile);
 #pragma unroll
     for (int i = 0; i < LOADS; i++) {
       const int r = (wave * LOADS + i) * RPL + lrow;          // row of the tile this lane brings a piece of
-      const uint32_t key = (uint32_t)min(t * PF_KEYS + r, last_row) * row_stride;   // behind the cache's end: masked, any row will do
+      const uint32_t key = (uint32_t)min(r, last_row - t * PF_KEYS) * row_stride;   // behind the cache's end: masked, any row will do
       dma16(rk, key + k_at(r, lp) * 16, 0, to + i * 1024);
       dma16(rv, key + v_at(r, lp) * 16, 0, to + TILE + i * 1024);
     }
@@ -369,7 +371,6 @@ int jsgrad_hip_attn_prefill(const void *q, const void *cache_k, const void *cach
   PrefillAttnArgs a = {};
   a.q = (const _Float16 *)q; a.cache_k = (const _Float16 *)cache_k; a.cache_v = (const _Float16 *)cache_v; a.out = (_Float16 *)out;
   a.S = seq_len; a.start_pos = start_pos; a.n_rep = n_heads / n_kv_heads; a.n_kv_heads = n_kv_heads; a.max_context = max_context;
-  JSG_REQUIRE((size_t)max_context * n_kv_heads * head_dim * 2 < (size_t)BUF_END, "jsgrad_hip_attn_prefill: a cache of %d positions is too long for 32-bit offsets", max_context);
   JSG_REQUIRE((size_t)seq_len * a.n_rep < (size_t)1 << 30, "jsgrad_hip_attn_prefill: seq_len %d", seq_len);
   a.scale_log2 = (float)(1.0 / sqrt((double)head_dim)) * 1.4426950408889634f;
   a.tiles = (seq_len * a.n_rep + PF_QROWS - 1) / PF_QROWS;
@@ -386,10 +387,10 @@ int jsgrad_hip_attn_prefill(const void *q, const void *cache_k, const void *cach
     const int fill = (int)((size_t)2 * state().cu_count / blocks), mean_tiles = (start_pos + seq_len / 2) / PF_KEYS + 1;
     if (mean_tiles >= 8) a.parts = fill < (int)sqrtf((float)mean_tiles) ? fill : (int)sqrtf((float)mean_tiles);
   }
+  if (a.parts > 1 && !sums.get(blocks * a.parts * 4 * (head_dim / 2 + 4) * 64 * sizeof(float))) a.parts = 1;
   if (a.parts > 1) {
     static int *counters = nullptr;
     if (!counters) JSG_HIP(hipGetSymbolAddress((void **)&counters, HIP_SYMBOL(pf_counters)));
-    if (int rc = sums.get(blocks * a.parts * 4 * (head_dim / 2 + 4) * 64 * sizeof(float))) return rc;
     a.ws = (float *)sums.p;
     a.counters = counters;
   }
