@@ -54,6 +54,10 @@ __device__ __forceinline__ i4_t dma_rsrc(const void *p) {
 __device__ __forceinline__ void dma16(i4_t rs, uint32_t voff, uint32_t soff, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rs), "s"(soff) : "memory");
 }
+// the same for bytes that are read once
+__device__ __forceinline__ void dma16_stream(i4_t rs, uint32_t voff, uint32_t soff, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds" ::"s"(lds), "v"(voff), "s"(rs), "s"(soff) : "memory");
+}
 // the same with four bytes per lane
 __device__ __forceinline__ void dma4(i4_t rs, uint32_t voff, uint32_t soff, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rs), "s"(soff) : "memory");
@@ -69,6 +73,8 @@ struct PoolBlock {
   ~PoolBlock() { if (p) jsgrad_hip_free(p); }
 };
 
+// gemm_few.hip: at most 16 rows, weights streamed past x in registers; *taken false: not for this call, nothing launched
+int gemm_few(int epi, int kind, const GemmArgs &a, int prof_kind, bool *taken);
 // gemm_tile.hip: the tiled kernels, any number of rows; epi: GEPI_*
 int gemm_tiled(int epi, int kind, const GemmArgs &a, int prof_kind);
 // gemm.hip: 8 MiB of device memory that belong to the several-row kernels (one launch at a time: the stream orders them)

@@ -1,5 +1,6 @@
 // Several-row linear layers, few rows: y[M][N] = x[M][K] . W[N][K]^T for 1 to 32 rows of fp16 activations (batched decode), fp32
-// accumulate, fp16 out, and the entry points for any number of rows (more rows: gemm_tile.hip).
+// accumulate, fp16 out, and the entry points for any number of rows (more rows: gemm_tile.hip; fp16 and short int8 matrices with
+// at most 16 rows: gemm_few.hip).
 //
 // What the reference computes (/root/reference/jsgrad/tensor.ts:2593-2605 `dot`, :3800 `linear`; Int8Linear.call
 // /root/reference/jsgrad/models/llama3.ts:35; NF4Linear.call :91-97): with more than one input row the weight operand is
@@ -657,6 +658,7 @@ template <int KIND, int EPI> static int dispatch_skinny(const GemmArgs &a, int p
 
 template <int EPI> static int dispatch_gemm(int kind, const GemmArgs &a, int prof_kind) {
   bool taken = false;
+  { const int rc = gemm_few(EPI, kind, a, prof_kind, &taken); if (taken || rc) return rc; }
   if (kind == JSGRAD_W_F16) { const int rc = dispatch_skinny<JSGRAD_W_F16, EPI>(a, prof_kind, &taken); if (taken) return rc; }
   // int8, at most 16 rows: the LDS-streamed kernel, except for matrices so small that its K parts cost more than they bring
   // (wo of the 8B shape, 16.8 MB: 9.7 us against 8.5 us with the direct-operand kernel; wq|wk|wv, 25 MB: 12.3 against 13.5)

@@ -1,0 +1,249 @@
+// At most 16 rows of fp16 activations (batched decode), fp16 or int8 weights: y[M][N] = x[M][K] . W[N][K]^T, float accumulation, fp16
+// out; what the reference computes is in gemm.hip.
+//
+// The launch is bound by reading W once.  A block of eight wavefronts stays on its compute unit and walks tiles of 16 weight rows;
+// the wavefronts split K, and a wavefront's share of x (16 rows of K / 8 elements, at most 128 registers) is in operand layout in
+// its registers for the whole launch, so x costs one read per block and no LDS traffic, and no barrier stands between a
+// wavefront and its weights.  Those come by direct global-to-LDS loads into a ring that belongs to the wavefront (16 KiB:
+// 128 KiB of every compute unit's LDS are on their way), 256 to 512 contiguous bytes of a row at a time: asked for in operand
+// layout (64 bytes of each of 16 rows per load) the same bytes take a quarter longer.  Per tile the eight partial sums are
+// added through LDS in wavefront order.
+// Tiles that are left after whole rounds over the compute units are dealt as halves of eight rows where that is enough for
+// everybody (w1|w3 of 14336 rows: 896 tiles on 256 units are 3.5 rounds instead of 4).
+#include <stdlib.h>
+
+#include "gemm.h"
+
+namespace jsg {
+
+constexpr int FW_WAVES = 8, FW_THREADS = FW_WAVES * 64;
+
+template <int KIND, int EPI, int SB> struct FwShape {
+  static constexpr int SLOT = 16 * SB;                        // bytes of a step: 16 rows x SB bytes
+  static constexpr int LOADS = SB / 64;                       // direct loads of 1 KiB per step
+  static constexpr int SCALE = KIND == JSGRAD_W_I8 ? 256 : 0; // a slot of row scales (a 4-byte load of all lanes fills 256 bytes)
+  static constexpr int RED = (EPI == GEPI_SWIGLU ? 2 : 1) * FW_WAVES * 1024;   // the wavefronts' sums
+  static constexpr int FIT = (160 * 1024 - RED) / (FW_WAVES * (SLOT + SCALE));
+  static constexpr int NS = FIT < 4 ? FIT : 4;                // steps on their way
+  static constexpr int RING = NS * (SLOT + SCALE);            // per wavefront
+  static constexpr int LDS = FW_WAVES * RING + RED;
+  static_assert(NS >= 2, "one step arrives while another is used");
+};
+
+// K = 8 wavefronts x PARTS steps x SB bytes of a weight row
+template <int KIND, int EPI, int SB, int PARTS, bool LONG> __global__ __launch_bounds__(FW_THREADS, 2) void few_rows_kernel(GemmArgs a, int tiles) {
+  typedef FwShape<KIND, EPI, SB> S;
+  constexpr int NMAT = EPI == GEPI_SWIGLU ? 2 : 1, LOADS = S::LOADS, NS = S::NS;
+  constexpr int KB = KIND == JSGRAD_W_F16 ? 2 : 1;            // bytes of a weight
+  constexpr int NFR = SB / 64;                                // 16-byte fragment reads of a lane per step
+  constexpr int MPR = KIND == JSGRAD_W_F16 ? 1 : 2;           // matrix instructions per fragment read
+  constexpr int NF = PARTS * NFR * MPR;                       // x fragments
+  static_assert(NF <= 32, "x fits 128 registers");
+  extern __shared__ __align__(16) unsigned char few_lds[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, lq = lane >> 4;
+  const int G = gridDim.x;
+  const uint32_t row_bytes = (uint32_t)a.K * KB, k_first = (uint32_t)wave * PARTS * SB;
+
+  // Units of this block: whole tiles blockIdx.x, + G, ..; what is left after whole rounds as halves, if they go round
+  const int whole = tiles / G, left = tiles - whole * G;
+  const bool halves = 2 * left <= G;
+  const bool more = (int)blockIdx.x < (halves ? 2 * left : left);
+  const int units = whole + (more ? 1 : 0), n_steps = units * NMAT * PARTS;
+  auto is_half = [&](int u) { return halves && u == whole; };
+  auto first_row = [&](int u) { return u < whole || !halves ? ((int)blockIdx.x + u * G) * 16 : whole * G * 16 + (int)blockIdx.x * 8; };
+  auto place = [&](int n, int q, const void *&w, const _Float16 *&s, int &row) {   // a tile never straddles two matrices
+    if constexpr (EPI == GEPI_SWIGLU) { w = q ? a.w1 : a.w0; s = q ? a.s1 : a.s0; row = n; }
+    else if constexpr (EPI == GEPI_ROPE_KV) {
+      const int which = n < a.n0 ? 0 : (n < a.n0 + a.n1 ? 1 : 2);
+      w = which == 0 ? a.w0 : (which == 1 ? a.w1 : a.w2);
+      s = which == 0 ? a.s0 : (which == 1 ? a.s1 : a.s2);
+      row = which == 0 ? n : (which == 1 ? n - a.n0 : n - a.n0 - a.n1);
+    } else { w = a.w0; s = a.s0; row = n; }
+  };
+
+  // A step's bytes lie in its slot row by row; 16-byte piece p of row r is kept at position p ^ swizzle(r), so that the 16
+  // rows of a fragment read hit different banks.  Row 8 begins with load LOADS / 2: a half unit issues that many.
+  auto swizzle = [](int r) { return SB % 256 == 0 ? r & 15 : (r >> 1) & 7; };
+  uint32_t vo[LOADS];
+#pragma unroll
+  for (int j = 0; j < LOADS; j++) {
+    const int o = j * 1024 + lane * 16, r = o / SB, p = (o % SB) / 16;
+    vo[j] = (uint32_t)r * row_bytes + (uint32_t)(p ^ swizzle(r)) * 16;
+  }
+  unsigned char *const ring = few_lds + wave * S::RING;
+  const uint32_t ring0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)ring;
+  auto issue = [&](int s) {
+    const int u = s / (NMAT * PARTS), q = s / PARTS % NMAT, part = s % PARTS;
+    const void *w; const _Float16 *sc; int row;
+    place(first_row(u), q, w, sc, row);
+    const i4_t rw = dma_rsrc((const unsigned char *)w + (size_t)row * row_bytes);
+    const uint32_t to = ring0 + (uint32_t)(s % NS) * (S::SLOT + S::SCALE), so = k_first + part * SB;
+    const bool half = is_half(u);
+#pragma unroll
+    for (int j = 0; j < LOADS; j++)
+      if (j < LOADS / 2 || !half) dma16_stream(rw, vo[j], so, to + j * 1024);
+    if constexpr (KIND == JSGRAD_W_I8) dma4(dma_rsrc(sc + row), (uint32_t)(lane & (half ? 3 : 7)) * 4, 0, to + S::SLOT);
+  };
+  constexpr int FULL = LOADS + (KIND == JSGRAD_W_I8 ? 1 : 0), HALF = LOADS / 2 + (KIND == JSGRAD_W_I8 ? 1 : 0);
+  // wait until step s has landed: what was issued behind it may stay in flight
+  auto landed = [&](int s) {
+    int behind = 0;
+#pragma unroll
+    for (int i = 1; i < NS; i++)
+      if (s + i < n_steps) behind += is_half((s + i) / (NMAT * PARTS)) ? HALF : FULL;
+    if (behind >= (NS - 1) * FULL) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 1) * FULL) : "memory");
+    else if (NS > 2 && behind >= FULL) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(FULL) : "memory");
+    else if (behind >= HALF) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(HALF) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  };
+
+  // x first: fragment f of read i holds the K elements that a lane finds in its 16 bytes of the weight row
+  h8_t xf[NF];
+  {
+    const _Float16 *xr = a.x + (size_t)min(l16, a.M - 1) * a.K + k_first / KB + lq * (16 / KB);   // rows past the end: never stored
+#pragma unroll
+    for (int f = 0; f < NF; f++) xf[f] = *(const h8_t *)(xr + (f / MPR) * (64 / KB) + (f % MPR) * 8);
+  }
+#pragma unroll
+  for (int i = 0; i < NS; i++)
+    if (i < n_steps) issue(i);
+  // Waited for here, or the compiler, which does not count the direct loads, would wait for all of them at the first use of x in
+  // every turn of the loop below.  Where there is hardly a second turn the steps behind the first need not have landed yet.
+  if constexpr (LONG)
+#pragma unroll
+    for (int f = 0; f < NF; f++) asm volatile("" : "+v"(xf[f]));
+
+  float *const red = (float *)(few_lds + FW_WAVES * S::RING);  // [matrix][wavefront][16 x rows][16 weight rows]
+  int s = 0;
+  for (int u = 0; u < units; u++) {
+#pragma unroll
+    for (int q = 0; q < NMAT; q++) {
+      f4_t acc = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int part = 0; part < PARTS; part++, s++) {
+        landed(s);
+        const unsigned char *const from = ring + (s % NS) * (S::SLOT + S::SCALE);
+        u4_t raw[NFR];
+#pragma unroll
+        for (int i = 0; i < NFR; i++) raw[i] = *(const u4_t *)(from + l16 * SB + ((i * 4 + lq) ^ swizzle(l16)) * 16);
+        h2_t scale = {};
+        if constexpr (KIND == JSGRAD_W_I8) {
+          const _Float16 v = *(const _Float16 *)(from + S::SLOT + l16 * 2);
+          scale = h2_t{v, v};
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");    // the slot is in registers: it is filled again
+        if (s + NS < n_steps) issue(s + NS);
+#pragma unroll
+        for (int i = 0; i < NFR; i++) {
+          if constexpr (KIND == JSGRAD_W_F16) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8_t, raw[i]), xf[part * NFR + i], acc, 0, 0, 0);
+          else {
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+              u4_t o;
+              uint32_t lo, hi;
+              i8x4_to_h2x2(raw[i][2 * h], lo, hi); o.x = pk_mul_h2(lo, scale); o.y = pk_mul_h2(hi, scale);
+              i8x4_to_h2x2(raw[i][2 * h + 1], lo, hi); o.z = pk_mul_h2(lo, scale); o.w = pk_mul_h2(hi, scale);
+              acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8_t, o), xf[(part * NFR + i) * 2 + h], acc, 0, 0, 0);
+            }
+          }
+        }
+      }
+      // lane: x row l16, weight rows 4 lq .. + 3
+      *(f4_t *)&red[(q * FW_WAVES + wave) * 256 + l16 * 16 + lq * 4] = acc;
+    }
+    lds_barrier();
+    if (tid < 256) {                                          // whole wavefronts
+      const int m = tid >> 4, c = tid & 15, n = first_row(u) + c;
+      float tot[NMAT];
+#pragma unroll
+      for (int q = 0; q < NMAT; q++) {
+        tot[q] = red[q * FW_WAVES * 256 + tid];
+#pragma unroll
+        for (int w = 1; w < FW_WAVES; w++) tot[q] += red[(q * FW_WAVES + w) * 256 + tid];
+      }
+      const bool mine = m < a.M && (c < 8 || !is_half(u));
+      const float own = rn16(tot[0]);
+      if constexpr (EPI == GEPI_SWIGLU) {
+        if (mine) a.y[(size_t)m * a.N + n] = (_Float16)(silu_act<_Float16>(own) * rn16(tot[NMAT - 1]));
+      } else if constexpr (EPI == GEPI_STORE) {
+        if (mine) a.y[(size_t)m * a.N + n] = (_Float16)(a.residual ? (float)a.residual[(size_t)m * a.N + n] + own : own);
+      } else {
+        const float other = dpp_f<0xB1>(own);                 // the neighbouring column: the other half of the rotary pair
+        if (mine) {
+          const int which = n < a.n0 ? 0 : (n < a.n0 + a.n1 ? 1 : 2);
+          const int nl = which == 0 ? n : (which == 1 ? n - a.n0 : n - a.n0 - a.n1);
+          const int b = m / a.seq_len, pos = a.start_pos + m % a.seq_len;
+          float v = own;
+          if (which < 2) {
+            const h2_t cs = *(const h2_t *)(a.rope_table + ((size_t)pos * (a.head_dim / 2) + ((nl % a.head_dim) >> 1)) * 2);
+            const float cc = (float)cs.x, dd = (float)cs.y;
+            v = nl & 1 ? other * dd + own * cc : own * cc - other * dd;
+          }
+          if (which == 0) a.y[(size_t)m * a.n0 + nl] = (_Float16)v;
+          else (which == 1 ? a.cache_k : a.cache_v)[((size_t)b * a.max_context + pos) * a.n1 + nl] = (_Float16)v;
+        }
+      }
+    }
+    if (u + 1 < units) lds_barrier();                         // the sums have been read
+  }
+}
+
+template <int KIND, int EPI, int SB, int PARTS, bool LONG> static int launch_few_as(const GemmArgs &a, int tiles, int grid, int prof_kind) {
+  constexpr int lds = FwShape<KIND, EPI, SB>::LDS;
+  static bool raised = false;
+  if (!raised) {
+    JSG_HIP(hipFuncSetAttribute((const void *)few_rows_kernel<KIND, EPI, SB, PARTS, LONG>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    raised = true;
+  }
+  JSG_LAUNCH(prof_kind, (few_rows_kernel<KIND, EPI, SB, PARTS, LONG>), dim3(grid), dim3(FW_THREADS), lds, a, tiles);
+  return 0;
+}
+// Two weight tiles or more per block: LONG (us, with and without: fp16 16384 x 2048 16.3 | 17.1, 2048 x 8192 9.2 | 8.7)
+template <int KIND, int EPI, int SB, int PARTS> static int launch_few(const GemmArgs &a, int prof_kind) {
+  const int tiles = a.N / 16, cus = state().cu_count, grid = 2 * tiles < cus ? 2 * tiles : cus;
+  if (tiles * (EPI == GEPI_SWIGLU ? 2 : 1) >= 2 * grid) return launch_few_as<KIND, EPI, SB, PARTS, true>(a, tiles, grid, prof_kind);
+  return launch_few_as<KIND, EPI, SB, PARTS, false>(a, tiles, grid, prof_kind);
+}
+
+// A wavefront's share of a weight row, in steps of 512, 384 or 256 bytes: long steps ask for long stretches of a row, the number
+// of steps is bounded by the registers x takes.
+template <int KIND, int EPI> static int gemm_few_kind(const GemmArgs &a, int prof_kind, bool *taken) {
+  constexpr bool F16 = KIND == JSGRAD_W_F16;
+  *taken = true;
+  const int share = a.K % (FW_WAVES * 64) ? 0 : a.K * (F16 ? 2 : 1) / FW_WAVES;
+  switch (share) {
+    case 256: return launch_few<KIND, EPI, 256, 1>(a, prof_kind);
+    case 384: return launch_few<KIND, EPI, 384, 1>(a, prof_kind);
+    case 512: return launch_few<KIND, EPI, 512, 1>(a, prof_kind);
+    case 2 * 384: return launch_few<KIND, EPI, 384, 2>(a, prof_kind);
+    case 2 * 512: return launch_few<KIND, EPI, 512, 2>(a, prof_kind);
+    case 3 * 512: if constexpr (F16) return launch_few<KIND, EPI, 512, 3>(a, prof_kind); else break;
+    case 4 * 512: if constexpr (F16) return launch_few<KIND, EPI, 512, 4>(a, prof_kind); else break;
+  }
+  *taken = false;
+  return 0;
+}
+template <int EPI> static int gemm_few_epi(int kind, const GemmArgs &a, int prof_kind, bool *taken) {
+  if (kind == JSGRAD_W_F16) return gemm_few_kind<JSGRAD_W_F16, EPI>(a, prof_kind, taken);
+  if (kind == JSGRAD_W_I8) return gemm_few_kind<JSGRAD_W_I8, EPI>(a, prof_kind, taken);
+  return 0;
+}
+
+int gemm_few(int epi, int kind, const GemmArgs &a, int prof_kind, bool *taken) {
+  *taken = false;
+  if (a.M > 16 || a.N % 16 || ((uintptr_t)a.s0 | (uintptr_t)a.s1 | (uintptr_t)a.s2) & 3) return 0;
+  // int8: the codes of a tile are half the bytes behind the same x, and the kernels of gemm.hip read whole 512-byte stretches of many
+  // tiles.  us, theirs | this one: 4096 x 4096, 2 / 8 / 16 rows 8.1 / 8.3 / 8.6 | 7.5 / 8.2 / 9.5, 6144 x 4096 11.9 / 12.0 / 12.0 |
+  // 10.2 / 10.9 / 12.0, 3072 x 8192 12.2 / 12.3 / 12.2 | 8.6 / 10.1 / 12.7, 5120 x 3072 9.9 / 10.4 / 11.2 | 7.0 / 7.5 / 8.1,
+  // 16384 x 3072 13.5 / 13.7 / 13.7 | 13.5 / 14.1 / 15.0, 28672 x 4096 26.6 / 26.8 / 27.2 | 28.2 / 28.7 / 30.3.
+  // fp16 is the faster here at every size measured: 2048 x 2048 6.2 / 6.3 / 6.3 | 4.5 / 4.5 / 5.1, 2048 x 8192 14.1 / 14.9 / 15.9 |
+  // 8.8 / 9.5 / 12.4, 16384 x 2048 23.6 / 23.7 / 24.4 | 16.3 / 17.2 / 18.2, 128256 x 2048 147 / 153 / 162 | 88 / 92 / 94 (6.0 TB/s).
+  const size_t codes = (size_t)a.N * (epi == GEPI_SWIGLU ? 2 : 1) * a.K;
+  if (kind == JSGRAD_W_I8 && (codes > (size_t)36 << 20 || (a.M > 8 && a.K > 3072))) return 0;
+  if (getenv("JSG_GEMM_NO_SKINNY") || getenv("JSG_GEMM_SKINNY_TILES") || getenv("JSG_SG_TPW")) return 0;   // tests that want one of the other kernels
+  if (epi == GEPI_STORE) return gemm_few_epi<GEPI_STORE>(kind, a, prof_kind, taken);
+  if (epi == GEPI_ROPE_KV) return gemm_few_epi<GEPI_ROPE_KV>(kind, a, prof_kind, taken);
+  return gemm_few_epi<GEPI_SWIGLU>(kind, a, prof_kind, taken);
+}
+
+}  // namespace jsg

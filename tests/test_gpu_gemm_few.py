@@ -1,0 +1,43 @@
+"""The kernel for at most 16 rows that streams fp16 or int8 weights past x in registers: every share of a weight row that it is built
+for, and every way its tiles are dealt (only halves, whole tiles with idle blocks, whole rounds and halves behind them, whole
+rounds and a ragged one).
+
+Tolerance: products and sums are those of the oracle's several-row Linear in another order (assert_close)."""
+import numpy as np
+import pytest
+
+import oracle as orc
+from denograd_amd.ffi import check
+from denograd_amd.tensor import Tensor
+from tests.helpers import assert_close
+from tests.test_gpu_rows import KINDS, dev, make_weight, sp, test_gemm_ffn_gate as ffn_gate, test_gemm_qkv_rope_writes_queries_and_cache as qkv_rope
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("kind,in_f", [("float16", k) for k in (1024, 1536, 2048, 3072, 4096, 6144, 8192)] + [("int8", k) for k in (2048, 3072, 4096, 6144, 8192)])
+@pytest.mark.parametrize("rows,out_f", [(16, 128), (8, 128), (5, 2176), (2, 4224), (7, 4224), (16, 6400)])
+def test_few_rows_against_oracle(hip, kind, in_f, rows, out_f):
+    rng = np.random.default_rng(rows + in_f)
+    w, s = make_weight(kind, out_f, in_f)
+    x = rng.standard_normal((rows, in_f)).astype(np.float16)
+    res = rng.standard_normal((rows, out_f)).astype(np.float16)
+    tw, ts = dev(w, s)
+    tx, tr = Tensor(x), Tensor(res)
+    lin = orc.linear(w, s, x, out_f, in_f, True)
+    for residual, ref in ((None, lin), (tr.ptr, (res.astype(np.float32) + lin).astype(np.float16).astype(np.float32))):
+        y = Tensor.full((rows + 1, out_f), 7.0, "float16")
+        check(hip.jsgrad_hip_gemm(KINDS[kind], tw.ptr, sp(ts), out_f, in_f, tx.ptr, rows, y.ptr, residual))
+        got = y.numpy()
+        assert np.all(got[rows] == 7.0)
+        assert_close(got[:rows].astype(np.float32), ref, True, f"{kind} {rows}x{out_f}x{in_f}", ulp_at=lin if residual else None)
+
+
+@pytest.mark.parametrize("kind,dim,hidden", [("float16", 2048, 4224), ("float16", 1536, 128), ("int8", 3072, 4224), ("int8", 4096, 2176)])
+def test_few_rows_ffn_gate(hip, kind, dim, hidden):
+    ffn_gate(hip, kind, 9, dim, hidden)
+
+
+@pytest.mark.parametrize("kind,hd,B,dim", [("float16", 64, 16, 3072), ("int8", 128, 3, 4096), ("int8", 128, 16, 2048)])
+def test_few_rows_qkv_rope(hip, kind, hd, B, dim):
+    qkv_rope(hip, kind, hd, B, 1, dim)
