@@ -8,6 +8,10 @@ namespace jsg {
 template <typename T> __global__ void fill_kernel(T *p, size_t n, T v) {
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) p[i] = v;
 }
+// The words travel as kernel arguments: a copy from host memory would have to be waited for, once per step.
+__global__ void set_state_kernel(int32_t *state, int token, int position) {
+  if (threadIdx.x == 0) { state[0] = token; state[1] = position; }
+}
 static unsigned grid_for(size_t n, int block) {
   size_t g = (n + block - 1) / block;
   size_t cap = (size_t)state().cu_count * 16;
@@ -347,6 +351,15 @@ int jsgrad_hip_memset(void *dst, int byte, size_t nbytes) {
   } else {
     hipLaunchKernelGGL(fill_kernel<uint8_t>, dim3(grid_for(nbytes, 256)), dim3(256), 0, state().stream, (uint8_t *)dst, nbytes, b);
   }
+  JSG_LAUNCHED();
+  return 0;
+}
+
+int jsgrad_hip_set_state(int32_t *dst, int token, int position) {
+  JSG_READY();
+  JSG_REQUIRE(dst, "jsgrad_hip_set_state: null pointer");
+  JSG_REQUIRE(!state().capturing, "jsgrad_hip_set_state during graph capture");   // a replay would repeat these values
+  hipLaunchKernelGGL(set_state_kernel, dim3(1), dim3(64), 0, state().stream, dst, token, position);
   JSG_LAUNCHED();
   return 0;
 }

@@ -420,7 +420,7 @@ class Transformer:
             raise ValueError(f"start_pos {start_pos} outside the KV cache of {self.max_context} positions")
         if not (0 <= token < self.vocab_size):
             raise ValueError(f"token {token} outside the vocabulary of {self.vocab_size}")
-        self.state.lazydata.copyin(np.array([token, start_pos], np.int32))
+        check(ffi.load().jsgrad_hip_set_state(self.state.ptr, token, start_pos))
         if start_pos != self._pos and self._ctx is not None:
             self._ctx.clear_attn_row()      # the position jumps: see _Scratch.clear_attn_row
         self._pos = start_pos
@@ -497,7 +497,7 @@ class Transformer:
         check(lib.jsgrad_hip_embed_rows(_KIND[emb.weight.dtype], emb.weight.ptr, emb.scale.ptr if emb.scale is not None else None, tok_dev.ptr, n, rows.h.ptr,
                                         self.dim, self.vocab_size))
         # the attention of a one-position call reads the position from the device state word, like the one-row kernels
-        self.state.lazydata.ensure_allocated().copyin(np.array([0, start_pos + seqlen - 1], np.int32))
+        check(lib.jsgrad_hip_set_state(self.state.ptr, 0, start_pos + seqlen - 1))
         ctx.clear_attn_row()     # the position moves by more than one: see _Scratch.clear_attn_row
         h = rows.h
         for layer in self.layers:

@@ -60,6 +60,9 @@ int jsgrad_hip_mem_info(size_t *host_out_live_bytes, size_t *host_out_idle_bytes
 /* Allocator._copyin / _copyout (allocator.ts:42-43).  copyout returns after the data is in host memory. */
 int jsgrad_hip_copyin(void *dst, const void *host_src, size_t nbytes);
 int jsgrad_hip_copyout(void *host_dst, const void *src, size_t nbytes);
+/* The two words of a model's step state, {token, position}, which the reference keeps as a one-element tensor and a bound
+ * Variable (models/llama3.ts:300-305, models/llama.ts:214-220): written in stream order, without waiting for the stream. */
+int jsgrad_hip_set_state(int32_t *state, int token, int position);
 /* BufferCopy between two device buffers (engine/realize.ts:92-122, Allocator._transfer allocator.ts:46). */
 int jsgrad_hip_copy(void *dst, const void *src, size_t nbytes);
 /* Tensor.zeros(...).contiguous().realize() for the KV cache (models/llama.ts:79): byte fill. */
