@@ -799,7 +799,10 @@ template <int EPI> static int gemm_tiled_epi(int kind, const GemmArgs &a, int pr
   const double elems = (double)a.N * NMAT * a.K;
   const float realise_us = (float)(elems * (kind == JSGRAD_W_I8 ? 3.0 : 2.5) / 4.5e6) + 2.0f * (EPI == GEPI_STORE ? 1 : NMAT + 1);
   const TileShape *qs = kind == JSGRAD_W_I8 ? QTILE_SHAPES_I8 : QTILE_SHAPES_NF4;
-  const Choice q = choose_tile(qs, N_QSHAPES, EPI, a.M, a.N * NMAT, a.K, ws_limit, nullptr);
+  // qtile_kernel brings scales by direct loads of four bytes; a pointer between two of those (a slice) is read half by half when
+  // the matrix is realised
+  const bool dwords = (((uintptr_t)a.s0 | (uintptr_t)a.s1 | (uintptr_t)a.s2) & 3) == 0;
+  const Choice q = dwords ? choose_tile(qs, N_QSHAPES, EPI, a.M, a.N * NMAT, a.K, ws_limit, nullptr) : Choice{0.0f, -1, 1};
   const size_t row = (size_t)a.K * 2;
   bool in_place = !pin && q.shape >= 0 && q.us < f.us + realise_us;
   PoolBlock block;

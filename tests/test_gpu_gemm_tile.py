@@ -13,6 +13,7 @@ from denograd_amd import ffi
 from denograd_amd.ffi import check
 from denograd_amd.tensor import Tensor
 from tests.helpers import assert_close
+from tests import test_gpu_rows as rows_tests
 from tests.test_gpu_rows import KINDS, dev, make_weight, sp
 
 pytestmark = pytest.mark.gpu
@@ -66,3 +67,23 @@ def test_tiled_gemm_captured_in_a_graph(hip, kind, in_f):
         check(hip.jsgrad_hip_gemm(KINDS[kind], tw.ptr, sp(ts), out_f, in_f, tx.ptr, rows, other.ptr, None))
         assert_close(other.numpy().astype(np.float32), ref, True, f"eager {kind}")
     check(hip.jsgrad_hip_graph_destroy(graph))
+
+
+@pytest.mark.parametrize("kind", ["int8", "nf4"])
+def test_scales_between_two_dwords(hip, monkeypatch, kind):
+    """Scales are halves and may lie at any even address (a slice of a longer tensor), in every entry point, at the row counts
+    that would otherwise read codes and scales in place; also in a capture, where the matrix is realised in scratch memory."""
+    held = {}
+
+    def slice_of_scales(t):
+        if id(t) not in held:                         # made by the first, eager, call: a capture copies nothing
+            held[id(t)] = t, Tensor(np.concatenate([np.full(1, 7.0, np.float16), t.numpy().reshape(-1)]))
+        return held[id(t)][1].ptr + 2
+
+    monkeypatch.setattr(rows_tests, "sp", slice_of_scales)
+    for rows in (33, 57, 130):
+        rows_tests.test_gemm_matches_several_row_linear(hip, kind, rows, 384, 512)
+        rows_tests.test_gemm_ffn_gate(hip, kind, rows, 256, 384)
+    rows_tests.test_gemm_qkv_rope_writes_queries_and_cache(hip, kind, 64, 1, 57, 512)
+    monkeypatch.setitem(globals(), "sp", slice_of_scales)
+    test_tiled_gemm_captured_in_a_graph(hip, kind, 4096)
