@@ -32,3 +32,26 @@ def test_attn_prefill_in_key_parts(hip, hd, H, KV, B, S, start):
     assert np.all(runs[0][B * S] == 5.0)
     assert all(np.array_equal(runs[0].view(np.uint16), r.view(np.uint16)) for r in runs)   # parts are folded in order, whoever is last
     assert np.max(np.abs(runs[0][:B * S].astype(np.float64) - attention_ref(q, ck, cv, B, S, start, H, KV, hd))) < 4e-3
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+def test_the_largest_probability_of_a_row_is_not_rounded(hip, hd):
+    """Two keys that a row can see, a tile apart, the later one larger by a factor of 2^5 to 2^8: its probability, the largest, is
+    exact in fp16 whatever the maximum was before, so what is off is the rounding of the other (2^-5 times 2^-11 of the
+    difference of two values), float sums, and half an fp16 unit of the result."""
+    S, start, ctx, small, large = 40, 100, 160, 3, 70
+    rng = np.random.default_rng(hd)
+    delta = np.linspace(5.0, 7.9, S) * np.log(2.0)
+    q = np.zeros((S, hd), np.float16)
+    q[:, 0] = delta / 4 * np.sqrt(hd)
+    ck = np.zeros((1, ctx, 1, hd), np.float16)
+    ck[0, :, 0, 0] = -4000
+    ck[0, small, 0, 0], ck[0, large, 0, 0] = 0, 4
+    cv = rng.standard_normal((1, ctx, 1, hd)).astype(np.float16)
+    tq, tk, tv, to = Tensor(q), Tensor(ck), Tensor(cv), Tensor.empty((S, hd), "float16")
+    check(hip.jsgrad_hip_attn_prefill(tq.ptr, tk.ptr, tv.ptr, to.ptr, 1, S, start, 1, 1, hd, ctx))
+    w = np.exp(-4.0 * q[:, :1].astype(np.float64) / np.sqrt(hd))
+    v = cv[0, :, 0].astype(np.float64)
+    ref = (v[large] + w * v[small]) / (1 + w)
+    half_unit = np.spacing(np.abs(ref).astype(np.float16)).astype(np.float64) / 2
+    assert np.all(np.abs(to.numpy().astype(np.float64) - ref) <= 1.01 * half_unit + 2.0 ** -16 * np.abs(v[large] - v[small]) + 2.0 ** -20)
