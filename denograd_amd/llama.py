@@ -420,7 +420,7 @@ class Transformer:
             raise ValueError(f"start_pos {start_pos} outside the KV cache of {self.max_context} positions")
         if not (0 <= token < self.vocab_size):
             raise ValueError(f"token {token} outside the vocabulary of {self.vocab_size}")
-        check(ffi.load().jsgrad_hip_set_state(self.state.ptr, token, start_pos))
+        check(ffi.load().jsgrad_hip_set_state(self.state.ptr, int(token), int(start_pos)))
         if start_pos != self._pos and self._ctx is not None:
             self._ctx.clear_attn_row()      # the position jumps: see _Scratch.clear_attn_row
         self._pos = start_pos

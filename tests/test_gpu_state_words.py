@@ -2,8 +2,9 @@
 import numpy as np
 import pytest
 
-from denograd_amd import ffi
+from denograd_amd import ffi, synthetic
 from denograd_amd.ffi import check
+from denograd_amd.llama3 import Llama3
 from denograd_amd.tensor import Tensor
 
 pytestmark = pytest.mark.gpu
@@ -22,3 +23,11 @@ def test_state_words_in_stream_order(hip, n):
 def test_null_state_is_refused(hip):
     with pytest.raises(ffi.HipError, match="null pointer"):
         check(hip.jsgrad_hip_set_state(None, 0, 0))
+
+
+@pytest.mark.parametrize("number", [int, float, np.int64, np.float32, np.array])
+def test_any_number_sets_the_state_of_a_model(hip, number):
+    cfg = synthetic.config("tiny16")
+    model = Llama3.from_config(cfg).load_weights(synthetic.random_state_dict(cfg, seed=0), quantized=True).model
+    model.set_state(number(7), number(3))
+    np.testing.assert_array_equal(model.state.numpy().reshape(-1), [7, 3])
