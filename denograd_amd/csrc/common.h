@@ -19,6 +19,16 @@ struct State {
   bool capturing = false;
 };
 State &state();
+
+// The workspace of the several-row kernels for the length of one call (runtime.hip).  Handing it back right behind the launches is
+// safe: one in-order stream serves every launch, so the next call that has it writes it after these launches have read it.  False,
+// and p stays null, during a graph capture, where nothing can be allocated and the block could not be promised to the replays,
+// and on a device without that much memory left: the caller has a way that needs none.
+struct Workspace {
+  void *p = nullptr;
+  bool get(size_t nbytes);
+  ~Workspace();
+};
 int attn_static_init(int dev);   // attention.hip: resolves the built-in attention workspace's device address (jsgrad_hip_init)
 int fail(const char *fmt, ...);
 int fail_hip(hipError_t e, const char *what);

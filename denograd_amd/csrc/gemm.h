@@ -63,16 +63,6 @@ __device__ __forceinline__ void dma4(i4_t rs, uint32_t voff, uint32_t soff, uint
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rs), "s"(soff) : "memory");
 }
 
-// A block of the allocator's pool for the length of one call.  Handing it back right behind the launches is safe: one
-// in-order stream serves every launch, so whoever gets the block next writes it after these launches have read it.  The pool
-// is bounded and gives memory back (runtime.hip).  False, and p stays null, during a graph capture, where nothing can be
-// allocated, and on a device without that much memory left: the caller has a way that needs none.
-struct PoolBlock {
-  void *p = nullptr;
-  bool get(size_t nbytes) { return !state().capturing && jsgrad_hip_malloc(nbytes, &p) == 0; }
-  ~PoolBlock() { if (p) jsgrad_hip_free(p); }
-};
-
 // gemm_few.hip: at most 16 rows, weights streamed past x in registers; *taken false: not for this call, nothing launched
 int gemm_few(int epi, int kind, const GemmArgs &a, int prof_kind, bool *taken);
 // gemm_tile.hip: the tiled kernels, any number of rows; epi: GEPI_*

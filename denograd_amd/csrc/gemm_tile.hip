@@ -660,6 +660,8 @@ static int realise(int kind, const void *w, const _Float16 *scale, int row0, int
 // ---------------------------------------------------------------- host side
 
 constexpr int TILE_COUNTERS = 4096;
+// What one call asks of the workspace at most: K parts' sums, and a realised matrix (w1|w3 of the 8B shape 235 MB, its lm_head 1 GB)
+constexpr size_t SUMS_LIMIT = (size_t)256 << 20, REALISED_LIMIT = (size_t)2 << 30;
 static __device__ int tile_counters[TILE_COUNTERS];
 
 template <int EPI> static int launch_tile256(const TileArgs &t, int prof_kind) {
@@ -740,6 +742,12 @@ static Choice choose_tile(const TileShape *shapes, int n_shapes, int epi, int M,
   return best;
 }
 
+static size_t sums_bytes(const TileShape *shapes, const Choice &c, int M, int weight_rows) {
+  if (c.split < 2) return 0;
+  const int bm = shapes[c.shape].bm, bn = shapes[c.shape].bn;
+  return (size_t)((M + bm - 1) / bm) * (weight_rows / bn) * c.split * bm * bn * 4;
+}
+
 template <int KIND, int EPI> static int launch_qshape(int s, const TileArgs &t, int prof_kind) {
   constexpr bool I8 = KIND == JSGRAD_W_I8;
   switch (s) {
@@ -777,21 +785,23 @@ template <int EPI> static int gemm_tiled_epi(int kind, const GemmArgs &a, int pr
   t.b_end[1] = n[0] + n[1];
 
   const char *pin = getenv("JSG_GEMM_TILE");                  // tests and measurements: "db", "wide", "tall" or "small" of the fp16 shapes, no K parts
-  const size_t ws_limit = state().capturing ? 0 : (size_t)256 << 20;
-  auto run = [&](const TileShape *shapes, int n_shapes, Choice c, int nmat_cols, auto launch) -> int {
-    PoolBlock sums;
-    if (c.split > 1) {
-      const int bm = shapes[c.shape].bm, bn = shapes[c.shape].bn;
-      if (!sums.get((size_t)((a.M + bm - 1) / bm) * (nmat_cols / bn) * c.split * bm * bn * 4)) c = choose_tile(shapes, n_shapes, EPI, a.M, nmat_cols, a.K, 0, pin);
-    }
+  const size_t ws_limit = state().capturing ? 0 : SUMS_LIMIT;
+  auto run = [&](const Choice &c, float *ws, auto launch) -> int {
     JSG_REQUIRE(c.shape >= 0, "jsgrad_hip_gemm: no tile shape for %d columns", t.ncols);
     t.split = c.split;
-    t.ws = (float *)sums.p;
+    t.ws = ws;
     return launch(c.shape, t, prof_kind);
+  };
+  Workspace ws;
+  // all of the output at once, its sums (if it has K parts) in the workspace
+  auto run_whole = [&](const TileShape *shapes, int n_shapes, Choice c, const char *pinned, auto launch) -> int {
+    const size_t sums = sums_bytes(shapes, c, a.M, a.N * NMAT);
+    if (sums && !ws.get(sums)) c = choose_tile(shapes, n_shapes, EPI, a.M, a.N * NMAT, a.K, 0, pinned);
+    return run(c, (float *)ws.p, launch);
   };
 
   Choice f = choose_tile(TILE_SHAPES, N_SHAPES, EPI, a.M, a.N * NMAT, a.K, ws_limit, pin);
-  if (kind == JSGRAD_W_F16) return run(TILE_SHAPES, N_SHAPES, f, a.N * NMAT, launch_shape<EPI>);
+  if (kind == JSGRAD_W_F16) return run_whole(TILE_SHAPES, N_SHAPES, f, pin, launch_shape<EPI>);
 
   // Quantised: dequantised as read, or realised first (memory at 4.5 TB/s, and 2 us a launch), whichever is estimated to be
   // done first: on the 8B shapes the line lies near a thousand rows.  Where there is no memory for the realised matrix (a
@@ -805,22 +815,26 @@ template <int EPI> static int gemm_tiled_epi(int kind, const GemmArgs &a, int pr
   const Choice q = dwords ? choose_tile(qs, N_QSHAPES, EPI, a.M, a.N * NMAT, a.K, ws_limit, nullptr) : Choice{0.0f, -1, 1};
   const size_t row = (size_t)a.K * 2;
   bool in_place = !pin && q.shape >= 0 && q.us < f.us + realise_us;
-  PoolBlock block;
-  if (!in_place) in_place = !block.get((size_t)a.N * NMAT * row) && !pin && q.shape >= 0;
-  if (in_place)
-    return kind == JSGRAD_W_I8 ? run(qs, N_QSHAPES, q, a.N * NMAT, launch_qshape<JSGRAD_W_I8, EPI>) : run(qs, N_QSHAPES, q, a.N * NMAT, launch_qshape<JSGRAD_W_NF4, EPI>);
-
-  // Realised into a block of the pool, all columns at once (as many as the realising kernel counts in 32 bits), or into the
-  // library's own scratch memory, as many columns at a time as fit.
-  size_t fit = ((size_t)1 << 32) / (a.K / 8) - 1;
-  _Float16 *out = (_Float16 *)block.p;
-  if (!out) {
-    size_t bytes = 0;
-    if (int rc = gemm_scratch((void **)&out, &bytes)) return rc;
-    fit = bytes / (NMAT * row);
+  // Realised into the workspace, with the K parts' sums behind it: all columns at once, or as many at a time as REALISED_LIMIT holds
+  size_t bytes = (size_t)a.N * NMAT * row < REALISED_LIMIT ? (size_t)a.N * NMAT * row : REALISED_LIMIT, sums = 0;
+  if (!in_place) {
+    sums = sums_bytes(TILE_SHAPES, f, a.M, a.N * NMAT);
+    if (!ws.get(bytes + sums)) {
+      sums = 0;
+      in_place = !ws.get(bytes) && !pin && q.shape >= 0;
+    }
   }
+  if (in_place)
+    return kind == JSGRAD_W_I8 ? run_whole(qs, N_QSHAPES, q, nullptr, launch_qshape<JSGRAD_W_I8, EPI>) : run_whole(qs, N_QSHAPES, q, nullptr, launch_qshape<JSGRAD_W_NF4, EPI>);
+
+  // ... or, without memory, in the library's own scratch
+  _Float16 *out = (_Float16 *)ws.p;
+  if (!out)
+    if (int rc = gemm_scratch((void **)&out, &bytes)) return rc;
+  const size_t fit = bytes / (NMAT * row);
   const int step = fit >= (size_t)a.N ? a.N : (int)(fit >= 128 ? fit / 128 * 128 : fit / 64 * 64);   // 64: the narrowest tile
   JSG_REQUIRE(step > 0, "jsgrad_hip_gemm: in_features %d is too long for these weights without memory to realise them in", a.K);
+  float *const sums_at = sums ? (float *)((unsigned char *)out + bytes) : nullptr;
   for (int c0 = 0; c0 < a.N; c0 += step) {
     const int nc = a.N - c0 < step ? a.N - c0 : step;
     t.col0 = c0;
@@ -838,8 +852,8 @@ template <int EPI> static int gemm_tiled_epi(int kind, const GemmArgs &a, int pr
           if (int rc = realise(kind, w[m], sc[m], lo - base, hi - lo, a.K, out + (size_t)(lo - c0) * a.K, prof_kind)) return rc;
       }
     }
-    if (nc != a.N) f = choose_tile(TILE_SHAPES, N_SHAPES, EPI, a.M, nc * NMAT, a.K, ws_limit, pin);
-    if (int rc = run(TILE_SHAPES, N_SHAPES, f, nc * NMAT, launch_shape<EPI>)) return rc;
+    if (nc != a.N || sums_bytes(TILE_SHAPES, f, a.M, a.N * NMAT) > sums) f = choose_tile(TILE_SHAPES, N_SHAPES, EPI, a.M, nc * NMAT, a.K, sums, pin);
+    if (int rc = run(f, sums_at, launch_shape<EPI>)) return rc;
   }
   return 0;
 }

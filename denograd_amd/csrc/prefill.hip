@@ -403,7 +403,7 @@ int jsgrad_hip_attn_prefill(const void *q, const void *cache_k, const void *cach
   // Fewer blocks than half of what the chip holds (two per CU): the keys are cut into parts.  Not during a graph capture,
   // where nothing can be allocated.
   const size_t blocks = (size_t)a.tiles * a.pairs;
-  PoolBlock sums;
+  Workspace sums;
   if (!state().capturing && blocks * 2 <= (size_t)2 * state().cu_count && blocks * 4 <= PF_COUNTERS) {
     // A tile takes 0.7-0.9 us and folding a part about as long, one after the other: least at about sqrt(tiles) parts, and nothing
     // to gain below eight.  (57 positions behind 1024, 24 heads of 128: 24.6 / 18.6 / 15.5 / 17.1 us in 1 / 2 / 4 / 8 parts;

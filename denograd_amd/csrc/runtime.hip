@@ -64,6 +64,12 @@ struct MemCache {
   size_t live_bytes = 0, idle_bytes = 0;
   size_t limit = 0;                                       // idle bytes beyond which the next stream wait gives them back
   bool enabled = true;                                    // LRU=0 switches the cache off (allocator.ts:73)
+  // The workspace of the several-row kernels: one block, as large as the largest request so far (or, in use, as the one that
+  // has it), kept from call to call.  It never becomes anybody's tensor.
+  void *ws = nullptr;
+  size_t ws_bytes = 0, ws_limit = (size_t)-1;
+  bool ws_busy = false;
+  size_t ws_refused = (size_t)-1, freed_since = 0;        // the least request that the device had no room for, bytes freed since
   // Frees arrive from finalisers on whatever thread runs them (ctypes releases the interpreter lock during a call), so the
   // books are kept under a lock; the stream waits and driver calls made while it is held are short and rare.
   std::mutex lock;
@@ -77,9 +83,15 @@ static size_t mem_class(size_t n) {
   const size_t step = n <= (64u << 10) ? 256 : n <= (4u << 20) ? (4u << 10) : n <= (256u << 20) ? (256u << 10) : (4u << 20);
   return (n + step - 1) / step * step;
 }
+static size_t mem_idle() { return g_mem.idle_bytes + (g_mem.ws_busy ? 0 : g_mem.ws_bytes); }
 // The stream must have been waited for.
 static int mem_release_idle() {
   hipError_t first = hipSuccess;
+  if (g_mem.ws && !g_mem.ws_busy) {
+    first = hipFree(g_mem.ws);
+    g_mem.ws = nullptr;
+    g_mem.ws_bytes = 0;
+  }
   for (auto &kv : g_mem.idle)
     for (void *p : kv.second) {
       const hipError_t e = hipFree(p);
@@ -88,6 +100,49 @@ static int mem_release_idle() {
   g_mem.idle.clear();
   g_mem.idle_bytes = 0;
   return first == hipSuccess ? 0 : fail_hip(first, "hipFree");
+}
+
+// A device that had no room for a request is not asked again, with a wait for the stream and every idle block given back, for
+// each launch of a pass: not before as many bytes have been freed, or jsgrad_hip_free_cache was called.
+bool Workspace::get(size_t nbytes) {
+  MemCache &m = g_mem;
+  if (p || state().capturing) return false;
+  std::lock_guard<std::mutex> guard(m.lock);
+  if (m.ws_busy || nbytes > m.ws_limit) return false;
+  if (m.ws_bytes < nbytes) {
+    if (nbytes >= m.ws_refused && m.freed_since < nbytes) return false;
+    const size_t cls = mem_class(nbytes);
+    if (m.ws) {                                           // what is queued still uses it
+      if (hipStreamSynchronize(state().stream) != hipSuccess) return false;
+      (void)hipFree(m.ws);
+      m.ws = nullptr;
+      m.ws_bytes = 0;
+    }
+    void *q = nullptr;
+    hipError_t e = hipMalloc(&q, cls);
+    if (e != hipSuccess && m.idle_bytes > 0) {
+      (void)hipGetLastError();
+      if (hipStreamSynchronize(state().stream) != hipSuccess || mem_release_idle()) return false;
+      e = hipMalloc(&q, cls);
+    }
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      m.ws_refused = nbytes;
+      m.freed_since = 0;
+      return false;
+    }
+    if (nbytes >= m.ws_refused) m.ws_refused = (size_t)-1;
+    m.ws = q;
+    m.ws_bytes = cls;
+  }
+  m.ws_busy = true;
+  p = m.ws;
+  return true;
+}
+Workspace::~Workspace() {
+  if (!p) return;
+  std::lock_guard<std::mutex> guard(g_mem.lock);
+  g_mem.ws_busy = false;
 }
 
 }  // namespace jsg
@@ -115,6 +170,7 @@ int jsgrad_hip_init(int device) {
     const char *lru = getenv("LRU"), *mb = getenv("JSGRAD_HIP_CACHE_MB");
     jsg::g_mem.enabled = !(lru && atoi(lru) == 0);
     jsg::g_mem.limit = mb ? (size_t)strtoull(mb, nullptr, 10) << 20 : p.totalGlobalMem / 8;
+    if (const char *ws = getenv("JSGRAD_HIP_WORKSPACE_MB")) jsg::g_mem.ws_limit = (size_t)strtoull(ws, nullptr, 10) << 20;
   }
   s.device = device;
   if (int e = jsg::attn_static_init(device)) return e;
@@ -150,12 +206,12 @@ int jsgrad_hip_malloc(size_t nbytes, void **host_out_ptr) {
     it->second.pop_back();
     m.idle_bytes -= cls;
   } else {
-    if (m.idle_bytes > m.limit) {
+    if (jsg::mem_idle() > m.limit) {
       JSG_HIP(hipStreamSynchronize(state().stream));
       if (int r = jsg::mem_release_idle()) return r;
     }
     hipError_t e = hipMalloc(&p, cls);
-    if (e != hipSuccess && m.idle_bytes > 0) {
+    if (e != hipSuccess && jsg::mem_idle() > 0) {
       // out of memory with blocks lying idle: give them back and ask again (allocator.ts:60-66)
       (void)hipGetLastError();
       JSG_HIP(hipStreamSynchronize(state().stream));
@@ -183,6 +239,7 @@ int jsgrad_hip_free(void *ptr) {
   const size_t cls = it->second;
   m.live.erase(it);
   m.live_bytes -= cls;
+  m.freed_since += cls;
   if (!m.enabled) {
     JSG_HIP(hipStreamSynchronize(state().stream));
     JSG_HIP(hipFree(ptr));
@@ -197,13 +254,14 @@ int jsgrad_hip_free_cache(void) {
   JSG_REQUIRE(!state().capturing, "jsgrad_hip_free_cache during graph capture");
   JSG_HIP(hipStreamSynchronize(state().stream));
   std::lock_guard<std::mutex> guard(jsg::g_mem.lock);
+  jsg::g_mem.ws_refused = (size_t)-1;
   return jsg::mem_release_idle();
 }
 int jsgrad_hip_mem_info(size_t *host_out_live_bytes, size_t *host_out_idle_bytes) {
   JSG_READY();
   std::lock_guard<std::mutex> guard(jsg::g_mem.lock);
   if (host_out_live_bytes) *host_out_live_bytes = jsg::g_mem.live_bytes;
-  if (host_out_idle_bytes) *host_out_idle_bytes = jsg::g_mem.idle_bytes;
+  if (host_out_idle_bytes) *host_out_idle_bytes = jsg::mem_idle();
   return 0;
 }
 int jsgrad_hip_copyin(void *dst, const void *host_src, size_t nbytes) {
@@ -234,7 +292,7 @@ int jsgrad_hip_sync(void) {
   JSG_HIP(hipStreamSynchronize(state().stream));
   {
     std::lock_guard<std::mutex> guard(jsg::g_mem.lock);
-    if (jsg::g_mem.idle_bytes > jsg::g_mem.limit) return jsg::mem_release_idle();
+    if (jsg::mem_idle() > jsg::g_mem.limit) return jsg::mem_release_idle();
   }
   return 0;
 }

@@ -50,7 +50,11 @@ int jsgrad_hip_cu_count(int *host_out);
  * the driver at the next jsgrad_hip_sync once more than JSGRAD_HIP_CACHE_MB (default: an eighth of the device) lies
  * idle, when hipMalloc runs out, or through jsgrad_hip_free_cache.  LRU=0 in the environment turns reuse off
  * (allocator.ts:73): free then waits for the stream and calls hipFree.  A pointer that jsgrad_hip_malloc did not hand
- * out, or a second free of one that it did, is an error. */
+ * out, or a second free of one that it did, is an error.
+ * The several-row calls (jsgrad_hip_gemm*, jsgrad_hip_attn_prefill) share one workspace, which grows to the largest request so far
+ * (at most 2.25 GB: a quantised matrix realised in fp16, and partial sums) and is kept, also with LRU=0; it counts as idle memory and
+ * is given back where idle blocks are.  JSGRAD_HIP_WORKSPACE_MB bounds a request (0: none); a call that cannot have its
+ * workspace, also because the device is full or a graph is being captured, does without and is slower. */
 int jsgrad_hip_malloc(size_t nbytes, void **host_out_ptr);
 int jsgrad_hip_free(void *ptr);
 /* LRUAllocator.free_cache (allocator.ts:65-70): wait for the stream and give every idle block back to the driver. */
