@@ -707,7 +707,6 @@ struct TileShape { int bm, bn, bk; float us; int per_cu; const char *pin; };
 static const TileShape TILE_SHAPES[] = {
   {64, 64, 64, 0.20f, 2, "small"},     // not for w1|w3 (its tiles come in pairs)
   {64, 128, 64, 0.33f, 1, "small"},
-  {128, 64, 64, 0.33f, 1, nullptr},    // not for w1|w3
   {128, 128, 64, 0.47f, 1, "tall"},
   {256, 128, 64, 0.85f, 1, "wide"},
   {256, 256, 64, 1.43f, 1, "db"},
@@ -761,10 +760,9 @@ template <int EPI> static int launch_shape(int s, const TileArgs &t, int prof_ki
   switch (s) {
     case 0: if constexpr (EPI != GEPI_SWIGLU) return launch_tile<EPI, 64, 64, 4>(t, prof_kind); else break;
     case 1: return launch_tile<EPI, 64, 128, 4>(t, prof_kind);
-    case 2: if constexpr (EPI != GEPI_SWIGLU) return launch_tile<EPI, 128, 64, 4>(t, prof_kind); else break;
-    case 3: return launch_tile<EPI, 128, 128, 4>(t, prof_kind);
-    case 4: return launch_tile<EPI, 256, 128, 3>(t, prof_kind);
-    case 5: return launch_tile256<EPI>(t, prof_kind);
+    case 2: return launch_tile<EPI, 128, 128, 4>(t, prof_kind);
+    case 3: return launch_tile<EPI, 256, 128, 3>(t, prof_kind);
+    case 4: return launch_tile256<EPI>(t, prof_kind);
   }
   return fail("jsgrad_hip_gemm: no tile shape");
 }
