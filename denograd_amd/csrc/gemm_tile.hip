@@ -703,16 +703,16 @@ template <int KIND, int EPI, int BM, int BN, int ST> static int launch_qtile(con
 
 // The shapes, with the K elements of a step, what a block takes for one, and how many blocks share a CU before they slow each
 // other down.  us per step, fitted to launches of 40 to 1500 rows over matrices of 2048 to 28672 columns and 2048 to 14336 rows.
-struct TileShape { int bm, bn, bk; float us; int per_cu; const char *pin; };
+struct TileShape { int bm, bn, bk; float us; int per_cu; };
 static const TileShape TILE_SHAPES[] = {
-  {64, 64, 64, 0.20f, 2, "small"},     // not for w1|w3 (its tiles come in pairs)
-  {64, 128, 64, 0.33f, 1, "small"},
-  {128, 128, 64, 0.47f, 1, "tall"},
-  {256, 128, 64, 0.85f, 1, "wide"},
-  {256, 256, 64, 1.43f, 1, "db"},
+  {64, 64, 64, 0.20f, 2},     // not for w1|w3 (its tiles come in pairs)
+  {64, 128, 64, 0.33f, 1},
+  {128, 128, 64, 0.47f, 1},
+  {256, 128, 64, 0.85f, 1},
+  {256, 256, 64, 1.43f, 1},
 };
-static const TileShape QTILE_SHAPES_I8[] = {{64, 64, 64, 0.28f, 1, nullptr}, {64, 128, 64, 0.44f, 1, nullptr}, {128, 128, 64, 0.58f, 1, nullptr}};
-static const TileShape QTILE_SHAPES_NF4[] = {{64, 64, 128, 0.60f, 1, nullptr}, {64, 128, 128, 0.95f, 1, nullptr}, {128, 128, 128, 1.50f, 1, nullptr}};
+static const TileShape QTILE_SHAPES_I8[] = {{64, 64, 64, 0.28f, 1}, {64, 128, 64, 0.44f, 1}, {128, 128, 64, 0.58f, 1}};
+static const TileShape QTILE_SHAPES_NF4[] = {{64, 64, 128, 0.60f, 1}, {64, 128, 128, 0.95f, 1}, {128, 128, 128, 1.50f, 1}};
 constexpr int N_SHAPES = sizeof(TILE_SHAPES) / sizeof(TILE_SHAPES[0]), N_QSHAPES = sizeof(QTILE_SHAPES_I8) / sizeof(QTILE_SHAPES_I8[0]);
 
 // Which shape and how many K parts: the least of an estimate of the launch's time (rounds of blocks over the CUs times
@@ -721,7 +721,23 @@ constexpr int N_SHAPES = sizeof(TILE_SHAPES) / sizeof(TILE_SHAPES[0]), N_QSHAPES
 // 41, 64x64 36, 256x128 in 8 parts 52; 371 x 2048 x 2048 64x64 10.4 | 128x64 15.6, 64x64 in 2 parts 11.9; 700 x 28672 x 4096
 // 256x128 178 | 128x128 227; 4096 x 4096 x 4096 256x256 98 | 256x128 116.
 struct Choice { float us; int shape, split; };
-static Choice choose_tile(const TileShape *shapes, int n_shapes, int epi, int M, int weight_rows, int K, size_t ws_limit, const char *pin) {
+// JSG_GEMM_TILE, for tests and measurements: rows x columns of a tile, optionally with K parts, of the fp16 kernels ("128x128",
+// "64x128/3"; quantised weights are then realised) or of qtile_kernel ("q64x64/3"); "small", "tall", "wide" and "db" name fp16
+// tiles from 64x64 (w1|w3: 64x128) to 256x256.  A tile that the output width does not allow is not taken.
+struct Pin { bool on = false, codes = false; int bm = 0, bn = 0, split = 1; };
+static Pin read_pin(int epi) {
+  Pin p;
+  const char *e = getenv("JSG_GEMM_TILE");
+  if (!e) return p;
+  p.on = true;
+  const struct { const char *name; int bm, bn; } names[] = {{"small", 64, epi == GEPI_SWIGLU ? 128 : 64}, {"tall", 128, 128}, {"wide", 256, 128}, {"db", 256, 256}};
+  for (const auto &n : names)
+    if (!strcmp(e, n.name)) { p.bm = n.bm; p.bn = n.bn; return p; }
+  p.codes = *e == 'q';
+  sscanf(e + (p.codes ? 1 : 0), "%dx%d/%d", &p.bm, &p.bn, &p.split);
+  return p;
+}
+static Choice choose_tile(const TileShape *shapes, int n_shapes, int epi, int M, int weight_rows, int K, size_t ws_limit, const Pin &pin) {
   const int cus = state().cu_count;
   Choice best = {0.0f, -1, 1};
   for (int s = 0; s < n_shapes; s++) {
@@ -729,12 +745,13 @@ static Choice choose_tile(const TileShape *shapes, int n_shapes, int epi, int M,
     if (weight_rows % c.bn || K % c.bk || (epi == GEPI_SWIGLU && c.bn < 128)) continue;
     const int tiles = ((M + c.bm - 1) / c.bm) * (weight_rows / c.bn), nk = K / c.bk;
     for (int d = 1; d <= 16; d++) {
-      if (d > 1 && (pin || c.bm * c.bn == 65536 || nk / d * c.bk < 256 || tiles > TILE_COUNTERS || tiles * d > 2 * cus || (size_t)tiles * d * c.bm * c.bn * 4 > ws_limit)) break;
+      if (d > 1 && (c.bm * c.bn == 65536 || nk < d || tiles > TILE_COUNTERS || (size_t)tiles * d * c.bm * c.bn * 4 > ws_limit)) break;
+      if (d > 1 && (pin.on ? d > pin.split : nk / d * c.bk < 256 || tiles * d > 2 * cus)) break;
       const int blocks = tiles * d, rounds = (blocks + cus * c.per_cu - 1) / (cus * c.per_cu);
       const float shared = c.per_cu > 1 && blocks > cus ? 1.7f : 1.0f;   // two blocks of a CU share its L1 and matrix cores
       float us = 5.0f + rounds * shared * c.us * ((nk + d - 1) / d);
       if (d > 1) us += 3.0f + (float)d * c.bm * c.bn * 4 / 120e3f;
-      if (pin && c.pin && !strcmp(pin, c.pin)) us = 0.0f;      // taken
+      if (pin.bm == c.bm && pin.bn == c.bn && d == pin.split) us = 0.0f;   // taken
       if (best.shape < 0 || us < best.us) best = {us, s, d};
     }
   }
@@ -782,7 +799,7 @@ template <int EPI> static int gemm_tiled_epi(int kind, const GemmArgs &a, int pr
   t.b_end[0] = n[0];
   t.b_end[1] = n[0] + n[1];
 
-  const char *pin = getenv("JSG_GEMM_TILE");                  // tests and measurements: "db", "wide", "tall" or "small" of the fp16 shapes, no K parts
+  const Pin pin = read_pin(EPI), none, &codes_pin = pin.codes ? pin : none;
   const size_t ws_limit = state().capturing ? 0 : SUMS_LIMIT;
   auto run = [&](const Choice &c, float *ws, auto launch) -> int {
     JSG_REQUIRE(c.shape >= 0, "jsgrad_hip_gemm: no tile shape for %d columns", t.ncols);
@@ -792,7 +809,7 @@ template <int EPI> static int gemm_tiled_epi(int kind, const GemmArgs &a, int pr
   };
   Workspace ws;
   // all of the output at once, its sums (if it has K parts) in the workspace
-  auto run_whole = [&](const TileShape *shapes, int n_shapes, Choice c, const char *pinned, auto launch) -> int {
+  auto run_whole = [&](const TileShape *shapes, int n_shapes, Choice c, const Pin &pinned, auto launch) -> int {
     const size_t sums = sums_bytes(shapes, c, a.M, a.N * NMAT);
     if (sums && !ws.get(sums)) c = choose_tile(shapes, n_shapes, EPI, a.M, a.N * NMAT, a.K, 0, pinned);
     return run(c, (float *)ws.p, launch);
@@ -810,20 +827,20 @@ template <int EPI> static int gemm_tiled_epi(int kind, const GemmArgs &a, int pr
   // qtile_kernel brings scales by direct loads of four bytes; a pointer between two of those (a slice) is read half by half when
   // the matrix is realised
   const bool dwords = (((uintptr_t)a.s0 | (uintptr_t)a.s1 | (uintptr_t)a.s2) & 3) == 0;
-  const Choice q = dwords ? choose_tile(qs, N_QSHAPES, EPI, a.M, a.N * NMAT, a.K, ws_limit, nullptr) : Choice{0.0f, -1, 1};
+  const Choice q = dwords ? choose_tile(qs, N_QSHAPES, EPI, a.M, a.N * NMAT, a.K, ws_limit, codes_pin) : Choice{0.0f, -1, 1};
   const size_t row = (size_t)a.K * 2;
-  bool in_place = !pin && q.shape >= 0 && q.us < f.us + realise_us;
+  bool in_place = (!pin.on || pin.codes) && q.shape >= 0 && q.us < f.us + realise_us;
   // Realised into the workspace, with the K parts' sums behind it: all columns at once, or as many at a time as REALISED_LIMIT holds
   size_t bytes = (size_t)a.N * NMAT * row < REALISED_LIMIT ? (size_t)a.N * NMAT * row : REALISED_LIMIT, sums = 0;
   if (!in_place) {
     sums = sums_bytes(TILE_SHAPES, f, a.M, a.N * NMAT);
     if (!ws.get(bytes + sums)) {
       sums = 0;
-      in_place = !ws.get(bytes) && !pin && q.shape >= 0;
+      in_place = !ws.get(bytes) && !pin.on && q.shape >= 0;
     }
   }
   if (in_place)
-    return kind == JSGRAD_W_I8 ? run_whole(qs, N_QSHAPES, q, nullptr, launch_qshape<JSGRAD_W_I8, EPI>) : run_whole(qs, N_QSHAPES, q, nullptr, launch_qshape<JSGRAD_W_NF4, EPI>);
+    return kind == JSGRAD_W_I8 ? run_whole(qs, N_QSHAPES, q, codes_pin, launch_qshape<JSGRAD_W_I8, EPI>) : run_whole(qs, N_QSHAPES, q, codes_pin, launch_qshape<JSGRAD_W_NF4, EPI>);
 
   // ... or, without memory, in the library's own scratch
   _Float16 *out = (_Float16 *)ws.p;

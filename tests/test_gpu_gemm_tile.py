@@ -1,5 +1,6 @@
-"""The tiled several-row kernels where they can go wrong: edges of the row tiles, output widths that only some shapes
-divide, one K tile, K parts, and quantised weights realised piece by piece while a graph is captured.
+"""The tiled several-row kernels where they can go wrong: every tile, with and without K parts, under every epilogue (pinned, since
+most sizes that are quick to check choose the smallest tile); edges of the row tiles and one K tile as chosen; and quantised
+weights realised piece by piece while a graph is captured.
 
 Tolerance: products and sums are those of the oracle's several-row Linear in another order (assert_close, an fp16 unit of the
 result or of the operands of the residual sum)."""
@@ -87,3 +88,28 @@ def test_scales_between_two_dwords(hip, monkeypatch, kind):
     rows_tests.test_gemm_qkv_rope_writes_queries_and_cache(hip, kind, 64, 1, 57, 512)
     monkeypatch.setitem(globals(), "sp", slice_of_scales)
     test_tiled_gemm_captured_in_a_graph(hip, kind, 4096)
+
+
+TILES = ["64x64", "64x64/3", "64x128", "64x128/3", "128x128", "128x128/2", "256x128", "256x128/5", "256x256"]
+CODE_TILES = ["q64x64", "q64x64/3", "q64x128", "q64x128/2", "q128x128", "q128x128/3"]
+
+
+@pytest.mark.parametrize("kind,tile", [(k, t) for k in ("float16", "int8") for t in TILES] + [(k, t) for k in ("int8", "nf4") for t in CODE_TILES])
+def test_every_tile_under_every_epilogue(hip, monkeypatch, kind, tile):
+    """Ragged row tiles (57 and 295 rows), K parts of unequal length (10 steps of 64, or 5 of 128, in 2, 3 or 5 parts); int8 under an
+    fp16 tile is realised first.  The plain epilogue also repeats itself bit for bit."""
+    monkeypatch.setenv("JSG_GEMM_TILE", tile)
+    for rows in (57, 295):
+        test_tiled_gemm_at_the_edges(hip, kind, rows, 768, 640)
+        if "64x64" not in tile:                               # tiles of w1|w3 come in pairs
+            rows_tests.test_gemm_ffn_gate(hip, kind, rows, 640, 384)
+    rows_tests.test_gemm_qkv_rope_writes_queries_and_cache(hip, kind, 64, 3, 19, 640)
+    rows_tests.test_gemm_qkv_rope_writes_queries_and_cache(hip, kind, 128, 5, 59, 640)
+
+
+@pytest.mark.parametrize("kind,rows,dim,hidden", [("int8", 57, 3072, 1024), ("nf4", 57, 3072, 1024), ("float16", 371, 2048, 1024), ("int8", 371, 2048, 1024)])
+def test_tiles_as_chosen_under_the_fused_epilogues(hip, kind, rows, dim, hidden):
+    """K parts under SwiGLU (57 rows: codes 64x128 in 8 parts; 371 rows: codes 128x128 in 5, fp16 64x128 in 2) and under the rotary
+    epilogue (64x64 in 8 or 12)."""
+    rows_tests.test_gemm_ffn_gate(hip, kind, rows, dim, hidden)
+    rows_tests.test_gemm_qkv_rope_writes_queries_and_cache(hip, kind, 128, 1, 57, dim)
