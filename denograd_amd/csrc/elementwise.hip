@@ -264,9 +264,9 @@ template <typename AT, bool VEC> __global__ __launch_bounds__(256) void nf4_quan
     else
 #pragma unroll
       for (int e = 0; e < 8; e++) v[e] = w[i * 8 + e];
-    float amax = 0.0f;
+    float amax = fabsf((float)v[0]);   // a maximum passes over what is not a number, but a block of nothing else has it for a scale
 #pragma unroll
-    for (int e = 0; e < 8; e++) amax = fmaxf(amax, fabsf((float)v[e]));
+    for (int e = 1; e < 8; e++) amax = fmaxf(amax, fabsf((float)v[e]));
     amax = fmaxf(amax, dpp_f<0xB1>(amax));
     amax = fmaxf(amax, dpp_f<0x4E>(amax));
     amax = fmaxf(amax, dpp_f<0x141>(amax));

@@ -51,3 +51,40 @@ def test_nf4_quantise(hip, act, name, offset):
     p, s = orc.nf4_quantize(w.astype(np.float32))
     assert np.array_equal(scale.numpy().view(np.uint16), np.asarray(s).reshape(-1).view(np.uint16))
     assert np.array_equal(packed.numpy()[offset:], np.asarray(p).reshape(-1))
+
+
+@pytest.mark.parametrize("act,name", [(ffi.F16, "float16"), (ffi.F32, "float32")])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_nf4_blocks_with_inf_or_nan(hip, act, name, offset):
+    """The maximum of a block passes over NaN; a block of nothing but NaN has NaN for its scale, so that it is not read back as zeros.
+    NaN, and what an infinite scale makes of infinities, get code 0; finite values beside an infinity get the code of zero."""
+    w = np.full((5, 64), 0.25, np.float32)
+    w[0] = np.nan
+    w[1, 1:] = np.nan
+    w[2, 60] = np.nan
+    w[3, 17] = np.inf
+    w[3, 18] = np.nan
+    flat = np.concatenate([np.zeros(offset, name), w.reshape(-1).astype(name)])
+    t, packed, scale = Tensor(flat), Tensor.zeros((w.size // 2 + offset,), "uint8"), Tensor.empty((5,), "float16")
+    check(hip.jsgrad_hip_nf4_quantize(t.ptr + offset * flat.itemsize, w.size, packed.ptr + offset, scale.ptr, act))
+    np.testing.assert_array_equal(scale.numpy(), np.array([np.nan, 0.25, 0.25, np.inf, 0.25], np.float16))
+    codes = np.where(np.isfinite(w), 15, 0)
+    codes[3] = np.where(np.isfinite(w[3]), 7, 0)
+    np.testing.assert_array_equal(packed.numpy()[offset:], (codes.reshape(-1, 2) @ np.array([16, 1])).astype(np.uint8))
+
+
+@pytest.mark.parametrize("act,name", [(ffi.F16, "float16"), (ffi.F32, "float32")])
+@pytest.mark.parametrize("in_f", [64, 264, 1003])
+def test_int8_rows_with_inf_or_nan(hip, act, name, in_f):
+    """The maximum of a row passes over NaN, whose code is 0; beside an infinity every code is 0."""
+    w = np.full((4, in_f), 0.25, np.float32)
+    w[0] = np.nan
+    w[1, in_f // 2] = np.nan
+    w[2, in_f - 1] = -np.inf
+    t, codes, scale = Tensor(w.astype(name)), Tensor.empty((4, in_f), "int8"), Tensor.empty((4,), "float16")
+    check(hip.jsgrad_hip_int8_quantize(t.ptr, 4, in_f, codes.ptr, scale.ptr, act))
+    s = np.float16(np.float32(0.25) * np.float32(np.float16(1 / 127)))
+    np.testing.assert_array_equal(scale.numpy(), np.array([0, s, np.inf, s], np.float16))
+    want = np.where(np.isnan(w), 0, 127)
+    want[2] = 0
+    np.testing.assert_array_equal(codes.numpy(), want)
