@@ -657,6 +657,80 @@ static int realise(int kind, const void *w, const _Float16 *scale, int row0, int
   return 0;
 }
 
+// ---------------------------------------------------------------- quantised weights, rows too long to realise
+//
+// For a call that may not allocate (a capture, a full device), whose codes cannot be read in place and of which not even 64 rows
+// realised in fp16 fit the library's own scratch (more than 65536 elements a row, w1|w3 32768).  No model has such rows; this keeps the
+// entry points from refusing them.  A wavefront makes two sums at a time, two neighbouring columns or the w1 and the w3 row of one.
+template <int KIND, int EPI> __global__ __launch_bounds__(256) void long_rows_kernel(GemmArgs a) {
+  __shared__ uint32_t pairs[KIND == JSGRAD_W_NF4 ? 256 : 1];
+  if constexpr (KIND == JSGRAD_W_NF4) {
+    pairs[threadIdx.x] = nf4_code_bits(threadIdx.x >> 4) | (nf4_code_bits(threadIdx.x & 15) << 16);
+    __syncthreads();
+  }
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int per_row = EPI == GEPI_SWIGLU ? a.N : a.N / 2;
+  const size_t items = (size_t)a.M * per_row;
+  for (size_t it = (size_t)blockIdx.x * 4 + wave; it < items; it += (size_t)gridDim.x * 4) {
+    const int m = (int)(it / per_row), i = (int)(it % per_row), n = EPI == GEPI_SWIGLU ? i : 2 * i;
+    int which = 0, nl = n;                                    // columns n and n + 1 are of one matrix: its boundaries are even
+    if constexpr (EPI == GEPI_ROPE_KV) {
+      which = n < a.n0 ? 0 : (n < a.n0 + a.n1 ? 1 : 2);
+      nl = which == 0 ? n : (which == 1 ? n - a.n0 : n - a.n0 - a.n1);
+    }
+    float sum[2];
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+      const int mat = EPI == GEPI_SWIGLU ? c : which;
+      const size_t row = (size_t)nl + (EPI == GEPI_SWIGLU ? 0 : c);
+      const unsigned char *w = (const unsigned char *)(mat == 0 ? a.w0 : (mat == 1 ? a.w1 : a.w2)) + row * (KIND == JSGRAD_W_I8 ? a.K : a.K / 2);
+      const _Float16 *sc = (mat == 0 ? a.s0 : (mat == 1 ? a.s1 : a.s2)) + row * (KIND == JSGRAD_W_I8 ? 1 : a.K / 64);
+      float v = 0.0f;
+      for (int k = lane * 8; k < a.K; k += 512) {
+        const h8_t x = *(const h8_t *)(a.x + (size_t)m * a.K + k);
+        const _Float16 s1 = sc[KIND == JSGRAD_W_I8 ? 0 : k / 64];
+        const h2_t s = {s1, s1};
+        u4_t o;
+        if constexpr (KIND == JSGRAD_W_I8) {
+          const uint2 q = *(const uint2 *)(w + k);
+          uint32_t lo, hi;
+          i8x4_to_h2x2(q.x, lo, hi); o.x = pk_mul_h2(lo, s); o.y = pk_mul_h2(hi, s);
+          i8x4_to_h2x2(q.y, lo, hi); o.z = pk_mul_h2(lo, s); o.w = pk_mul_h2(hi, s);
+        } else {
+          const uint32_t q = *(const uint32_t *)(w + k / 2);
+#pragma unroll
+          for (int b = 0; b < 4; b++) o[b] = pk_mul_h2(pairs[(q >> (8 * b)) & 0xffu], s);
+        }
+        const h8_t wv = __builtin_bit_cast(h8_t, o);
+#pragma unroll
+        for (int e = 0; e < 8; e++) v = __builtin_fmaf((float)x[e], (float)wv[e], v);
+      }
+      sum[c] = wave_sum(v);
+    }
+    if (lane != 0) continue;
+    if constexpr (EPI == GEPI_SWIGLU) a.y[(size_t)m * a.N + n] = (_Float16)swiglu(sum[0], sum[1]);
+    else if constexpr (EPI == GEPI_STORE) {
+#pragma unroll
+      for (int c = 0; c < 2; c++) {
+        const size_t at = (size_t)m * a.N + n + c;
+        a.y[at] = (_Float16)(a.residual ? (float)a.residual[at] + rn16(sum[c]) : sum[c]);
+      }
+    } else {
+      const int b = m / a.seq_len, pos = a.start_pos + m % a.seq_len;
+      float ev = rn16(sum[0]), od = rn16(sum[1]);
+      if (which < 2) {
+        const _Float16 *cs = a.rope_table + ((size_t)pos * (a.head_dim / 2) + ((nl % a.head_dim) >> 1)) * 2;
+        const float c = (float)cs[0], d = (float)cs[1], e = ev;
+        ev = e * c - od * d;
+        od = e * d + od * c;
+      }
+      _Float16 *to = which == 0 ? a.y + (size_t)m * a.n0 + nl : (which == 1 ? a.cache_k : a.cache_v) + ((size_t)b * a.max_context + pos) * a.n1 + nl;
+      to[0] = (_Float16)ev;
+      to[1] = (_Float16)od;
+    }
+  }
+}
+
 // ---------------------------------------------------------------- host side
 
 constexpr int TILE_COUNTERS = 4096;
@@ -848,7 +922,12 @@ template <int EPI> static int gemm_tiled_epi(int kind, const GemmArgs &a, int pr
     if (int rc = gemm_scratch((void **)&out, &bytes)) return rc;
   const size_t fit = bytes / (NMAT * row);
   const int step = fit >= (size_t)a.N ? a.N : (int)(fit >= 128 ? fit / 128 * 128 : fit / 64 * 64);   // 64: the narrowest tile
-  JSG_REQUIRE(step > 0, "jsgrad_hip_gemm: in_features %d is too long for these weights without memory to realise them in", a.K);
+  if (step == 0) {
+    const dim3 grid((unsigned)state().cu_count * 8), block(256);
+    if (kind == JSGRAD_W_I8) JSG_LAUNCH(prof_kind, (long_rows_kernel<JSGRAD_W_I8, EPI>), grid, block, 0, a);
+    else JSG_LAUNCH(prof_kind, (long_rows_kernel<JSGRAD_W_NF4, EPI>), grid, block, 0, a);
+    return 0;
+  }
   float *const sums_at = sums ? (float *)((unsigned char *)out + bytes) : nullptr;
   for (int c0 = 0; c0 < a.N; c0 += step) {
     const int nc = a.N - c0 < step ? a.N - c0 : step;

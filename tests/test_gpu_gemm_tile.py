@@ -113,3 +113,46 @@ def test_tiles_as_chosen_under_the_fused_epilogues(hip, kind, rows, dim, hidden)
     epilogue (64x64 in 8 or 12)."""
     rows_tests.test_gemm_ffn_gate(hip, kind, rows, dim, hidden)
     rows_tests.test_gemm_qkv_rope_writes_queries_and_cache(hip, kind, 128, 1, 57, dim)
+
+
+class Captured:
+    """The library with its several-row products captured in a graph, which is then launched."""
+
+    def __init__(self, hip):
+        self.hip = hip
+
+    def __getattr__(self, name):
+        f = getattr(self.hip, name)
+        if not name.startswith("jsgrad_hip_gemm"):
+            return f
+
+        def call(*args):
+            graph = C.c_void_p()
+            check(self.hip.jsgrad_hip_graph_begin())
+            try:
+                status = f(*args)
+            finally:
+                check(self.hip.jsgrad_hip_graph_end(C.byref(graph)))
+            if status == 0:
+                check(self.hip.jsgrad_hip_graph_launch(graph))
+                check(self.hip.jsgrad_hip_sync())
+            check(self.hip.jsgrad_hip_graph_destroy(graph))
+            return status
+        return call
+
+
+@pytest.mark.parametrize("kind", ["int8", "nf4"])
+def test_rows_too_long_for_the_scratch_memory(hip, monkeypatch, kind):
+    """Captured, with codes that are not read in place (int8: scales between two dwords; nf4: an odd number of 64-blocks), and of which
+    64 rows realised in fp16 exceed 8 MiB: served all the same, under every epilogue."""
+    held = []
+
+    def slice_of_scales(t):
+        held.append(Tensor(np.concatenate([np.full(1, 7.0, np.float16), t.numpy().reshape(-1)])))
+        return held[-1].ptr + 2
+
+    if kind == "int8":
+        monkeypatch.setattr(rows_tests, "sp", slice_of_scales)
+    rows_tests.test_gemm_matches_several_row_linear(Captured(hip), kind, 3, 128, 65600)
+    rows_tests.test_gemm_ffn_gate(Captured(hip), kind, 35, 32832, 128)
+    rows_tests.test_gemm_qkv_rope_writes_queries_and_cache(Captured(hip), kind, 64, 1, 3, 65600)
