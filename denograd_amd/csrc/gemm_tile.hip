@@ -775,25 +775,28 @@ template <int KIND, int EPI, int BM, int BN, int ST> static int launch_qtile(con
   return 0;
 }
 
-// The shapes, with the K elements of a step, what a block takes for one, and how many blocks share a CU before they slow each
-// other down.  us per step, fitted to launches of 40 to 1500 rows over matrices of 2048 to 28672 columns and 2048 to 14336 rows.
-struct TileShape { int bm, bn, bk; float us; int per_cu; };
+// The shapes, with the K elements of a step and four times fitted to 684 launches of 33 to 4096 rows over the matrices of the 1B, 3B and
+// 8B models, each under every shape (weights from memory; an estimate is off by 6-10 % r.m.s., nf4 3 %): us of a step of blocks that
+// have a compute unit each, what fill adds to it when every unit has one (they share memory and power), us of a step of a
+// round when there are several, and of a round's end.
+struct TileShape { int bm, bn, bk; float step, fill, round_step, end; };
 static const TileShape TILE_SHAPES[] = {
-  {64, 64, 64, 0.20f, 2},     // not for w1|w3 (its tiles come in pairs)
-  {64, 128, 64, 0.33f, 1},
-  {128, 128, 64, 0.47f, 1},
-  {256, 128, 64, 0.85f, 1},
-  {256, 256, 64, 1.43f, 1},
+  {64, 64, 64, 0.25f, 0.02f, 0.21f, 0.0f},     // not for w1|w3 (its tiles come in pairs)
+  {64, 128, 64, 0.29f, 0.08f, 0.39f, 0.0f},
+  {128, 128, 64, 0.37f, 0.13f, 0.54f, 0.3f},
+  {256, 128, 64, 0.58f, 0.28f, 0.90f, 0.8f},
+  {256, 256, 64, 0.95f, 0.43f, 1.50f, 3.2f},
 };
-static const TileShape QTILE_SHAPES_I8[] = {{64, 64, 64, 0.28f, 1}, {64, 128, 64, 0.44f, 1}, {128, 128, 64, 0.58f, 1}};
-static const TileShape QTILE_SHAPES_NF4[] = {{64, 64, 128, 0.60f, 1}, {64, 128, 128, 0.95f, 1}, {128, 128, 128, 1.50f, 1}};
+static const TileShape QTILE_SHAPES_I8[] = {{64, 64, 64, 0.27f, 0.03f, 0.18f, 0.0f}, {64, 128, 64, 0.39f, 0.04f, 0.32f, 0.5f}, {128, 128, 64, 0.56f, 0.08f, 0.51f, 1.2f}};
+static const TileShape QTILE_SHAPES_NF4[] = {{64, 64, 128, 0.57f, 0.03f, 0.45f, 0.3f}, {64, 128, 128, 0.86f, 0.08f, 0.72f, 1.3f}, {128, 128, 128, 1.4f, 0.12f, 1.6f, 2.3f}};
 constexpr int N_SHAPES = sizeof(TILE_SHAPES) / sizeof(TILE_SHAPES[0]), N_QSHAPES = sizeof(QTILE_SHAPES_I8) / sizeof(QTILE_SHAPES_I8[0]);
 
-// Which shape and how many K parts: the least of an estimate of the launch's time (rounds of blocks over the CUs times
-// steps per block, a fixed 5 us for start and first tiles, for K parts 3 us and the last arriver's reading of all sums at
-// a CU's 64 bytes a clock).  Examples, us, this choice | the neighbours: 371 x 2048 x 8192 128x128 in 4 parts 29.5 | in 2 parts
-// 41, 64x64 36, 256x128 in 8 parts 52; 371 x 2048 x 2048 64x64 10.4 | 128x64 15.6, 64x64 in 2 parts 11.9; 700 x 28672 x 4096
-// 256x128 178 | 128x128 227; 4096 x 4096 x 4096 256x256 98 | 256x128 116.
+// Which shape and how many K parts: the least of an estimate of the launch's time (4.5 us for start and first tiles; for K parts 2 us
+// and the sums' way through memory).  Over those launches the choice is 1 % slower than the best shape on average, 4 % at the
+// ninth decile.  Examples, us, this choice | others: 371 x 2048 x 8192 128x128 in 5 parts 24.4 | in 3 parts 28.9,
+// 64x64 38.6, 256x128 in 8 parts 34.9; 371 x 2048 x 2048 64x128 in 2 parts 12.4 | in one 14.2, 64x64 12.7; 700 x 28672 x 4096 256x128
+// 182 | 256x256 190, 128x128 216; 2048 x 6144 x 4096 256x256 84 | 256x128 107, 128x128 106; 1200 x 2048 x 2048 128x128 18.4 |
+// 256x128 25.9.
 struct Choice { float us; int shape, split; };
 // JSG_GEMM_TILE, for tests and measurements: rows x columns of a tile, optionally with K parts, of the fp16 kernels ("128x128",
 // "64x128/3"; quantised weights are then realised) or of qtile_kernel ("q64x64/3"); "small", "tall", "wide" and "db" name fp16
@@ -821,10 +824,10 @@ static Choice choose_tile(const TileShape *shapes, int n_shapes, int epi, int M,
     for (int d = 1; d <= 16; d++) {
       if (d > 1 && (c.bm * c.bn == 65536 || nk < d || tiles > TILE_COUNTERS || (size_t)tiles * d * c.bm * c.bn * 4 > ws_limit)) break;
       if (d > 1 && (pin.on ? d > pin.split : nk / d * c.bk < 256 || tiles * d > 2 * cus)) break;
-      const int blocks = tiles * d, rounds = (blocks + cus * c.per_cu - 1) / (cus * c.per_cu);
-      const float shared = c.per_cu > 1 && blocks > cus ? 1.7f : 1.0f;   // two blocks of a CU share its L1 and matrix cores
-      float us = 5.0f + rounds * shared * c.us * ((nk + d - 1) / d);
-      if (d > 1) us += 3.0f + (float)d * c.bm * c.bn * 4 / 120e3f;
+      const int blocks = tiles * d, steps = (nk + d - 1) / d;
+      const float fill = (float)blocks / cus;
+      float us = 4.5f + (fill <= 1.0f ? (c.step + c.fill * fill) * steps + c.end : ((blocks + cus - 1) / cus) * (c.round_step * steps + c.end));
+      if (d > 1) us += 2.0f + (float)d * c.bm * c.bn * 4 / 80e3f * (fill > 1.0f ? fill : 1.0f);
       if (pin.bm == c.bm && pin.bn == c.bn && d == pin.split) us = 0.0f;   // taken
       if (best.shape < 0 || us < best.us) best = {us, s, d};
     }
@@ -892,11 +895,13 @@ template <int EPI> static int gemm_tiled_epi(int kind, const GemmArgs &a, int pr
   Choice f = choose_tile(TILE_SHAPES, N_SHAPES, EPI, a.M, a.N * NMAT, a.K, ws_limit, pin);
   if (kind == JSGRAD_W_F16) return run_whole(TILE_SHAPES, N_SHAPES, f, pin, launch_shape<EPI>);
 
-  // Quantised: dequantised as read, or realised first (memory at 4.5 TB/s, and 2 us a launch), whichever is estimated to be
-  // done first: on the 8B shapes the line lies near a thousand rows.  Where there is no memory for the realised matrix (a
-  // capture, a full device) the codes are read in place whenever a shape takes them.
-  const double elems = (double)a.N * NMAT * a.K;
-  const float realise_us = (float)(elems * (kind == JSGRAD_W_I8 ? 3.0 : 2.5) / 4.5e6) + 2.0f * (EPI == GEPI_STORE ? 1 : NMAT + 1);
+  // Quantised: dequantised as read, or realised first, whichever is estimated to be done first.  Where there is no memory for the
+  // realised matrix (a capture, a full device) the codes are read in place whenever a shape takes them.  Realising: codes in and halves
+  // out at 8.8 TB/s, slower where the last level cache cannot hold them until they are read (w1|w3 of the 8B shape, 352 MB: 60 us), a
+  // launch per matrix.  On the matrices of the 8B model int8 is realised from 640 to 1800 rows on, nf4 from 320 to 640 (and read in
+  // place again in narrow bands above that, where the fp16 tiles begin another round).
+  const float moved = (float)((double)a.N * NMAT * a.K * (kind == JSGRAD_W_I8 ? 3.0 : 2.5)), big = moved - 150e6f;
+  const float realise_us = moved / 8.8e6f + (big > 0.0f ? big / 17e6f : 0.0f) + 3.2f + 4.5f * (EPI == GEPI_STORE ? 0 : EPI == GEPI_SWIGLU ? 1 : 2);
   const TileShape *qs = kind == JSGRAD_W_I8 ? QTILE_SHAPES_I8 : QTILE_SHAPES_NF4;
   // qtile_kernel brings scales by direct loads of four bytes; a pointer between two of those (a slice) is read half by half when
   // the matrix is realised
