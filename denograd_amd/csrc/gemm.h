@@ -1,4 +1,4 @@
-// What the several-row kernels share: gemm.hip (few rows), gemm_tile.hip (more than that), prefill.hip (causal attention).
+// What the several-row kernels share: gemm.hip (few rows), gemm_tile.hip and gemm_staged.hip (more than that), prefill.hip (causal attention).
 #pragma once
 #include "common.h"
 
@@ -67,7 +67,8 @@ __device__ __forceinline__ void dma4(i4_t rs, uint32_t voff, uint32_t soff, uint
 int gemm_few(int epi, int kind, const GemmArgs &a, int prof_kind, bool *taken);
 // gemm_tile.hip: the tiled kernels, any number of rows; epi: GEPI_*
 int gemm_tiled(int epi, int kind, const GemmArgs &a, int prof_kind);
-// gemm.hip: 8 MiB of device memory that belong to the several-row kernels (one launch at a time: the stream orders them)
-int gemm_scratch(void **host_out, size_t *host_out_bytes);
+// gemm_staged.hip: quantised weights dequantised on their way into LDS, any number of rows; bm: 32 (32x128 tiles, not for w1|w3), 128
+// (128x128) or 256 (256x256; the output, w1 and w3 counted together, is then a multiple of 256)
+int gemm_staged(int epi, int kind, int bm, const GemmArgs &a, int prof_kind);
 
 }  // namespace jsg

@@ -669,13 +669,6 @@ template <int EPI> static int dispatch_gemm(int kind, const GemmArgs &a, int pro
   if (kind == JSGRAD_W_NF4) { const int rc = dispatch_skinny<JSGRAD_W_NF4, EPI>(a, prof_kind, &taken); if (taken) return rc; }
   return gemm_tiled(EPI, kind, a, prof_kind);
 }
-int gemm_scratch(void **host_out, size_t *host_out_bytes) {
-  static void *p = nullptr;
-  if (!p) JSG_HIP(hipGetSymbolAddress(&p, HIP_SYMBOL(sg_scratch)));
-  *host_out = p;
-  *host_out_bytes = SG_WS_BYTES;
-  return 0;
-}
 
 // largest column tile any configuration uses: output widths must be multiples of it
 constexpr int GEMM_N_ALIGN = 128;

@@ -30,13 +30,11 @@ namespace jsg {
 constexpr int TILE_BK = 64;
 constexpr int TILE_THREADS = 512;
 
-// One launch of a tiled kernel: columns [col0, col0 + ncols) of the output.
 struct TileArgs {
   GemmArgs g;                          // output side: y, residual, rope, cache, M, N, K
-  const void *b[3];                    // weight rows of those columns (fp16, or codes), up to three matrices on top of each other
+  const void *b[3];                    // weight rows (fp16, or codes), up to three matrices on top of each other
   const _Float16 *s[3];                // codes: their scales
   int b_end[2];                        // ends of the first two (SWIGLU: b[0] is w1, b[1] is w3, row for row)
-  int col0, ncols;
   int split;                           // K parts
   float *ws;                           // split > 1: [tile][part][BM * BN] floats
   int *counters;                       // split > 1: one per tile, zero, and zero again afterwards
@@ -62,7 +60,7 @@ __device__ __forceinline__ void turn_barrier_lds() {
 struct TileId { int tile, part, m0, col; };
 template <int BM, int CW> __device__ __forceinline__ TileId tile_id(const TileArgs &t) {
   constexpr int GROUP = 4;
-  const int tiles_m = (t.g.M + BM - 1) / BM, tiles_n = t.ncols / CW, nblocks = tiles_m * tiles_n * t.split;
+  const int tiles_m = (t.g.M + BM - 1) / BM, tiles_n = t.g.N / CW, nblocks = tiles_m * tiles_n * t.split;
   int bid = blockIdx.x;
   const int per = nblocks / 8;
   if (bid < per * 8) bid = (bid & 7) * per + (bid >> 3);
@@ -335,7 +333,7 @@ template <int EPI> __global__ __launch_bounds__(TILE_THREADS, 2) void tile256_ke
 
   constexpr int C16 = EPI == GEPI_SWIGLU ? 2 : 4;
   _Float16 *ep = (_Float16 *)tile_lds + wave * 64 * (C16 * 16 + 8);
-  tile_epilogue<EPI, 8, C16, 4>(a, ep, m0 + g * 128, t.col0 + id.col + wn * C16 * 16, [&](int i, int j, int c) {
+  tile_epilogue<EPI, 8, C16, 4>(a, ep, m0 + g * 128, id.col + wn * C16 * 16, [&](int i, int j, int c) {
     if constexpr (EPI == GEPI_SWIGLU) return swiglu(acc[i >> 2][i & 3][0][j][c], acc[i >> 2][i & 3][1][j][c]);
     else return acc[i >> 2][i & 3][j >> 1][j & 1][c];
   });
@@ -436,7 +434,7 @@ template <int EPI, int BM, int BN, int ST> __global__ __launch_bounds__(TILE_THR
   constexpr int C16 = EPI == GEPI_SWIGLU ? TN / 2 : TN, RB = TM < 4 ? TM : 4;
   _Float16 *ep = (_Float16 *)tile_lds + wave * RB * 16 * (C16 * 16 + 8);
   static_assert((size_t)8 * RB * 16 * (C16 * 16 + 8) * 2 <= tile_lds_bytes<EPI, BM, BN, ST>(), "the turning pieces fit the tiles' LDS");
-  tile_epilogue<EPI, TM, C16, RB>(a, ep, m0 + g * TM * 16, t.col0 + id.col + wn * C16 * 16, [&](int i, int j, int c) {
+  tile_epilogue<EPI, TM, C16, RB>(a, ep, m0 + g * TM * 16, id.col + wn * C16 * 16, [&](int i, int j, int c) {
     if constexpr (EPI == GEPI_SWIGLU) return swiglu(acc[i][j][c], acc[i][j + TN / 2][c]);
     else return acc[i][j][c];
   });
@@ -595,7 +593,7 @@ template <int KIND, int EPI, int BM, int BN, int ST> __global__ __launch_bounds_
   constexpr int C16 = EPI == GEPI_SWIGLU ? 1 : TN, RB = 4;
   _Float16 *ep = (_Float16 *)tile_lds + wave * RB * 16 * (C16 * 16 + 8);
   static_assert((size_t)4 * RB * 16 * (C16 * 16 + 8) * 2 <= (size_t)ST * BUF, "the turning pieces fit the stages' LDS");
-  tile_epilogue<EPI, TM, C16, RB>(a, ep, m0, t.col0 + id.col + wave * C16 * 16, [&](int i, int j, int c) {
+  tile_epilogue<EPI, TM, C16, RB>(a, ep, m0, id.col + wave * C16 * 16, [&](int i, int j, int c) {
     if constexpr (EPI == GEPI_SWIGLU) return swiglu(acc[i][0][c], acc[i][1][c]);
     else return acc[i][j][c];
   });
@@ -603,16 +601,15 @@ template <int KIND, int EPI, int BM, int BN, int ST> __global__ __launch_bounds_
 
 // ---------------------------------------------------------------- quantised weights, realised in fp16
 //
-// Rows [row0, row0 + rows) of one matrix to out[rows][K].  A thread makes eight elements at a time, so a wavefront's store is 1 KiB
+// One matrix to out[rows][K].  A thread makes eight elements at a time, so a wavefront's store is 1 KiB
 // without gaps (nf4 with 64 bytes per thread: 3.0 TB/s of codes in and halves out), and has four such pieces in flight.
-template <int KIND> __global__ __launch_bounds__(256) void realise_kernel(const unsigned char *w, const _Float16 *scale, _Float16 *out, int row0, size_t pieces, int ppr) {
+template <int KIND> __global__ __launch_bounds__(256) void realise_kernel(const unsigned char *w, const _Float16 *scale, _Float16 *out, size_t pieces, int ppr) {
   __shared__ uint32_t pairs[KIND == JSGRAD_W_NF4 ? 256 : 1];
   if constexpr (KIND == JSGRAD_W_NF4) {
     pairs[threadIdx.x] = nf4_code_bits(threadIdx.x >> 4) | (nf4_code_bits(threadIdx.x & 15) << 16);
     __syncthreads();
   }
   constexpr int U = 4;
-  const size_t first = (size_t)row0 * ppr;
   for (size_t i0 = (size_t)blockIdx.x * (256 * U) + threadIdx.x; i0 < pieces; i0 += (size_t)gridDim.x * (256 * U)) {
     uint2 q[U];
     _Float16 s1[U];
@@ -620,11 +617,11 @@ template <int KIND> __global__ __launch_bounds__(256) void realise_kernel(const 
     for (int u = 0; u < U; u++) {
       const size_t i = i0 + u * 256 < pieces ? i0 + u * 256 : pieces - 1;
       if constexpr (KIND == JSGRAD_W_I8) {
-        q[u] = *(const uint2 *)(w + (first + i) * 8);
-        s1[u] = scale[row0 + (int)((uint32_t)i / (uint32_t)ppr)];
+        q[u] = *(const uint2 *)(w + i * 8);
+        s1[u] = scale[(uint32_t)i / (uint32_t)ppr];
       } else {
-        q[u].x = *(const uint32_t *)(w + (first + i) * 4);
-        s1[u] = scale[(first + i) >> 3];                      // a block of 64 is eight pieces
+        q[u].x = *(const uint32_t *)(w + i * 4);
+        s1[u] = scale[i >> 3];                      // a block of 64 is eight pieces
       }
     }
 #pragma unroll
@@ -646,89 +643,15 @@ template <int KIND> __global__ __launch_bounds__(256) void realise_kernel(const 
   }
 }
 
-static int realise(int kind, const void *w, const _Float16 *scale, int row0, int rows, int K, _Float16 *out, int prof_kind) {
+static int realise(int kind, const void *w, const _Float16 *scale, int rows, int K, _Float16 *out, int prof_kind) {
   const int ppr = K / 8;                                      // pieces per row
   const size_t pieces = (size_t)rows * ppr;
   JSG_REQUIRE(pieces < (size_t)1 << 32, "jsgrad_hip_gemm: a matrix of %d x %d is too large", rows, K);
   const size_t want = (pieces + 1023) / 1024;
   const int grid = (int)(want < (size_t)16 * state().cu_count ? want : (size_t)16 * state().cu_count);
-  if (kind == JSGRAD_W_I8) JSG_LAUNCH(prof_kind, realise_kernel<JSGRAD_W_I8>, dim3(grid), dim3(256), 0, (const unsigned char *)w, scale, out, row0, pieces, ppr);
-  else JSG_LAUNCH(prof_kind, realise_kernel<JSGRAD_W_NF4>, dim3(grid), dim3(256), 0, (const unsigned char *)w, scale, out, row0, pieces, ppr);
+  if (kind == JSGRAD_W_I8) JSG_LAUNCH(prof_kind, realise_kernel<JSGRAD_W_I8>, dim3(grid), dim3(256), 0, (const unsigned char *)w, scale, out, pieces, ppr);
+  else JSG_LAUNCH(prof_kind, realise_kernel<JSGRAD_W_NF4>, dim3(grid), dim3(256), 0, (const unsigned char *)w, scale, out, pieces, ppr);
   return 0;
-}
-
-// ---------------------------------------------------------------- quantised weights, rows too long to realise
-//
-// For a call that may not allocate (a capture, a full device), whose codes cannot be read in place and of which not even 64 rows
-// realised in fp16 fit the library's own scratch (more than 65536 elements a row, w1|w3 32768).  No model has such rows; this keeps the
-// entry points from refusing them.  A wavefront makes two sums at a time, two neighbouring columns or the w1 and the w3 row of one.
-template <int KIND, int EPI> __global__ __launch_bounds__(256) void long_rows_kernel(GemmArgs a) {
-  __shared__ uint32_t pairs[KIND == JSGRAD_W_NF4 ? 256 : 1];
-  if constexpr (KIND == JSGRAD_W_NF4) {
-    pairs[threadIdx.x] = nf4_code_bits(threadIdx.x >> 4) | (nf4_code_bits(threadIdx.x & 15) << 16);
-    __syncthreads();
-  }
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  const int per_row = EPI == GEPI_SWIGLU ? a.N : a.N / 2;
-  const size_t items = (size_t)a.M * per_row;
-  for (size_t it = (size_t)blockIdx.x * 4 + wave; it < items; it += (size_t)gridDim.x * 4) {
-    const int m = (int)(it / per_row), i = (int)(it % per_row), n = EPI == GEPI_SWIGLU ? i : 2 * i;
-    int which = 0, nl = n;                                    // columns n and n + 1 are of one matrix: its boundaries are even
-    if constexpr (EPI == GEPI_ROPE_KV) {
-      which = n < a.n0 ? 0 : (n < a.n0 + a.n1 ? 1 : 2);
-      nl = which == 0 ? n : (which == 1 ? n - a.n0 : n - a.n0 - a.n1);
-    }
-    float sum[2];
-#pragma unroll
-    for (int c = 0; c < 2; c++) {
-      const int mat = EPI == GEPI_SWIGLU ? c : which;
-      const size_t row = (size_t)nl + (EPI == GEPI_SWIGLU ? 0 : c);
-      const unsigned char *w = (const unsigned char *)(mat == 0 ? a.w0 : (mat == 1 ? a.w1 : a.w2)) + row * (KIND == JSGRAD_W_I8 ? a.K : a.K / 2);
-      const _Float16 *sc = (mat == 0 ? a.s0 : (mat == 1 ? a.s1 : a.s2)) + row * (KIND == JSGRAD_W_I8 ? 1 : a.K / 64);
-      float v = 0.0f;
-      for (int k = lane * 8; k < a.K; k += 512) {
-        const h8_t x = *(const h8_t *)(a.x + (size_t)m * a.K + k);
-        const _Float16 s1 = sc[KIND == JSGRAD_W_I8 ? 0 : k / 64];
-        const h2_t s = {s1, s1};
-        u4_t o;
-        if constexpr (KIND == JSGRAD_W_I8) {
-          const uint2 q = *(const uint2 *)(w + k);
-          uint32_t lo, hi;
-          i8x4_to_h2x2(q.x, lo, hi); o.x = pk_mul_h2(lo, s); o.y = pk_mul_h2(hi, s);
-          i8x4_to_h2x2(q.y, lo, hi); o.z = pk_mul_h2(lo, s); o.w = pk_mul_h2(hi, s);
-        } else {
-          const uint32_t q = *(const uint32_t *)(w + k / 2);
-#pragma unroll
-          for (int b = 0; b < 4; b++) o[b] = pk_mul_h2(pairs[(q >> (8 * b)) & 0xffu], s);
-        }
-        const h8_t wv = __builtin_bit_cast(h8_t, o);
-#pragma unroll
-        for (int e = 0; e < 8; e++) v = __builtin_fmaf((float)x[e], (float)wv[e], v);
-      }
-      sum[c] = wave_sum(v);
-    }
-    if (lane != 0) continue;
-    if constexpr (EPI == GEPI_SWIGLU) a.y[(size_t)m * a.N + n] = (_Float16)swiglu(sum[0], sum[1]);
-    else if constexpr (EPI == GEPI_STORE) {
-#pragma unroll
-      for (int c = 0; c < 2; c++) {
-        const size_t at = (size_t)m * a.N + n + c;
-        a.y[at] = (_Float16)(a.residual ? (float)a.residual[at] + rn16(sum[c]) : sum[c]);
-      }
-    } else {
-      const int b = m / a.seq_len, pos = a.start_pos + m % a.seq_len;
-      float ev = rn16(sum[0]), od = rn16(sum[1]);
-      if (which < 2) {
-        const _Float16 *cs = a.rope_table + ((size_t)pos * (a.head_dim / 2) + ((nl % a.head_dim) >> 1)) * 2;
-        const float c = (float)cs[0], d = (float)cs[1], e = ev;
-        ev = e * c - od * d;
-        od = e * d + od * c;
-      }
-      _Float16 *to = which == 0 ? a.y + (size_t)m * a.n0 + nl : (which == 1 ? a.cache_k : a.cache_v) + ((size_t)b * a.max_context + pos) * a.n1 + nl;
-      to[0] = (_Float16)ev;
-      to[1] = (_Float16)od;
-    }
-  }
 }
 
 // ---------------------------------------------------------------- host side
@@ -745,7 +668,7 @@ template <int EPI> static int launch_tile256(const TileArgs &t, int prof_kind) {
     JSG_HIP(hipFuncSetAttribute((const void *)tile256_kernel<EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
     raised = true;
   }
-  const int tiles = ((t.g.M + 255) / 256) * (t.ncols / (EPI == GEPI_SWIGLU ? 128 : 256));
+  const int tiles = ((t.g.M + 255) / 256) * (t.g.N / (EPI == GEPI_SWIGLU ? 128 : 256));
   JSG_LAUNCH(prof_kind, (tile256_kernel<EPI>), dim3(tiles), dim3(TILE_THREADS), lds, t);
   return 0;
 }
@@ -757,7 +680,7 @@ template <int EPI, int BM, int BN, int ST> static int launch_tile(const TileArgs
     JSG_HIP(hipFuncSetAttribute((const void *)tile_kernel<EPI, BM, BN, ST>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
     raised = true;
   }
-  const int tiles = ((t.g.M + BM - 1) / BM) * (t.ncols / (EPI == GEPI_SWIGLU ? BN / 2 : BN));
+  const int tiles = ((t.g.M + BM - 1) / BM) * (t.g.N / (EPI == GEPI_SWIGLU ? BN / 2 : BN));
   JSG_LAUNCH(prof_kind, (tile_kernel<EPI, BM, BN, ST>), dim3(tiles * t.split), dim3(TILE_THREADS), lds, t);
   return 0;
 }
@@ -770,7 +693,7 @@ template <int KIND, int EPI, int BM, int BN, int ST> static int launch_qtile(con
     JSG_HIP(hipFuncSetAttribute((const void *)qtile_kernel<KIND, EPI, BM, BN, ST>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
     raised = true;
   }
-  const int tiles = ((t.g.M + BM - 1) / BM) * (t.ncols / (EPI == GEPI_SWIGLU ? BN / 2 : BN));
+  const int tiles = ((t.g.M + BM - 1) / BM) * (t.g.N / (EPI == GEPI_SWIGLU ? BN / 2 : BN));
   JSG_LAUNCH(prof_kind, (qtile_kernel<KIND, EPI, BM, BN, ST>), dim3(tiles * t.split), dim3(QT_THREADS), lds, t);
   return 0;
 }
@@ -789,7 +712,10 @@ static const TileShape TILE_SHAPES[] = {
 };
 static const TileShape QTILE_SHAPES_I8[] = {{64, 64, 64, 0.27f, 0.03f, 0.18f, 0.0f}, {64, 128, 64, 0.39f, 0.04f, 0.32f, 0.5f}, {128, 128, 64, 0.56f, 0.08f, 0.51f, 1.2f}};
 static const TileShape QTILE_SHAPES_NF4[] = {{64, 64, 128, 0.57f, 0.03f, 0.45f, 0.3f}, {64, 128, 128, 0.86f, 0.08f, 0.72f, 1.3f}, {128, 128, 128, 1.4f, 0.12f, 1.6f, 2.3f}};
-constexpr int N_SHAPES = sizeof(TILE_SHAPES) / sizeof(TILE_SHAPES[0]), N_QSHAPES = sizeof(QTILE_SHAPES_I8) / sizeof(QTILE_SHAPES_I8[0]);
+// gemm_staged.hip; 32x128 not for w1|w3
+static const TileShape STAGED_SHAPES_I8[] = {{32, 128, 64, 0.45f, 0.10f, 0.30f, 0.5f}, {128, 128, 64, 0.77f, 0.09f, 0.60f, 1.2f}, {256, 256, 64, 1.1f, 0.48f, 1.7f, 8.0f}};
+static const TileShape STAGED_SHAPES_NF4[] = {{32, 128, 64, 0.55f, 0.15f, 0.35f, 0.5f}, {128, 128, 64, 0.88f, 0.10f, 0.66f, 0.7f}, {256, 256, 64, 1.5f, 0.34f, 1.95f, 8.4f}};
+constexpr int N_SHAPES = sizeof(TILE_SHAPES) / sizeof(TILE_SHAPES[0]), N_QSHAPES = sizeof(QTILE_SHAPES_I8) / sizeof(QTILE_SHAPES_I8[0]), N_STAGED = sizeof(STAGED_SHAPES_I8) / sizeof(STAGED_SHAPES_I8[0]);
 
 // Which shape and how many K parts: the least of an estimate of the launch's time (4.5 us for start and first tiles; for K parts 2 us
 // and the sums' way through memory).  Over those launches the choice is 1 % slower than the best shape on average, 4 % at the
@@ -799,19 +725,18 @@ constexpr int N_SHAPES = sizeof(TILE_SHAPES) / sizeof(TILE_SHAPES[0]), N_QSHAPES
 // 256x128 25.9.
 struct Choice { float us; int shape, split; };
 // JSG_GEMM_TILE, for tests and measurements: rows x columns of a tile, optionally with K parts, of the fp16 kernels ("128x128",
-// "64x128/3"; quantised weights are then realised) or of qtile_kernel ("q64x64/3"); "small", "tall", "wide" and "db" name fp16
-// tiles from 64x64 (w1|w3: 64x128) to 256x256.  A tile that the output width does not allow is not taken.
-struct Pin { bool on = false, codes = false; int bm = 0, bn = 0, split = 1; };
+// "64x128/3"; quantised weights are then realised), of qtile_kernel ("q64x64/3") or of the staged kernel ("s256x256"); "small", "tall",
+// "wide" and "db" name fp16 tiles from 64x64 (w1|w3: 64x128) to 256x256.  A tile that the output width does not allow is not taken.
+struct Pin { char family = 0; int bm = 0, bn = 0, split = 1; };   // family: 't', 'q' or 's'; 0: no pin
 static Pin read_pin(int epi) {
   Pin p;
   const char *e = getenv("JSG_GEMM_TILE");
   if (!e) return p;
-  p.on = true;
+  p.family = *e == 'q' || (*e == 's' && e[1] != 'm') ? *e : 't';
   const struct { const char *name; int bm, bn; } names[] = {{"small", 64, epi == GEPI_SWIGLU ? 128 : 64}, {"tall", 128, 128}, {"wide", 256, 128}, {"db", 256, 256}};
   for (const auto &n : names)
     if (!strcmp(e, n.name)) { p.bm = n.bm; p.bn = n.bn; return p; }
-  p.codes = *e == 'q';
-  sscanf(e + (p.codes ? 1 : 0), "%dx%d/%d", &p.bm, &p.bn, &p.split);
+  sscanf(e + (p.family != 't'), "%dx%d/%d", &p.bm, &p.bn, &p.split);
   return p;
 }
 static Choice choose_tile(const TileShape *shapes, int n_shapes, int epi, int M, int weight_rows, int K, size_t ws_limit, const Pin &pin) {
@@ -819,11 +744,11 @@ static Choice choose_tile(const TileShape *shapes, int n_shapes, int epi, int M,
   Choice best = {0.0f, -1, 1};
   for (int s = 0; s < n_shapes; s++) {
     const TileShape &c = shapes[s];
-    if (weight_rows % c.bn || K % c.bk || (epi == GEPI_SWIGLU && c.bn < 128)) continue;
+    if (weight_rows % c.bn || K % c.bk || (epi == GEPI_SWIGLU && (c.bn < 128 || c.bm < 64))) continue;
     const int tiles = ((M + c.bm - 1) / c.bm) * (weight_rows / c.bn), nk = K / c.bk;
     for (int d = 1; d <= 16; d++) {
       if (d > 1 && (c.bm * c.bn == 65536 || nk < d || tiles > TILE_COUNTERS || (size_t)tiles * d * c.bm * c.bn * 4 > ws_limit)) break;
-      if (d > 1 && (pin.on ? d > pin.split : nk / d * c.bk < 256 || tiles * d > 2 * cus)) break;
+      if (d > 1 && (pin.family ? d > pin.split : nk / d * c.bk < 256 || tiles * d > 2 * cus)) break;
       const int blocks = tiles * d, steps = (nk + d - 1) / d;
       const float fill = (float)blocks / cus;
       float us = 4.5f + (fill <= 1.0f ? (c.step + c.fill * fill) * steps + c.end : ((blocks + cus - 1) / cus) * (c.round_step * steps + c.end));
@@ -871,90 +796,67 @@ template <int EPI> static int gemm_tiled_epi(int kind, const GemmArgs &a, int pr
   static int *counters = nullptr;
   if (!counters) JSG_HIP(hipGetSymbolAddress((void **)&counters, HIP_SYMBOL(tile_counters)));
   t.counters = counters;
-  t.ncols = a.N;
   for (int q = 0; q < 3; q++) { t.b[q] = w[q]; t.s[q] = sc[q]; }
   t.b_end[0] = n[0];
   t.b_end[1] = n[0] + n[1];
 
-  const Pin pin = read_pin(EPI), none, &codes_pin = pin.codes ? pin : none;
+  const Pin pin = read_pin(EPI), none;
+  auto pinned = [&](char family) -> const Pin & { return pin.family == family ? pin : none; };
   const size_t ws_limit = state().capturing ? 0 : SUMS_LIMIT;
-  auto run = [&](const Choice &c, float *ws, auto launch) -> int {
-    JSG_REQUIRE(c.shape >= 0, "jsgrad_hip_gemm: no tile shape for %d columns", t.ncols);
+  const int wrows = a.N * NMAT;
+  auto run = [&](const Choice &c, float *sums, auto launch) -> int {
+    JSG_REQUIRE(c.shape >= 0, "jsgrad_hip_gemm: no tile shape for %d columns", a.N);
     t.split = c.split;
-    t.ws = ws;
+    t.ws = sums;
     return launch(c.shape, t, prof_kind);
   };
   Workspace ws;
-  // all of the output at once, its sums (if it has K parts) in the workspace
-  auto run_whole = [&](const TileShape *shapes, int n_shapes, Choice c, const Pin &pinned, auto launch) -> int {
-    const size_t sums = sums_bytes(shapes, c, a.M, a.N * NMAT);
-    if (sums && !ws.get(sums)) c = choose_tile(shapes, n_shapes, EPI, a.M, a.N * NMAT, a.K, 0, pinned);
+  // the K parts' sums, if there are parts, in the workspace
+  auto run_whole = [&](const TileShape *shapes, int n_shapes, Choice c, const Pin &p, auto launch) -> int {
+    const size_t sums = sums_bytes(shapes, c, a.M, wrows);
+    if (sums && !ws.get(sums)) c = choose_tile(shapes, n_shapes, EPI, a.M, wrows, a.K, 0, p);
     return run(c, (float *)ws.p, launch);
   };
 
-  Choice f = choose_tile(TILE_SHAPES, N_SHAPES, EPI, a.M, a.N * NMAT, a.K, ws_limit, pin);
-  if (kind == JSGRAD_W_F16) return run_whole(TILE_SHAPES, N_SHAPES, f, pin, launch_shape<EPI>);
+  Choice f = choose_tile(TILE_SHAPES, N_SHAPES, EPI, a.M, wrows, a.K, ws_limit, pinned('t'));
+  if (kind == JSGRAD_W_F16) return run_whole(TILE_SHAPES, N_SHAPES, f, pinned('t'), launch_shape<EPI>);
 
-  // Quantised: dequantised as read, or realised first, whichever is estimated to be done first.  Where there is no memory for the
-  // realised matrix (a capture, a full device) the codes are read in place whenever a shape takes them.  Realising: codes in and halves
-  // out at 8.8 TB/s, slower where the last level cache cannot hold them until they are read (w1|w3 of the 8B shape, 352 MB: 60 us), a
-  // launch per matrix.  On the matrices of the 8B model int8 is realised from 640 to 1800 rows on, nf4 from 320 to 640 (and read in
-  // place again in narrow bands above that, where the fp16 tiles begin another round).
-  const float moved = (float)((double)a.N * NMAT * a.K * (kind == JSGRAD_W_I8 ? 3.0 : 2.5)), big = moved - 150e6f;
-  const float realise_us = moved / 8.8e6f + (big > 0.0f ? big / 17e6f : 0.0f) + 3.2f + 4.5f * (EPI == GEPI_STORE ? 0 : EPI == GEPI_SWIGLU ? 1 : 2);
+  // Quantised: dequantised as read (qtile_kernel), dequantised on the way into LDS (gemm_staged.hip), or realised first, whichever is
+  // estimated to be done first; without memory for the realised matrix (a capture, a full device) one of the first two.  Realising:
+  // codes in and halves out at 8.8 TB/s, slower where the last level cache cannot hold them until they are read (w1|w3 of the 8B
+  // shape, 352 MB: 60 us), a launch per matrix.  On the matrices of the 8B model int8 is realised from 640 to 1800 rows on, nf4 from 320 to 640
+  // (with narrow bands back and forth where a round of blocks ends); the staged kernel comes first in between for w1|w3 and, of the two
+  // that need no memory, from 200 (nf4) or 1400 rows (int8) on.
+  const float moved = (float)((double)wrows * a.K * (kind == JSGRAD_W_I8 ? 3.0 : 2.5)), big = moved - 150e6f;
+  const float realise_us = pin.family == 't' ? 0.0f : moved / 8.8e6f + (big > 0.0f ? big / 17e6f : 0.0f) + 3.2f + 4.5f * (EPI == GEPI_STORE ? 0 : EPI == GEPI_SWIGLU ? 1 : 2);
   const TileShape *qs = kind == JSGRAD_W_I8 ? QTILE_SHAPES_I8 : QTILE_SHAPES_NF4;
-  // qtile_kernel brings scales by direct loads of four bytes; a pointer between two of those (a slice) is read half by half when
-  // the matrix is realised
+  // qtile_kernel brings scales by direct loads of four bytes; a pointer between two of those (a slice) is read half by half elsewhere
   const bool dwords = (((uintptr_t)a.s0 | (uintptr_t)a.s1 | (uintptr_t)a.s2) & 3) == 0;
-  const Choice q = dwords ? choose_tile(qs, N_QSHAPES, EPI, a.M, a.N * NMAT, a.K, ws_limit, codes_pin) : Choice{0.0f, -1, 1};
-  const size_t row = (size_t)a.K * 2;
-  bool in_place = (!pin.on || pin.codes) && q.shape >= 0 && q.us < f.us + realise_us;
-  // Realised into the workspace, with the K parts' sums behind it: all columns at once, or as many at a time as REALISED_LIMIT holds
-  size_t bytes = (size_t)a.N * NMAT * row < REALISED_LIMIT ? (size_t)a.N * NMAT * row : REALISED_LIMIT, sums = 0;
-  if (!in_place) {
-    sums = sums_bytes(TILE_SHAPES, f, a.M, a.N * NMAT);
-    if (!ws.get(bytes + sums)) {
-      sums = 0;
-      in_place = !ws.get(bytes) && !pin.on && q.shape >= 0;
-    }
-  }
-  if (in_place)
-    return kind == JSGRAD_W_I8 ? run_whole(qs, N_QSHAPES, q, codes_pin, launch_qshape<JSGRAD_W_I8, EPI>) : run_whole(qs, N_QSHAPES, q, codes_pin, launch_qshape<JSGRAD_W_NF4, EPI>);
-
-  // ... or, without memory, in the library's own scratch
-  _Float16 *out = (_Float16 *)ws.p;
-  if (!out)
-    if (int rc = gemm_scratch((void **)&out, &bytes)) return rc;
-  const size_t fit = bytes / (NMAT * row);
-  const int step = fit >= (size_t)a.N ? a.N : (int)(fit >= 128 ? fit / 128 * 128 : fit / 64 * 64);   // 64: the narrowest tile
-  if (step == 0) {
-    const dim3 grid((unsigned)state().cu_count * 8), block(256);
-    if (kind == JSGRAD_W_I8) JSG_LAUNCH(prof_kind, (long_rows_kernel<JSGRAD_W_I8, EPI>), grid, block, 0, a);
-    else JSG_LAUNCH(prof_kind, (long_rows_kernel<JSGRAD_W_NF4, EPI>), grid, block, 0, a);
-    return 0;
-  }
-  float *const sums_at = sums ? (float *)((unsigned char *)out + bytes) : nullptr;
-  for (int c0 = 0; c0 < a.N; c0 += step) {
-    const int nc = a.N - c0 < step ? a.N - c0 : step;
-    t.col0 = c0;
-    t.ncols = nc;
-    t.b[0] = out;
-    t.b[1] = t.b[2] = out + (size_t)nc * a.K;
-    t.b_end[0] = t.b_end[1] = nc;
-    if constexpr (EPI == GEPI_SWIGLU) {
-      for (int m = 0; m < 2; m++)
-        if (int rc = realise(kind, w[m], sc[m], c0, nc, a.K, out + (size_t)m * nc * a.K, prof_kind)) return rc;
-    } else {
-      for (int m = 0, base = 0; m < 3; base += n[m++]) {
-        const int lo = c0 > base ? c0 : base, hi = c0 + nc < base + n[m] ? c0 + nc : base + n[m];
-        if (lo < hi)
-          if (int rc = realise(kind, w[m], sc[m], lo - base, hi - lo, a.K, out + (size_t)(lo - c0) * a.K, prof_kind)) return rc;
+  const Choice q = dwords ? choose_tile(qs, N_QSHAPES, EPI, a.M, wrows, a.K, ws_limit, pinned('q')) : Choice{0.0f, -1, 1};
+  const TileShape *ss = kind == JSGRAD_W_I8 ? STAGED_SHAPES_I8 : STAGED_SHAPES_NF4;
+  const Choice st = choose_tile(ss, N_STAGED, EPI, a.M, wrows, a.K, 0, pinned('s'));   // takes every call
+  const bool staged = q.shape < 0 || st.us < q.us;
+  const size_t bytes = (size_t)wrows * a.K * 2;
+  if (f.shape >= 0 && f.us + realise_us < (staged ? st.us : q.us) && bytes <= REALISED_LIMIT) {
+    // into the workspace, with the K parts' sums behind it
+    const size_t sums = sums_bytes(TILE_SHAPES, f, a.M, wrows);
+    if (!ws.get(bytes + sums) && sums && ws.get(bytes)) f = choose_tile(TILE_SHAPES, N_SHAPES, EPI, a.M, wrows, a.K, 0, pinned('t'));
+    if (ws.p) {
+      _Float16 *const out = (_Float16 *)ws.p;
+      const int n_mats = EPI == GEPI_ROPE_KV ? 3 : NMAT;
+      for (int m = 0, base = 0; m < n_mats; m++) {
+        const int rows = EPI == GEPI_ROPE_KV ? n[m] : a.N;
+        if (int rc = realise(kind, w[m], sc[m], rows, a.K, out + (size_t)base * a.K, prof_kind)) return rc;
+        base += rows;
       }
+      t.b[0] = out;
+      t.b[1] = t.b[2] = out + (size_t)a.N * a.K;
+      t.b_end[0] = t.b_end[1] = a.N;
+      return run(f, (float *)((unsigned char *)ws.p + bytes), launch_shape<EPI>);
     }
-    if (nc != a.N || sums_bytes(TILE_SHAPES, f, a.M, a.N * NMAT) > sums) f = choose_tile(TILE_SHAPES, N_SHAPES, EPI, a.M, nc * NMAT, a.K, sums, pin);
-    if (int rc = run(f, sums_at, launch_shape<EPI>)) return rc;
   }
-  return 0;
+  if (staged) return gemm_staged(EPI, kind, ss[st.shape].bm, a, prof_kind);
+  return kind == JSGRAD_W_I8 ? run_whole(qs, N_QSHAPES, q, pinned('q'), launch_qshape<JSGRAD_W_I8, EPI>) : run_whole(qs, N_QSHAPES, q, pinned('q'), launch_qshape<JSGRAD_W_NF4, EPI>);
 }
 
 int gemm_tiled(int epi, int kind, const GemmArgs &a, int prof_kind) {
