@@ -55,3 +55,19 @@ def test_the_largest_probability_of_a_row_is_not_rounded(hip, hd):
     ref = (v[large] + w * v[small]) / (1 + w)
     half_unit = np.spacing(np.abs(ref).astype(np.float16)).astype(np.float64) / 2
     assert np.all(np.abs(to.numpy().astype(np.float64) - ref) <= 1.01 * half_unit + 2.0 ** -16 * np.abs(v[large] - v[small]) + 2.0 ** -20)
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("KV,n_rep,B,S,start", [(3, 1, 3, 130, 5), (3, 3, 5, 37, 70), (1, 5, 2, 131, 0), (2, 6, 3, 9, 200), (7, 7, 1, 61, 3), (1, 16, 3, 17, 64), (5, 33, 1, 6, 1)])
+def test_attn_prefill_any_head_geometry(hip, hd, KV, n_rep, B, S, start):
+    """Row, block and head numbers are divided by reciprocals: numbers of heads, kv heads and tiles that are not powers of two.  Nothing
+    behind the last row is written."""
+    H, ctx = KV * n_rep, start + S + 3
+    rng = np.random.default_rng(H + S)
+    q = rng.standard_normal((B * S, H * hd)).astype(np.float16)
+    ck, cv = (rng.standard_normal((B, ctx, KV, hd)).astype(np.float16) for _ in range(2))
+    tq, tk, tv, to = Tensor(q), Tensor(ck), Tensor(cv), Tensor.full((B * S + 1, H * hd), 5.0, "float16")
+    check(hip.jsgrad_hip_attn_prefill(tq.ptr, tk.ptr, tv.ptr, to.ptr, B, S, start, H, KV, hd, ctx))
+    got = to.numpy()
+    assert np.all(got[B * S] == 5.0)
+    assert np.max(np.abs(got[:B * S].astype(np.float64) - attention_ref(q, ck, cv, B, S, start, H, KV, hd))) < 4e-3
