@@ -698,31 +698,31 @@ template <int KIND, int EPI, int BM, int BN, int ST> static int launch_qtile(con
   return 0;
 }
 
-// The shapes, with the K elements of a step and four times fitted to 684 launches of 33 to 4096 rows over the matrices of the 1B, 3B and
-// 8B models, each under every shape (weights from memory; an estimate is off by 6-10 % r.m.s., nf4 3 %): us of a step of blocks that
-// have a compute unit each, what fill adds to it when every unit has one (they share memory and power), us of a step of a
-// round when there are several, and of a round's end.
+// The shapes, with the K elements of a step and four times: us of a step of blocks that have a compute unit each, what fill adds to it
+// when every unit has one (they share memory and power), us of a step of a round when there are several, and of a round's end.
+// Fitted to 33 to 4096 rows over the matrices of the 1B, 3B and 8B models, each under every shape that could matter, weights in memory
+// and in the last level cache, for the choice rather than for the single time (an estimate is off by 5-10 % r.m.s.).
 struct TileShape { int bm, bn, bk; float step, fill, round_step, end; };
 static const TileShape TILE_SHAPES[] = {
-  {64, 64, 64, 0.25f, 0.02f, 0.21f, 0.0f},     // not for w1|w3 (its tiles come in pairs)
-  {64, 128, 64, 0.29f, 0.08f, 0.39f, 0.0f},
-  {128, 128, 64, 0.37f, 0.13f, 0.54f, 0.3f},
-  {256, 128, 64, 0.58f, 0.28f, 0.90f, 0.8f},
-  {256, 256, 64, 0.95f, 0.43f, 1.50f, 3.2f},
+  {64, 64, 64, 0.19f, 0.03f, 0.22f, 0.0f},     // not for w1|w3 (its tiles come in pairs)
+  {64, 128, 64, 0.27f, 0.064f, 0.37f, 0.0f},
+  {128, 128, 64, 0.38f, 0.13f, 0.63f, 0.3f},
+  {256, 128, 64, 0.55f, 0.32f, 0.85f, 1.0f},
+  {256, 256, 64, 0.82f, 0.39f, 1.3f, 3.0f},
 };
-static const TileShape QTILE_SHAPES_I8[] = {{64, 64, 64, 0.27f, 0.03f, 0.18f, 0.0f}, {64, 128, 64, 0.39f, 0.04f, 0.32f, 0.5f}, {128, 128, 64, 0.56f, 0.08f, 0.51f, 1.2f}};
-static const TileShape QTILE_SHAPES_NF4[] = {{64, 64, 128, 0.57f, 0.03f, 0.45f, 0.3f}, {64, 128, 128, 0.86f, 0.08f, 0.72f, 1.3f}, {128, 128, 128, 1.4f, 0.12f, 1.6f, 2.3f}};
+static const TileShape QTILE_SHAPES_I8[] = {{64, 64, 64, 0.25f, 0.024f, 0.18f, 0.03f}, {64, 128, 64, 0.35f, 0.03f, 0.36f, 0.57f}, {128, 128, 64, 0.52f, 0.087f, 0.50f, 1.2f}};
+static const TileShape QTILE_SHAPES_NF4[] = {{64, 64, 128, 0.51f, 0.062f, 0.43f, 0.3f}, {64, 128, 128, 0.86f, 0.075f, 0.70f, 0.74f}, {128, 128, 128, 1.6f, 0.13f, 1.4f, 3.2f}};
 // gemm_staged.hip; 32x128 not for w1|w3
-static const TileShape STAGED_SHAPES_I8[] = {{32, 128, 64, 0.45f, 0.10f, 0.30f, 0.5f}, {128, 128, 64, 0.77f, 0.09f, 0.60f, 1.2f}, {256, 256, 64, 1.1f, 0.48f, 1.7f, 8.0f}};
-static const TileShape STAGED_SHAPES_NF4[] = {{32, 128, 64, 0.55f, 0.15f, 0.35f, 0.5f}, {128, 128, 64, 0.88f, 0.10f, 0.66f, 0.7f}, {256, 256, 64, 1.5f, 0.34f, 1.95f, 8.4f}};
+static const TileShape STAGED_SHAPES_I8[] = {{32, 128, 64, 0.48f, 0.1f, 0.36f, 0.5f}, {128, 128, 64, 0.88f, 0.09f, 0.61f, 1.2f}, {256, 256, 64, 1.1f, 0.43f, 1.7f, 6.0f}};
+static const TileShape STAGED_SHAPES_NF4[] = {{32, 128, 64, 0.53f, 0.17f, 0.29f, 0.5f}, {128, 128, 64, 0.92f, 0.09f, 0.71f, 0.7f}, {256, 256, 64, 1.4f, 0.29f, 1.9f, 7.8f}};
 constexpr int N_SHAPES = sizeof(TILE_SHAPES) / sizeof(TILE_SHAPES[0]), N_QSHAPES = sizeof(QTILE_SHAPES_I8) / sizeof(QTILE_SHAPES_I8[0]), N_STAGED = sizeof(STAGED_SHAPES_I8) / sizeof(STAGED_SHAPES_I8[0]);
 
-// Which shape and how many K parts: the least of an estimate of the launch's time (4.5 us for start and first tiles; for K parts 2 us
-// and the sums' way through memory).  Over those launches the choice is 1 % slower than the best shape on average, 4 % at the
-// ninth decile.  Examples, us, this choice | others: 371 x 2048 x 8192 128x128 in 5 parts 24.4 | in 3 parts 28.9,
-// 64x64 38.6, 256x128 in 8 parts 34.9; 371 x 2048 x 2048 64x128 in 2 parts 12.4 | in one 14.2, 64x64 12.7; 700 x 28672 x 4096 256x128
-// 182 | 256x256 190, 128x128 216; 2048 x 6144 x 4096 256x256 84 | 256x128 107, 128x128 106; 1200 x 2048 x 2048 128x128 18.4 |
-// 256x128 25.9.
+// Which shape and how many K parts: the least of an estimate of the launch's time (4.5 us for start and first tiles; for K parts 1.7 us
+// and the sums' way through memory).  Over the measured sizes the choice is 0.7 % slower than the best shape on average, 2.5 % at
+// the ninth decile.  Examples, us with weights from memory, this choice | others: 371 x 2048 x 8192 128x128 in 5 parts 26.3 | in 3 parts
+// 32.2, 64x128 in 2 32.9, 256x128 in 7 34.4; 371 x 2048 x 2048 64x64 12.7 | 64x128 in 2 parts 12.4, in one 15.5; 700 x 28672 x 4096
+// 256x128 185 | 256x256 188, 128x128 223; 2048 x 6144 x 4096 256x256 90 | 128x128 111, 256x128 112; int8 codes, 57 x 5120 x 3072 64x64 in
+// 3 parts 11.2 | 64x128 in 5 12.4, 64x64 in 6 12.9.
 struct Choice { float us; int shape, split; };
 // JSG_GEMM_TILE, for tests and measurements: rows x columns of a tile, optionally with K parts, of the fp16 kernels ("128x128",
 // "64x128/3"; quantised weights are then realised), of qtile_kernel ("q64x64/3") or of the staged kernel ("s256x256"); "small", "tall",
@@ -752,7 +752,7 @@ static Choice choose_tile(const TileShape *shapes, int n_shapes, int epi, int M,
       const int blocks = tiles * d, steps = (nk + d - 1) / d;
       const float fill = (float)blocks / cus;
       float us = 4.5f + (fill <= 1.0f ? (c.step + c.fill * fill) * steps + c.end : ((blocks + cus - 1) / cus) * (c.round_step * steps + c.end));
-      if (d > 1) us += 2.0f + (float)d * c.bm * c.bn * 4 / 80e3f * (fill > 1.0f ? fill : 1.0f);
+      if (d > 1) us += 1.7f + (float)d * c.bm * c.bn * 4 / 83e3f * (fill > 1.0f ? fill : 1.0f);
       if (pin.bm == c.bm && pin.bn == c.bn && d == pin.split) us = 0.0f;   // taken
       if (best.shape < 0 || us < best.us) best = {us, s, d};
     }
@@ -823,12 +823,11 @@ template <int EPI> static int gemm_tiled_epi(int kind, const GemmArgs &a, int pr
 
   // Quantised: dequantised as read (qtile_kernel), dequantised on the way into LDS (gemm_staged.hip), or realised first, whichever is
   // estimated to be done first; without memory for the realised matrix (a capture, a full device) one of the first two.  Realising:
-  // codes in and halves out at 8.8 TB/s, slower where the last level cache cannot hold them until they are read (w1|w3 of the 8B
-  // shape, 352 MB: 60 us), a launch per matrix.  On the matrices of the 8B model int8 is realised from 640 to 1800 rows on, nf4 from 320 to 640
-  // (with narrow bands back and forth where a round of blocks ends); the staged kernel comes first in between for w1|w3 and, of the two
-  // that need no memory, from 200 (nf4) or 1400 rows (int8) on.
-  const float moved = (float)((double)wrows * a.K * (kind == JSGRAD_W_I8 ? 3.0 : 2.5)), big = moved - 150e6f;
-  const float realise_us = pin.family == 't' ? 0.0f : moved / 8.8e6f + (big > 0.0f ? big / 17e6f : 0.0f) + 3.2f + 4.5f * (EPI == GEPI_STORE ? 0 : EPI == GEPI_SWIGLU ? 1 : 2);
+  // codes in and halves out at 8.5 TB/s, slower where the last level cache cannot hold them until they are read (w1|w3 of the 8B
+  // shape, 352 MB: 60 us), a launch per matrix.  On the matrices of the 8B model int8 is realised from 1000 to 1700 rows on, nf4 from 320 to
+  // 640 (with narrow bands back and forth where a round of blocks ends); for w1|w3 the staged kernel comes first in between.
+  const float moved = (float)((double)wrows * a.K * (kind == JSGRAD_W_I8 ? 3.0 : 2.5)), big = moved - 120e6f;
+  const float realise_us = pin.family == 't' ? 0.0f : moved / 8.5e6f + (big > 0.0f ? big / 18e6f : 0.0f) + 3.7f + 4.5f * (EPI == GEPI_STORE ? 0 : EPI == GEPI_SWIGLU ? 1 : 2);
   const TileShape *qs = kind == JSGRAD_W_I8 ? QTILE_SHAPES_I8 : QTILE_SHAPES_NF4;
   // qtile_kernel brings scales by direct loads of four bytes; a pointer between two of those (a slice) is read half by half elsewhere
   const bool dwords = (((uintptr_t)a.s0 | (uintptr_t)a.s1 | (uintptr_t)a.s2) & 3) == 0;

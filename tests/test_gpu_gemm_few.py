@@ -33,6 +33,14 @@ def test_few_rows_against_oracle(hip, kind, in_f, rows, out_f):
         assert_close(got[:rows].astype(np.float32), ref, True, f"{kind} {rows}x{out_f}x{in_f}", ulp_at=lin if residual else None)
 
 
+@pytest.mark.parametrize("kind,in_f,rows,out_f", [("float16", k, r, n) for k in (1024, 1536, 2048, 3072, 4096, 6144, 8192) for r, n in ((3, 8320), (2, 11392))] +
+                         [("int8", 2048, 3, 8320), ("int8", 3072, 9, 8320), ("int8", 4096, 3, 8320), ("int8", 2048, 2, 11392), ("int8", 3072, 2, 11392)])
+def test_few_rows_with_several_rounds_of_tiles(hip, kind, in_f, rows, out_f):
+    """Outputs of 8192 and more give a block two tiles and more, whose steps follow each other through its ring (and x is waited for in
+    front of them): two rounds and halves behind them, two rounds and a ragged third."""
+    test_few_rows_against_oracle(hip, kind, in_f, rows, out_f)
+
+
 @pytest.mark.parametrize("kind,dim,hidden", [("float16", 2048, 4224), ("float16", 1536, 128), ("int8", 3072, 4224), ("int8", 4096, 2176)])
 def test_few_rows_ffn_gate(hip, kind, dim, hidden):
     ffn_gate(hip, kind, 9, dim, hidden)

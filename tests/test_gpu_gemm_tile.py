@@ -109,7 +109,7 @@ def test_every_tile_under_every_epilogue(hip, monkeypatch, kind, tile):
 @pytest.mark.parametrize("kind,rows,dim,hidden", [("int8", 57, 3072, 1024), ("nf4", 57, 3072, 1024), ("float16", 371, 2048, 1024), ("int8", 371, 2048, 1024)])
 def test_tiles_as_chosen_under_the_fused_epilogues(hip, kind, rows, dim, hidden):
     """K parts under SwiGLU (57 rows: codes 64x128 in 6 or 8 parts; 371 rows: fp16 and codes 64x128 in 2) and under the rotary epilogue
-    (64x64 in 8)."""
+    (64x64 in 4 or 8)."""
     rows_tests.test_gemm_ffn_gate(hip, kind, rows, dim, hidden)
     rows_tests.test_gemm_qkv_rope_writes_queries_and_cache(hip, kind, 128, 1, 57, dim)
 
