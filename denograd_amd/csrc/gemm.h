@@ -67,8 +67,8 @@ __device__ __forceinline__ void dma4(i4_t rs, uint32_t voff, uint32_t soff, uint
 int gemm_few(int epi, int kind, const GemmArgs &a, int prof_kind, bool *taken);
 // gemm_tile.hip: the tiled kernels, any number of rows; epi: GEPI_*
 int gemm_tiled(int epi, int kind, const GemmArgs &a, int prof_kind);
-// gemm_staged.hip: quantised weights dequantised on their way into LDS, any number of rows; bm: 32 (32x128 tiles, not for w1|w3), 128
-// (128x128) or 256 (256x256; the output, w1 and w3 counted together, is then a multiple of 256)
-int gemm_staged(int epi, int kind, int bm, const GemmArgs &a, int prof_kind);
+// gemm_staged.hip: quantised weights dequantised on their way into LDS, any number of rows; tiles of bm x bn: 32x128 (not for w1|w3),
+// 128x128, 256x128 or 256x256 (the output, w1 and w3 counted together, is then a multiple of 256)
+int gemm_staged(int epi, int kind, int bm, int bn, const GemmArgs &a, int prof_kind);
 
 }  // namespace jsg

@@ -1,5 +1,5 @@
 // Several-row linear layers, few rows: y[M][N] = x[M][K] . W[N][K]^T for 1 to 32 rows of fp16 activations (batched decode), fp32
-// accumulate, fp16 out, and the entry points for any number of rows (more rows: gemm_tile.hip; fp16 and short int8 matrices with
+// accumulate, fp16 out, and the entry points for any number of rows (more rows: gemm_tile.hip and gemm_staged.hip; fp16 and short int8 matrices with
 // at most 16 rows: gemm_few.hip).
 //
 // What the reference computes (/root/reference/jsgrad/tensor.ts:2593-2605 `dot`, :3800 `linear`; Int8Linear.call

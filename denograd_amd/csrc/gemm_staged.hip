@@ -11,8 +11,8 @@
 // v_mfma_f32_32x32x16_f16.  Both operands are K-contiguous in memory, so a lane's 8-element operand fragment is one 128-bit LDS read.
 // LDS rows are padded by 8 halves, which spreads the 32 rows of a fragment read over all banks.
 //
-// Two loop shapes.  128x128, or 32x128 for few rows, out of one LDS buffer (two barriers per K tile, the next tile prefetched into
-// registers) with three blocks per CU, whose wavefronts cover each other's barriers and conversions.  256x256 out of two, one block per CU (one
+// Two loop shapes.  128x128, 256x128, or 32x128 for few rows, out of one LDS buffer (two barriers per K tile, the next tile prefetched
+// into registers) with two or three blocks per CU, whose wavefronts cover each other's barriers and conversions.  256x256 out of two, one block per CU (one
 // wavefront per SIMD): one barrier per K tile, and the instruction order of a K tile is spelled out so that fragment reads,
 // conversion, LDS writes and the requests of the tile after next sit between the matrix instructions.
 #include <type_traits>
@@ -373,19 +373,20 @@ template <int KIND, int EPI, int WGM, int WGN, int TM, int TN, bool DB = false> 
   JSG_LAUNCH(prof_kind, (staged_kernel<KIND, EPI, WGM, WGN, TM, TN, DB>), dim3(tiles), dim3(STAGED_THREADS), lds, a);
   return 0;
 }
-template <int KIND, int EPI> static int gemm_staged_as(int bm, const GemmArgs &a, int prof_kind) {
-  if (bm == 256) return launch_staged<KIND, EPI, 2, 2, 4, 4, true>(a, prof_kind);
+template <int KIND, int EPI> static int gemm_staged_as(int bm, int bn, const GemmArgs &a, int prof_kind) {
+  if (bn == 256) return launch_staged<KIND, EPI, 2, 2, 4, 4, true>(a, prof_kind);
+  if (bm == 256) return launch_staged<KIND, EPI, 2, 2, 4, 2>(a, prof_kind);
   if constexpr (EPI != GEPI_SWIGLU)
     if (bm == 32) return launch_staged<KIND, EPI, 1, 4, 1, 1>(a, prof_kind);
   return launch_staged<KIND, EPI, 2, 2, 2, 2>(a, prof_kind);
 }
-template <int KIND> static int gemm_staged_kind(int epi, int bm, const GemmArgs &a, int prof_kind) {
-  if (epi == GEPI_STORE) return gemm_staged_as<KIND, GEPI_STORE>(bm, a, prof_kind);
-  if (epi == GEPI_ROPE_KV) return gemm_staged_as<KIND, GEPI_ROPE_KV>(bm, a, prof_kind);
-  return gemm_staged_as<KIND, GEPI_SWIGLU>(bm, a, prof_kind);
+template <int KIND> static int gemm_staged_kind(int epi, int bm, int bn, const GemmArgs &a, int prof_kind) {
+  if (epi == GEPI_STORE) return gemm_staged_as<KIND, GEPI_STORE>(bm, bn, a, prof_kind);
+  if (epi == GEPI_ROPE_KV) return gemm_staged_as<KIND, GEPI_ROPE_KV>(bm, bn, a, prof_kind);
+  return gemm_staged_as<KIND, GEPI_SWIGLU>(bm, bn, a, prof_kind);
 }
-int gemm_staged(int epi, int kind, int bm, const GemmArgs &a, int prof_kind) {
-  return kind == JSGRAD_W_I8 ? gemm_staged_kind<JSGRAD_W_I8>(epi, bm, a, prof_kind) : gemm_staged_kind<JSGRAD_W_NF4>(epi, bm, a, prof_kind);
+int gemm_staged(int epi, int kind, int bm, int bn, const GemmArgs &a, int prof_kind) {
+  return kind == JSGRAD_W_I8 ? gemm_staged_kind<JSGRAD_W_I8>(epi, bm, bn, a, prof_kind) : gemm_staged_kind<JSGRAD_W_NF4>(epi, bm, bn, a, prof_kind);
 }
 
 }  // namespace jsg

@@ -5,9 +5,10 @@
 // /root/reference/jsgrad/models/llama3.ts:35; NF4Linear.call :91-97): with more than one input row the weight operand is
 // expanded over the rows, so a quantised weight is first realised in fp16, W = RN16(code * scale), and the products of
 // two fp16 values are then summed in float.  So it is here.  With many rows `realise_kernel` writes that matrix once per call
-// (int8 8B w1|w3: 117 MB in, 235 MB out, ~75 us, where the product takes 5.4 ms at 32768 rows) and the fp16 kernels serve the
+// (int8 8B w1|w3: 117 MB in, 235 MB out, ~60 us, where the product takes 5.4 ms at 32768 rows) and the fp16 kernels serve the
 // three formats.  With some hundred rows or fewer the writing and reading of the realised matrix would be most of the
-// time; `qtile_kernel` keeps the codes in LDS and dequantises a fragment as it is read.
+// time; `qtile_kernel` keeps the codes in LDS and dequantises a fragment as it is read.  In between, and without memory, the kernel of
+// gemm_staged.hip has sizes where it comes first.
 //
 // Both operands are K-contiguous in memory (x rows, W rows), so an operand fragment of v_mfma_f32_16x16x32_f16 (8 K elements
 // of one row per lane) is one 16-byte LDS read.  The 16x16 instruction is used because the chip is power-limited under this
@@ -713,8 +714,8 @@ static const TileShape TILE_SHAPES[] = {
 static const TileShape QTILE_SHAPES_I8[] = {{64, 64, 64, 0.25f, 0.024f, 0.18f, 0.03f}, {64, 128, 64, 0.35f, 0.03f, 0.36f, 0.57f}, {128, 128, 64, 0.52f, 0.087f, 0.50f, 1.2f}};
 static const TileShape QTILE_SHAPES_NF4[] = {{64, 64, 128, 0.51f, 0.062f, 0.43f, 0.3f}, {64, 128, 128, 0.86f, 0.075f, 0.70f, 0.74f}, {128, 128, 128, 1.6f, 0.13f, 1.4f, 3.2f}};
 // gemm_staged.hip; 32x128 not for w1|w3
-static const TileShape STAGED_SHAPES_I8[] = {{32, 128, 64, 0.48f, 0.1f, 0.36f, 0.5f}, {128, 128, 64, 0.88f, 0.09f, 0.61f, 1.2f}, {256, 256, 64, 1.1f, 0.43f, 1.7f, 6.0f}};
-static const TileShape STAGED_SHAPES_NF4[] = {{32, 128, 64, 0.53f, 0.17f, 0.29f, 0.5f}, {128, 128, 64, 0.92f, 0.09f, 0.71f, 0.7f}, {256, 256, 64, 1.4f, 0.29f, 1.9f, 7.8f}};
+static const TileShape STAGED_SHAPES_I8[] = {{32, 128, 64, 0.48f, 0.1f, 0.36f, 0.5f}, {128, 128, 64, 0.88f, 0.09f, 0.61f, 1.2f}, {256, 128, 64, 1.13f, 0.16f, 1.04f, 2.5f}, {256, 256, 64, 1.1f, 0.43f, 1.7f, 6.0f}};
+static const TileShape STAGED_SHAPES_NF4[] = {{32, 128, 64, 0.53f, 0.17f, 0.29f, 0.5f}, {128, 128, 64, 0.92f, 0.09f, 0.71f, 0.7f}, {256, 128, 64, 1.2f, 0.17f, 1.03f, 2.0f}, {256, 256, 64, 1.4f, 0.29f, 1.9f, 7.8f}};
 constexpr int N_SHAPES = sizeof(TILE_SHAPES) / sizeof(TILE_SHAPES[0]), N_QSHAPES = sizeof(QTILE_SHAPES_I8) / sizeof(QTILE_SHAPES_I8[0]), N_STAGED = sizeof(STAGED_SHAPES_I8) / sizeof(STAGED_SHAPES_I8[0]);
 
 // Which shape and how many K parts: the least of an estimate of the launch's time (4.5 us for start and first tiles; for K parts 1.7 us
@@ -854,7 +855,7 @@ template <int EPI> static int gemm_tiled_epi(int kind, const GemmArgs &a, int pr
       return run(f, (float *)((unsigned char *)ws.p + bytes), launch_shape<EPI>);
     }
   }
-  if (staged) return gemm_staged(EPI, kind, ss[st.shape].bm, a, prof_kind);
+  if (staged) return gemm_staged(EPI, kind, ss[st.shape].bm, ss[st.shape].bn, a, prof_kind);
   return kind == JSGRAD_W_I8 ? run_whole(qs, N_QSHAPES, q, pinned('q'), launch_qshape<JSGRAD_W_I8, EPI>) : run_whole(qs, N_QSHAPES, q, pinned('q'), launch_qshape<JSGRAD_W_NF4, EPI>);
 }
 

@@ -207,7 +207,9 @@ int jsgrad_hip_embed_rows(int kind, const void *table, const void *scale, const 
 int jsgrad_hip_rmsnorm_rows(const void *x, const void *weight, void *y, int rows, int dim, float eps);
 
 /* Linear.call / Int8Linear.call / NF4Linear.call (nn/index.ts:411, llama3.ts:35,91-97) on x[rows][in_f]:
- * y[rows][out_f] = x . W^T (+ residual[rows][out_f] added after the cast, models/llama.ts:125-126). */
+ * y[rows][out_f] = x . W^T (+ residual[rows][out_f] added after the cast, models/llama.ts:125-126).
+ * This call, the next two and jsgrad_hip_attn_prefill sum in float, in an order that a call repeats but that depends on the number of
+ * rows and on whether the workspace is to be had (not in a graph capture): a row may differ by a rounding of the result. */
 int jsgrad_hip_gemm(int kind, const void *w, const void *scale, int out_f, int in_f, const void *x, int rows, void *y, const void *residual);
 
 /* wq/wk/wv + apply_rotary_emb + KV-cache assign (models/llama.ts:61-87) for rows = B * seq_len positions starting

@@ -90,7 +90,7 @@ def test_scales_between_two_dwords(hip, monkeypatch, kind):
 
 
 TILES = ["64x64", "64x64/3", "64x128", "64x128/3", "128x128", "128x128/2", "256x128", "256x128/5", "256x256"]
-CODE_TILES = ["q64x64", "q64x64/3", "q64x128", "q64x128/2", "q128x128", "q128x128/3", "s32x128", "s128x128", "s256x256"]
+CODE_TILES = ["q64x64", "q64x64/3", "q64x128", "q64x128/2", "q128x128", "q128x128/3", "s32x128", "s128x128", "s256x128", "s256x256"]
 
 
 @pytest.mark.parametrize("kind,tile", [(k, t) for k in ("float16", "int8") for t in TILES] + [(k, t) for k in ("int8", "nf4") for t in CODE_TILES])
