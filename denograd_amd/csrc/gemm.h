@@ -1,5 +1,9 @@
 // What the several-row kernels share: gemm.hip (few rows), gemm_tile.hip and gemm_staged.hip (more than that), prefill.hip (causal attention).
 #pragma once
+#include <stdlib.h>
+#include <string.h>
+#include <unistd.h>
+
 #include "common.h"
 
 namespace jsg {
@@ -20,6 +24,7 @@ struct GemmArgs {
   const _Float16 *rope_table;         // [2*max_context][hd/2][2]
   _Float16 *cache_k, *cache_v;        // [B][max_context][n1]
   int seq_len, start_pos, head_dim, max_context;
+  bool pins;                          // some variable of the environment begins with JSG_: a test may want a certain kernel or tile
 };
 
 __device__ __forceinline__ uint32_t pk_mul_h2(uint32_t a, h2_t s) {
@@ -63,8 +68,18 @@ __device__ __forceinline__ void dma4(i4_t rs, uint32_t voff, uint32_t soff, uint
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rs), "s"(soff) : "memory");
 }
 
+// What a test asks for, or null.  Looking a variable up costs a walk through the environment, so a call makes one walk for all of them.
+inline bool any_pins() {
+  for (char **e = environ; *e; e++)
+    if (!strncmp(*e, "JSG_", 4)) return true;
+  return false;
+}
+inline const char *pin_env(const GemmArgs &a, const char *name) { return a.pins ? getenv(name) : nullptr; }
+
 // gemm_few.hip: at most 16 rows, weights streamed past x in registers; *taken false: not for this call, nothing launched
 int gemm_few(int epi, int kind, const GemmArgs &a, int prof_kind, bool *taken);
+// gemm_group.hip: at most 32 rows, wherever the weight-streaming kernels of gemm.hip are slower; *taken as above
+int gemm_group(int epi, int kind, const GemmArgs &a, int prof_kind, bool *taken);
 // gemm_tile.hip: the tiled kernels, any number of rows; epi: GEPI_*
 int gemm_tiled(int epi, int kind, const GemmArgs &a, int prof_kind);
 // gemm_staged.hip: quantised weights dequantised on their way into LDS, any number of rows; tiles of bm x bn: 32x128 (not for w1|w3),

@@ -1,14 +1,12 @@
 // Several-row linear layers, few rows: y[M][N] = x[M][K] . W[N][K]^T for 1 to 32 rows of fp16 activations (batched decode), fp32
-// accumulate, fp16 out, and the entry points for any number of rows (more rows: gemm_tile.hip and gemm_staged.hip; fp16 and short int8 matrices with
+// accumulate, fp16 out, and the entry points for any number of rows (more rows: gemm_tile.hip and gemm_staged.hip; wide or long matrices with up to
+// 32 rows: gemm_group.hip; fp16 and short int8 matrices with
 // at most 16 rows: gemm_few.hip).
 //
 // What the reference computes (/root/reference/jsgrad/tensor.ts:2593-2605 `dot`, :3800 `linear`; Int8Linear.call
 // /root/reference/jsgrad/models/llama3.ts:35; NF4Linear.call :91-97): with more than one input row the weight operand is
 // expanded over the rows, so a quantised weight is first realised in fp16, W = RN16(code * scale), and the products of
 // two fp16 values are then summed in float.  v_pk_mul_f16 of the exact fp16 code by the fp16 scale is that single rounding.
-#include <stdlib.h>
-#include <string.h>
-
 #include <type_traits>
 
 #include "gemm.h"
@@ -594,7 +592,7 @@ template <int EPI, int TPW> static int launch_stream(const GemmArgs &a, int prof
   if (groups > SG_MAX_GROUPS) return 0;
   int best = 0;
   double best_score = 0.0;
-  const char *pin = getenv("JSG_SG_SPLITK");
+  const char *pin = pin_env(a, "JSG_SG_SPLITK");
   for (int d = 1; d <= nchunks && d <= 16; d++) {
     if (nchunks % d) continue;
     const int units = groups * d;
@@ -632,10 +630,10 @@ template <int EPI, int TPW> static int launch_stream(const GemmArgs &a, int prof
 // measured faster than two on every shape of the 8B model (lm_head 97 us against 105), although x is read twice as often.
 template <int EPI> static int dispatch_stream(const GemmArgs &a, int prof_kind, bool *taken) {
   *taken = false;
-  if (getenv("JSG_GEMM_NO_STREAM")) return 0;
+  if (pin_env(a, "JSG_GEMM_NO_STREAM")) return 0;
   if constexpr (EPI == GEPI_SWIGLU) return launch_stream<EPI, 2>(a, prof_kind, taken);
   else {
-    const char *pin = getenv("JSG_SG_TPW");                  // "1" or "2": tests run both
+    const char *pin = pin_env(a, "JSG_SG_TPW");                  // "1" or "2": tests run both
     if (!(pin && pin[0] == '2')) {
       const int rc = launch_stream<EPI, 1>(a, prof_kind, taken);
       if (*taken || rc) return rc;
@@ -648,9 +646,9 @@ template <int EPI> static int dispatch_stream(const GemmArgs &a, int prof_kind, 
 // rows per block that is half as often.  Measured on the lm_head (8016 tiles) the two-tile shape is no faster and moves
 // more HBM bytes (1.5x the weights against 1.24x), so it is only taken when pinned.
 template <int KIND, int EPI> static int dispatch_skinny(const GemmArgs &a, int prof_kind, bool *taken) {
-  *taken = a.M <= 32 && a.K % SkFmt<KIND>::KC == 0 && a.K / SkFmt<KIND>::KC >= 2 && a.N % 16 == 0 && !getenv("JSG_GEMM_NO_SKINNY");
+  *taken = a.M <= 32 && a.K % SkFmt<KIND>::KC == 0 && a.K / SkFmt<KIND>::KC >= 2 && a.N % 16 == 0 && !pin_env(a, "JSG_GEMM_NO_SKINNY");
   if (!*taken) return 0;
-  const char *pin = getenv("JSG_GEMM_SKINNY_TILES");     // "1" or "2": tests run small matrices through both
+  const char *pin = pin_env(a, "JSG_GEMM_SKINNY_TILES");     // "1" or "2": tests run small matrices through both
   const bool two = a.N % 32 == 0 && pin && pin[0] == '2';
   if (a.M <= 16) return two ? launch_skinny<KIND, EPI, 1, 2>(a, prof_kind) : launch_skinny<KIND, EPI, 1, 1>(a, prof_kind);
   return two ? launch_skinny<KIND, EPI, 2, 2>(a, prof_kind) : launch_skinny<KIND, EPI, 2, 1>(a, prof_kind);
@@ -658,13 +656,18 @@ template <int KIND, int EPI> static int dispatch_skinny(const GemmArgs &a, int p
 
 template <int EPI> static int dispatch_gemm(int kind, const GemmArgs &a, int prof_kind) {
   bool taken = false;
+  if (const char *e = pin_env(a, "JSG_GEMM_TILE"); e && *e == 'g') {   // tests
+    const int rc = gemm_group(EPI, kind, a, prof_kind, &taken);
+    if (taken || rc) return rc;
+  }
   { const int rc = gemm_few(EPI, kind, a, prof_kind, &taken); if (taken || rc) return rc; }
-  if (kind == JSGRAD_W_F16) { const int rc = dispatch_skinny<JSGRAD_W_F16, EPI>(a, prof_kind, &taken); if (taken) return rc; }
   // int8, at most 16 rows: the LDS-streamed kernel, except for matrices so small that its K parts cost more than they bring
   // (wo of the 8B shape, 16.8 MB: 9.7 us against 8.5 us with the direct-operand kernel; wq|wk|wv, 25 MB: 12.3 against 13.5)
   static const size_t stream_min = getenv("JSG_SG_MIN_BYTES") ? (size_t)atoll(getenv("JSG_SG_MIN_BYTES")) : (size_t)20 << 20;
   const bool small_matrix = EPI == GEPI_STORE && (size_t)a.N * (size_t)a.K < stream_min;
   if (kind == JSGRAD_W_I8 && !small_matrix) { const int rc = dispatch_stream<EPI>(a, prof_kind, &taken); if (taken || rc) return rc; }
+  { const int rc = gemm_group(EPI, kind, a, prof_kind, &taken); if (taken || rc) return rc; }
+  if (kind == JSGRAD_W_F16) { const int rc = dispatch_skinny<JSGRAD_W_F16, EPI>(a, prof_kind, &taken); if (taken) return rc; }
   if (kind == JSGRAD_W_I8) { const int rc = dispatch_skinny<JSGRAD_W_I8, EPI>(a, prof_kind, &taken); if (taken) return rc; }
   if (kind == JSGRAD_W_NF4) { const int rc = dispatch_skinny<JSGRAD_W_NF4, EPI>(a, prof_kind, &taken); if (taken) return rc; }
   return gemm_tiled(EPI, kind, a, prof_kind);
@@ -697,6 +700,7 @@ int jsgrad_hip_gemm(int kind, const void *w, const void *scale, int out_f, int i
   JSG_REQUIRE(out_f > 0 && out_f % GEMM_N_ALIGN == 0, "jsgrad_hip_gemm: out_features %d must be a positive multiple of %d", out_f, GEMM_N_ALIGN);
   JSG_REQUIRE(aligned16(w) && aligned16(x) && aligned16(y) && aligned16(residual), "jsgrad_hip_gemm: w, x, y and residual must be 16-byte aligned");
   GemmArgs a = {};
+  a.pins = any_pins();
   a.w0 = w; a.s0 = (const _Float16 *)scale; a.n0 = out_f;
   a.M = rows; a.N = out_f; a.K = in_f;
   a.x = (const _Float16 *)x; a.y = (_Float16 *)y; a.residual = (const _Float16 *)residual;
@@ -720,6 +724,7 @@ int jsgrad_hip_gemm_qkv_rope(int kind, const void *wq, const void *sq, const voi
   JSG_REQUIRE(start_pos >= 0 && start_pos + seq_len <= max_context, "jsgrad_hip_gemm_qkv_rope: positions [%d, %d) outside the cache of %d", start_pos,
               start_pos + seq_len, max_context);
   GemmArgs a = {};
+  a.pins = any_pins();
   a.w0 = wq; a.w1 = wk; a.w2 = wv;
   a.s0 = (const _Float16 *)sq; a.s1 = (const _Float16 *)sk; a.s2 = (const _Float16 *)sv;
   a.n0 = nq; a.n1 = nkv; a.n2 = nkv;
@@ -739,6 +744,7 @@ int jsgrad_hip_gemm_ffn_gate(int kind, const void *w1, const void *s1, const voi
   JSG_REQUIRE(hidden > 0 && hidden % GEMM_N_ALIGN == 0, "jsgrad_hip_gemm_ffn_gate: hidden_dim %d must be a positive multiple of %d", hidden, GEMM_N_ALIGN);
   JSG_REQUIRE(aligned16(w1) && aligned16(w3) && aligned16(x) && aligned16(y), "jsgrad_hip_gemm_ffn_gate: w1, w3, x and g must be 16-byte aligned");
   GemmArgs a = {};
+  a.pins = any_pins();
   a.w0 = w1; a.w1 = w3; a.s0 = (const _Float16 *)s1; a.s1 = (const _Float16 *)s3;
   a.n0 = hidden; a.n1 = hidden;
   a.M = rows; a.N = hidden; a.K = dim;

@@ -10,8 +10,6 @@
 // added through LDS in wavefront order.
 // Tiles that are left after whole rounds over the compute units are dealt as halves of eight rows where that is enough for
 // everybody (w1|w3 of 14336 rows: 896 tiles on 256 units are 3.5 rounds instead of 4).
-#include <stdlib.h>
-
 #include "gemm.h"
 
 namespace jsg {
@@ -238,9 +236,12 @@ int gemm_few(int epi, int kind, const GemmArgs &a, int prof_kind, bool *taken) {
   // 16384 x 3072 13.5 / 13.7 / 13.7 | 13.5 / 14.1 / 15.0, 28672 x 4096 26.6 / 26.8 / 27.2 | 28.2 / 28.7 / 30.3.
   // fp16 is the faster here at every size measured: 2048 x 2048 6.2 / 6.3 / 6.3 | 4.5 / 4.5 / 5.1, 2048 x 8192 14.1 / 14.9 / 15.9 |
   // 8.8 / 9.5 / 12.4, 16384 x 2048 23.6 / 23.7 / 24.4 | 16.3 / 17.2 / 18.2, 128256 x 2048 147 / 153 / 162 | 88 / 92 / 94 (6.0 TB/s).
+  // fp16 rows of 16 KiB behind more than 8 rows of x go to gemm_group.hip, which reads x from LDS: 2048 x 8192, 16 rows 12.8 | 10.9 there, 3072 x 8192
+  // 15.5 | 12.8 (8 rows 9.8 | 10.7, 12.6 | 12.6).
+  if (kind == JSGRAD_W_F16 && a.M > 8 && a.K > 4096) return 0;
   const size_t codes = (size_t)a.N * (epi == GEPI_SWIGLU ? 2 : 1) * a.K;
   if (kind == JSGRAD_W_I8 && (codes > (size_t)36 << 20 || (a.M > 8 && a.K > 3072))) return 0;
-  if (getenv("JSG_GEMM_NO_SKINNY") || getenv("JSG_GEMM_SKINNY_TILES") || getenv("JSG_SG_TPW")) return 0;   // tests that want one of the other kernels
+  if (pin_env(a, "JSG_GEMM_NO_SKINNY") || pin_env(a, "JSG_GEMM_SKINNY_TILES") || pin_env(a, "JSG_SG_TPW")) return 0;   // tests that want one of the other kernels
   if (epi == GEPI_STORE) return gemm_few_epi<GEPI_STORE>(kind, a, prof_kind, taken);
   if (epi == GEPI_ROPE_KV) return gemm_few_epi<GEPI_ROPE_KV>(kind, a, prof_kind, taken);
   return gemm_few_epi<GEPI_SWIGLU>(kind, a, prof_kind, taken);

@@ -21,76 +21,11 @@
 //
 // Eight wavefronts, two per SIMD, as two groups that take turns (half a phase apart, a barrier per turn): while one group's
 // matrix instructions run, the other reads its next fragments and asks for tiles further on.
-#include <stdlib.h>
-#include <string.h>
+#include <algorithm>
 
-#include "gemm.h"
+#include "gemm_tile.h"
 
 namespace jsg {
-
-constexpr int TILE_BK = 64;
-constexpr int TILE_THREADS = 512;
-
-struct TileArgs {
-  GemmArgs g;                          // output side: y, residual, rope, cache, M, N, K
-  const void *b[3];                    // weight rows (fp16, or codes), up to three matrices on top of each other
-  const _Float16 *s[3];                // codes: their scales
-  int b_end[2];                        // ends of the first two (SWIGLU: b[0] is w1, b[1] is w3, row for row)
-  int split;                           // K parts
-  float *ws;                           // split > 1: [tile][part][BM * BN] floats
-  int *counters;                       // split > 1: one per tile, zero, and zero again afterwards
-};
-
-template <int N> __device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
-__device__ __forceinline__ void turn_barrier() {
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("s_barrier" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-}
-// ... after this wavefront's LDS reads have arrived
-__device__ __forceinline__ void turn_barrier_lds() {
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-}
-
-// Block id -> tile (and K part): blocks are dealt to the eight XCDs round-robin, so ids are first made contiguous per XCD; K
-// parts of a tile are neighbours, then GROUP row tiles share each column tile, so that the blocks resident on one XCD share
-// operand tiles in its L2.  (GROUP 2 / 4 / 8 / 16 at 32768 x 4096 x 14336: 1453 / 1451 / 1413 / 1334 TFLOP/s, at
-// 32768 x 28672 x 4096: 1392 / 1422 / 1440 / 1318.)
-struct TileId { int tile, part, m0, col; };
-template <int BM, int CW> __device__ __forceinline__ TileId tile_id(const TileArgs &t) {
-  constexpr int GROUP = 4;
-  const int tiles_m = (t.g.M + BM - 1) / BM, tiles_n = t.g.N / CW, nblocks = tiles_m * tiles_n * t.split;
-  int bid = blockIdx.x;
-  const int per = nblocks / 8;
-  if (bid < per * 8) bid = (bid & 7) * per + (bid >> 3);
-  TileId r;
-  r.part = bid % t.split;
-  r.tile = bid / t.split;
-  const int in_group = GROUP * tiles_n, first_m = (r.tile / in_group) * GROUP, gsz = min(tiles_m - first_m, GROUP);
-  r.m0 = (first_m + (r.tile % in_group) % gsz) * BM;
-  r.col = ((r.tile % in_group) / gsz) * CW;
-  return r;
-}
-
-// Where row r of a weight tile of BN rows lies: the matrix and its row.  Boundaries are multiples of 64, so the 8 or 16 rows of a
-// load, or of a fragment, never straddle two matrices.
-struct WeightRow { int mat, row; };
-template <int EPI, int BN> __device__ __forceinline__ WeightRow weight_row(const TileArgs &t, int col, int r) {
-  if constexpr (EPI == GEPI_SWIGLU) return r < BN / 2 ? WeightRow{0, col + r} : WeightRow{1, col + r - BN / 2};
-  else {
-    const int n = col + r;
-    if (n < t.b_end[0]) return {0, n};
-    if (n < t.b_end[1]) return {1, n - t.b_end[0]};
-    return {2, n - t.b_end[1]};
-  }
-}
-template <typename T> __device__ __forceinline__ const T *pick(const T *const (&p)[3], int i) { return i == 0 ? p[0] : (i == 1 ? p[1] : p[2]); }
-template <int EPI, int BN> __device__ __forceinline__ const unsigned char *weight_ptr(const TileArgs &t, int col, int r, size_t row_bytes) {
-  const WeightRow w = weight_row<EPI, BN>(t, col, r);
-  return (const unsigned char *)pick(t.b, w.mat) + (size_t)w.row * row_bytes;
-}
 
 // ---- epilogue of one wavefront: R16 x C16 tiles of 16x16 outputs.  The weight fragment is the first MFMA operand, so a lane
 // holds output row lane % 16 and the four neighbouring columns 4 * (lane / 16) + 0..3 of a tile.  Stored from there an
@@ -131,45 +66,11 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs &a, _Float16 *ep, i
       const int m = mrow + i0 * 16 + row, n = ncol + piece * 8;
       const h8_t v = *(const h8_t *)&ep[row * RS + piece * 8];
       if (m >= a.M) continue;
-      if constexpr (EPI == GEPI_SWIGLU) {
-        *(h8_t *)&a.y[(size_t)m * a.N + n] = v;
-      } else if constexpr (EPI == GEPI_STORE) {
-        h8_t o = v;
-        if (a.residual) {
-#pragma unroll
-          for (int c = 0; c < 8; c++) o[c] = (_Float16)((float)res[p][c] + (float)v[c]);
-        }
-        *(h8_t *)&a.y[(size_t)m * a.N + n] = o;
-      } else {
-        // wq | wk | wv columns; q and k get the interleaved-pair rotation (llama.ts:17-32), k and v go to the cache rows.
-        // Eight neighbouring columns are four pairs of one head of one matrix (every boundary is a multiple of 8).
-        const int b = m / a.seq_len, pos = a.start_pos + m % a.seq_len;
-        const int which = n < a.n0 ? 0 : (n < a.n0 + a.n1 ? 1 : 2);
-        const int nl = which == 0 ? n : (which == 1 ? n - a.n0 : n - a.n0 - a.n1);
-        h8_t o = v;
-        if (which < 2) {
-          const int pair = (nl % a.head_dim) >> 1;
-          const h8_t cs = *(const h8_t *)(a.rope_table + ((size_t)pos * (a.head_dim / 2) + pair) * 2);   // cos, sin of four pairs
-#pragma unroll
-          for (int h = 0; h < 4; h++) {
-            const float ev = (float)v[2 * h], od = (float)v[2 * h + 1];
-            const float c = (float)cs[2 * h], d = (float)cs[2 * h + 1];
-            o[2 * h] = (_Float16)(ev * c - od * d);
-            o[2 * h + 1] = (_Float16)(ev * d + od * c);
-          }
-        }
-        if (which == 0) *(h8_t *)&a.y[(size_t)m * a.n0 + nl] = o;
-        else {
-          _Float16 *cache = which == 1 ? a.cache_k : a.cache_v;
-          *(h8_t *)&cache[((size_t)b * a.max_context + pos) * a.n1 + nl] = o;
-        }
-      }
+      store_piece<EPI>(a, m, n, v, res[EPI == GEPI_STORE ? p : 0]);
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the reads, before the next rows overwrite the piece
   }
 }
-// silu(w1 x) * (w3 x), each GEMM output and the product stored as fp16 (llama.ts:108-110)
-__device__ __forceinline__ float swiglu(float gate, float up) { return silu_act<_Float16>(rn16(gate)) * rn16(up); }
 
 // ---- K parts: every part leaves its sums in the workspace, the last of a tile's parts to arrive adds them in K order, so the
 // result does not depend on who is last.  False: this block was not the last.
@@ -703,19 +604,19 @@ template <int KIND, int EPI, int BM, int BN, int ST> static int launch_qtile(con
 // when every unit has one (they share memory and power), us of a step of a round when there are several, and of a round's end.
 // Fitted to 33 to 4096 rows over the matrices of the 1B, 3B and 8B models, each under every shape that could matter, weights in memory
 // and in the last level cache, for the choice rather than for the single time (an estimate is off by 5-10 % r.m.s.).
-struct TileShape { int bm, bn, bk; float step, fill, round_step, end; };
+struct TileShape { int bm, bn, bk; float step, fill, round_step, end; bool pairs = true; };   // pairs: w1|w3 as well
 static const TileShape TILE_SHAPES[] = {
-  {64, 64, 64, 0.19f, 0.03f, 0.22f, 0.0f},     // not for w1|w3 (its tiles come in pairs)
+  {64, 64, 64, 0.19f, 0.03f, 0.22f, 0.0f, false},
   {64, 128, 64, 0.27f, 0.064f, 0.37f, 0.0f},
   {128, 128, 64, 0.38f, 0.13f, 0.63f, 0.3f},
   {256, 128, 64, 0.55f, 0.32f, 0.85f, 1.0f},
   {256, 256, 64, 0.82f, 0.39f, 1.3f, 3.0f},
 };
-static const TileShape QTILE_SHAPES_I8[] = {{64, 64, 64, 0.25f, 0.024f, 0.18f, 0.03f}, {64, 128, 64, 0.35f, 0.03f, 0.36f, 0.57f}, {128, 128, 64, 0.52f, 0.087f, 0.50f, 1.2f}};
-static const TileShape QTILE_SHAPES_NF4[] = {{64, 64, 128, 0.51f, 0.062f, 0.43f, 0.3f}, {64, 128, 128, 0.86f, 0.075f, 0.70f, 0.74f}, {128, 128, 128, 1.6f, 0.13f, 1.4f, 3.2f}};
-// gemm_staged.hip; 32x128 not for w1|w3
-static const TileShape STAGED_SHAPES_I8[] = {{32, 128, 64, 0.48f, 0.1f, 0.36f, 0.5f}, {128, 128, 64, 0.88f, 0.09f, 0.61f, 1.2f}, {256, 128, 64, 1.13f, 0.16f, 1.04f, 2.5f}, {256, 256, 64, 1.1f, 0.43f, 1.7f, 6.0f}};
-static const TileShape STAGED_SHAPES_NF4[] = {{32, 128, 64, 0.53f, 0.17f, 0.29f, 0.5f}, {128, 128, 64, 0.92f, 0.09f, 0.71f, 0.7f}, {256, 128, 64, 1.2f, 0.17f, 1.03f, 2.0f}, {256, 256, 64, 1.4f, 0.29f, 1.9f, 7.8f}};
+static const TileShape QTILE_SHAPES_I8[] = {{64, 64, 64, 0.25f, 0.024f, 0.18f, 0.03f, false}, {64, 128, 64, 0.35f, 0.03f, 0.36f, 0.57f}, {128, 128, 64, 0.52f, 0.087f, 0.50f, 1.2f}};
+static const TileShape QTILE_SHAPES_NF4[] = {{64, 64, 128, 0.51f, 0.062f, 0.43f, 0.3f, false}, {64, 128, 128, 0.86f, 0.075f, 0.70f, 0.74f}, {128, 128, 128, 1.6f, 0.13f, 1.4f, 3.2f}};
+// gemm_staged.hip
+static const TileShape STAGED_SHAPES_I8[] = {{32, 128, 64, 0.48f, 0.1f, 0.36f, 0.5f, false}, {128, 128, 64, 0.88f, 0.09f, 0.61f, 1.2f}, {256, 128, 64, 1.13f, 0.16f, 1.04f, 2.5f}, {256, 256, 64, 1.1f, 0.43f, 1.7f, 6.0f}};
+static const TileShape STAGED_SHAPES_NF4[] = {{32, 128, 64, 0.53f, 0.17f, 0.29f, 0.5f, false}, {128, 128, 64, 0.92f, 0.09f, 0.71f, 0.7f}, {256, 128, 64, 1.2f, 0.17f, 1.03f, 2.0f}, {256, 256, 64, 1.4f, 0.29f, 1.9f, 7.8f}};
 constexpr int N_SHAPES = sizeof(TILE_SHAPES) / sizeof(TILE_SHAPES[0]), N_QSHAPES = sizeof(QTILE_SHAPES_I8) / sizeof(QTILE_SHAPES_I8[0]), N_STAGED = sizeof(STAGED_SHAPES_I8) / sizeof(STAGED_SHAPES_I8[0]);
 
 // Which shape and how many K parts: the least of an estimate of the launch's time (4.5 us for start and first tiles; for K parts 1.7 us
@@ -729,9 +630,9 @@ struct Choice { float us; int shape, split; };
 // "64x128/3"; quantised weights are then realised), of qtile_kernel ("q64x64/3") or of the staged kernel ("s256x256"); "small", "tall",
 // "wide" and "db" name fp16 tiles from 64x64 (w1|w3: 64x128) to 256x256.  A tile that the output width does not allow is not taken.
 struct Pin { char family = 0; int bm = 0, bn = 0, split = 1; };   // family: 't', 'q' or 's'; 0: no pin
-static Pin read_pin(int epi) {
+static Pin read_pin(int epi, const GemmArgs &a) {
   Pin p;
-  const char *e = getenv("JSG_GEMM_TILE");
+  const char *e = pin_env(a, "JSG_GEMM_TILE");
   if (!e) return p;
   p.family = *e == 'q' || (*e == 's' && e[1] != 'm') ? *e : 't';
   const struct { const char *name; int bm, bn; } names[] = {{"small", 64, epi == GEPI_SWIGLU ? 128 : 64}, {"tall", 128, 128}, {"wide", 256, 128}, {"db", 256, 256}};
@@ -745,7 +646,7 @@ static Choice choose_tile(const TileShape *shapes, int n_shapes, int epi, int M,
   Choice best = {0.0f, -1, 1};
   for (int s = 0; s < n_shapes; s++) {
     const TileShape &c = shapes[s];
-    if (weight_rows % c.bn || K % c.bk || (epi == GEPI_SWIGLU && (c.bn < 128 || c.bm < 64))) continue;
+    if (weight_rows % c.bn || K % c.bk || (epi == GEPI_SWIGLU && !c.pairs)) continue;
     const int tiles = ((M + c.bm - 1) / c.bm) * (weight_rows / c.bn), nk = K / c.bk;
     for (int d = 1; d <= 16; d++) {
       if (d > 1 && (c.bm * c.bn == 65536 || nk < d || tiles > TILE_COUNTERS || (size_t)tiles * d * c.bm * c.bn * 4 > ws_limit)) break;
@@ -792,16 +693,11 @@ template <int EPI> static int gemm_tiled_epi(int kind, const GemmArgs &a, int pr
   const void *const w[3] = {a.w0, a.w1, a.w2};
   const _Float16 *const sc[3] = {a.s0, a.s1, a.s2};
   const int n[3] = {EPI == GEPI_ROPE_KV ? a.n0 : a.N, EPI == GEPI_ROPE_KV ? a.n1 : 0, EPI == GEPI_ROPE_KV ? a.n2 : 0};   // rows on top of each other
-  TileArgs t = {};
-  t.g = a;
   static int *counters = nullptr;
   if (!counters) JSG_HIP(hipGetSymbolAddress((void **)&counters, HIP_SYMBOL(tile_counters)));
-  t.counters = counters;
-  for (int q = 0; q < 3; q++) { t.b[q] = w[q]; t.s[q] = sc[q]; }
-  t.b_end[0] = n[0];
-  t.b_end[1] = n[0] + n[1];
+  TileArgs t = tile_args(EPI, a, counters);
 
-  const Pin pin = read_pin(EPI), none;
+  const Pin pin = read_pin(EPI, a), none;
   auto pinned = [&](char family) -> const Pin & { return pin.family == family ? pin : none; };
   const size_t ws_limit = state().capturing ? 0 : SUMS_LIMIT;
   const int wrows = a.N * NMAT;
@@ -820,7 +716,17 @@ template <int EPI> static int gemm_tiled_epi(int kind, const GemmArgs &a, int pr
   };
 
   Choice f = choose_tile(TILE_SHAPES, N_SHAPES, EPI, a.M, wrows, a.K, ws_limit, pinned('t'));
-  if (kind == JSGRAD_W_F16) return run_whole(TILE_SHAPES, N_SHAPES, f, pinned('t'), launch_shape<EPI>);
+  const GroupChoice g = pin.family ? GroupChoice() : choose_group(EPI, kind, a, ws_limit);
+  // the group kernel, if it is estimated to be done before `us`
+  auto group_first = [&](float us, bool *taken) -> int {
+    *taken = false;
+    return g.shape >= 0 && g.us < us ? run_group(EPI, kind, a, g, prof_kind, taken) : 0;
+  };
+  bool taken;
+  if (kind == JSGRAD_W_F16) {
+    if (const int rc = group_first(f.us, &taken); rc || taken) return rc;
+    return run_whole(TILE_SHAPES, N_SHAPES, f, pinned('t'), launch_shape<EPI>);
+  }
 
   // Quantised: dequantised as read (qtile_kernel), dequantised on the way into LDS (gemm_staged.hip), or realised first, whichever is
   // estimated to be done first; without memory for the realised matrix (a capture, a full device) one of the first two.  Realising:
@@ -836,6 +742,7 @@ template <int EPI> static int gemm_tiled_epi(int kind, const GemmArgs &a, int pr
   const TileShape *ss = kind == JSGRAD_W_I8 ? STAGED_SHAPES_I8 : STAGED_SHAPES_NF4;
   const Choice st = choose_tile(ss, N_STAGED, EPI, a.M, wrows, a.K, 0, pinned('s'));   // takes every call
   const bool staged = q.shape < 0 || st.us < q.us;
+  if (const int rc = group_first(std::min(staged ? st.us : q.us, f.shape >= 0 ? f.us + realise_us : st.us), &taken); rc || taken) return rc;
   const size_t bytes = (size_t)wrows * a.K * 2;
   if (f.shape >= 0 && f.us + realise_us < (staged ? st.us : q.us) && bytes <= REALISED_LIMIT) {
     // into the workspace, with the K parts' sums behind it

@@ -1,0 +1,56 @@
+"""The kernel that shares a tile's K range among the wavefronts of a block (some dozens of rows), pinned: every tile, with and without
+K parts, under every epilogue, at ragged row tiles and where turns of its ring run out: one stage in all (one group has work), fewer
+turns than the ring holds, a last turn with stages for some groups only.
+
+Tolerance: products and sums are those of the oracle's several-row Linear in another order (assert_close)."""
+import numpy as np
+import pytest
+
+from denograd_amd.tensor import Tensor
+from tests import test_gpu_gemm_tile as tile_tests
+from tests import test_gpu_rows as rows_tests
+from tests.test_gpu_gemm_tile import test_tiled_gemm_at_the_edges as check_gemm
+
+pytestmark = pytest.mark.gpu
+
+TILES = ["g16x64", "g16x64/3", "g16x128", "g16x128/2", "g32x64", "g32x64/5", "g32x128", "g32x128/3", "g64x64", "g64x64/3", "g64x128", "g64x128/2"]
+
+
+@pytest.mark.parametrize("kind", ["float16", "int8", "nf4"])
+@pytest.mark.parametrize("tile", TILES)
+def test_every_group_tile(hip, monkeypatch, kind, tile):
+    monkeypatch.setenv("JSG_GEMM_TILE", tile)
+    for rows, out_f, in_f in ((2, 128, 128), (16, 256, 1152), (19, 128, 640), (57, 768, 640), (64, 128, 2048), (100, 256, 1408)):
+        check_gemm(hip, kind, rows, out_f, in_f)
+    for rows in (5, 57):
+        rows_tests.test_gemm_ffn_gate(hip, kind, rows, 640, 384)
+    rows_tests.test_gemm_qkv_rope_writes_queries_and_cache(hip, kind, 64, 3, 19, 640)
+    rows_tests.test_gemm_qkv_rope_writes_queries_and_cache(hip, kind, 128, 5, 9, 640)
+    if kind != "nf4":
+        check_gemm(hip, kind, 33, 128, 64)
+        check_gemm(hip, kind, 9, 128, 8256)
+
+
+@pytest.mark.parametrize("kind", ["float16", "int8", "nf4"])
+def test_as_chosen(hip, monkeypatch, kind):
+    """Calls that come to the group kernel by their sizes (more than one round of the streaming kernel's blocks, long rows, 33 to 64 rows of
+    short ones), the same calls in a capture (no memory for K parts), and with scales at an odd multiple of two bytes."""
+    sizes = ((20, 4224, 1024), (31, 256, 8192), (12, 256, 9216), (40, 384, 1024), (57, 128, 2048))
+    for rows, out_f, in_f in sizes:
+        check_gemm(hip, kind, rows, out_f, in_f)
+        check_gemm(tile_tests.Captured(hip), kind, rows, out_f, in_f)
+    for rows in (9, 24, 57):
+        rows_tests.test_gemm_ffn_gate(hip, kind, rows, 1024, 4224)
+        rows_tests.test_gemm_ffn_gate(tile_tests.Captured(hip), kind, rows, 1024, 4224)
+    rows_tests.test_gemm_qkv_rope_writes_queries_and_cache(hip, kind, 64, 3, 9, 3072)
+    if kind == "float16":
+        return
+    held = []
+
+    def slice_of_scales(t):
+        held.append(Tensor(np.concatenate([np.full(1, 7.0, np.float16), t.numpy().reshape(-1)])))
+        return held[-1].ptr + 2
+
+    monkeypatch.setattr(tile_tests, "sp", slice_of_scales)
+    for rows, out_f, in_f in sizes:
+        check_gemm(hip, kind, rows, out_f, in_f)
