@@ -230,14 +230,13 @@ template <int EPI> static int gemm_few_epi(int kind, const GemmArgs &a, int prof
 int gemm_few(int epi, int kind, const GemmArgs &a, int prof_kind, bool *taken) {
   *taken = false;
   if (a.M > 16 || a.N % 16 || ((uintptr_t)a.s0 | (uintptr_t)a.s1 | (uintptr_t)a.s2) & 3) return 0;
-  // int8: the codes of a tile are half the bytes behind the same x, and the kernels of gemm.hip read whole 512-byte stretches of many
-  // tiles.  us, theirs | this one: 4096 x 4096, 2 / 8 / 16 rows 8.1 / 8.3 / 8.6 | 7.5 / 8.2 / 9.5, 6144 x 4096 11.9 / 12.0 / 12.0 |
-  // 10.2 / 10.9 / 12.0, 3072 x 8192 12.2 / 12.3 / 12.2 | 8.6 / 10.1 / 12.7, 5120 x 3072 9.9 / 10.4 / 11.2 | 7.0 / 7.5 / 8.1,
-  // 16384 x 3072 13.5 / 13.7 / 13.7 | 13.5 / 14.1 / 15.0, 28672 x 4096 26.6 / 26.8 / 27.2 | 28.2 / 28.7 / 30.3.
-  // fp16 is the faster here at every size measured: 2048 x 2048 6.2 / 6.3 / 6.3 | 4.5 / 4.5 / 5.1, 2048 x 8192 14.1 / 14.9 / 15.9 |
+  // int8: the codes of a tile are half the bytes behind the same x, and a tile is over in a step or two; gemm_group.hip keeps its ring full
+  // over wide matrices.  us, 8 / 16 rows, that one | this one: 5120 x 3072 9.2 / 9.3 | 7.7 / 8.5, 3072 x 8192 10.6 / 10.9 | 10.5 / 12.7, 16384 x 2048
+  // 10.9 / 10.5 | 10.7 / 11.1, 6144 x 4096 10.4 / 10.7 | 10.7 / 12.0, 16384 x 3072 13.3 / 13.2 | 14.1 / 15.0, 28672 x 4096 22.2 / 22.1 | 28.7 / 30.3.
+  // fp16, skinny_gemm_kernel | this one, 2 / 8 / 16 rows: 2048 x 2048 6.2 / 6.3 / 6.3 | 4.5 / 4.5 / 5.1, 2048 x 8192 14.1 / 14.9 / 15.9 |
   // 8.8 / 9.5 / 12.4, 16384 x 2048 23.6 / 23.7 / 24.4 | 16.3 / 17.2 / 18.2, 128256 x 2048 147 / 153 / 162 | 88 / 92 / 94 (6.0 TB/s).
   // fp16 rows of 16 KiB behind more than 8 rows of x go to gemm_group.hip, which reads x from LDS: 2048 x 8192, 16 rows 12.8 | 10.9 there, 3072 x 8192
-  // 15.5 | 12.8 (8 rows 9.8 | 10.7, 12.6 | 12.6).
+  // 15.5 | 12.8 (8 rows 9.8 | 10.9, 12.6 | 13.0).
   if (kind == JSGRAD_W_F16 && a.M > 8 && a.K > 4096) return 0;
   const size_t codes = (size_t)a.N * (epi == GEPI_SWIGLU ? 2 : 1) * a.K;
   if (kind == JSGRAD_W_I8 && (codes > (size_t)36 << 20 || (a.M > 8 && a.K > 3072))) return 0;

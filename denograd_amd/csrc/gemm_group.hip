@@ -7,10 +7,10 @@
 // wavefronts of a group split the tile's columns, so a weight is dequantised once per block and a piece of x is read by WN wavefronts.
 // Fragments are read a turn ahead of the matrix instructions that use them, one barrier per turn.  The groups' sums are
 // added in LDS in group order; K parts over blocks as in gemm_tile.hip, in part order.
-// Measured (weights from memory, us, the kernels it took the sizes from | this one): 24 rows, int8 16384 x 3072 22.8 | 17.2, 28672 x 4096
-// 50 | 34 (3.5 TB/s), 128256 x 3072 213 | 100; fp16 16384 x 2048 23.8 | 16.1, 128256 x 3072 265 | 126 (6.2 TB/s), 4096 x 14336 36 | 22.6; nf4
-// 28672 x 4096 46 | 26, with 8 rows 36.7 | 22.5.  From 33 rows on a turn is as much LDS and matrix work as it takes its bytes to arrive
-// (16384 x 3072 int8, 57 rows: 1.2 us a turn of 48 KiB), and it is level with the tiled kernels but for nf4 (21 | 17.5) and short rows.
+// Measured (weights from memory, us, the kernels it took the sizes from | this one): 16 rows, int8 28672 x 4096 27.0 | 22.1 (5.3 TB/s), 4096 x 14336 17.8 |
+// 15.8; 24 rows, int8 16384 x 3072 22.8 | 15.0, 128256 x 3072 213 | 77; fp16 16384 x 2048 23.8 | 14.7, 128256 x 3072 265 | 126 (6.2 TB/s), 4096 x 14336
+// 36 | 23; nf4 28672 x 4096 46 | 25, with 8 rows 36.7 | 21.7.  From 33 rows on LDS reads and matrix instructions of a turn take as long as its bytes to
+// arrive, and it is ahead by less: 57 rows, 16384 x 3072 int8 19.5 | 17.5, nf4 21.4 | 18.4, 128256 x 3072 int8 112 | 104.
 #include <type_traits>
 
 #include "gemm_tile.h"
@@ -19,32 +19,35 @@ namespace jsg {
 
 constexpr int GROUP_THREADS = 512;
 
-// bytes of an LDS row of weights (one stage), K elements of a stage
-template <int KIND> struct GFmt {
-  static constexpr int KS = KIND == JSGRAD_W_NF4 ? 128 : 64;
-  static constexpr int WB = KIND == JSGRAD_W_F16 ? 128 : 64;
+// A stage of a group: WB bytes (64 or 128) of every weight row, as 16-byte pieces; a lane's piece is the operands of STEPS matrix instructions, and
+// x is read in the order of K that this makes: lane quarter lq, step s of piece group p: elements (p * 4 + lq) * 8 * STEPS + 8 s .. + 7.
+template <int KIND, int WB> struct GFmt {
+  static constexpr int STEPS = KIND == JSGRAD_W_F16 ? 1 : (KIND == JSGRAD_W_I8 ? 2 : 4);
+  static constexpr int PG = WB / 64;                          // piece groups: four pieces, one per lane quarter
+  static constexpr int KF = PG * STEPS, KS = KF * 32;         // steps and K elements of a stage
 };
-template <int KIND, int BM, int BN, int WN, int ST> struct GShape {
-  typedef GFmt<KIND> F;
+template <int KIND, int WB, int BM, int BN, int WN, int ST> struct GShape {
+  typedef GFmt<KIND, WB> F;
   static constexpr int G = 8 / WN;                            // K groups
-  static constexpr int X = BM * F::KS * 2, W = BN * F::WB;    // bytes of a group's stage
-  static constexpr int TURN = G * (X + W) + (KIND == JSGRAD_W_NF4 ? 2048 : 0);   // nf4: 256 bytes of scales per wavefront
+  static constexpr int X = BM * F::KS * 2, W = BN * WB;       // bytes of a group's stage
+  static constexpr int SCALES = KIND == JSGRAD_W_NF4 ? 256 * F::PG : 0;   // per wavefront
+  static constexpr int TURN = G * (X + W) + 8 * SCALES;
   static constexpr int TABLE = KIND == JSGRAD_W_NF4 ? 16384 : (KIND == JSGRAD_W_I8 ? 2048 : 0);   // nf4: 16 copies of the table of code pairs; int8: row scales
   static constexpr int RED = G * BM * (BN + 4) * 4;
   static constexpr int LDS = (TURN * ST > RED ? TURN * ST : RED) + TABLE;
   static_assert(LDS + 64 <= 160 * 1024, "LDS of one compute unit");
 };
 
-template <int KIND, int EPI, int BM, int BN, int WN, int ST> __global__ __launch_bounds__(GROUP_THREADS, 2) void group_kernel(TileArgs t) {
-  typedef GFmt<KIND> F;
-  typedef GShape<KIND, BM, BN, WN, ST> S;
+template <int KIND, int EPI, int WB, int BM, int BN, int WN, int ST> __global__ __launch_bounds__(GROUP_THREADS, 2) void group_kernel(TileArgs t) {
+  typedef GFmt<KIND, WB> F;
+  typedef GShape<KIND, WB, BM, BN, WN, ST> S;
   const GemmArgs &a = t.g;
   extern __shared__ __align__(16) unsigned char group_lds[];
-  constexpr int G = S::G, KS = F::KS, KF = KS / 32, TM = BM / 16, TN = BN / 16 / WN;
+  constexpr int G = S::G, KS = F::KS, KF = F::KF, PG = F::PG, STEPS = F::STEPS, TM = BM / 16, TN = BN / 16 / WN;
   constexpr int XI = S::X / 1024, WI = S::W / 1024;           // direct loads of 1 KiB per group and turn: eight x rows, or 1024 / WB weight rows
   constexpr int NX = G * XI / 8, NW = G * WI / 8;             // ... and per wavefront
   static_assert(NX * 8 == G * XI && NW * 8 == G * WI && TN >= 1, "every wavefront issues the same loads");
-  constexpr int NLD = NX + NW + (KIND == JSGRAD_W_NF4 ? 1 : 0);
+  constexpr int NLD = NX + NW + (KIND == JSGRAD_W_NF4 ? PG : 0);
   constexpr int CW = EPI == GEPI_SWIGLU ? BN / 2 : BN;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, lq = lane >> 4;
   const int kg = wave / WN, wn = wave % WN;
@@ -62,6 +65,11 @@ template <int KIND, int EPI, int BM, int BN, int WN, int ST> __global__ __launch
   const uint32_t x_bytes = (uint32_t)a.K * 2, w_bytes = KIND == JSGRAD_W_F16 ? a.K * 2 : (KIND == JSGRAD_W_I8 ? a.K : a.K / 2);
   const int nst = a.K / KS, k0 = (int)((long long)id.part * nst / t.split), ns = (int)((long long)(id.part + 1) * nst / t.split) - k0;
   const int turns = (ns + G - 1) / G;
+  // Weight rows whose distance is a multiple of 4 KiB: blocks start their walk through K at different turns and wrap around, so that they
+  // don't queue at the same offset of such rows for the same memory channels (28672 x 4096, us: int8, 8 rows 30.1 -> 26.4, 24 rows 33.9 ->
+  // 32.2; fp16, 24 rows in 32x64 tiles 46.3 -> 41.9, but in 32x128 47 -> 55 and 57 rows 49.3 -> 56.7; other distances and K parts: 1 % slower).
+  const int first = BM <= 32 && (KIND != JSGRAD_W_F16 || BM * BN < 4096) && t.split == 1 && w_bytes % 4096 == 0 ? (int)((unsigned)(id.col / CW) % (unsigned)turns) : 0;
+  auto turn_of = [&](int turn) { const int r = turn + first; return r >= turns ? r - turns : r; };
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)group_lds;
   const i4_t ra = dma_rsrc(a.x + (size_t)m0 * a.K);
   uint32_t va[NX], la[NX];
@@ -73,7 +81,7 @@ template <int KIND, int EPI, int BM, int BN, int WN, int ST> __global__ __launch
     va[i] = (uint32_t)min(r8 + (lane >> 3), a.M - 1 - m0) * x_bytes + (uint32_t)((lane & 7) ^ (lane >> 3)) * 16 + sl * 128;   // rows past the end are computed and never stored
     la[i] = lds0 + ga[i] * (S::X + S::W) + in * 1024;
   }
-  constexpr int RPL = 1024 / F::WB;                           // weight rows of a load
+  constexpr int RPL = 1024 / WB;                           // weight rows of a load
   i4_t rb[NW];
   uint32_t lb[NW];
   int gb[NW];
@@ -84,21 +92,24 @@ template <int KIND, int EPI, int BM, int BN, int WN, int ST> __global__ __launch
     rb[i] = dma_rsrc(weight_ptr<EPI, BN>(t, id.col, idx % WI * RPL, w_bytes));
     lb[i] = lds0 + gb[i] * (S::X + S::W) + S::X + idx % WI * 1024;
   }
-  const uint32_t vb = F::WB == 128 ? (uint32_t)(lane >> 3) * w_bytes + (uint32_t)((lane & 7) ^ (lane >> 3)) * 16
-                                   : (uint32_t)(lane >> 2) * w_bytes + (uint32_t)((lane & 3) ^ (lane >> 4)) * 16;
+  const uint32_t vb = WB == 128 ? (uint32_t)(lane >> 3) * w_bytes + (uint32_t)((lane & 7) ^ (lane >> 3)) * 16
+                                   : (uint32_t)(lane >> 2) * w_bytes + (uint32_t)((lane & 3) ^ ((lane >> 3) & 3)) * 16;
   // scales of this wavefront's rows (one matrix: a wavefront's columns never straddle two)
   const int my_row = wn * TN * 16;
   const WeightRow sr = weight_row<EPI, BN>(t, id.col, my_row);
   i4_t rs;
   if constexpr (KIND != JSGRAD_W_F16) rs = dma_rsrc(pick(t.s, sr.mat) + (size_t)sr.row * (KIND == JSGRAD_W_I8 ? 1 : a.K / 64));
   const uint32_t vs = KIND == JSGRAD_W_I8 ? (uint32_t)(lane & (TN * 8 - 1)) * 4 : (uint32_t)(lane & (TN * 16 - 1)) * (a.K / 32);
-  auto load = [&](int turn, int buf) {
+  auto load = [&](int at, int buf) {
+    const int turn = turn_of(at);
     const uint32_t base = (uint32_t)buf * S::TURN;
 #pragma unroll
     for (int i = 0; i < NX; i++) dma16(ra, va[i], (uint32_t)(k0 + min(turn * G + ga[i], ns - 1)) * (KS * 2), base + la[i]);
 #pragma unroll
-    for (int i = 0; i < NW; i++) dma16_stream(rb[i], vb, (uint32_t)(k0 + min(turn * G + gb[i], ns - 1)) * F::WB, base + lb[i]);
-    if constexpr (KIND == JSGRAD_W_NF4) dma4(rs, vs, (uint32_t)(k0 + min(turn * G + kg, ns - 1)) * 4, lds0 + base + G * (S::X + S::W) + wave * 256);
+    for (int i = 0; i < NW; i++) dma16_stream(rb[i], vb, (uint32_t)(k0 + min(turn * G + gb[i], ns - 1)) * WB, base + lb[i]);
+    if constexpr (KIND == JSGRAD_W_NF4)
+#pragma unroll
+      for (int p = 0; p < PG; p++) dma4(rs, vs, (uint32_t)((k0 + min(turn * G + kg, ns - 1)) * PG + p) * 4, lds0 + base + G * (S::X + S::W) + wave * S::SCALES + p * 256);
   };
 
   f4_t acc[TM][TN];
@@ -108,58 +119,61 @@ template <int KIND, int EPI, int BM, int BN, int WN, int ST> __global__ __launch
     for (int j = 0; j < TN; j++) acc[i][j] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
   struct Frags {
     h8_t x[KF][TM];
-    u4_t w[KF][TN];                                           // fp16: the fragment; int8: eight codes in two words; nf4: in one
-    h2_t s[TN];                                               // nf4: the scales of the stage's two blocks
+    u4_t w[PG][TN];
+    h2_t s[PG][TN];                                           // nf4: the scales of the piece group's two blocks
   };
   Frags fr[2];
   auto read = [&](int buf, Frags &f) {
     const unsigned char *px = group_lds + buf * S::TURN + kg * (S::X + S::W) + l16 * 128;
-    const unsigned char *pw = group_lds + buf * S::TURN + kg * (S::X + S::W) + S::X + (my_row + l16) * F::WB;
+    const unsigned char *pw = group_lds + buf * S::TURN + kg * (S::X + S::W) + S::X + (my_row + l16) * WB;
 #pragma unroll
-    for (int k = 0; k < KF; k++) {
-      const uint32_t sw = (uint32_t)(((k & 1) * 4 + lq) ^ (l16 & 7)) * 16;
+    for (int p = 0; p < PG; p++) {
 #pragma unroll
-      for (int i = 0; i < TM; i++) f.x[k][i] = *(const h8_t *)(px + (k / 2) * BM * 128 + i * 2048 + sw);
+      for (int s = 0; s < STEPS; s++) {
+        const int piece = (p * 4 + lq) * STEPS + s;
+        const unsigned char *from = px + (piece >> 3) * (BM * 128) + ((piece & 7) ^ (l16 & 7)) * 16;
+#pragma unroll
+        for (int i = 0; i < TM; i++) f.x[p * STEPS + s][i] = *(const h8_t *)(from + i * 2048);
+      }
+      const uint32_t at = (WB == 128 ? (p * 4 + lq) ^ (l16 & 7) : lq ^ ((l16 >> 1) & 3)) * 16;
 #pragma unroll
       for (int j = 0; j < TN; j++) {
-        const unsigned char *pr = pw + j * 16 * F::WB;
-        if constexpr (KIND == JSGRAD_W_F16) f.w[k][j] = *(const u4_t *)(pr + sw);
-        else if constexpr (KIND == JSGRAD_W_I8) {
-          const uint2 q = *(const uint2 *)(pr + (uint32_t)((k * 2 + (lq >> 1)) ^ (l16 >> 2)) * 16 + (lq & 1) * 8);
-          f.w[k][j].x = q.x;
-          f.w[k][j].y = q.y;
-        } else f.w[k][j].x = *(const uint32_t *)(pr + (uint32_t)(k ^ (l16 >> 2)) * 16 + lq * 4);
+        f.w[p][j] = *(const u4_t *)(pw + j * 16 * WB + at);
+        if constexpr (KIND == JSGRAD_W_NF4) f.s[p][j] = *(const h2_t *)(group_lds + buf * S::TURN + G * (S::X + S::W) + wave * S::SCALES + p * 256 + (j * 16 + l16) * 4);
       }
     }
-    if constexpr (KIND == JSGRAD_W_NF4)
-#pragma unroll
-      for (int j = 0; j < TN; j++) f.s[j] = *(const h2_t *)(group_lds + buf * S::TURN + G * (S::X + S::W) + wave * 256 + (j * 16 + l16) * 4);
   };
   h2_t scale[TN];
   const uint32_t *const tab = table + l16;
-  auto compute = [&](const Frags &f) {
+  auto compute = [&](int turn, const Frags &f) {
+    if (turn_of(turn) * G + kg >= ns) return;                 // the last turn may not have a stage for every group
 #pragma unroll
-    for (int k = 0; k < KF; k++)
+    for (int p = 0; p < PG; p++)
 #pragma unroll
       for (int j = 0; j < TN; j++) {
-        u4_t o;
-        if constexpr (KIND == JSGRAD_W_F16) o = f.w[k][j];
-        else if constexpr (KIND == JSGRAD_W_I8) {
-          uint32_t lo, hi;
-          i8x4_to_h2x2(f.w[k][j].x, lo, hi); o.x = pk_mul_h2(lo, scale[j]); o.y = pk_mul_h2(hi, scale[j]);
-          i8x4_to_h2x2(f.w[k][j].y, lo, hi); o.z = pk_mul_h2(lo, scale[j]); o.w = pk_mul_h2(hi, scale[j]);
-        } else {
-          const _Float16 s1 = k / 2 ? f.s[j].y : f.s[j].x;
-          const h2_t s = {s1, s1};
-          const uint32_t c = f.w[k][j].x;
-          o.x = pk_mul_h2(tab[(c & 0xffu) * 16], s);
-          o.y = pk_mul_h2(tab[((c >> 8) & 0xffu) * 16], s);
-          o.z = pk_mul_h2(tab[((c >> 16) & 0xffu) * 16], s);
-          o.w = pk_mul_h2(tab[(c >> 24) * 16], s);
-        }
-        const h8_t b = __builtin_bit_cast(h8_t, o);
+        const u4_t raw = f.w[p][j];
+        const uint32_t wds[4] = {raw.x, raw.y, raw.z, raw.w};
+        const _Float16 s1 = lq < 2 ? f.s[p][j].x : f.s[p][j].y;
+        const h2_t sv = {s1, s1};
 #pragma unroll
-        for (int i = 0; i < TM; i++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b, f.x[k][i], acc[i][j], 0, 0, 0);
+        for (int s = 0; s < STEPS; s++) {
+          u4_t o;
+          if constexpr (KIND == JSGRAD_W_F16) o = raw;
+          else if constexpr (KIND == JSGRAD_W_I8) {
+            uint32_t lo, hi;
+            i8x4_to_h2x2(wds[2 * s], lo, hi); o.x = pk_mul_h2(lo, scale[j]); o.y = pk_mul_h2(hi, scale[j]);
+            i8x4_to_h2x2(wds[2 * s + 1], lo, hi); o.z = pk_mul_h2(lo, scale[j]); o.w = pk_mul_h2(hi, scale[j]);
+          } else {
+            const uint32_t c = wds[s];
+            o.x = pk_mul_h2(tab[(c & 0xffu) * 16], sv);
+            o.y = pk_mul_h2(tab[((c >> 8) & 0xffu) * 16], sv);
+            o.z = pk_mul_h2(tab[((c >> 16) & 0xffu) * 16], sv);
+            o.w = pk_mul_h2(tab[(c >> 24) * 16], sv);
+          }
+          const h8_t b = __builtin_bit_cast(h8_t, o);
+#pragma unroll
+          for (int i = 0; i < TM; i++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b, f.x[p * STEPS + s][i], acc[i][j], 0, 0, 0);
+        }
       }
   };
 
@@ -197,18 +211,17 @@ template <int KIND, int EPI, int BM, int BN, int WN, int ST> __global__ __launch
   int turn = 1;
   for (; turn + 1 < turns; turn += 2) {
     step(turn, 1);
-    compute(fr[0]);
+    compute(turn - 1, fr[0]);
     __builtin_amdgcn_sched_barrier(0);
     step(turn + 1, 0);
-    compute(fr[1]);
+    compute(turn, fr[1]);
     __builtin_amdgcn_sched_barrier(0);
   }
-  const bool own_last = (turns - 1) * G + kg < ns;            // the last turn may not have a stage for every group
   if (turn < turns) {
     step(turn, 1);
-    compute(fr[0]);
-    if (own_last) compute(fr[1]);
-  } else if (own_last) compute(fr[0]);
+    compute(turn - 1, fr[0]);
+    compute(turn, fr[1]);
+  } else compute(turn - 1, fr[0]);
 
   // ---- the groups' sums through LDS (every load has landed and been read)
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -290,27 +303,29 @@ template <int KIND, int EPI, int BM, int BN, int WN, int ST> __global__ __launch
   }
 }
 
-template <int KIND, int EPI, int BM, int BN, int WN, int ST> static int launch_group_as(const TileArgs &t, int prof_kind) {
-  constexpr int lds = GShape<KIND, BM, BN, WN, ST>::LDS;
+template <int KIND, int EPI, int WB, int BM, int BN, int WN, int ST> static int launch_group_as(const TileArgs &t, int prof_kind) {
+  constexpr int lds = GShape<KIND, WB, BM, BN, WN, ST>::LDS;
   static bool raised = false;
   if (!raised) {
-    JSG_HIP(hipFuncSetAttribute((const void *)group_kernel<KIND, EPI, BM, BN, WN, ST>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    JSG_HIP(hipFuncSetAttribute((const void *)group_kernel<KIND, EPI, WB, BM, BN, WN, ST>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
     raised = true;
   }
   const int tiles = ((t.g.M + BM - 1) / BM) * (t.g.N / (EPI == GEPI_SWIGLU ? BN / 2 : BN));
-  JSG_LAUNCH(prof_kind, (group_kernel<KIND, EPI, BM, BN, WN, ST>), dim3(tiles * t.split), dim3(GROUP_THREADS), lds, t);
+  JSG_LAUNCH(prof_kind, (group_kernel<KIND, EPI, WB, BM, BN, WN, ST>), dim3(tiles * t.split), dim3(GROUP_THREADS), lds, t);
   return 0;
 }
 
-// Turns in LDS: as many as fit, four at most for 32 and 64 rows (more only lengthens the way to the first)
+// Turns in LDS: as many as fit.  Stages have 128 bytes of a weight row, whole cache lines for eight rows per load: with 64 bytes of sixteen rows int8
+// codes came at three quarters of the rate (us, 64 | 128: 16384 x 3072, 16 rows 16.7 | 13.2, 28672 x 4096 27.4 | 22.1, 24 rows 32.7 | 26.6, 128256 x 3072 101 |
+// 77; nf4 28672 x 4096, 24 rows 29 | 25).  nf4 behind 64 rows of x, where that many K elements of x leave no room for a third turn, keeps 64.
 template <int KIND, int EPI> static int launch_group_kind(int bm, int bn, const TileArgs &t, int prof_kind) {
   constexpr bool NF4 = KIND == JSGRAD_W_NF4, F16 = KIND == JSGRAD_W_F16;
-  if (bm == 16 && bn == 64) return launch_group_as<KIND, EPI, 16, 64, 2, F16 ? 3 : (NF4 ? 4 : 6)>(t, prof_kind);
-  if (bm == 16 && bn == 128) return launch_group_as<KIND, EPI, 16, 128, 2, F16 || NF4 ? 2 : 3>(t, prof_kind);
-  if (bm == 32 && bn == 64) return launch_group_as<KIND, EPI, 32, 64, NF4 ? 4 : 2, F16 ? 3 : (NF4 ? 5 : 4)>(t, prof_kind);
-  if (bm == 32 && bn == 128) return launch_group_as<KIND, EPI, 32, 128, 4, F16 ? 3 : (NF4 ? 4 : 6)>(t, prof_kind);
-  if (bm == 64 && bn == 64) return launch_group_as<KIND, EPI, 64, 64, NF4 ? 4 : 2, F16 ? 2 : 3>(t, prof_kind);
-  if (bm == 64 && bn == 128) return launch_group_as<KIND, EPI, 64, 128, 4, F16 ? 3 : (NF4 ? 2 : 4)>(t, prof_kind);
+  if (bm == 16 && bn == 64) return launch_group_as<KIND, EPI, 128, 16, 64, NF4 ? 4 : 2, 3>(t, prof_kind);
+  if (bm == 16 && bn == 128) return launch_group_as<KIND, EPI, 128, 16, 128, F16 ? 2 : 4, F16 || NF4 ? 2 : 3>(t, prof_kind);
+  if (bm == 32 && bn == 64) return launch_group_as<KIND, EPI, 128, 32, 64, F16 ? 2 : 4, F16 ? 3 : (NF4 ? 2 : 4)>(t, prof_kind);
+  if (bm == 32 && bn == 128) return launch_group_as<KIND, EPI, 128, 32, 128, 4, NF4 ? 2 : 3>(t, prof_kind);
+  if (bm == 64 && bn == 64) return launch_group_as<KIND, EPI, NF4 ? 64 : 128, 64, 64, F16 ? 2 : 4, F16 ? 2 : 3>(t, prof_kind);
+  if (bm == 64 && bn == 128) return launch_group_as<KIND, EPI, NF4 ? 64 : 128, 64, 128, 4, F16 ? 3 : 2>(t, prof_kind);
   return fail("jsgrad_hip_gemm: no tile shape");
 }
 
@@ -330,18 +345,20 @@ static int launch_group(int epi, int kind, int bm, int bn, const TileArgs &t, in
 // added to it when all units have one, a turn when there are several rounds of blocks, and a round's end.  Fitted to 8 to 57 rows over the matrices
 // of the 1B, 3B and 8B models in the three formats, weights from memory, each under every shape and number of K parts that could
 // matter; the choice is 2 % slower than the best shape on average.
-struct GroupShape { int bm, bn, groups; float step, fill, round_step, end; };
+struct GroupShape { int bm, bn, stage, groups; float step, fill, round_step, end; };   // stage: K elements
 constexpr int N_GROUP = 6;
 static const GroupShape GROUP_SHAPES[3][N_GROUP] = {   // fp16, int8, nf4
-  {{16, 64, 4, 0.46f, 0.40f, 0.95f, 0.96f}, {16, 128, 4, 1.20f, 0.89f, 2.15f, 0.66f}, {32, 64, 4, 0.52f, 0.51f, 1.12f, 1.06f}, {32, 128, 2, 0.47f, 0.61f, 1.03f, 1.11f}, {64, 64, 4, 1.07f, 0.52f, 1.67f, 1.34f}, {64, 128, 2, 0.55f, 0.89f, 1.31f, 2.10f}},
-  {{16, 64, 4, 0.55f, 0.21f, 0.91f, 1.04f}, {16, 128, 4, 0.93f, 0.49f, 1.56f, 1.36f}, {32, 64, 4, 0.54f, 0.26f, 0.95f, 1.44f}, {32, 128, 2, 0.46f, 0.49f, 0.90f, 1.84f}, {64, 64, 4, 0.70f, 0.41f, 1.20f, 2.01f}, {64, 128, 2, 0.42f, 0.62f, 1.03f, 2.32f}},
-  {{16, 64, 4, 1.00f, 0.34f, 1.60f, 1.10f}, {16, 128, 4, 1.79f, 0.56f, 2.57f, 1.64f}, {32, 64, 2, 0.64f, 0.23f, 1.01f, 1.35f}, {32, 128, 2, 1.14f, 0.54f, 1.70f, 1.61f}, {64, 64, 2, 0.72f, 0.30f, 1.13f, 2.08f}, {64, 128, 2, 1.02f, 0.83f, 1.72f, 3.47f}},
+  {{16, 64, 64, 4, 0.44f, 0.43f, 0.91f, 1.3f}, {16, 128, 64, 4, 1.19f, 0.89f, 2.06f, 1.1f}, {32, 64, 64, 4, 0.52f, 0.51f, 1.07f, 1.5f}, {32, 128, 64, 2, 0.46f, 0.60f, 0.98f, 1.6f}, {64, 64, 64, 4, 1.06f, 0.54f, 1.64f, 1.6f}, {64, 128, 64, 2, 0.54f, 0.88f, 1.27f, 2.4f}},
+  {{16, 64, 128, 4, 0.62f, 0.37f, 1.21f, 1.7f}, {16, 128, 128, 2, 0.54f, 0.42f, 1.03f, 1.8f}, {32, 64, 128, 2, 0.39f, 0.29f, 0.77f, 1.7f}, {32, 128, 128, 2, 0.64f, 0.60f, 1.23f, 2.4f}, {64, 64, 128, 2, 0.53f, 0.45f, 1.03f, 2.4f}, {64, 128, 128, 2, 0.82f, 1.11f, 1.70f, 3.6f}},
+  {{16, 64, 256, 2, 0.87f, 0.26f, 1.33f, 1.6f}, {16, 128, 256, 2, 1.69f, 0.45f, 2.27f, 1.9f}, {32, 64, 256, 2, 1.25f, 0.30f, 1.77f, 1.9f}, {32, 128, 256, 2, 1.94f, 0.63f, 2.56f, 2.5f}, {64, 64, 128, 2, 0.83f, 0.26f, 1.18f, 2.5f}, {64, 128, 128, 2, 1.06f, 0.81f, 1.70f, 3.8f}},
 };
+// The K parts' sums of a launch lie in memory that belongs to the library: they are also there in a graph capture and on a full device, and
+// one in-order stream serves every launch.
 constexpr int GROUP_COUNTERS = 4096;
-constexpr size_t GROUP_SUMS = (size_t)64 << 20;               // what the K parts' sums may take
+constexpr size_t GROUP_SUMS = (size_t)8 << 20;
+static __device__ __align__(256) unsigned char group_sums[GROUP_SUMS];
 static __device__ int group_counters[GROUP_COUNTERS];
 
-static int stage_of(int kind) { return kind == JSGRAD_W_NF4 ? 128 : 64; }
 static size_t group_bytes(const GroupShape &s, int M, int weight_rows, int split) {
   return split < 2 ? 0 : (size_t)((M + s.bm - 1) / s.bm) * (weight_rows / s.bn) * split * s.bm * s.bn * 4;
 }
@@ -351,23 +368,23 @@ static bool group_pin(const GemmArgs &a, int &bm, int &bn, int &split) {
   split = 1;
   return e && *e == 'g' && sscanf(e + 1, "%dx%d/%d", &bm, &bn, &split) >= 2;
 }
-GroupChoice choose_group(int epi, int kind, const GemmArgs &a, size_t ws_limit) {
+GroupChoice choose_group(int epi, int kind, const GemmArgs &a) {
   GroupChoice best;
   int bm = 0, bn = 0, split = 0;
   const bool pin = group_pin(a, bm, bn, split);
   // scales come by direct loads of four bytes; with more rows than a tile has the weights would be read twice
-  if (a.K % stage_of(kind) || ((uintptr_t)a.s0 | (uintptr_t)a.s1 | (uintptr_t)a.s2) & 3 || (!pin && a.M > 64)) return best;
-  const int cus = state().cu_count, weight_rows = a.N * (epi == GEPI_SWIGLU ? 2 : 1), stages = a.K / stage_of(kind);
+  if (((uintptr_t)a.s0 | (uintptr_t)a.s1 | (uintptr_t)a.s2) & 3 || (!pin && a.M > 64)) return best;
+  const int cus = state().cu_count, weight_rows = a.N * (epi == GEPI_SWIGLU ? 2 : 1);
   for (int i = 0; i < N_GROUP; i++) {
     const GroupShape &s = GROUP_SHAPES[kind - JSGRAD_W_F16][i];
-    if (pin && (s.bm != bm || s.bn != bn)) continue;
-    if (weight_rows % s.bn) continue;
+    const int stages = a.K / s.stage;
+    if (weight_rows % s.bn || a.K % s.stage || (pin && (s.bm != bm || s.bn != bn))) continue;
     const int tiles = ((a.M + s.bm - 1) / s.bm) * (weight_rows / s.bn);
     for (int d = 1; d <= 16 && d <= stages; d++) {
       if (pin && d != (split < stages ? split : stages)) continue;
       const int blocks = tiles * d, turns = ((stages + d - 1) / d + s.groups - 1) / s.groups;
       // parts of at least two turns, and not more than two blocks for every unit
-      if (d > 1 && (tiles > GROUP_COUNTERS || group_bytes(s, a.M, weight_rows, d) > ws_limit || (!pin && (turns < 2 || blocks > 2 * cus)))) break;
+      if (d > 1 && (tiles > GROUP_COUNTERS || group_bytes(s, a.M, weight_rows, d) > GROUP_SUMS || (!pin && (turns < 2 || blocks > 2 * cus)))) break;
       const float fill = (float)blocks / cus;
       float us = 3.5f + (fill <= 1.0f ? (s.step + s.fill * fill) * turns + s.end : ((blocks + cus - 1) / cus) * (s.round_step * turns + s.end));
       if (d > 1) us += 1.7f + (float)d * s.bm * s.bn * 4 / 83e3f * (fill > 1.0f ? fill : 1.0f);
@@ -377,17 +394,17 @@ GroupChoice choose_group(int epi, int kind, const GemmArgs &a, size_t ws_limit) 
   return best;
 }
 
-int run_group(int epi, int kind, const GemmArgs &a, const GroupChoice &c, int prof_kind, bool *taken) {
+int run_group(int epi, int kind, const GemmArgs &a, const GroupChoice &c, int prof_kind) {
   static int *counters = nullptr;
-  if (!counters) JSG_HIP(hipGetSymbolAddress((void **)&counters, HIP_SYMBOL(group_counters)));
+  static float *sums = nullptr;
+  if (!sums) {
+    JSG_HIP(hipGetSymbolAddress((void **)&counters, HIP_SYMBOL(group_counters)));
+    JSG_HIP(hipGetSymbolAddress((void **)&sums, HIP_SYMBOL(group_sums)));
+  }
   const GroupShape &s = GROUP_SHAPES[kind - JSGRAD_W_F16][c.shape];
-  const size_t bytes = group_bytes(s, a.M, a.N * (epi == GEPI_SWIGLU ? 2 : 1), c.split);
-  Workspace ws;
-  *taken = !bytes || ws.get(bytes);
-  if (!*taken) return 0;
   TileArgs t = tile_args(epi, a, counters);
   t.split = c.split;
-  t.ws = (float *)ws.p;
+  t.ws = sums;
   return launch_group(epi, kind, s.bm, s.bn, t, prof_kind);
 }
 
@@ -396,19 +413,20 @@ int gemm_group(int epi, int kind, const GemmArgs &a, int prof_kind, bool *taken)
   int bm, bn, split;
   const bool pin = group_pin(a, bm, bn, split);
   if (!pin) {
-    if (a.M > 32 || pin_env(a, "JSG_GEMM_TILE") || pin_env(a, "JSG_GEMM_NO_SKINNY") || pin_env(a, "JSG_GEMM_SKINNY_TILES") || pin_env(a, "JSG_SG_TPW")) return 0;   // tests that want one of the other kernels
+    if (a.M > 32 || pin_env(a, "JSG_GEMM_TILE") || pin_env(a, "JSG_GEMM_NO_SKINNY") || pin_env(a, "JSG_GEMM_SKINNY_TILES")) return 0;   // tests that want one of the other kernels
     // One round of skinny_gemm_kernel's blocks over short rows: no K parts whose sums have to travel.  us, that | this one: 24 rows, fp16
     // 2048 x 2048 7.5 | 7.5, 3072 x 2048 8.1 | 8.1, 3072 x 3072 9.9 | 9.3, 2048 x 8192 18.7 | 11.5, 5120 x 3072 17.5 | 10.5; int8
-    // 2048 x 2048 6.7 | 7.6, 3072 x 3072 8.6 | 9.1, 4096 x 4096 10.5 | 10.1, 6144 x 4096 17.5 | 12.1, 28672 x 4096 50 | 34; nf4
-    // 4096 x 4096 9.3 | 10.7, 3072 x 8192 14.8 | 12.9, 28672 x 4096 46 | 26; 8 rows, nf4 4096 x 4096 7.8 | 9.1, 3072 x 8192 10.7 | 11.5,
-    // 4096 x 14336 16.2 | 16.3, 6144 x 4096 11.3 | 11.4, 28672 x 4096 36.7 | 22.5.
+    // 2048 x 2048 6.7 | 7.8, 3072 x 3072 8.6 | 9.0, 4096 x 4096 10.5 | 10.1, 6144 x 4096 17.5 | 11.4, 28672 x 4096 50 | 27; nf4
+    // 4096 x 4096 9.3 | 10.9, 3072 x 8192 14.8 | 12.9, 28672 x 4096 46 | 25; 16 rows, int8 4096 x 4096 9.1 | 9.6, 6144 x 4096 13.5 | 10.7; 8 rows, nf4
+    // 4096 x 4096 7.8 | 9.4, 3072 x 8192 10.7 | 11.5 (16 rows 11.6 | 11.8), 6144 x 4096 11.3 | 10.7, 28672 x 4096 36.7 | 21.7.
     const int rows = a.N * (epi == GEPI_SWIGLU ? 2 : 1);
-    const int longest = kind == JSGRAD_W_F16 ? 2048 : (kind == JSGRAD_W_I8 ? (a.M <= 16 ? 4096 : 3072) : (a.M <= 16 ? 8192 : 4096));
+    const int longest = kind == JSGRAD_W_F16 ? 2048 : (kind == JSGRAD_W_I8 ? (a.M <= 16 ? 4096 : 3072) : (a.M <= 8 ? 8192 : 4096));
     if (a.K % 512 || a.K < 1024 || (rows <= 16 * state().cu_count && a.K <= longest)) return 0;
   }
-  const GroupChoice c = choose_group(epi, kind, a, GROUP_SUMS);   // without memory for K parts, as in a capture, the kernels of gemm.hip
+  const GroupChoice c = choose_group(epi, kind, a);
   if (c.shape < 0) return pin ? fail("jsgrad_hip_gemm: no tile shape") : 0;
-  return run_group(epi, kind, a, c, prof_kind, taken);
+  *taken = true;
+  return run_group(epi, kind, a, c, prof_kind);
 }
 
 }  // namespace jsg

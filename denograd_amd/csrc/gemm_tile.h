@@ -123,8 +123,7 @@ inline TileArgs tile_args(int epi, const GemmArgs &a, int *counters) {
 
 // gemm_group.hip: at most 64 rows.  The estimate of its fastest shape for a call; shape < 0: not for this call.
 struct GroupChoice { float us = 0.0f; int shape = -1, split = 1; };
-GroupChoice choose_group(int epi, int kind, const GemmArgs &a, size_t ws_limit);
-// *taken false: no memory for the K parts' sums, nothing launched
-int run_group(int epi, int kind, const GemmArgs &a, const GroupChoice &c, int prof_kind, bool *taken);
+GroupChoice choose_group(int epi, int kind, const GemmArgs &a);
+int run_group(int epi, int kind, const GemmArgs &a, const GroupChoice &c, int prof_kind);
 
 }  // namespace jsg

@@ -716,15 +716,19 @@ template <int EPI> static int gemm_tiled_epi(int kind, const GemmArgs &a, int pr
   };
 
   Choice f = choose_tile(TILE_SHAPES, N_SHAPES, EPI, a.M, wrows, a.K, ws_limit, pinned('t'));
-  const GroupChoice g = pin.family ? GroupChoice() : choose_group(EPI, kind, a, ws_limit);
-  // the group kernel, if it is estimated to be done before `us`
-  auto group_first = [&](float us, bool *taken) -> int {
-    *taken = false;
-    return g.shape >= 0 && g.us < us ? run_group(EPI, kind, a, g, prof_kind, taken) : 0;
+  // At most 64 rows: the group kernel, where its estimate is the least.  The estimates of the tiled kernels are without the rate at which
+  // they can draw weights with so few rows (57 rows, from 12 MB on: fp16 4.6 TB/s, codes 3.9, and for codes a seventh too low below that): us,
+  // theirs measured | the group kernel: fp16 16384 x 3072 25.5 | 24.2, 28672 x 4096 52.5 | 49.4; int8 16384 x 2048 15.3 | 13.6, 16384 x 3072
+  // 18.8 | 17.5, 128256 x 3072 112 | 104; nf4 16384 x 3072 20.9 | 18.4, 28672 x 4096 34.5 | 31.6; with K parts level, 3072 x 8192 int8 14.9 | 15.4.
+  const GroupChoice g = pin.family ? GroupChoice() : choose_group(EPI, kind, a);
+  auto group_first = [&](float us) {
+    if (g.shape < 0) return false;
+    const float mb = (float)((double)wrows * a.K * (kind == JSGRAD_W_F16 ? 2.0 : (kind == JSGRAD_W_I8 ? 1.0 : 0.5)) * 1e-6);
+    if (g.split == 1 && mb > 12.0f) us = kind == JSGRAD_W_F16 ? std::max(us, 3.8f + mb / 4.6f) : std::max(us * 1.15f, 3.8f + mb / 3.9f);
+    return g.us < us;
   };
-  bool taken;
   if (kind == JSGRAD_W_F16) {
-    if (const int rc = group_first(f.us, &taken); rc || taken) return rc;
+    if (group_first(f.us)) return run_group(EPI, kind, a, g, prof_kind);
     return run_whole(TILE_SHAPES, N_SHAPES, f, pinned('t'), launch_shape<EPI>);
   }
 
@@ -742,7 +746,7 @@ template <int EPI> static int gemm_tiled_epi(int kind, const GemmArgs &a, int pr
   const TileShape *ss = kind == JSGRAD_W_I8 ? STAGED_SHAPES_I8 : STAGED_SHAPES_NF4;
   const Choice st = choose_tile(ss, N_STAGED, EPI, a.M, wrows, a.K, 0, pinned('s'));   // takes every call
   const bool staged = q.shape < 0 || st.us < q.us;
-  if (const int rc = group_first(std::min(staged ? st.us : q.us, f.shape >= 0 ? f.us + realise_us : st.us), &taken); rc || taken) return rc;
+  if (group_first(std::min(staged ? st.us : q.us, f.shape >= 0 ? f.us + realise_us : st.us))) return run_group(EPI, kind, a, g, prof_kind);
   const size_t bytes = (size_t)wrows * a.K * 2;
   if (f.shape >= 0 && f.us + realise_us < (staged ? st.us : q.us) && bytes <= REALISED_LIMIT) {
     // into the workspace, with the K parts' sums behind it

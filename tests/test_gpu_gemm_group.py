@@ -20,13 +20,14 @@ TILES = ["g16x64", "g16x64/3", "g16x128", "g16x128/2", "g32x64", "g32x64/5", "g3
 @pytest.mark.parametrize("tile", TILES)
 def test_every_group_tile(hip, monkeypatch, kind, tile):
     monkeypatch.setenv("JSG_GEMM_TILE", tile)
-    for rows, out_f, in_f in ((2, 128, 128), (16, 256, 1152), (19, 128, 640), (57, 768, 640), (64, 128, 2048), (100, 256, 1408)):
+    k = 2 if kind == "nf4" else 1                             # stages are 64 elements, of int8 128, of nf4 256 (128 with 64 rows)
+    for rows, out_f, in_f in ((2, 128, 128 * k), (16, 256, 1152 * k), (19, 128, 640 * k), (57, 768, 640 * k), (64, 128, 2048), (57, 4224, 512), (100, 256, 1408 * k)):
         check_gemm(hip, kind, rows, out_f, in_f)
     for rows in (5, 57):
-        rows_tests.test_gemm_ffn_gate(hip, kind, rows, 640, 384)
-    rows_tests.test_gemm_qkv_rope_writes_queries_and_cache(hip, kind, 64, 3, 19, 640)
-    rows_tests.test_gemm_qkv_rope_writes_queries_and_cache(hip, kind, 128, 5, 9, 640)
-    if kind != "nf4":
+        rows_tests.test_gemm_ffn_gate(hip, kind, rows, 640 * k, 384)
+    rows_tests.test_gemm_qkv_rope_writes_queries_and_cache(hip, kind, 64, 3, 19, 640 * k)
+    rows_tests.test_gemm_qkv_rope_writes_queries_and_cache(hip, kind, 128, 5, 9, 640 * k)
+    if kind == "float16":
         check_gemm(hip, kind, 33, 128, 64)
         check_gemm(hip, kind, 9, 128, 8256)
 
@@ -34,7 +35,7 @@ def test_every_group_tile(hip, monkeypatch, kind, tile):
 @pytest.mark.parametrize("kind", ["float16", "int8", "nf4"])
 def test_as_chosen(hip, monkeypatch, kind):
     """Calls that come to the group kernel by their sizes (more than one round of the streaming kernel's blocks, long rows, 33 to 64 rows of
-    short ones), the same calls in a capture (no memory for K parts), and with scales at an odd multiple of two bytes."""
+    short ones), the same calls in a capture, and with scales at an odd multiple of two bytes."""
     sizes = ((20, 4224, 1024), (31, 256, 8192), (12, 256, 9216), (40, 384, 1024), (57, 128, 2048))
     for rows, out_f, in_f in sizes:
         check_gemm(hip, kind, rows, out_f, in_f)
