@@ -243,20 +243,23 @@ template <int EPI> __global__ __launch_bounds__(TILE_THREADS, 2) void tile256_ke
 
 // ---------------------------------------------------------------- smaller tiles, K parts
 //
-// The same eight wavefronts as 2 x 4 over a BM x BN tile, a phase per K tile (two groups half a phase apart as above), ST tiles
-// in LDS, of which ST - 1 are on their way or being read.  For inputs of some dozens to some hundred rows, where 256 x 256
+// The same eight wavefronts over a BM x BN tile, each group (half the rows) as WR x 4 / WR, a phase per K tile (two groups half a phase apart as
+// above), ST tiles in LDS, of which ST - 1 are on their way or being read.  Tiles of 192 and 256 rows: WR 2, i.e. 48 or 64 rows x 64
+// columns to a wavefront, since a group's turn is its fragment reads: 14 or 16 of them for 24 or 32 matrix instructions, 20 with 128 x 32 (256 rows: 1-3 %).  For inputs of some dozens to some hundred rows, where 256 x 256
 // tiles would leave most of the chip idle.  What bounds it, from builds with parts of the loop left out (128 x 128, 64 K
 // tiles, us): nothing but barriers 3, matrix instructions 15, direct loads 18 (the 64 bytes a clock of a CU's L1), fragment
-// reads 21 (each group reads alone and waits), all of it 30.
+// reads 21 (each group reads alone and waits), all of it 30.  192 rows: 371 x 16384 x 2048 31.7 us, with 256 35.3 (36 % of its rows past the end);
+// 700 x 6144 x 4096 45.1 | 50.2, 1100 x 16384 x 2048 85 | 96, 320 x 4096 x 14336 in parts 54.8, with 128 rows 67.8.
 template <int EPI, int BM, int BN, int ST> constexpr size_t tile_lds_bytes() { return (size_t)(BM + BN) * 128 * ST; }
-template <int EPI, int BM, int BN, int ST> __global__ __launch_bounds__(TILE_THREADS, 2) void tile_kernel(TileArgs t) {
+template <int EPI, int BM, int BN, int ST, int WR> __global__ __launch_bounds__(TILE_THREADS, 2) void tile_kernel(TileArgs t) {
   const GemmArgs &a = t.g;
   extern __shared__ __align__(16) unsigned char tile_lds[];
-  constexpr int TM = BM / 32, TN = BN / 64, NLD = (BM + BN) / 64, BUF = (BM + BN) * 128;
+  constexpr int TM = BM / 32 / WR, TN = BN / 64 * WR, NLD = (BM + BN) / 64, BUF = (BM + BN) * 128;
   static_assert(EPI != GEPI_SWIGLU || TN % 2 == 0, "a wavefront holds the w1 and the w3 tile of the same columns");
   constexpr int CW = EPI == GEPI_SWIGLU ? BN / 2 : BN;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, lq = lane >> 4;
-  const int g = wave >> 2, wn = wave & 3;
+  const int g = wave >> 2, wr = (wave & 3) / (4 / WR), wn = (wave & 3) % (4 / WR);
+  const int my_row = (g * WR + wr) * TM * 16;                 // first row of this wavefront in the tile
   const TileId id = tile_id<BM, CW>(t);
   const int m0 = id.m0;
 
@@ -290,7 +293,7 @@ template <int EPI, int BM, int BN, int ST> __global__ __launch_bounds__(TILE_THR
   h8_t af[2][TM], bf[2][TN];
   const uint32_t sw0 = (uint32_t)(lq ^ (l16 & 7)) * 16, sw1 = sw0 ^ 64;
   auto read = [&](int buf) {
-    const unsigned char *pa = tile_lds + buf * BUF + (g * TM * 16 + l16) * 128, *pb = tile_lds + buf * BUF + BM * 128 + l16 * 128;
+    const unsigned char *pa = tile_lds + buf * BUF + (my_row + l16) * 128, *pb = tile_lds + buf * BUF + BM * 128 + l16 * 128;
 #pragma unroll
     for (int k = 0; k < 2; k++) {
       const uint32_t sw = k ? sw1 : sw0;
@@ -336,7 +339,7 @@ template <int EPI, int BM, int BN, int ST> __global__ __launch_bounds__(TILE_THR
   constexpr int C16 = EPI == GEPI_SWIGLU ? TN / 2 : TN, RB = TM < 4 ? TM : 4;
   _Float16 *ep = (_Float16 *)tile_lds + wave * RB * 16 * (C16 * 16 + 8);
   static_assert((size_t)8 * RB * 16 * (C16 * 16 + 8) * 2 <= tile_lds_bytes<EPI, BM, BN, ST>(), "the turning pieces fit the tiles' LDS");
-  tile_epilogue<EPI, TM, C16, RB>(a, ep, m0 + g * TM * 16, id.col + wn * C16 * 16, [&](int i, int j, int c) {
+  tile_epilogue<EPI, TM, C16, RB>(a, ep, m0 + my_row, id.col + wn * C16 * 16, [&](int i, int j, int c) {
     if constexpr (EPI == GEPI_SWIGLU) return swiglu(acc[i][j][c], acc[i][j + TN / 2][c]);
     else return acc[i][j][c];
   });
@@ -574,16 +577,16 @@ template <int EPI> static int launch_tile256(const TileArgs &t, int prof_kind) {
   JSG_LAUNCH(prof_kind, (tile256_kernel<EPI>), dim3(tiles), dim3(TILE_THREADS), lds, t);
   return 0;
 }
-template <int EPI, int BM, int BN, int ST> static int launch_tile(const TileArgs &t, int prof_kind) {
+template <int EPI, int BM, int BN, int ST, int WR = 1> static int launch_tile(const TileArgs &t, int prof_kind) {
   constexpr int lds = (int)tile_lds_bytes<EPI, BM, BN, ST>();
   static_assert(lds + 64 <= 160 * 1024, "LDS of one compute unit");
   static bool raised = false;
   if (!raised) {
-    JSG_HIP(hipFuncSetAttribute((const void *)tile_kernel<EPI, BM, BN, ST>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    JSG_HIP(hipFuncSetAttribute((const void *)tile_kernel<EPI, BM, BN, ST, WR>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
     raised = true;
   }
   const int tiles = ((t.g.M + BM - 1) / BM) * (t.g.N / (EPI == GEPI_SWIGLU ? BN / 2 : BN));
-  JSG_LAUNCH(prof_kind, (tile_kernel<EPI, BM, BN, ST>), dim3(tiles * t.split), dim3(TILE_THREADS), lds, t);
+  JSG_LAUNCH(prof_kind, (tile_kernel<EPI, BM, BN, ST, WR>), dim3(tiles * t.split), dim3(TILE_THREADS), lds, t);
   return 0;
 }
 
@@ -609,6 +612,7 @@ static const TileShape TILE_SHAPES[] = {
   {64, 64, 64, 0.19f, 0.03f, 0.22f, 0.0f, false},
   {64, 128, 64, 0.27f, 0.064f, 0.37f, 0.0f},
   {128, 128, 64, 0.38f, 0.13f, 0.63f, 0.3f},
+  {192, 128, 64, 0.51f, 0.26f, 0.73f, 1.5f},
   {256, 128, 64, 0.55f, 0.32f, 0.85f, 1.0f},
   {256, 256, 64, 0.82f, 0.39f, 1.3f, 3.0f},
 };
@@ -620,8 +624,7 @@ static const TileShape STAGED_SHAPES_NF4[] = {{32, 128, 64, 0.53f, 0.17f, 0.29f,
 constexpr int N_SHAPES = sizeof(TILE_SHAPES) / sizeof(TILE_SHAPES[0]), N_QSHAPES = sizeof(QTILE_SHAPES_I8) / sizeof(QTILE_SHAPES_I8[0]), N_STAGED = sizeof(STAGED_SHAPES_I8) / sizeof(STAGED_SHAPES_I8[0]);
 
 // Which shape and how many K parts: the least of an estimate of the launch's time (4.5 us for start and first tiles; for K parts 1.7 us
-// and the sums' way through memory).  Over the measured sizes the choice is 0.7 % slower than the best shape on average, 2.5 % at
-// the ninth decile.  Examples, us with weights from memory, this choice | others: 371 x 2048 x 8192 128x128 in 5 parts 26.3 | in 3 parts
+// and the sums' way through memory).  Over the measured sizes the choice is 0.9 % slower than the best shape on average.  Examples, us with weights from memory, this choice | others: 371 x 2048 x 8192 128x128 in 5 parts 26.3 | in 3 parts
 // 32.2, 64x128 in 2 32.9, 256x128 in 7 34.4; 371 x 2048 x 2048 64x64 12.7 | 64x128 in 2 parts 12.4, in one 15.5; 700 x 28672 x 4096
 // 256x128 185 | 256x256 188, 128x128 223; 2048 x 6144 x 4096 256x256 90 | 128x128 111, 256x128 112; int8 codes, 57 x 5120 x 3072 64x64 in
 // 3 parts 11.2 | 64x128 in 5 12.4, 64x64 in 6 12.9.
@@ -682,8 +685,9 @@ template <int EPI> static int launch_shape(int s, const TileArgs &t, int prof_ki
     case 0: if constexpr (EPI != GEPI_SWIGLU) return launch_tile<EPI, 64, 64, 4>(t, prof_kind); else break;
     case 1: return launch_tile<EPI, 64, 128, 4>(t, prof_kind);
     case 2: return launch_tile<EPI, 128, 128, 4>(t, prof_kind);
-    case 3: return launch_tile<EPI, 256, 128, 3>(t, prof_kind);
-    case 4: return launch_tile256<EPI>(t, prof_kind);
+    case 3: return launch_tile<EPI, 192, 128, 3, 2>(t, prof_kind);
+    case 4: return launch_tile<EPI, 256, 128, 3, 2>(t, prof_kind);
+    case 5: return launch_tile256<EPI>(t, prof_kind);
   }
   return fail("jsgrad_hip_gemm: no tile shape");
 }
