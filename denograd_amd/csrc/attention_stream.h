@@ -13,10 +13,21 @@
 
 namespace jsg {
 
-constexpr int ATT_STREAM_CHUNK_MIN = 32;   // shorter chunks finish no sooner and only add partial results for the merge to fetch
-__host__ __device__ __forceinline__ int att_stream_chunk_rows(int T, int nsplit) {
+// Rows per chunk for T visible positions of `pairs` (sequence, kv head) pairs: at least T / nsplit, and not so few that the merge costs
+// more than the chunks save.  A block asks for 64 (head_dim 64) or 32 rows (head_dim 128) at once and for five times as many in two
+// rounds, so what one block takes in two rounds is one chunk and nothing to merge.  us, chunks of 32 | 64 | 128 | 160 rows: head_dim 64, 5 sequences
+// 300 positions 8.7 | 7.8 | 8.8 | 9.1, 600 11.2 | 9.1 | 9.4 | 9.5, 1000 14.1 | 10.2 | 10.4 | 10.3, 16 sequences 300 10.6 | 9.6 | 9.5 | 9.8, 1000
+// 15.9 | 15.8 | 15.1 | 14.5, 2 sequences 2048 20.5 | 13.3 | 11.3 | 11.0; head_dim 128, 5 sequences 300 9.5 | 9.6 | 10.5 | 10.9, 600 12.1 | 11.2 | 11.2 |
+// 11.5, 1000 15.3 | 13.0 | 12.9 | 12.7, 32 sequences 200 15.1 | 13.8 | 12.8 | 12.6; in one chunk: 90 positions, 5 sequences 7.7 -> 7.0, 32 10.3 -> 7.9
+// (130 positions, 2 sequences 7.6 -> 7.9, 5 8.0 -> 8.1, 8 9.0 -> 8.1).
+template <int HD> __device__ __forceinline__ int att_stream_chunk_rows(int T, int nsplit, int pairs) {
+  int most = HD == 64 ? 64 : 32;
+  if (T <= (HD == 64 ? ATT_CHUNK_MAX : (pairs >= 40 ? 160 : 96))) most = ATT_CHUNK_MAX;
+  else if (pairs >= 128) most = HD == 64 && T >= 600 ? 160 : 128;
+  else if (T >= 800) most = HD == 64 && T >= 1400 ? 160 : 128;
+  else if (T >= 400) most = 64;
   const int c = (T + nsplit - 1) / nsplit;
-  return c < ATT_STREAM_CHUNK_MIN ? ATT_STREAM_CHUNK_MIN : c;
+  return c < most ? most : c;
 }
 
 // NW wavefronts per block.  COHERENT: q and the output cross between blocks of the same launch.
@@ -286,6 +297,24 @@ template <typename AT, int HD, int NREP, int NW, bool COHERENT> struct AttnStrea
       }
       __syncthreads();
     }
+    // output element i of the kv head's query heads: its P.V sum times 1 / (sum of the weights)
+    auto store_out = [&](int i, float O, float inv) {
+      AT *dst = (AT *)a.out + (size_t)g * NREP * HD + i;
+      const float r = Act<AT>::rn(O * inv);                   // the cast of the P.V result
+      if (a.out_tagged != nullptr) tw_store(a.out_tagged + (size_t)g * NREP * HD + i, a.out_tag, r);
+      else if constexpr (COHERENT) st_coherent(dst, (AT)r);
+      else *dst = (AT)r;
+    };
+    if (n_active == 1) {                                      // nothing to merge: the weight of the one chunk is 1
+      for (int i = tid; i < NREP * HD; i += nthreads) {
+        const int j = i / HD, d = i % HD;
+        float v = 0.0f;
+#pragma unroll
+        for (int w = 0; w < SLOTS; w++) v += sm.o_part[w][j][d];
+        store_out(i, v, 1.0f / sm.l_sh[j]);
+      }
+      return;
+    }
     float *mine = a.partial + ((size_t)g * a.nsplit + split) * NREP * (HD + 2);
     for (int i = tid; i < NREP * HD; i += nthreads) {
       const int j = i / HD, d = i % HD;
@@ -341,14 +370,6 @@ template <typename AT, int HD, int NREP, int NW, bool COHERENT> struct AttnStrea
     }
     __syncthreads();
     // ... then every thread sums its output elements over the chunks in chunk order, two elements at a time
-    auto finish = [&](int i, float O) {
-      const int j = i / HD, d = i % HD;
-      AT *dst = (AT *)a.out + (size_t)(g * NREP + j) * HD + d;
-      const float r = Act<AT>::rn(O * sm.l_sh[j]);  // the cast of the P.V result
-      if (a.out_tagged != nullptr) tw_store(a.out_tagged + (size_t)(g * NREP + j) * HD + d, a.out_tag, r);
-      else if constexpr (COHERENT) st_coherent(dst, (AT)r);
-      else *dst = (AT)r;
-    };
     auto ld_part = [&](const float *po, int s) { return ld_coherent(po + (size_t)(s < n_active ? s : n_active - 1) * NREP * (HD + 2)); };
     constexpr bool PAIRS = NREP * HD > NW * 64;              // more elements than threads: a thread has at least two
     for (int i0 = tid; i0 < NREP * HD; i0 += (PAIRS ? 2 : 1) * nthreads) {
@@ -386,8 +407,8 @@ template <typename AT, int HD, int NREP, int NW, bool COHERENT> struct AttnStrea
         Oa = add(parta, ja, s0, Oa);
         if constexpr (PAIRS) Ob = add(partb, jb, s0, Ob);
       }
-      finish(i0, Oa);
-      if (two) finish(i1, Ob);
+      store_out(i0, Oa, sm.l_sh[ja]);
+      if (two) store_out(i1, Ob, sm.l_sh[jb]);
     }
     if (tid == 0) __hip_atomic_store(&a.counters[g], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }

@@ -1,0 +1,36 @@
+"""Attention of many sequences at one new position each, where the chunks' length changes with the position and the number of
+sequences: one chunk in all (nothing to merge), the first with two, and both sides of every line between lengths.  One workspace
+serves all positions in turn, so each launch leaves its counters as it found them.
+
+Tolerance: the float64 result rounded to fp16 and the float sums in another order, as in test_gpu_rows."""
+import numpy as np
+import pytest
+
+from denograd_amd.ffi import check
+from denograd_amd.tensor import Tensor
+from tests.test_gpu_rows import attention_ref
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("hd,B,H,KV,positions", [
+    (64, 2, 8, 2, (1, 64, 65, 256, 257, 300, 799, 800, 1399, 1400, 1)),
+    (128, 2, 6, 2, (1, 32, 33, 160, 161, 399, 400, 799, 800, 160, 1500)),
+    (64, 20, 8, 8, (256, 257, 599, 600, 3)), (128, 20, 16, 8, (160, 161, 600, 97)),
+    (64, 3, 8, 1, (70, 300)), (128, 3, 8, 1, (70, 300)),
+])
+def test_attn_decode_batch_at_the_chunk_lines(hip, hd, B, H, KV, positions):
+    rng = np.random.default_rng(hd + B)
+    ctx = max(positions) + 5
+    q = rng.standard_normal((B, H * hd)).astype(np.float16)
+    ck, cv = (rng.standard_normal((B, ctx, KV, hd)).astype(np.float16) for _ in range(2))
+    tq, tk, tv = Tensor(q), Tensor(ck), Tensor(cv)
+    ws = Tensor.zeros((hip.jsgrad_hip_attn_batch_workspace_bytes(B, H, KV, hd),), "uint8")
+    for T in positions:
+        st = Tensor(np.array([0, T - 1], np.int32))
+        out = Tensor.full((B + 1, H * hd), 7.0, "float16")
+        check(hip.jsgrad_hip_attn_decode_batch(tq.ptr, tk.ptr, tv.ptr, st.ptr, out.ptr, ws.ptr, B, H, KV, hd, ctx))
+        got = out.numpy().astype(np.float64)
+        assert np.all(got[B] == 7.0)
+        ref = attention_ref(q, ck, cv, B, 1, T - 1, H, KV, hd)
+        assert np.max(np.abs(got[:B] - ref)) < 4e-3, T
