@@ -36,6 +36,7 @@ SIGNATURES: dict[str, tuple[list, object]] = {
     "jsgrad_hip_mem_info": ([C.POINTER(_sz), C.POINTER(_sz)], _i32),
     "jsgrad_hip_copyin": ([_vp, _vp, _sz], _i32),
     "jsgrad_hip_set_state": ([_vp, _i32, _i32], _i32),
+    "jsgrad_hip_read_step": ([_vp, _vp, _vp, _vp], _i32),
     "jsgrad_hip_copyout": ([_vp, _vp, _sz], _i32),
     "jsgrad_hip_copy": ([_vp, _vp, _sz], _i32),
     "jsgrad_hip_memset": ([_vp, _i32, _sz], _i32),

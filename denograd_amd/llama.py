@@ -327,6 +327,17 @@ class Transformer:
         check(ffi.load().jsgrad_hip_attn_decode_status(self._ctx.workspace.ptr, self.n_heads, self.n_kv_heads, self.dim // self.n_heads, C.byref(e)))
         return e.value
 
+    def read_token(self) -> int:
+        """The token of the last step (state[0]), once everything queued is done: one wait for it and for the error word of the
+        step's attention launches.  Raises as check_errors does."""
+        ctx = self._prepare()
+        words = (C.c_int32 * 2)()
+        check(ffi.load().jsgrad_hip_read_step(self.state.ptr, ctx.attn_wo_ws.ptr if ctx.attn_wo_ws is not None else None,
+                                              None if ctx.fuse_attn_wo else ctx.workspace.ptr, words))
+        if words[1]:
+            self.check_errors()
+        return words[0]
+
     def check_errors(self) -> None:
         """Raise if a bounded wait inside an attention launch ran out since the model was made (another process holding
         compute units, or a device fault): the tokens after that point are not to be trusted.  Called wherever the host

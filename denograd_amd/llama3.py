@@ -227,10 +227,8 @@ class Llama3:
     # ---- inference (token ids in, token ids out)
     def _call(self, tok: int) -> int:
         """llama3.ts:334-337: one model call and the per-token device->host read."""
-        res = self.model.call(np.array([[tok]], np.int32), self.start_pos, self.temperature, self.top_k, self.top_p, self.alpha_f, self.alpha_p)
-        tok = int(res.item())
-        self.model.check_errors()
-        return tok
+        self.model.call(np.array([[tok]], np.int32), self.start_pos, self.temperature, self.top_k, self.top_p, self.alpha_f, self.alpha_p)
+        return self.model.read_token()
 
     def _prefill(self, toks: list[int]) -> None:
         """llama3.ts:297-312: skip the shared prefix of the previous prompt when starting over, then feed tokens one at a time."""

@@ -67,6 +67,11 @@ int jsgrad_hip_copyout(void *host_dst, const void *src, size_t nbytes);
 /* The two words of a model's step state, {token, position}, which the reference keeps as a one-element tensor and a bound
  * Variable (models/llama3.ts:300-305, models/llama.ts:214-220): written in stream order, without waiting for the stream. */
 int jsgrad_hip_set_state(int32_t *state, int token, int position);
+/* The read of a token per step that the reference's loop has (`.item()`, models/llama3.ts:334-337), with the error word of the step's
+ * attention launches beside it: waits for everything queued, then host_out_words = {state[0], error}.  attn_wo_workspace: of
+ * jsgrad_hip_attn_wo, or null and attn_workspace: of jsgrad_hip_attn_decode, or both null (error 0).  An error word is left as it is:
+ * jsgrad_hip_attn_wo_status / jsgrad_hip_attn_decode_status say and do the rest. */
+int jsgrad_hip_read_step(const int32_t *state, const void *attn_wo_workspace, const void *attn_workspace, int32_t *host_out_words);
 /* BufferCopy between two device buffers (engine/realize.ts:92-122, Allocator._transfer allocator.ts:46). */
 int jsgrad_hip_copy(void *dst, const void *src, size_t nbytes);
 /* Tensor.zeros(...).contiguous().realize() for the KV cache (models/llama.ts:79): byte fill. */

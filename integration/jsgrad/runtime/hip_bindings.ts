@@ -22,6 +22,7 @@ const SYMBOLS = {
   jsgrad_hip_copyin: { parameters: [P, B, U], result: I }, // dst, host_src, nbytes
   jsgrad_hip_copyout: { parameters: [B, P, U], result: I }, // host_dst, src, nbytes
   jsgrad_hip_set_state: { parameters: [P, I, I], result: I }, // state, token, position
+  jsgrad_hip_read_step: { parameters: [P, P, P, B], result: I }, // state, attn_wo_workspace, attn_workspace, host_out_words
   jsgrad_hip_copy: { parameters: [P, P, U], result: I }, // dst, src, nbytes
   jsgrad_hip_memset: { parameters: [P, I, U], result: I }, // dst, byte, nbytes
   jsgrad_hip_sync: { parameters: [], result: I },
