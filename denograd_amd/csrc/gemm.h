@@ -24,6 +24,9 @@ struct GemmArgs {
   const _Float16 *rope_table;         // [2*max_context][hd/2][2]
   _Float16 *cache_k, *cache_v;        // [B][max_context][n1]
   int seq_len, start_pos, head_dim, max_context;
+  // x is to be RMSNorm'ed first: gemm_few.hip does that in registers, for the others x is normed in memory
+  const _Float16 *norm_w;             // [K] or null
+  float eps, inv_k;                   // inv_k: float(1 / K)
   bool pins;                          // some variable of the environment begins with JSG_: a test may want a certain kernel or tile
 };
 
@@ -66,6 +69,21 @@ __device__ __forceinline__ void dma16_stream(i4_t rs, uint32_t voff, uint32_t so
 // the same with four bytes per lane
 __device__ __forceinline__ void dma4(i4_t rs, uint32_t voff, uint32_t soff, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rs), "s"(soff) : "memory");
+}
+
+// RMSNorm.call (nn/index.ts:586-588) with the rounding points of rmsnorm_rows_kernel: the factor of a row with this sum of squares, and
+// eight elements of it
+__device__ __forceinline__ float norm_factor(const GemmArgs &a, float sum) { return __fsqrt_rn(__fdiv_rn(1.0f, __fadd_rn(__fmul_rn(sum, a.inv_k), a.eps))); }
+__device__ __forceinline__ h8_t norm_piece(h8_t x, float r, h8_t w) {
+  h8_t n;
+#pragma unroll
+  for (int e = 0; e < 8; e++) n[e] = (_Float16)__fmul_rn((float)x[e], r);
+  return n * w;
+}
+__device__ __forceinline__ float square_sum(h8_t x, float s) {
+#pragma unroll
+  for (int e = 0; e < 8; e++) s = fmaf((float)x[e], (float)x[e], s);
+  return s;
 }
 
 // What a test asks for, or null.  Looking a variable up costs a walk through the environment, so a call makes one walk for all of them.

@@ -329,13 +329,23 @@ template <int KIND, int EPI> static int dispatch_skinny(const GemmArgs &a, int p
   return two ? launch_skinny<KIND, EPI, 2, 2>(a, prof_kind) : launch_skinny<KIND, EPI, 2, 1>(a, prof_kind);
 }
 
-template <int EPI> static int dispatch_gemm(int kind, const GemmArgs &a, int prof_kind) {
+// x normed into xn, which is what the product reads then
+static int norm_first(GemmArgs &a, _Float16 *xn) {
+  if (const int rc = jsgrad_hip_rmsnorm_rows(a.x, a.norm_w, xn, a.M, a.K, a.eps)) return rc;
+  a.x = xn;
+  a.norm_w = nullptr;
+  return 0;
+}
+template <int EPI> static int dispatch_gemm(int kind, GemmArgs a, int prof_kind, _Float16 *xn = nullptr) {
   bool taken = false;
-  if (const char *e = pin_env(a, "JSG_GEMM_TILE"); e && *e == 'g') {   // tests
-    const int rc = gemm_group(EPI, kind, a, prof_kind, &taken);
+  const char *const pin = pin_env(a, "JSG_GEMM_TILE");
+  const bool group = pin && *pin == 'g';                      // tests
+  if (!group) {
+    const int rc = gemm_few(EPI, kind, a, prof_kind, &taken);
     if (taken || rc) return rc;
   }
-  { const int rc = gemm_few(EPI, kind, a, prof_kind, &taken); if (taken || rc) return rc; }
+  if (a.norm_w)
+    if (const int rc = norm_first(a, xn)) return rc;
   { const int rc = gemm_group(EPI, kind, a, prof_kind, &taken); if (taken || rc) return rc; }
   if (kind == JSGRAD_W_F16) { const int rc = dispatch_skinny<JSGRAD_W_F16, EPI>(a, prof_kind, &taken); if (taken) return rc; }
   if (kind == JSGRAD_W_I8) { const int rc = dispatch_skinny<JSGRAD_W_I8, EPI>(a, prof_kind, &taken); if (taken) return rc; }
@@ -356,42 +366,48 @@ static int check_gemm(const char *who, int kind, int rows, int in_f) {
   return 0;
 }
 
-}  // namespace jsg
+// An input that is normed first: its norm's weights, and rows of memory for the result where no kernel norms x on its way
+struct NormFirst { const void *weight; float eps; void *xn; };
+static int set_norm(const char *who, const NormFirst *norm, GemmArgs &a) {
+  if (!norm) return 0;
+  JSG_REQUIRE(norm->weight && norm->xn, "%s: null pointer argument", who);
+  JSG_REQUIRE(aligned16(norm->weight) && aligned16(norm->xn), "%s: the norm's weight and xn must be 16-byte aligned", who);
+  a.norm_w = (const _Float16 *)norm->weight;
+  a.eps = norm->eps;
+  a.inv_k = (float)(1.0 / (double)a.K);
+  return 0;
+}
 
-using namespace jsg;
-
-extern "C" {
-
-int jsgrad_hip_gemm(int kind, const void *w, const void *scale, int out_f, int in_f, const void *x, int rows, void *y, const void *residual) {
-  JSG_READY();
-  if (int rc = check_gemm("jsgrad_hip_gemm", kind, rows, in_f)) return rc;
-  JSG_REQUIRE(w && x && y, "jsgrad_hip_gemm: null pointer argument");
-  JSG_REQUIRE(kind == JSGRAD_W_F16 || scale, "jsgrad_hip_gemm: quantised weights need their scales");
-  JSG_REQUIRE(out_f > 0 && out_f % GEMM_N_ALIGN == 0, "jsgrad_hip_gemm: out_features %d must be a positive multiple of %d", out_f, GEMM_N_ALIGN);
-  JSG_REQUIRE(aligned16(w) && aligned16(x) && aligned16(y) && aligned16(residual), "jsgrad_hip_gemm: w, x, y and residual must be 16-byte aligned");
+static int plain_gemm(const char *who, const NormFirst *norm, int kind, const void *w, const void *scale, int out_f, int in_f, const void *x, int rows,
+                      void *y, const void *residual) {
+  if (int rc = check_gemm(who, kind, rows, in_f)) return rc;
+  JSG_REQUIRE(w && x && y, "%s: null pointer argument", who);
+  JSG_REQUIRE(kind == JSGRAD_W_F16 || scale, "%s: quantised weights need their scales", who);
+  JSG_REQUIRE(out_f > 0 && out_f % GEMM_N_ALIGN == 0, "%s: out_features %d must be a positive multiple of %d", who, out_f, GEMM_N_ALIGN);
+  JSG_REQUIRE(aligned16(w) && aligned16(x) && aligned16(y) && aligned16(residual), "%s: w, x, y and residual must be 16-byte aligned", who);
   GemmArgs a = {};
   a.pins = any_pins();
   a.w0 = w; a.s0 = (const _Float16 *)scale; a.n0 = out_f;
   a.M = rows; a.N = out_f; a.K = in_f;
   a.x = (const _Float16 *)x; a.y = (_Float16 *)y; a.residual = (const _Float16 *)residual;
-  return dispatch_gemm<GEPI_STORE>(kind, a, PROF_GEMM);
+  if (int rc = set_norm(who, norm, a)) return rc;
+  return dispatch_gemm<GEPI_STORE>(kind, a, PROF_GEMM, norm ? (_Float16 *)norm->xn : nullptr);
 }
 
-int jsgrad_hip_gemm_qkv_rope(int kind, const void *wq, const void *sq, const void *wk, const void *sk, const void *wv, const void *sv, const void *x,
-                             int rows, int seq_len, int start_pos, const void *rope_table, void *q_out, void *cache_k, void *cache_v, int dim,
-                             int n_heads, int n_kv_heads, int head_dim, int max_context) {
-  JSG_READY();
-  if (int rc = check_gemm("jsgrad_hip_gemm_qkv_rope", kind, rows, dim)) return rc;
-  JSG_REQUIRE(wq && wk && wv && x && rope_table && q_out && cache_k && cache_v, "jsgrad_hip_gemm_qkv_rope: null pointer argument");
-  JSG_REQUIRE(kind == JSGRAD_W_F16 || (sq && sk && sv), "jsgrad_hip_gemm_qkv_rope: quantised weights need their scales");
-  JSG_REQUIRE(head_dim > 0 && head_dim % 8 == 0 && n_heads > 0 && n_kv_heads > 0, "jsgrad_hip_gemm_qkv_rope: bad head geometry (head_dim a multiple of 8)");
+static int qkv_rope_gemm(const char *who, const NormFirst *norm, int kind, const void *wq, const void *sq, const void *wk, const void *sk, const void *wv, const void *sv,
+                         const void *x, int rows, int seq_len, int start_pos, const void *rope_table, void *q_out, void *cache_k, void *cache_v, int dim,
+                         int n_heads, int n_kv_heads, int head_dim, int max_context) {
+  if (int rc = check_gemm(who, kind, rows, dim)) return rc;
+  JSG_REQUIRE(wq && wk && wv && x && rope_table && q_out && cache_k && cache_v, "%s: null pointer argument", who);
+  JSG_REQUIRE(kind == JSGRAD_W_F16 || (sq && sk && sv), "%s: quantised weights need their scales", who);
+  JSG_REQUIRE(head_dim > 0 && head_dim % 8 == 0 && n_heads > 0 && n_kv_heads > 0, "%s: bad head geometry (head_dim a multiple of 8)", who);
   JSG_REQUIRE(aligned16(wq) && aligned16(wk) && aligned16(wv) && aligned16(x) && aligned16(rope_table) && aligned16(q_out) && aligned16(cache_k) && aligned16(cache_v),
-              "jsgrad_hip_gemm_qkv_rope: weights, x, rope_table, q_out and the caches must be 16-byte aligned");
+              "%s: weights, x, rope_table, q_out and the caches must be 16-byte aligned", who);
   const int nq = n_heads * head_dim, nkv = n_kv_heads * head_dim;
-  JSG_REQUIRE(nq % GEMM_N_ALIGN == 0 && nkv % GEMM_N_ALIGN == 0, "jsgrad_hip_gemm_qkv_rope: n_heads*head_dim %d and n_kv_heads*head_dim %d must be multiples of %d", nq, nkv,
+  JSG_REQUIRE(nq % GEMM_N_ALIGN == 0 && nkv % GEMM_N_ALIGN == 0, "%s: n_heads*head_dim %d and n_kv_heads*head_dim %d must be multiples of %d", who, nq, nkv,
               GEMM_N_ALIGN);
-  JSG_REQUIRE(seq_len > 0 && rows % seq_len == 0, "jsgrad_hip_gemm_qkv_rope: %d rows are not whole sequences of %d", rows, seq_len);
-  JSG_REQUIRE(start_pos >= 0 && start_pos + seq_len <= max_context, "jsgrad_hip_gemm_qkv_rope: positions [%d, %d) outside the cache of %d", start_pos,
+  JSG_REQUIRE(seq_len > 0 && rows % seq_len == 0, "%s: %d rows are not whole sequences of %d", who, rows, seq_len);
+  JSG_REQUIRE(start_pos >= 0 && start_pos + seq_len <= max_context, "%s: positions [%d, %d) outside the cache of %d", who, start_pos,
               start_pos + seq_len, max_context);
   GemmArgs a = {};
   a.pins = any_pins();
@@ -402,24 +418,71 @@ int jsgrad_hip_gemm_qkv_rope(int kind, const void *wq, const void *sq, const voi
   a.x = (const _Float16 *)x; a.y = (_Float16 *)q_out;
   a.rope_table = (const _Float16 *)rope_table; a.cache_k = (_Float16 *)cache_k; a.cache_v = (_Float16 *)cache_v;
   a.seq_len = seq_len; a.start_pos = start_pos; a.head_dim = head_dim; a.max_context = max_context;
-  return dispatch_gemm<GEPI_ROPE_KV>(kind, a, PROF_GEMM);
+  if (int rc = set_norm(who, norm, a)) return rc;
+  return dispatch_gemm<GEPI_ROPE_KV>(kind, a, PROF_GEMM, norm ? (_Float16 *)norm->xn : nullptr);
 }
 
-int jsgrad_hip_gemm_ffn_gate(int kind, const void *w1, const void *s1, const void *w3, const void *s3, const void *x, int rows, void *y, int dim,
-                             int hidden) {
-  JSG_READY();
-  if (int rc = check_gemm("jsgrad_hip_gemm_ffn_gate", kind, rows, dim)) return rc;
-  JSG_REQUIRE(w1 && w3 && x && y, "jsgrad_hip_gemm_ffn_gate: null pointer argument");
-  JSG_REQUIRE(kind == JSGRAD_W_F16 || (s1 && s3), "jsgrad_hip_gemm_ffn_gate: quantised weights need their scales");
-  JSG_REQUIRE(hidden > 0 && hidden % GEMM_N_ALIGN == 0, "jsgrad_hip_gemm_ffn_gate: hidden_dim %d must be a positive multiple of %d", hidden, GEMM_N_ALIGN);
-  JSG_REQUIRE(aligned16(w1) && aligned16(w3) && aligned16(x) && aligned16(y), "jsgrad_hip_gemm_ffn_gate: w1, w3, x and g must be 16-byte aligned");
+static int ffn_gate_gemm(const char *who, const NormFirst *norm, int kind, const void *w1, const void *s1, const void *w3, const void *s3,
+                         const void *x, int rows, void *y, int dim, int hidden) {
+  if (int rc = check_gemm(who, kind, rows, dim)) return rc;
+  JSG_REQUIRE(w1 && w3 && x && y, "%s: null pointer argument", who);
+  JSG_REQUIRE(kind == JSGRAD_W_F16 || (s1 && s3), "%s: quantised weights need their scales", who);
+  JSG_REQUIRE(hidden > 0 && hidden % GEMM_N_ALIGN == 0, "%s: hidden_dim %d must be a positive multiple of %d", who, hidden, GEMM_N_ALIGN);
+  JSG_REQUIRE(aligned16(w1) && aligned16(w3) && aligned16(x) && aligned16(y), "%s: w1, w3, x and g must be 16-byte aligned", who);
   GemmArgs a = {};
   a.pins = any_pins();
   a.w0 = w1; a.w1 = w3; a.s0 = (const _Float16 *)s1; a.s1 = (const _Float16 *)s3;
   a.n0 = hidden; a.n1 = hidden;
   a.M = rows; a.N = hidden; a.K = dim;
   a.x = (const _Float16 *)x; a.y = (_Float16 *)y;
-  return dispatch_gemm<GEPI_SWIGLU>(kind, a, PROF_GEMM);
+  if (int rc = set_norm(who, norm, a)) return rc;
+  return dispatch_gemm<GEPI_SWIGLU>(kind, a, PROF_GEMM, norm ? (_Float16 *)norm->xn : nullptr);
+}
+
+}  // namespace jsg
+
+using namespace jsg;
+
+extern "C" {
+
+int jsgrad_hip_gemm(int kind, const void *w, const void *scale, int out_f, int in_f, const void *x, int rows, void *y, const void *residual) {
+  JSG_READY();
+  return plain_gemm("jsgrad_hip_gemm", nullptr, kind, w, scale, out_f, in_f, x, rows, y, residual);
+}
+int jsgrad_hip_gemm_norm(int kind, const void *w, const void *scale, int out_f, int in_f, const void *x, const void *norm_weight, float eps, void *xn,
+                         int rows, void *y) {
+  JSG_READY();
+  const NormFirst norm = {norm_weight, eps, xn};
+  return plain_gemm("jsgrad_hip_gemm_norm", &norm, kind, w, scale, out_f, in_f, x, rows, y, nullptr);
+}
+
+int jsgrad_hip_gemm_qkv_rope(int kind, const void *wq, const void *sq, const void *wk, const void *sk, const void *wv, const void *sv, const void *x,
+                             int rows, int seq_len, int start_pos, const void *rope_table, void *q_out, void *cache_k, void *cache_v, int dim,
+                             int n_heads, int n_kv_heads, int head_dim, int max_context) {
+  JSG_READY();
+  return qkv_rope_gemm("jsgrad_hip_gemm_qkv_rope", nullptr, kind, wq, sq, wk, sk, wv, sv, x, rows,
+                       seq_len, start_pos, rope_table, q_out, cache_k, cache_v, dim, n_heads, n_kv_heads, head_dim, max_context);
+}
+int jsgrad_hip_gemm_qkv_rope_norm(int kind, const void *wq, const void *sq, const void *wk, const void *sk, const void *wv, const void *sv,
+                                  const void *x, const void *norm_weight, float eps, void *xn, int rows, int seq_len, int start_pos,
+                                  const void *rope_table, void *q_out, void *cache_k, void *cache_v, int dim, int n_heads, int n_kv_heads,
+                                  int head_dim, int max_context) {
+  JSG_READY();
+  const NormFirst norm = {norm_weight, eps, xn};
+  return qkv_rope_gemm("jsgrad_hip_gemm_qkv_rope_norm", &norm, kind, wq, sq, wk, sk, wv, sv, x, rows,
+                       seq_len, start_pos, rope_table, q_out, cache_k, cache_v, dim, n_heads, n_kv_heads, head_dim, max_context);
+}
+
+int jsgrad_hip_gemm_ffn_gate(int kind, const void *w1, const void *s1, const void *w3, const void *s3, const void *x, int rows, void *y, int dim,
+                             int hidden) {
+  JSG_READY();
+  return ffn_gate_gemm("jsgrad_hip_gemm_ffn_gate", nullptr, kind, w1, s1, w3, s3, x, rows, y, dim, hidden);
+}
+int jsgrad_hip_gemm_ffn_gate_norm(int kind, const void *w1, const void *s1, const void *w3, const void *s3, const void *x, const void *norm_weight,
+                                  float eps, void *xn, int rows, void *y, int dim, int hidden) {
+  JSG_READY();
+  const NormFirst norm = {norm_weight, eps, xn};
+  return ffn_gate_gemm("jsgrad_hip_gemm_ffn_gate_norm", &norm, kind, w1, s1, w3, s3, x, rows, y, dim, hidden);
 }
 
 }  // extern "C"

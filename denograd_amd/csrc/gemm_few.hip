@@ -102,9 +102,35 @@ template <int KIND, int EPI, int SB, int PARTS, bool LONG> __global__ __launch_b
 #pragma unroll
     for (int f = 0; f < NF; f++) xf[f] = *(const h8_t *)(xr + (f / MPR) * (64 / KB) + (f % MPR) * 8);
   }
+  constexpr bool NORM = NF <= 16;                             // with the norm's weights x takes twice the registers
+  const bool norm = NORM && a.norm_w;
+  if constexpr (NORM)
+    if (norm) {
+      // Normed in registers: sums over a wavefront's share, the eight shares through LDS in order.  Using x waits for all loads before it and behind
+      // it, so the first step goes out ahead of that and the others behind.
+      h8_t wf[NF];
+      const _Float16 *wr = a.norm_w + k_first / KB + lq * (16 / KB);
+#pragma unroll
+      for (int f = 0; f < NF; f++) wf[f] = *(const h8_t *)(wr + (f / MPR) * (64 / KB) + (f % MPR) * 8);
+      if (n_steps > 0) issue(0);
+      float ss = 0.0f;
+#pragma unroll
+      for (int f = 0; f < NF; f++) ss = square_sum(xf[f], ss);
+      ss = add_xor32(add_xor16(ss));
+      float *const part = (float *)(few_lds + FW_WAVES * S::RING);
+      if (lq == 0) part[wave * 16 + l16] = ss;
+      lds_barrier();
+      float tot = part[l16];
+#pragma unroll
+      for (int w = 1; w < FW_WAVES; w++) tot += part[w * 16 + l16];
+      const float r = norm_factor(a, tot);
+#pragma unroll
+      for (int f = 0; f < NF; f++) xf[f] = norm_piece(xf[f], r, wf[f]);
+      lds_barrier();                                          // the sums have been read
+    }
 #pragma unroll
   for (int i = 0; i < NS; i++)
-    if (i < n_steps) issue(i);
+    if (i < n_steps && !(i == 0 && norm)) issue(i);
   // Waited for here, or the compiler, which does not count the direct loads, would wait for all of them at the first use of x in
   // every turn of the loop below.  Where there is hardly a second turn the steps behind the first need not have landed yet.
   if constexpr (LONG)
@@ -238,6 +264,11 @@ int gemm_few(int epi, int kind, const GemmArgs &a, int prof_kind, bool *taken) {
   // fp16 rows of 16 KiB behind more than 8 rows of x go to gemm_group.hip, which reads x from LDS: 2048 x 8192, 16 rows 12.8 | 10.9 there, 3072 x 8192
   // 15.5 | 12.8 (8 rows 9.8 | 10.9, 12.6 | 13.0).
   if (kind == JSGRAD_W_F16 && a.M > 8 && a.K > 4096) return 0;
+  // A norm in front is done in registers, x and the norm's weights at once: rows of half the length at most.  us per decode step, norms as launches of
+  // their own (33 of the 1B shape) | here: 1B shape 2 rows 897 | 832, 5 rows 903 | 846, 12 rows 968 | 908, 16 rows 1006 | 944; int8 14 layers of the 3B shape
+  // with 6 rows 830 | 810, of the 8B shape with 4 rows 1131 | 1113.  In gemm_group.hip, whose blocks read all of x for it and norm every fragment, it
+  // costs more than the launches: 8B int8 16 rows 3321 | 3403, 8B NF4 16 layers 8 rows 1403 | 1467.
+  if (a.norm_w && a.K > 4096) return 0;
   const size_t codes = (size_t)a.N * (epi == GEPI_SWIGLU ? 2 : 1) * a.K;
   if (kind == JSGRAD_W_I8 && (codes > (size_t)36 << 20 || (a.M > 8 && a.K > 3072))) return 0;
   if (pin_env(a, "JSG_GEMM_NO_SKINNY") || pin_env(a, "JSG_GEMM_SKINNY_TILES") || pin_env(a, "JSG_SG_TPW")) return 0;   // tests that want one of the other kernels

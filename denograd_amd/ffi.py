@@ -78,6 +78,9 @@ SIGNATURES: dict[str, tuple[list, object]] = {
     "jsgrad_hip_gemm": ([_i32, _vp, _vp, _i32, _i32, _vp, _i32, _vp, _vp], _i32),
     "jsgrad_hip_gemm_qkv_rope": ([_i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32], _i32),
     "jsgrad_hip_gemm_ffn_gate": ([_i32, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _i32, _i32], _i32),
+    "jsgrad_hip_gemm_norm": ([_i32, _vp, _vp, _i32, _i32, _vp, _vp, _f32, _vp, _i32, _vp], _i32),
+    "jsgrad_hip_gemm_qkv_rope_norm": ([_i32, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _f32, _vp, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32], _i32),
+    "jsgrad_hip_gemm_ffn_gate_norm": ([_i32, _vp, _vp, _vp, _vp, _vp, _vp, _f32, _vp, _i32, _vp, _i32, _i32], _i32),
     "jsgrad_hip_attn_prefill": ([_vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32], _i32),
     "jsgrad_hip_attn_batch_workspace_bytes": ([_i32, _i32, _i32, _i32], _sz),
     "jsgrad_hip_attn_decode_batch": ([_vp, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32], _i32),

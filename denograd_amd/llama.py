@@ -48,16 +48,20 @@ class Attention:
         if self.cache_kv is None or self.cache_kv.shape[1] != bsz:
             self.cache_kv = Tensor.zeros((2, bsz, self.max_context, self.n_kv_heads, self.head_dim), dtype, device)
 
-    def call_rows(self, xn: Tensor, bsz: int, seqlen: int, start_pos: int, state: Tensor, freqs_cis: Tensor, rows: "_RowScratch", residual: Tensor, out: Tensor) -> Tensor:
-        """Several positions and/or sequences: xn [bsz*seqlen, dim] is the normed input; out = residual + wo(attention)."""
+    def call_rows(self, xn: Tensor, bsz: int, seqlen: int, start_pos: int, state: Tensor, freqs_cis: Tensor, rows: "_RowScratch", residual: Tensor, out: Tensor,
+                  norm: RMSNorm | None = None) -> Tensor:
+        """Several positions and/or sequences: xn [bsz*seqlen, dim] is the normed input, or what norm is to be applied to; out = residual + wo(attention)."""
         lib = ffi.load()
         half = self.cache_kv.nbytes // 2
         ck, cv = self.cache_kv.ptr, self.cache_kv.ptr + half
         n = bsz * seqlen
         sp = lambda l: l.scale.ptr if l.scale is not None else None
-        check(lib.jsgrad_hip_gemm_qkv_rope(self.wq.kind, self.wq.weight.ptr, sp(self.wq), self.wk.weight.ptr, sp(self.wk), self.wv.weight.ptr, sp(self.wv),
-                                           xn.ptr, n, seqlen, start_pos, freqs_cis.ptr, rows.q.ptr, ck, cv,
-                                           self.dim, self.n_heads, self.n_kv_heads, self.head_dim, self.max_context))
+        weights = (self.wq.kind, self.wq.weight.ptr, sp(self.wq), self.wk.weight.ptr, sp(self.wk), self.wv.weight.ptr, sp(self.wv), xn.ptr)
+        rest = (n, seqlen, start_pos, freqs_cis.ptr, rows.q.ptr, ck, cv, self.dim, self.n_heads, self.n_kv_heads, self.head_dim, self.max_context)
+        if norm is None:
+            check(lib.jsgrad_hip_gemm_qkv_rope(*weights, *rest))
+        else:
+            check(lib.jsgrad_hip_gemm_qkv_rope_norm(*weights, norm.weight.ptr, norm.eps, rows.xn.ptr, *rest))
         if seqlen == 1:
             check(lib.jsgrad_hip_attn_decode_batch(rows.q.ptr, ck, cv, state.ptr, rows.attn.ptr, rows.workspace.ptr, bsz,
                                                    self.n_heads, self.n_kv_heads, self.head_dim, self.max_context))
@@ -101,11 +105,16 @@ class FeedForward:
                                              ctx.g.ptr, self.dim, self.hidden_dim, act_code(x.dtype)))
         return self.w2.call(ctx.g, out=out, residual=x)
 
-    def call_rows(self, xn: Tensor, n: int, rows: "_RowScratch", residual: Tensor, out: Tensor) -> Tensor:
-        """out = residual + w2( silu(w1 xn) * (w3 xn) ) for n rows of normed input."""
+    def call_rows(self, xn: Tensor, n: int, rows: "_RowScratch", residual: Tensor, out: Tensor, norm: RMSNorm | None = None) -> Tensor:
+        """out = residual + w2( silu(w1 xn) * (w3 xn) ) for n rows of normed input, or of what norm is to be applied to."""
         lib = ffi.load()
         sp = lambda l: l.scale.ptr if l.scale is not None else None
-        check(lib.jsgrad_hip_gemm_ffn_gate(self.w1.kind, self.w1.weight.ptr, sp(self.w1), self.w3.weight.ptr, sp(self.w3), xn.ptr, n, rows.g.ptr, self.dim, self.hidden_dim))
+        weights = (self.w1.kind, self.w1.weight.ptr, sp(self.w1), self.w3.weight.ptr, sp(self.w3), xn.ptr)
+        rest = (n, rows.g.ptr, self.dim, self.hidden_dim)
+        if norm is None:
+            check(lib.jsgrad_hip_gemm_ffn_gate(*weights, *rest))
+        else:
+            check(lib.jsgrad_hip_gemm_ffn_gate_norm(*weights, norm.weight.ptr, norm.eps, rows.xn.ptr, *rest))
         check(lib.jsgrad_hip_gemm(self.w2.kind, self.w2.weight.ptr, sp(self.w2), self.dim, self.hidden_dim, rows.g.ptr, n, out.ptr, residual.ptr))
         return out
 
@@ -124,8 +133,10 @@ class TransformerBlock:
     def call_rows(self, x: Tensor, bsz: int, seqlen: int, start_pos: int, state: Tensor, freqs_cis: Tensor, rows: "_RowScratch") -> Tensor:
         """TransformerBlock.call (llama.ts:124-127) on x [bsz*seqlen, dim]; the result is written back into x."""
         lib, n = ffi.load(), bsz * seqlen
-        check(lib.jsgrad_hip_rmsnorm_rows(x.ptr, self.attention_norm.weight.ptr, rows.xn.ptr, n, self.attention.dim, self.attention_norm.eps))
-        h = self.attention.call_rows(rows.xn, bsz, seqlen, start_pos, state, freqs_cis, rows, residual=x, out=rows.h2)
+        h = self.attention.call_rows(x, bsz, seqlen, start_pos, state, freqs_cis, rows, residual=x, out=rows.h2, norm=self.attention_norm)
+        if type(self.feed_forward).call_rows is FeedForward.call_rows:
+            return self.feed_forward.call_rows(h, n, rows, residual=h, out=x, norm=self.ffn_norm)
+        # a feed forward of the caller's own takes its rows normed
         check(lib.jsgrad_hip_rmsnorm_rows(h.ptr, self.ffn_norm.weight.ptr, rows.xn.ptr, n, self.attention.dim, self.ffn_norm.eps))
         return self.feed_forward.call_rows(rows.xn, n, rows, residual=h, out=x)
 
@@ -527,9 +538,8 @@ class Transformer:
             if seqlen > 1 and self.vocab_size % 128 == 0 and out.kind != ffi.W_F32:
                 # the reference applies the lm_head to all seqlen rows before selecting the last (llama.ts:210), i.e. with
                 # the weight expanded over rows: the several-row kernel reproduces that arithmetic for the row that is kept
-                check(lib.jsgrad_hip_rmsnorm_rows(last.ptr, self.norm.weight.ptr, rows.xn.ptr, 1, self.dim, self.norm.eps))
-                check(lib.jsgrad_hip_gemm(out.kind, out.weight.ptr, out.scale.ptr if out.scale is not None else None, self.vocab_size, self.dim, rows.xn.ptr, 1,
-                                          ctx.logits.ptr, None))
+                check(lib.jsgrad_hip_gemm_norm(out.kind, out.weight.ptr, out.scale.ptr if out.scale is not None else None, self.vocab_size, self.dim, last.ptr,
+                                               self.norm.weight.ptr, self.norm.eps, rows.xn.ptr, 1, ctx.logits.ptr))
             else:
                 out.call(Tensor(buffer=last.lazydata.view(self.dim, "float16", 0), shape=(self.dim,), dtype="float16", device=self.device), out=ctx.logits, norm=self.norm)
             self._set_sampling(temperature, top_k, top_p, alpha_f, alpha_p)
@@ -537,9 +547,8 @@ class Transformer:
             check(lib.jsgrad_hip_copy(rows.next_tokens.ptr, self.state.ptr, 4))
             self._pos = start_pos + seqlen
         else:
-            check(lib.jsgrad_hip_rmsnorm_rows(last.ptr, self.norm.weight.ptr, rows.xn.ptr, bsz, self.dim, self.norm.eps))
-            check(lib.jsgrad_hip_gemm(out.kind, out.weight.ptr, out.scale.ptr if out.scale is not None else None, self.vocab_size, self.dim, rows.xn.ptr, bsz,
-                                      rows.logits.ptr, None))
+            check(lib.jsgrad_hip_gemm_norm(out.kind, out.weight.ptr, out.scale.ptr if out.scale is not None else None, self.vocab_size, self.dim, last.ptr,
+                                           self.norm.weight.ptr, self.norm.eps, rows.xn.ptr, bsz, rows.logits.ptr))
             check(lib.jsgrad_hip_argmax_rows(rows.logits.ptr, bsz, self.vocab_size, rows.next_tokens.ptr))
         return Tensor(buffer=rows.next_tokens.lazydata.view(bsz, "int32", 0), shape=(bsz,), dtype="int32", device=self.device)
 

@@ -229,6 +229,18 @@ int jsgrad_hip_gemm_qkv_rope(int kind, const void *wq, const void *sq, const voi
 int jsgrad_hip_gemm_ffn_gate(int kind, const void *w1, const void *s1, const void *w3, const void *s3, const void *x, int rows, void *g, int dim,
                              int hidden);
 
+/* The three calls above behind a norm (TransformerBlock.call, models/llama.ts:124-127, and Transformer.forward, :209-210): x is the input of the norm.
+ * The result is that of jsgrad_hip_rmsnorm_rows(x, norm_weight, xn, rows, K, eps) and the call on xn, but for the order in which the
+ * squares are added.  xn: scratch, x's size, 16-byte aligned, not x; written unless the product's kernel norms on its way. */
+int jsgrad_hip_gemm_norm(int kind, const void *w, const void *scale, int out_f, int in_f, const void *x, const void *norm_weight, float eps, void *xn,
+                         int rows, void *y);
+int jsgrad_hip_gemm_qkv_rope_norm(int kind, const void *wq, const void *sq, const void *wk, const void *sk, const void *wv, const void *sv,
+                                  const void *x, const void *norm_weight, float eps, void *xn, int rows, int seq_len, int start_pos,
+                                  const void *rope_table, void *q_out, void *cache_k, void *cache_v, int dim, int n_heads, int n_kv_heads,
+                                  int head_dim, int max_context);
+int jsgrad_hip_gemm_ffn_gate_norm(int kind, const void *w1, const void *s1, const void *w3, const void *s3, const void *x, const void *norm_weight,
+                                  float eps, void *xn, int rows, void *g, int dim, int hidden);
+
 /* repeat_kv + scaled_dot_product_attention with the causal mask triu(start_pos + 1) (models/llama.ts:89-95,208;
  * tensor.ts:3920-3934): query row s of sequence b sees cache rows [0, start_pos + s].  q / out: [B*seq_len][n_heads*head_dim]. */
 int jsgrad_hip_attn_prefill(const void *q, const void *cache_k, const void *cache_v, void *out, int batch, int seq_len, int start_pos, int n_heads,

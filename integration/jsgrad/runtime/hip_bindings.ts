@@ -59,6 +59,9 @@ const SYMBOLS = {
   jsgrad_hip_gemm: { parameters: [I, P, P, I, I, P, I, P, P], result: I }, // kind, w, scale, out_f, in_f, x, rows, y, residual
   jsgrad_hip_gemm_qkv_rope: { parameters: [I, P, P, P, P, P, P, P, I, I, I, P, P, P, P, I, I, I, I, I], result: I }, // kind, wq, sq, wk, sk, wv, sv, x, rows, seq_len, start_pos, rope_table, q_out, cache_k, cache_v, dim, n_heads, n_kv_heads, head_dim, max_context
   jsgrad_hip_gemm_ffn_gate: { parameters: [I, P, P, P, P, P, I, P, I, I], result: I }, // kind, w1, s1, w3, s3, x, rows, g, dim, hidden
+  jsgrad_hip_gemm_norm: { parameters: [I, P, P, I, I, P, P, F, P, I, P], result: I }, // kind, w, scale, out_f, in_f, x, norm_weight, eps, xn, rows, y
+  jsgrad_hip_gemm_qkv_rope_norm: { parameters: [I, P, P, P, P, P, P, P, P, F, P, I, I, I, P, P, P, P, I, I, I, I, I], result: I }, // kind, wq, sq, wk, sk, wv, sv, x, norm_weight, eps, xn, rows, seq_len, start_pos, rope_table, q_out, cache_k, cache_v, dim, n_heads, n_kv_heads, head_dim, max_context
+  jsgrad_hip_gemm_ffn_gate_norm: { parameters: [I, P, P, P, P, P, P, F, P, I, P, I, I], result: I }, // kind, w1, s1, w3, s3, x, norm_weight, eps, xn, rows, g, dim, hidden
   jsgrad_hip_attn_prefill: { parameters: [P, P, P, P, I, I, I, I, I, I, I], result: I }, // q, cache_k, cache_v, out, batch, seq_len, start_pos, n_heads, n_kv_heads, head_dim, max_context
   jsgrad_hip_attn_batch_workspace_bytes: { parameters: [I, I, I, I], result: U }, // batch, n_heads, n_kv_heads, head_dim
   jsgrad_hip_attn_decode_batch: { parameters: [P, P, P, P, P, P, I, I, I, I, I], result: I }, // q, cache_k, cache_v, state, out, workspace, batch, n_heads, n_kv_heads, head_dim, max_context

@@ -1,0 +1,106 @@
+"""Products whose input is normed on the way: rows in the registers of the kernel for few of them, others through a pass over memory.  Every such call against the norm and the product as two calls.
+
+Tolerance: the two add a row's squares in another order, which moves its factor by a float rounding or two and with it an element of the
+normed row by one fp16 rounding where it lay that close to a tie: assert_close's bound for a norm in front (composed)."""
+import numpy as np
+import pytest
+
+import oracle as orc
+from denograd_amd import ffi
+from denograd_amd.ffi import check
+from denograd_amd.tensor import Tensor
+from tests.helpers import assert_close
+from tests.test_gpu_gemm_tile import Captured
+from tests.test_gpu_rows import KINDS, dev, make_weight, sp
+
+pytestmark = pytest.mark.gpu
+EPS = 1e-5
+
+
+def rows_and_norm(hip, rows, dim, seed=0):
+    rng = np.random.default_rng(seed + rows + dim)
+    x = (rng.standard_normal((rows, dim)) * 3).astype(np.float16)
+    x[rows // 2] = 0.0                                        # eps alone under the root
+    x[-1] *= np.float16(40.0)
+    nw = (1.0 + 0.3 * rng.standard_normal(dim)).astype(np.float16)
+    tx, tn, xn = Tensor(x), Tensor(nw), Tensor.full((rows, dim), 9.0, "float16")
+    check(hip.jsgrad_hip_rmsnorm_rows(tx.ptr, tn.ptr, xn.ptr, rows, dim, EPS))
+    return tx, tn, xn
+
+
+def check_plain(hip, kind, rows, out_f, in_f, captured=False):
+    tx, tn, xn = rows_and_norm(hip, rows, in_f)
+    w, s = make_weight(kind, out_f, in_f)
+    tw, ts = dev(w, s)
+    scratch, y = Tensor.full((rows, in_f), 9.0, "float16"), Tensor.full((rows + 1, out_f), 7.0, "float16")
+    call = Captured(hip).jsgrad_hip_gemm_norm if captured else hip.jsgrad_hip_gemm_norm
+    check(call(KINDS[kind], tw.ptr, sp(ts), out_f, in_f, tx.ptr, tn.ptr, EPS, scratch.ptr, rows, y.ptr))
+    got = y.numpy()
+    assert np.all(got[rows] == 7.0)
+    normed = xn.numpy()
+    assert np.all(np.isfinite(got[:rows]))
+    many = np.concatenate([normed, normed]) if rows == 1 else normed   # one row of the several-row arithmetic
+    assert_close(got[:rows].astype(np.float32), orc.linear(w, s, many, out_f, in_f, True)[:rows], True, f"{kind} {rows}x{out_f}x{in_f}", composed=True)
+
+
+@pytest.mark.parametrize("kind", ["float16", "int8", "nf4"])
+@pytest.mark.parametrize("rows,out_f,in_f", [(1, 2176, 2048), (5, 384, 1024), (16, 128, 1536), (7, 4224, 2048), (2, 8320, 3072), (16, 4224, 4096), (9, 256, 4096), (3, 128, 64),
+                                             (16, 4224, 512), (5, 128, 4608), (12, 256, 9216), (17, 256, 2048), (70, 384, 1024)])
+def test_normed_gemm(hip, kind, rows, out_f, in_f):
+    check_plain(hip, kind, rows, out_f, in_f)
+    check_plain(hip, kind, rows, out_f, in_f, captured=True)
+
+
+@pytest.mark.parametrize("kind", ["float16", "int8", "nf4"])
+@pytest.mark.parametrize("tile", ["g16x64", "g32x64/3"])
+def test_normed_in_front_of_the_group_kernel(hip, monkeypatch, kind, tile):
+    """A kernel that does not norm: through memory."""
+    monkeypatch.setenv("JSG_GEMM_TILE", tile)
+    for rows, out_f, in_f in ((2, 128, 256), (16, 256, 2304), (5, 128, 1280), (13, 256, 4096)):
+        check_plain(hip, kind, rows, out_f, in_f)
+
+
+@pytest.mark.parametrize("kind", ["float16", "int8", "nf4"])
+@pytest.mark.parametrize("rows,dim,hidden", [(5, 2048, 4224), (16, 4096, 2176), (16, 2048, 384), (4, 4608, 128), (24, 1024, 384)])
+def test_normed_ffn_gate(hip, kind, rows, dim, hidden):
+    tx, tn, xn = rows_and_norm(hip, rows, dim, 1)
+    (w1, s1), (w3, s3) = make_weight(kind, hidden, dim), make_weight(kind, hidden, dim)
+    t1, ts1 = dev(w1, s1)
+    t3, ts3 = dev(w3, s3)
+    scratch, got, ref = (Tensor.full((rows, n), 9.0, "float16") for n in (dim, hidden, hidden))
+    check(hip.jsgrad_hip_gemm_ffn_gate(KINDS[kind], t1.ptr, sp(ts1), t3.ptr, sp(ts3), xn.ptr, rows, ref.ptr, dim, hidden))
+    check(hip.jsgrad_hip_gemm_ffn_gate_norm(KINDS[kind], t1.ptr, sp(ts1), t3.ptr, sp(ts3), tx.ptr, tn.ptr, EPS, scratch.ptr, rows, got.ptr, dim, hidden))
+    assert_close(got.numpy().astype(np.float32), ref.numpy().astype(np.float32), True, f"{kind} {rows}", composed=True)
+
+
+@pytest.mark.parametrize("kind", ["float16", "int8", "nf4"])
+@pytest.mark.parametrize("batch,seq,dim", [(5, 1, 2048), (16, 1, 4096), (2, 7, 3072), (3, 9, 1024)])
+def test_normed_qkv_rope(hip, kind, batch, seq, dim):
+    hd, heads, kv, context, start, rows = 64, 8, 2, 32, 3, batch * seq
+    tx, tn, xn = rows_and_norm(hip, rows, dim, 2)
+    weights, held = [], []
+    for n in (heads * hd, kv * hd, kv * hd):
+        w, ts = dev(*make_weight(kind, n, dim))
+        held += [w, ts]
+        weights += [w.ptr, sp(ts)]
+    table = Tensor.zeros((2 * context, hd // 2, 2), "float16")
+    check(hip.jsgrad_hip_rope_table(table.ptr, hd, 2 * context, 500000.0, ffi.F16))
+    scratch, outs = Tensor.full((rows, dim), 9.0, "float16"), []
+    for norm in (False, True):
+        q = Tensor.full((rows, heads * hd), 7.0, "float16")
+        caches = [Tensor.full((batch, context, kv * hd), 7.0, "float16") for _ in range(2)]
+        rest = (rows, seq, start, table.ptr, q.ptr, caches[0].ptr, caches[1].ptr, dim, heads, kv, hd, context)
+        if norm:
+            check(hip.jsgrad_hip_gemm_qkv_rope_norm(KINDS[kind], *weights, tx.ptr, tn.ptr, EPS, scratch.ptr, *rest))
+        else:
+            check(hip.jsgrad_hip_gemm_qkv_rope(KINDS[kind], *weights, xn.ptr, *rest))
+        outs.append([t.numpy().astype(np.float32) for t in (q, *caches)])
+    for name, a, b in zip("qkv", *outs):
+        assert_close(b, a, True, name, composed=True)
+
+
+def test_misaligned_and_missing_norm_arguments_are_refused(hip):
+    t = Tensor.zeros((4096,), "float16")
+    args = lambda nw, xn: (KINDS["float16"], t.ptr, None, 128, 64, t.ptr, nw, EPS, xn, 2, t.ptr)
+    for nw, xn in ((None, t.ptr), (t.ptr, None), (t.ptr + 2, t.ptr), (t.ptr, t.ptr + 8)):
+        assert hip.jsgrad_hip_gemm_norm(*args(nw, xn)) != 0
