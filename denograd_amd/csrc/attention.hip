@@ -32,13 +32,13 @@ __global__ __launch_bounds__(NW * 64) void attn_decode_kernel(AttnArgs a) {
 }
 JSG_TRACE_ENTRY(jsgrad_hip_attn_decode_trace)
 
-// Many sequences at the same position (grid y; the chunks in grid z, so that the blocks that have one are neighbours: blocks go round the
-// compute units, and with the chunks of a sequence side by side those of 20 sequences of one chunk each, the other seven empty, shared every eighth
+// Many sequences at the same position (grid y; a pair's blocks in grid z, so that the blocks that have work are neighbours: blocks go round the
+// compute units, and with the blocks of a sequence side by side those of 20 sequences of one block each, the other seven empty, shared every eighth
 // unit: 12.3 us, 24 sequences with six empty ones 7.7): blocks of 4 wavefronts that stream their rows (attention_stream.h).
 constexpr int ATT_STREAM_NW = 4;
 template <int HD, int NREP>
 __global__ __launch_bounds__(ATT_STREAM_NW * 64) void attn_decode_stream_kernel(AttnArgs a) {
-  typedef AttnStream<_Float16, HD, NREP, ATT_STREAM_NW, false> A;
+  typedef AttnStream<HD, NREP, ATT_STREAM_NW> A;
   __shared__ typename A::Smem sm;
   const int g = blockIdx.x, split = blockIdx.z;
   if (const int z = blockIdx.y) {   // sequence z: its own rows of q / out / cache / workspace
@@ -49,27 +49,16 @@ __global__ __launch_bounds__(ATT_STREAM_NW * 64) void attn_decode_stream_kernel(
     a.counters += z * a.n_kv_heads;
     a.partial += z * a.partial_bstride;
   }
-  const int pos = __builtin_amdgcn_readfirstlane(a.st[1]);
-  if (pos < 0 || pos >= a.max_context) return;
-  const int T = pos + 1;
-  const int chunk = att_stream_chunk_rows<HD>(T, a.nsplit, a.pairs);  // <= ATT_CHUNK_MAX, checked on the host against max_context
-  const int n_active = (T + chunk - 1) / chunk;
-  if (split >= n_active) return;
-  A::item(a, sm, g, split, T, chunk, n_active);
+  A::item(a, sm, g, split, [&](int T) { return att_stream_blocks<HD, ATT_STREAM_NW>(T, a.nsplit); });
 }
 
-// splits of the streaming launch: enough that a chunk fits the LDS score buffer, no more than the merge can index there, and
-// as many blocks as the device holds at once (5 per CU at this kernel's registers): the sequences fill the chip by
-// themselves, every extra split only adds its fixed cost (query load, partial store, counter, merge), and a launch of one
-// full round of blocks has no thinly filled second round (16 sequences x 8 kv heads at 2100 positions: 34.5 us with 5 blocks
-// per CU, 35.7 us with 4 or 8, 37.8 us with 10)
-static int stream_nsplit(int max_context, int heads_x_batch) {
-  int by_lds = (max_context + ATT_CHUNK_MAX - 1) / ATT_CHUNK_MAX;
-  int wanted = (max_context + 31) / 32;
-  if (wanted > 64) wanted = 64;
-  const int fill = (5 * state().cu_count + heads_x_batch - 1) / heads_x_batch;
-  if (wanted > fill) wanted = fill;
-  return by_lds > wanted ? by_lds : wanted;
+// Blocks per (sequence, kv head) of the streaming launch: one block to a compute unit, whose rows on their way (32 KB) are enough, for every
+// block more is a longer merge.  us, head_dim 128, 2050 positions, 1 | 2 | 3 | 4 | 6 | 8 blocks: 16 sequences of 8 kv heads 34.4 | 29.0 | 33.1 | 30.6 | 30.1 |
+// 31.1, 8 sequences 32.5 | 21.9 | 18.1 | 18.0 | 19.8 | 17.9; 1000 positions, 24 sequences 21.8 | 24.8 | 25.7 | 23.4 | 24.8 | 24.8, 32 27.6 | 29.1 | 29.1 | 30.4 |
+// 30.9 | 32.1.  With more pairs than units some have two: three to a unit, 40 sequences 39.7 | 37.2 | 36.3 | 36.7 | 38.0 | 39.0.
+static int stream_nsplit(int pairs) {
+  const int cu = state().cu_count, n = (pairs > cu ? 3 : 1) * cu / pairs;
+  return n < 1 ? 1 : (n > 64 ? 64 : n);
 }
 
 template <typename AT, int HD, int NW> static int launch_attn(const AttnArgs &a, int n_rep) {
@@ -89,10 +78,9 @@ template <typename AT, int HD, int NW> static int launch_attn(const AttnArgs &a,
   return 0;
 }
 template <int HD> static int launch_attn_stream(const AttnArgs &a, int n_rep, int batch) {
-  dim3 grid(a.n_kv_heads, batch, a.nsplit), block(ATT_STREAM_NW * 64);
 #define JSG_REP(N)                                                                                   \
   case N:                                                                                            \
-    JSG_LAUNCH(PROF_ATTN, (attn_decode_stream_kernel<HD, N>), grid, block, 0, a);                      \
+    JSG_LAUNCH(PROF_ATTN, (attn_decode_stream_kernel<HD, N>), dim3(a.n_kv_heads, batch, a.nsplit), dim3(ATT_STREAM_NW * 64), 0, a); \
     break;
   switch (n_rep) {
     JSG_REP(1) JSG_REP(2) JSG_REP(3) JSG_REP(4) JSG_REP(8)
@@ -161,7 +149,7 @@ int jsgrad_hip_attn_decode_batch(const void *q, const void *cache_k, const void 
   a.q = q; a.cache_k = cache_k; a.cache_v = cache_v; a.st = st; a.out = out;
   a.counters = (int *)workspace;                                   // [batch][n_kv_heads], densely packed
   a.partial = (float *)((char *)workspace + (size_t)batch * counter_bytes);
-  a.n_kv_heads = n_kv_heads; a.nsplit = stream_nsplit(max_context, n_kv_heads * batch); a.pairs = n_kv_heads * batch; a.max_context = max_context;
+  a.n_kv_heads = n_kv_heads; a.nsplit = stream_nsplit(n_kv_heads * batch); a.max_context = max_context;
   a.scale = (float)(1.0 / sqrt((double)head_dim));
   a.q_bstride = (size_t)n_heads * head_dim * sizeof(_Float16);
   a.cache_bstride = (size_t)max_context * n_kv_heads * head_dim * sizeof(_Float16);

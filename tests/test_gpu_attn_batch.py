@@ -34,3 +34,32 @@ def test_attn_decode_batch_at_the_chunk_lines(hip, hd, B, H, KV, positions):
         assert np.all(got[B] == 7.0)
         ref = attention_ref(q, ck, cv, B, 1, T - 1, H, KV, hd)
         assert np.max(np.abs(got[:B] - ref)) < 4e-3, T
+
+
+@pytest.mark.parametrize("hd,B,H,KV,positions", [
+    (64, 1, 8, 2, (1, 31, 32, 33, 127, 128, 129, 385, 2100, 4096, 9000)), (128, 1, 12, 4, (15, 16, 17, 64, 65, 257, 1025, 8200)),   # many blocks to a pair
+    (64, 16, 16, 16, (128, 129, 400, 513, 5)), (128, 16, 16, 16, (64, 193, 256, 257, 500)),   # one
+    (64, 41, 32, 8, (50, 900)), (128, 41, 24, 8, (50, 450)),   # more pairs than compute units
+    (64, 4, 16, 2, (40, 700)), (128, 4, 16, 2, (40, 700)), (64, 4, 6, 2, (40, 700)), (128, 3, 2, 1, (40, 700)),
+])
+def test_attn_decode_batch_at_the_edges_of_tiles(hip, hd, B, H, KV, positions):
+    """Part tiles, wavefronts and blocks with no or one tile, merges of one and of several batches of blocks, every number of query heads per kv
+    head.  The cache behind the position holds no numbers, which must not be met by a weight of zero."""
+    rng = np.random.default_rng(hd + B + H)
+    ctx = max(positions) + 5
+    q = rng.standard_normal((B, H * hd)).astype(np.float16)
+    ck, cv = (rng.standard_normal((B, ctx, KV, hd)).astype(np.float16) for _ in range(2))
+    tq = Tensor(q)
+    ws = Tensor.zeros((hip.jsgrad_hip_attn_batch_workspace_bytes(B, H, KV, hd),), "uint8")
+    for T in positions:
+        k, v = ck.copy(), cv.copy()
+        k[:, T:], v[:, T:] = np.nan, np.inf
+        tk, tv = Tensor(k), Tensor(v)
+        st = Tensor(np.array([0, T - 1], np.int32))
+        for _ in range(2):                                    # the counters come back to zero
+            out = Tensor.full((B + 1, H * hd), 7.0, "float16")
+            check(hip.jsgrad_hip_attn_decode_batch(tq.ptr, tk.ptr, tv.ptr, st.ptr, out.ptr, ws.ptr, B, H, KV, hd, ctx))
+            got = out.numpy().astype(np.float64)
+            assert np.all(got[B] == 7.0)
+            ref = attention_ref(q, ck, cv, B, 1, T - 1, H, KV, hd)
+            assert np.max(np.abs(got[:B] - ref)) < 4e-3, T
