@@ -13,6 +13,16 @@ from tests.test_gpu_gemm_tile import test_tiled_gemm_at_the_edges as check_gemm
 
 pytestmark = pytest.mark.gpu
 
+
+@pytest.fixture(autouse=True)
+def own_numbers():
+    """The stream of random numbers that the other files share goes on where it was."""
+    before = rows_tests.RNG.bit_generator.state
+    rows_tests.RNG.bit_generator.state = np.random.default_rng(5).bit_generator.state
+    yield
+    rows_tests.RNG.bit_generator.state = before
+
+
 TILES = ["g16x64", "g16x64/3", "g16x128", "g16x128/2", "g32x64", "g32x64/5", "g32x128", "g32x128/3", "g64x64", "g64x64/3", "g64x128", "g64x128/2"]
 
 

@@ -9,11 +9,23 @@ import oracle as orc
 from denograd_amd import ffi
 from denograd_amd.ffi import check
 from denograd_amd.tensor import Tensor
+from tests import test_gpu_rows as rows_tests
 from tests.helpers import assert_close
 from tests.test_gpu_gemm_tile import Captured
 from tests.test_gpu_rows import KINDS, dev, make_weight, sp
 
 pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def own_numbers():
+    """The stream of random numbers that the other files share goes on where it was."""
+    before = rows_tests.RNG.bit_generator.state
+    rows_tests.RNG.bit_generator.state = np.random.default_rng(5).bit_generator.state
+    yield
+    rows_tests.RNG.bit_generator.state = before
+
+
 EPS = 1e-5
 
 

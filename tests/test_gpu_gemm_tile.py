@@ -161,9 +161,11 @@ def test_long_rows_without_memory(hip, monkeypatch, kind):
 @pytest.mark.parametrize("tile", ["192x128", "192x128/3"])
 def test_tiles_of_192_rows(hip, monkeypatch, kind, tile):
     """Three row tiles to a wavefront: whole and ragged tiles of 192 rows under every epilogue."""
+    before = rows_tests.RNG.bit_generator.state               # the stream that the files share goes on where it was
     monkeypatch.setenv("JSG_GEMM_TILE", tile)
     for rows in (57, 192, 193, 371):
         test_tiled_gemm_at_the_edges(hip, kind, rows, 768, 640)
         rows_tests.test_gemm_ffn_gate(hip, kind, rows, 640, 384)
     rows_tests.test_gemm_qkv_rope_writes_queries_and_cache(hip, kind, 64, 4, 50, 640)
     rows_tests.test_gemm_qkv_rope_writes_queries_and_cache(hip, kind, 128, 5, 59, 640)
+    rows_tests.RNG.bit_generator.state = before
