@@ -324,50 +324,53 @@ __global__ void embed_rows_kernel(int kind, const void *table, const _Float16 *s
 }
 
 // RMSNorm.call (nn/index.ts:586-588), one block per row.  A thread keeps its 16-byte chunks of the row (and of the weight)
-// in registers between the sum of squares and the scaling: one round of loads.  MAXCH chunks per thread (d <= 2048 * MAXCH);
-// longer rows take the two-pass loop.
-template <int MAXCH>
-__global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const _Float16 *x, const _Float16 *w, _Float16 *y, int d, float eps, float inv_d) {
-  __shared__ float red[4];
+// in registers between the sum of squares and the scaling: one round of loads.  CHUNKS 0: longer rows, in two passes.
+template <int THREADS, int CHUNKS>
+__global__ __launch_bounds__(THREADS) void rmsnorm_rows_kernel(const _Float16 *x, const _Float16 *w, _Float16 *y, int d, float eps, float inv_d) {
+  constexpr int NW = THREADS / 64;
+  __shared__ float red[NW];
+  auto total = [&](float ss) {
+    ss = wave_sum(ss);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+    __syncthreads();
+    float t[NW];
+#pragma unroll
+    for (int i = 0; i < NW; i++) t[i] = red[i];
+#pragma unroll
+    for (int n = NW / 2; n > 0; n /= 2)
+#pragma unroll
+      for (int i = 0; i < n; i++) t[i] = t[2 * i] + t[2 * i + 1];
+    return t[0];
+  };
   const _Float16 *xr = x + (size_t)blockIdx.x * d;
   _Float16 *yr = y + (size_t)blockIdx.x * d;
   float ss = 0.0f;
-  if constexpr (MAXCH > 0) {
-    const int nch = d / 8;
-    h8_t xv[MAXCH], wv[MAXCH];
+  if constexpr (CHUNKS > 0) {
+    h8_t xv[CHUNKS] = {}, wv[CHUNKS] = {};
 #pragma unroll
-    for (int c = 0; c < MAXCH; c++) {
-      const int i = threadIdx.x + c * 256;
-      if (i < nch) { xv[c] = *(const h8_t *)(xr + i * 8); wv[c] = *(const h8_t *)(w + i * 8); }
+    for (int c = 0; c < CHUNKS; c++) {
+      const int i = (threadIdx.x + c * THREADS) * 8;
+      if (i < d) { xv[c] = *(const h8_t *)(xr + i); wv[c] = *(const h8_t *)(w + i); }
     }
 #pragma unroll
-    for (int c = 0; c < MAXCH; c++)
-      if (threadIdx.x + c * 256 < nch)
+    for (int c = 0; c < CHUNKS; c++)
 #pragma unroll
-        for (int e = 0; e < 8; e++) { const float f = (float)xv[c][e]; ss = fmaf(f, f, ss); }
-    ss = wave_sum(ss);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
-    __syncthreads();
-    const float tot = (red[0] + red[1]) + (red[2] + red[3]);
-    const float r = __fsqrt_rn(__fdiv_rn(1.0f, __fadd_rn(__fmul_rn(tot, inv_d), eps)));
+      for (int e = 0; e < 8; e++) { const float f = (float)xv[c][e]; ss = fmaf(f, f, ss); }
+    const float r = __fsqrt_rn(__fdiv_rn(1.0f, __fadd_rn(__fmul_rn(total(ss), inv_d), eps)));
 #pragma unroll
-    for (int c = 0; c < MAXCH; c++) {
-      const int i = threadIdx.x + c * 256;
-      if (i < nch) {
+    for (int c = 0; c < CHUNKS; c++) {
+      const int i = (threadIdx.x + c * THREADS) * 8;
+      if (i < d) {
         h8_t o;
 #pragma unroll
         for (int e = 0; e < 8; e++) o[e] = (_Float16)__fmul_rn(rn16(__fmul_rn((float)xv[c][e], r)), (float)wv[c][e]);
-        *(h8_t *)(yr + i * 8) = o;
+        *(h8_t *)(yr + i) = o;
       }
     }
   } else {
-    for (int i = threadIdx.x; i < d; i += 256) { const float f = (float)xr[i]; ss = fmaf(f, f, ss); }
-    ss = wave_sum(ss);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
-    __syncthreads();
-    const float tot = (red[0] + red[1]) + (red[2] + red[3]);
-    const float r = __fsqrt_rn(__fdiv_rn(1.0f, __fadd_rn(__fmul_rn(tot, inv_d), eps)));
-    for (int i = threadIdx.x; i < d; i += 256) {
+    for (int i = threadIdx.x; i < d; i += THREADS) { const float f = (float)xr[i]; ss = fmaf(f, f, ss); }
+    const float r = __fsqrt_rn(__fdiv_rn(1.0f, __fadd_rn(__fmul_rn(total(ss), inv_d), eps)));
+    for (int i = threadIdx.x; i < d; i += THREADS) {
       const float v = rn16(__fmul_rn((float)xr[i], r));
       yr[i] = (_Float16)__fmul_rn(v, (float)w[i]);
     }
@@ -480,9 +483,18 @@ int jsgrad_hip_rmsnorm_rows(const void *x, const void *w, void *y, int rows, int
   JSG_READY();
   JSG_REQUIRE(x && w && y && rows > 0 && d > 0, "jsgrad_hip_rmsnorm_rows: bad argument");
   const float inv_d = (float)(1.0 / (double)d);
-  if (d % 8 == 0 && d <= 2048) JSG_LAUNCH(PROF_RMSNORM, rmsnorm_rows_kernel<1>, dim3(rows), dim3(256), 0, (const _Float16 *)x, (const _Float16 *)w, (_Float16 *)y, d, eps, inv_d);
-  else if (d % 8 == 0 && d <= 8192) JSG_LAUNCH(PROF_RMSNORM, rmsnorm_rows_kernel<4>, dim3(rows), dim3(256), 0, (const _Float16 *)x, (const _Float16 *)w, (_Float16 *)y, d, eps, inv_d);
-  else JSG_LAUNCH(PROF_RMSNORM, rmsnorm_rows_kernel<0>, dim3(rows), dim3(256), 0, (const _Float16 *)x, (const _Float16 *)w, (_Float16 *)y, d, eps, inv_d);
+  // A few rows are one latency chain, shortest with one chunk per thread; thousands of rows fill the chip either way, and larger blocks leave gaps.
+  // us, 256 threads of up to four chunks | one chunk each: 16 x 3072 2.12 | 1.84, 16 x 4096 2.19 | 1.90, 32768 x 3072 69.8 | 73.7, 16 x 8192 2.78 | 2.14, 371 x 8192
+  // 4.55 | 4.15, 4096 x 8192 24.3 | 26.5; a step of 16 sequences of the 8B int8 shape (65 norms) 3127 | 3106.
+#define JSG_NORM(THREADS, CHUNKS)                                                                                       \
+  JSG_LAUNCH(PROF_RMSNORM, (rmsnorm_rows_kernel<THREADS, CHUNKS>), dim3(rows), dim3(THREADS), 0, (const _Float16 *)x,    \
+             (const _Float16 *)w, (_Float16 *)y, d, eps, inv_d)
+  if (d % 8 == 0 && d <= 2048) JSG_NORM(256, 1);
+  else if (d % 8 == 0 && d <= 8192 && rows > 1024) JSG_NORM(256, 4);
+  else if (d % 8 == 0 && d <= 4096) JSG_NORM(512, 1);
+  else if (d % 8 == 0 && d <= 8192) JSG_NORM(1024, 1);
+  else JSG_NORM(256, 0);
+#undef JSG_NORM
   return 0;
 }
 

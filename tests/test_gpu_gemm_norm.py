@@ -116,3 +116,13 @@ def test_misaligned_and_missing_norm_arguments_are_refused(hip):
     args = lambda nw, xn: (KINDS["float16"], t.ptr, None, 128, 64, t.ptr, nw, EPS, xn, 2, t.ptr)
     for nw, xn in ((None, t.ptr), (t.ptr, None), (t.ptr + 2, t.ptr), (t.ptr, t.ptr + 8)):
         assert hip.jsgrad_hip_gemm_norm(*args(nw, xn)) != 0
+
+
+@pytest.mark.parametrize("rows,dim", [(3, 8), (19, 2040), (3, 2048), (3, 2056), (19, 4096), (3, 4104), (5, 8192), (3, 8200), (3, 4098), (1025, 2056), (1025, 8192)])
+def test_rmsnorm_rows_of_every_length(hip, rows, dim):
+    """Both sides of every line between block sizes and chunks; the sums' order is the only difference (assert_close)."""
+    tx, tn, xn = rows_and_norm(hip, rows, dim, 3)
+    got, x, w = xn.numpy(), tx.numpy(), tn.numpy()
+    some = sorted({0, rows // 2, rows - 1})
+    ref = np.stack([orc.rmsnorm(x[r], w, EPS, True) for r in some])
+    assert_close(got[some].astype(np.float32), ref, True, f"{rows}x{dim}")
