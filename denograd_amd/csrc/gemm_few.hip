@@ -268,7 +268,8 @@ int gemm_few(int epi, int kind, const GemmArgs &a, int prof_kind, bool *taken) {
   // their own (33 of the 1B shape) | here: 1B shape 2 rows 897 | 832, 5 rows 903 | 846, 12 rows 968 | 908, 16 rows 1006 | 944; int8 14 layers of the 3B shape
   // with 6 rows 830 | 810, of the 8B shape with 4 rows 1131 | 1113.  In gemm_group.hip, whose blocks read all of x for it and norm every fragment, it
   // costs more than the launches: 8B int8 16 rows 3321 | 3403, 8B NF4 16 layers 8 rows 1403 | 1467.
-  if (a.norm_w && a.K > 4096) return 0;
+  // The norm's weights are read here in 16-byte pieces; from any other address in memory first.
+  if (a.norm_w && (a.K > 4096 || (uintptr_t)a.norm_w & 15)) return 0;
   const size_t codes = (size_t)a.N * (epi == GEPI_SWIGLU ? 2 : 1) * a.K;
   if (kind == JSGRAD_W_I8 && (codes > (size_t)36 << 20 || (a.M > 8 && a.K > 3072))) return 0;
   if (pin_env(a, "JSG_GEMM_NO_SKINNY") || pin_env(a, "JSG_GEMM_SKINNY_TILES") || pin_env(a, "JSG_SG_TPW")) return 0;   // tests that want one of the other kernels

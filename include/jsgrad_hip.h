@@ -231,7 +231,8 @@ int jsgrad_hip_gemm_ffn_gate(int kind, const void *w1, const void *s1, const voi
 
 /* The three calls above behind a norm (TransformerBlock.call, models/llama.ts:124-127, and Transformer.forward, :209-210): x is the input of the norm.
  * The result is that of jsgrad_hip_rmsnorm_rows(x, norm_weight, xn, rows, K, eps) and the call on xn, but for the order in which the
- * squares are added.  xn: scratch, x's size, 16-byte aligned, not x; written unless the product's kernel norms on its way. */
+ * squares are added.  xn: scratch, x's size, 16-byte aligned, not x; written unless the product's kernel norms on its way.  norm_weight may lie at
+ * any address that jsgrad_hip_rmsnorm_rows takes. */
 int jsgrad_hip_gemm_norm(int kind, const void *w, const void *scale, int out_f, int in_f, const void *x, const void *norm_weight, float eps, void *xn,
                          int rows, void *y);
 int jsgrad_hip_gemm_qkv_rope_norm(int kind, const void *wq, const void *sq, const void *wk, const void *sk, const void *wv, const void *sv,

@@ -2,12 +2,15 @@
 
 Tolerance: the two add a row's squares in another order, which moves its factor by a float rounding or two and with it an element of the
 normed row by one fp16 rounding where it lay that close to a tie: assert_close's bound for a norm in front (composed)."""
+import types
+
 import numpy as np
 import pytest
 
 import oracle as orc
-from denograd_amd import ffi
+from denograd_amd import ffi, synthetic
 from denograd_amd.ffi import check
+from denograd_amd.llama3 import Llama3
 from denograd_amd.tensor import Tensor
 from tests import test_gpu_rows as rows_tests
 from tests.helpers import assert_close
@@ -114,8 +117,47 @@ def test_normed_qkv_rope(hip, kind, batch, seq, dim):
 def test_misaligned_and_missing_norm_arguments_are_refused(hip):
     t = Tensor.zeros((4096,), "float16")
     args = lambda nw, xn: (KINDS["float16"], t.ptr, None, 128, 64, t.ptr, nw, EPS, xn, 2, t.ptr)
-    for nw, xn in ((None, t.ptr), (t.ptr, None), (t.ptr + 2, t.ptr), (t.ptr, t.ptr + 8)):
+    for nw, xn in ((None, t.ptr), (t.ptr, None), (t.ptr, t.ptr + 8)):
         assert hip.jsgrad_hip_gemm_norm(*args(nw, xn)) != 0
+
+
+@pytest.mark.parametrize("kind", ["float16", "int8", "nf4"])
+@pytest.mark.parametrize("rows,dim", [(5, 2048), (20, 1024), (70, 512)])
+def test_norm_weights_at_any_even_address(hip, monkeypatch, kind, rows, dim):
+    """A slice of a longer tensor as the norm's weights, in all three calls: what jsgrad_hip_rmsnorm_rows takes."""
+    held = []
+
+    def sliced(hip, rows, dim, seed=0):
+        tx, tn, xn = whole(hip, rows, dim, seed)
+        held.append(Tensor(np.concatenate([np.full(1, 7.0, np.float16), tn.numpy()])))
+        return tx, types.SimpleNamespace(ptr=held[-1].ptr + 2), xn
+
+    whole = rows_and_norm
+    monkeypatch.setitem(globals(), "rows_and_norm", sliced)
+    check_plain(hip, kind, rows, 384, dim)
+    check_plain(hip, kind, rows, 384, dim, captured=True)
+    test_normed_ffn_gate(hip, kind, rows, dim, 256)
+    test_normed_qkv_rope(hip, kind, rows, 1, dim)
+
+
+def test_a_model_whose_norm_weights_are_slices(hip):
+    """A prompt and several sequences at once, against the same model with norm weights of their own."""
+    cfg = synthetic.config("tiny16")
+    prompt = np.arange(1, 25, dtype=np.int32).reshape(2, 12)
+    out = []
+    for sliced in (False, True):
+        model = Llama3.from_config(cfg).load_weights(synthetic.random_state_dict(cfg, seed=0), quantized=True).model
+        if sliced:
+            for norm in [n for layer in model.layers for n in (layer.attention_norm, layer.ffn_norm)] + [model.norm]:
+                longer = Tensor(np.concatenate([np.full(1, 7.0, np.float16), norm.weight.numpy().reshape(-1)]))
+                norm.weight = Tensor(buffer=longer.lazydata.view(cfg["dim"], "float16", 2), shape=(cfg["dim"],), dtype="float16", device=longer.device)
+        model.forward_rows(prompt[:1], 0)
+        out.append([model.logits.numpy().astype(np.float32)])
+        model.forward_rows(prompt, 0)
+        model.forward_rows(prompt[:, :1].copy(), 12)
+        out[-1].append(model.rows_logits().numpy().astype(np.float32))
+    for a, b in zip(*out):
+        assert_close(b, a, True, "logits", composed=True)
 
 
 @pytest.mark.parametrize("rows,dim", [(3, 8), (19, 2040), (3, 2048), (3, 2056), (19, 4096), (3, 4104), (5, 8192), (3, 8200), (3, 4098), (1025, 2056), (1025, 8192)])
