@@ -66,6 +66,19 @@ def test_normed_gemm(hip, kind, rows, out_f, in_f):
     check_plain(hip, kind, rows, out_f, in_f, captured=True)
 
 
+@pytest.mark.parametrize("kind", ["float16", "int8"])
+@pytest.mark.parametrize("rows,out_f,in_f", [(1, 256, 8192), (5, 384, 6144), (8, 1024, 8192), (5, 384, 8192)])
+def test_rows_too_long_to_norm_in_registers_take_the_kernel_of_normed_rows(hip, kind, rows, out_f, in_f):
+    """Normed in memory, the call is that of two calls, bit for bit."""
+    tx, tn, xn = rows_and_norm(hip, rows, in_f)
+    w, s = make_weight(kind, out_f, in_f)
+    tw, ts = dev(w, s)
+    scratch, got, ref = Tensor.full((rows, in_f), 9.0, "float16"), Tensor.full((rows, out_f), 7.0, "float16"), Tensor.full((rows, out_f), 7.0, "float16")
+    check(hip.jsgrad_hip_gemm(KINDS[kind], tw.ptr, sp(ts), out_f, in_f, xn.ptr, rows, ref.ptr, None))
+    check(hip.jsgrad_hip_gemm_norm(KINDS[kind], tw.ptr, sp(ts), out_f, in_f, tx.ptr, tn.ptr, EPS, scratch.ptr, rows, got.ptr))
+    assert np.array_equal(got.numpy().view(np.uint16), ref.numpy().view(np.uint16))
+
+
 @pytest.mark.parametrize("kind", ["float16", "int8", "nf4"])
 @pytest.mark.parametrize("tile", ["g16x64", "g32x64/3"])
 def test_normed_in_front_of_the_group_kernel(hip, monkeypatch, kind, tile):
