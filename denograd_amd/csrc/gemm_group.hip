@@ -98,8 +98,13 @@ template <int KIND, int EPI, int WB, int BM, int BN, int WN, int ST> __global__ 
   const int my_row = wn * TN * 16;
   const WeightRow sr = weight_row<EPI, BN>(t, id.col, my_row);
   i4_t rs;
-  if constexpr (KIND != JSGRAD_W_F16) rs = dma_rsrc(pick(t.s, sr.mat) + (size_t)sr.row * (KIND == JSGRAD_W_I8 ? 1 : a.K / 64));
-  const uint32_t vs = KIND == JSGRAD_W_I8 ? (uint32_t)(lane & (TN * 8 - 1)) * 4 : (uint32_t)(lane & (TN * 16 - 1)) * (a.K / 32);
+  uint32_t odd = 0;                                           // int8 scales between two words: loaded from the word they begin in, and lying a half further on
+  if constexpr (KIND != JSGRAD_W_F16) {
+    const _Float16 *const from = pick(t.s, sr.mat) + (size_t)sr.row * (KIND == JSGRAD_W_I8 ? 1 : a.K / 64);
+    if constexpr (KIND == JSGRAD_W_I8) odd = (uint32_t)((uintptr_t)from >> 1) & 1;
+    rs = dma_rsrc(from - odd);
+  }
+  const uint32_t vs = KIND == JSGRAD_W_I8 ? min((uint32_t)lane, TN * 8 - 1 + odd) * 4 : (uint32_t)(lane & (TN * 16 - 1)) * (a.K / 32);
   auto load = [&](int at, int buf) {
     const int turn = turn_of(at);
     const uint32_t base = (uint32_t)buf * S::TURN;
@@ -201,7 +206,7 @@ template <int KIND, int EPI, int WB, int BM, int BN, int WN, int ST> __global__ 
       if (turn == 0)
 #pragma unroll
         for (int j = 0; j < TN; j++) {
-          const _Float16 v = *(const _Float16 *)(group_lds + (S::LDS - S::TABLE) + wave * 256 + (j * 16 + l16) * 2);
+          const _Float16 v = *(const _Float16 *)(group_lds + (S::LDS - S::TABLE) + wave * 256 + (j * 16 + l16 + odd) * 2);
           scale[j] = h2_t{v, v};
         }
     buf = buf + 1 == ST ? 0 : buf + 1;
@@ -372,8 +377,10 @@ GroupChoice choose_group(int epi, int kind, const GemmArgs &a) {
   GroupChoice best;
   int bm = 0, bn = 0, split = 0;
   const bool pin = group_pin(a, bm, bn, split);
-  // scales come by direct loads of four bytes; with more rows than a tile has the weights would be read twice
-  if (((uintptr_t)a.s0 | (uintptr_t)a.s1 | (uintptr_t)a.s2) & 3 || (!pin && a.M > 64)) return best;
+  // Scales come by direct loads of four bytes: int8's, once per block, from any even address (us with scales at an odd multiple of two bytes, the
+  // kernels below | here: 9 x 128256 x 1024 85.8 | 32.8, 7 x w1|w3 of 14336 x 3072 37.0 | 18.8); nf4's, every turn, from whole words only.
+  // With more rows than a tile has the weights would be read twice.
+  if (((uintptr_t)a.s0 | (uintptr_t)a.s1 | (uintptr_t)a.s2) & (kind == JSGRAD_W_I8 ? 1 : 3) || (!pin && a.M > 64)) return best;
   const int cus = state().cu_count, weight_rows = a.N * (epi == GEPI_SWIGLU ? 2 : 1);
   for (int i = 0; i < N_GROUP; i++) {
     const GroupShape &s = GROUP_SHAPES[kind - JSGRAD_W_F16][i];

@@ -6,6 +6,8 @@ Tolerance: products and sums are those of the oracle's several-row Linear in ano
 import numpy as np
 import pytest
 
+from denograd_amd import ffi
+from denograd_amd.ffi import check
 from denograd_amd.tensor import Tensor
 from tests import test_gpu_gemm_tile as tile_tests
 from tests import test_gpu_rows as rows_tests
@@ -65,3 +67,23 @@ def test_as_chosen(hip, monkeypatch, kind):
     monkeypatch.setattr(tile_tests, "sp", slice_of_scales)
     for rows, out_f, in_f in sizes:
         check_gemm(hip, kind, rows, out_f, in_f)
+
+
+@pytest.mark.parametrize("rows,out_f,in_f", [(1, 4224, 1024), (9, 256, 8192), (16, 8320, 512), (24, 4224, 1024), (57, 128, 2048)])
+@pytest.mark.parametrize("tile", ["", "g16x64", "g16x128", "g32x64/3", "g32x128", "g64x64", "g64x128/2"])
+def test_int8_scales_between_two_words_take_the_same_kernel(hip, monkeypatch, rows, out_f, in_f, tile):
+    """The bits of the call with scales at a multiple of four bytes, in every tile (8, 16 or 32 words of scales to a wavefront, one more here) and as
+    chosen; the last scale is the last half of its allocation."""
+    rng = np.random.default_rng(rows)
+    w, s = rows_tests.make_weight("int8", out_f, in_f)
+    x = Tensor(rng.standard_normal((rows, in_f)).astype(np.float16))
+    tw, ts = Tensor(w), Tensor(s)
+    odd = Tensor(np.concatenate([np.full(1, 7.0, np.float16), s.reshape(-1)]))
+    if tile:
+        monkeypatch.setenv("JSG_GEMM_TILE", tile)
+    out = []
+    for scales in (ts.ptr, odd.ptr + 2):
+        y = Tensor.full((rows, out_f), 7.0, "float16")
+        check(hip.jsgrad_hip_gemm(ffi.W_I8, tw.ptr, scales, out_f, in_f, x.ptr, rows, y.ptr, None))
+        out.append(y.numpy().view(np.uint16))
+    assert np.array_equal(*out)
