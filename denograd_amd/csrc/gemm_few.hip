@@ -261,17 +261,23 @@ int gemm_few(int epi, int kind, const GemmArgs &a, int prof_kind, bool *taken) {
   // 10.9 / 10.5 | 10.7 / 11.1, 6144 x 4096 10.4 / 10.7 | 10.7 / 12.0, 16384 x 3072 13.3 / 13.2 | 14.1 / 15.0, 28672 x 4096 22.2 / 22.1 | 28.7 / 30.3.
   // fp16, skinny_gemm_kernel | this one, 2 / 8 / 16 rows: 2048 x 2048 6.2 / 6.3 / 6.3 | 4.5 / 4.5 / 5.1, 2048 x 8192 14.1 / 14.9 / 15.9 |
   // 8.8 / 9.5 / 12.4, 16384 x 2048 23.6 / 23.7 / 24.4 | 16.3 / 17.2 / 18.2, 128256 x 2048 147 / 153 / 162 | 88 / 92 / 94 (6.0 TB/s).
-  // fp16 rows of 16 KiB behind more than 8 rows of x go to gemm_group.hip, which reads x from LDS: 2048 x 8192, 16 rows 12.8 | 10.9 there, 3072 x 8192
-  // 15.5 | 12.8 (8 rows 9.8 | 10.9, 12.6 | 13.0).
-  if (kind == JSGRAD_W_F16 && a.M > 8 && a.K > 4096) return 0;
+  // fp16 rows of more than 4096 elements (6144 and 8192 come here): the more rows of x a block reads for its few tiles, the nearer gemm_group.hip, which reads x from LDS, comes.  us,
+  // 9 / 12 / 16 rows, that one | this one: 1024 x 6144 9.9 / 10.0 / 10.1 | 7.5 / 8.3 / 9.3, 2048 x 6144 10.5 / 10.6 / 10.8 | 8.4 / 9.0 / 10.1, 4096 x 6144
+  // 13.2 / 13.2 / 13.3 | 12.1 / 12.8 / 13.9, 8192 x 6144 19.2 / 19.4 / 19.4 | 19.4 / 20.0 / 20.9, 20480 x 6144 58.0 / 58.5 / 58.7 | 40.6 / 41.5 / 42.6;
+  // 2048 x 8192 11.0 / 11.1 / 11.3 | 9.8 / 11.2 / 12.7, 3072 x 8192 12.9 / 12.9 / 13.0 | 12.6 / 13.9 / 15.3, 4096 x 8192 17.3 / 17.3 / 17.3 | 14.7 / 16.0 /
+  // 17.5, 8192 x 8192 26.5 / 26.7 / 26.7 | 25.1 / 25.9 / 27.0, 12032 x 8192 38.5 / 38.7 / 38.8 | 34.2 / 35.0 / 36.4.
+  const int rows = a.N * (epi == GEPI_SWIGLU ? 2 : 1);
+  const size_t elements = (size_t)rows * a.K;
+  if (kind == JSGRAD_W_F16 && a.K > 4096 &&
+      (a.K > 6144 ? rows > 1024 && rows <= 3072 && a.M > (rows <= 2048 ? 12 : 9) : rows > 2048 && elements < (size_t)80 << 20 && a.M > (rows <= 6144 ? 13 : 8)))
+    return 0;
   // A norm in front is done in registers, x and the norm's weights at once: rows of half the length at most.  us per decode step, norms as launches of
   // their own (33 of the 1B shape) | here: 1B shape 2 rows 897 | 832, 5 rows 903 | 846, 12 rows 968 | 908, 16 rows 1006 | 944; int8 14 layers of the 3B shape
   // with 6 rows 830 | 810, of the 8B shape with 4 rows 1131 | 1113.  In gemm_group.hip, whose blocks read all of x for it and norm every fragment, it
   // costs more than the launches: 8B int8 16 rows 3321 | 3403, 8B NF4 16 layers 8 rows 1403 | 1467.
   // The norm's weights are read here in 16-byte pieces; from any other address in memory first.
   if (a.norm_w && (a.K > 4096 || (uintptr_t)a.norm_w & 15)) return 0;
-  const size_t codes = (size_t)a.N * (epi == GEPI_SWIGLU ? 2 : 1) * a.K;
-  if (kind == JSGRAD_W_I8 && (codes > (size_t)36 << 20 || (a.M > 8 && a.K > 3072))) return 0;
+  if (kind == JSGRAD_W_I8 && (elements > (size_t)36 << 20 || (a.M > 8 && a.K > 3072))) return 0;
   if (pin_env(a, "JSG_GEMM_NO_SKINNY") || pin_env(a, "JSG_GEMM_SKINNY_TILES") || pin_env(a, "JSG_SG_TPW")) return 0;   // tests that want one of the other kernels
   if (epi == GEPI_STORE) return gemm_few_epi<GEPI_STORE>(kind, a, prof_kind, taken);
   if (epi == GEPI_ROPE_KV) return gemm_few_epi<GEPI_ROPE_KV>(kind, a, prof_kind, taken);

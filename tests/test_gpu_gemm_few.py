@@ -49,3 +49,18 @@ def test_few_rows_ffn_gate(hip, kind, dim, hidden):
 @pytest.mark.parametrize("kind,hd,B,dim", [("float16", 64, 16, 3072), ("int8", 128, 3, 4096), ("int8", 128, 16, 2048)])
 def test_few_rows_qkv_rope(hip, kind, hd, B, dim):
     qkv_rope(hip, kind, hd, B, 1, dim)
+
+
+@pytest.mark.parametrize("most,out_f,in_f", [(16, 1024, 8192), (12, 2048, 8192), (9, 3072, 8192), (16, 4096, 8192), (16, 2048, 6144), (13, 4096, 6144), (16, 14336, 6144)])
+def test_long_fp16_rows_up_to_the_number_where_another_kernel_is_faster(hip, most, out_f, in_f):
+    """A row's sums do not depend on the rows beside it, so the first rows of a call have the bits of the call of those rows alone exactly where both
+    take this kernel; behind the line the sums are in another order."""
+    w, x = Tensor.randn((out_f * in_f,), "float16", 1, 0.05), Tensor.randn((17 * in_f,), "float16", 2, 1.0)
+    out = []
+    for rows in (8, most, most + 1):
+        y = Tensor.empty((rows, out_f), "float16")
+        check(hip.jsgrad_hip_gemm(KINDS["float16"], w.ptr, None, out_f, in_f, x.ptr, rows, y.ptr, None))
+        out.append(y.numpy().view(np.uint16)[:8])
+    few, at, behind = out
+    assert np.array_equal(at, few)
+    assert not np.array_equal(behind, few)
