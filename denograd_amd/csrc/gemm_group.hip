@@ -422,13 +422,21 @@ int gemm_group(int epi, int kind, const GemmArgs &a, int prof_kind, bool *taken)
   if (!pin) {
     if (a.M > 32 || pin_env(a, "JSG_GEMM_TILE") || pin_env(a, "JSG_GEMM_NO_SKINNY") || pin_env(a, "JSG_GEMM_SKINNY_TILES")) return 0;   // tests that want one of the other kernels
     // One round of skinny_gemm_kernel's blocks over short rows: no K parts whose sums have to travel.  us, that | this one: 24 rows, fp16
-    // 2048 x 2048 7.5 | 7.5, 3072 x 2048 8.1 | 8.1, 3072 x 3072 9.9 | 9.3, 2048 x 8192 18.7 | 11.5, 5120 x 3072 17.5 | 10.5; int8
-    // 2048 x 2048 6.7 | 7.8, 3072 x 3072 8.6 | 9.0, 4096 x 4096 10.5 | 10.1, 6144 x 4096 17.5 | 11.4, 28672 x 4096 50 | 27; nf4
-    // 4096 x 4096 9.3 | 10.9, 3072 x 8192 14.8 | 12.9, 28672 x 4096 46 | 25; 16 rows, int8 4096 x 4096 9.1 | 9.6, 6144 x 4096 13.5 | 10.7; 8 rows, nf4
-    // 4096 x 4096 7.8 | 9.4, 3072 x 8192 10.7 | 11.5 (16 rows 11.6 | 11.8), 6144 x 4096 11.3 | 10.7, 28672 x 4096 36.7 | 21.7.
-    const int rows = a.N * (epi == GEPI_SWIGLU ? 2 : 1);
-    const int longest = kind == JSGRAD_W_F16 ? 2048 : (kind == JSGRAD_W_I8 ? (a.M <= 16 ? 4096 : 3072) : (a.M <= 8 ? 8192 : 4096));
-    if (a.K % 512 || a.K < 1024 || (rows <= 16 * state().cu_count && a.K <= longest)) return 0;
+    // 2048 x 2048 7.5 | 7.5, 3072 x 2048 8.1 | 8.1, 3072 x 3072 9.9 | 9.3, 4096 x 3072 9.9 | 10.5, 4096 x 3584 11.3 | 11.1, 2048 x 8192 18.7 | 11.5; int8
+    // 1024 x 4096 8.7 | 8.2, 2048 x 4096 8.9 | 9.6, 4096 x 3584 9.2 | 10.2, 4096 x 4096 10.2 | 10.3, 4096 x 4608 11.0 | 10.8, 6144 x 4096 17.5 | 11.4, 28672 x 4096 50 | 27; nf4
+    // 4096 x 4096 9.3 | 10.9, 4096 x 5120 12.0 | 12.4, 4096 x 6144 12.8 | 12.6, 3072 x 8192 14.8 | 12.9, 28672 x 4096 46 | 25; 16 rows, int8 4096 x 4096
+    // 9.1 | 9.6, 2560 x 5120 9.9 | 9.0, 3840 x 5120 10.1 | 10.5 (w1|w3 of 2048 x 5120 14.2 | 12.0), 4096 x 5632 10.2 | 10.8, 6144 x 4096 13.5 | 10.7; nf4 4096 x 6144 10.3 | 10.9, 4096 x 8192
+    // 11.9 | 12.1, 4096 x 10240 14.8 | 13.4; 8 rows, nf4 4096 x 4096 7.8 | 9.4, 3072 x 8192 10.7 | 11.5, 6144 x 4096 11.3 | 10.7, 28672 x 4096 36.7 | 21.7.
+    // Where this one finds four or five parts for a unit each (up to 3072 weight rows) the line lies lower.
+    const int rows = a.N * (epi == GEPI_SWIGLU ? 2 : 1), round = 16 * state().cu_count;
+    const bool wide = rows > 3072;
+    const int longest = kind == JSGRAD_W_F16 ? (wide ? 3072 : 2048)
+                      : kind == JSGRAD_W_I8 ? (a.M <= 16 ? (wide && epi != GEPI_SWIGLU ? 5632 : 4096) : (rows > 1024 ? 4096 : 3072))
+                                            : (a.M <= (wide ? 16 : 8) ? 8192 : (wide ? 5120 : 4096));
+    if (a.K % 512 || a.K < 1024 || (rows <= round && a.K <= longest)) return 0;
+    // ... whose blocks have w1 and w3 at once: nf4, us, 2 / 16 / 32 rows, 4096 x 2048 10.4 / 10.4 / 11.9 | 9.8 / 9.6 / 9.9, x 3072 10.8 / 10.9 / 12.5 | 10.7 / 10.7 /
+    // 12.3, x 3584 10.1 / 10.3 / 12.2 | 11.1 / 11.2 / 12.8, x 4096 10.7 / 11.1 / 13.0 | 11.8 / 11.8 / 14.0, x 5120 15.3 / 16.1 / 18.7 | 12.9 / 13.4 / 16.0
+    if (kind == JSGRAD_W_NF4 && epi == GEPI_SWIGLU && a.N <= round && a.K > 3072 && a.K <= 4096) return 0;
   }
   const GroupChoice c = choose_group(epi, kind, a);
   if (c.shape < 0) return pin ? fail("jsgrad_hip_gemm: no tile shape") : 0;

@@ -87,3 +87,39 @@ def test_int8_scales_between_two_words_take_the_same_kernel(hip, monkeypatch, ro
         check(hip.jsgrad_hip_gemm(ffi.W_I8, tw.ptr, scales, out_f, in_f, x.ptr, rows, y.ptr, None))
         out.append(y.numpy().view(np.uint16))
     assert np.array_equal(*out)
+
+
+@pytest.mark.parametrize("kind,rows,out_f,in_f,skinny", [
+    ("float16", 24, 4096, 3072, True), ("float16", 24, 4096, 3584, False), ("float16", 24, 3072, 2048, True), ("float16", 24, 3072, 2560, False),
+    ("int8", 16, 4096, 5632, True), ("int8", 12, 4096, 6144, False), ("int8", 16, 3072, 4096, True), ("int8", 16, 3072, 4608, False),
+    ("int8", 24, 2048, 4096, True), ("int8", 24, 1024, 4096, False), ("int8", 24, 4096, 4608, False),
+    ("nf4", 16, 4096, 8192, True), ("nf4", 16, 4096, 8704, False), ("nf4", 16, 3072, 4608, False), ("nf4", 8, 3072, 8192, True),
+    ("nf4", 17, 4096, 5120, True), ("nf4", 17, 4096, 5632, False)])
+def test_lines_to_the_kernel_for_short_rows(hip, monkeypatch, kind, rows, out_f, in_f, skinny):
+    """Which kernel a call comes to, by its bits: the K groups and parts of this one add the sums in another order."""
+    w = Tensor.randn((out_f * in_f // 2,), "float16", 1, 0.05)    # as fp16, half of the rows twice; as codes, any bits are some
+    s = None if kind == "float16" else Tensor.full((out_f * (in_f // 64),), 0.01, "float16")
+    x = Tensor.randn((rows * in_f,), "float16", 2, 1.0)
+    if kind == "float16":
+        w = Tensor(np.concatenate([w.numpy(), w.numpy()]))
+    out = []
+    for pin in ("", "1"):
+        if pin:
+            monkeypatch.setenv("JSG_GEMM_SKINNY_TILES", pin)
+        y = Tensor.empty((rows, out_f), "float16")
+        check(hip.jsgrad_hip_gemm(rows_tests.KINDS[kind], w.ptr, s.ptr if s is not None else None, out_f, in_f, x.ptr, rows, y.ptr, None))
+        out.append(y.numpy().view(np.uint16))
+    assert np.array_equal(*out) == skinny
+
+
+@pytest.mark.parametrize("rows,hidden,dim,skinny", [(2, 4096, 4096, True), (24, 2560, 3584, True), (16, 4096, 3072, False), (16, 4096, 4608, False), (16, 4224, 4096, False)])
+def test_lines_to_the_kernel_for_short_rows_of_nf4_gates(hip, monkeypatch, rows, hidden, dim, skinny):
+    w, s, x = Tensor.randn((hidden * dim // 2,), "float16", 1, 0.05), Tensor.full((hidden * dim // 64,), 0.01, "float16"), Tensor.randn((rows * dim,), "float16", 2, 1.0)
+    out = []
+    for pin in ("", "1"):
+        if pin:
+            monkeypatch.setenv("JSG_GEMM_SKINNY_TILES", pin)
+        y = Tensor.empty((rows, hidden), "float16")
+        check(hip.jsgrad_hip_gemm_ffn_gate(ffi.W_NF4, w.ptr, s.ptr, w.ptr + hidden * dim // 2, s.ptr, x.ptr, rows, y.ptr, dim, hidden))
+        out.append(y.numpy().view(np.uint16))
+    assert np.array_equal(*out) == skinny
