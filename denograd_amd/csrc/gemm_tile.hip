@@ -750,6 +750,10 @@ template <int EPI> static int gemm_tiled_epi(int kind, const GemmArgs &a, int pr
   const TileShape *ss = kind == JSGRAD_W_I8 ? STAGED_SHAPES_I8 : STAGED_SHAPES_NF4;
   const Choice st = choose_tile(ss, N_STAGED, EPI, a.M, wrows, a.K, 0, pinned('s'));   // takes every call
   const bool staged = q.shape < 0 || st.us < q.us;
+  // int8 rows of 512 codes: a block of the group kernel, which has its unit to itself, is over in a turn or two, and there are rounds of them.  us, 16 rows,
+  // that | the staged kernel, several of whose blocks share a unit: 65536 x 512 12.7 | 11.4, 128256 x 512 23.4 | 17.5 (x 1024 32.5 | 35 and more).
+  if constexpr (EPI != GEPI_SWIGLU)
+    if (!pin.family && kind == JSGRAD_W_I8 && a.M <= 32 && a.K <= 512 && wrows > 192 * state().cu_count) return gemm_staged(EPI, kind, 32, 128, a, prof_kind);
   if (group_first(std::min(staged ? st.us : q.us, f.shape >= 0 ? f.us + realise_us : st.us))) return run_group(EPI, kind, a, g, prof_kind);
   const size_t bytes = (size_t)wrows * a.K * 2;
   if (f.shape >= 0 && f.us + realise_us < (staged ? st.us : q.us) && bytes <= REALISED_LIMIT) {

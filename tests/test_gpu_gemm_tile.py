@@ -169,3 +169,12 @@ def test_tiles_of_192_rows(hip, monkeypatch, kind, tile):
     rows_tests.test_gemm_qkv_rope_writes_queries_and_cache(hip, kind, 64, 4, 50, 640)
     rows_tests.test_gemm_qkv_rope_writes_queries_and_cache(hip, kind, 128, 5, 59, 640)
     rows_tests.RNG.bit_generator.state = before
+
+
+@pytest.mark.parametrize("rows,captured", [(2, False), (16, True), (32, False), (33, False)])
+def test_many_short_int8_rows(hip, rows, captured):
+    """Up to 32 rows behind more than 192 weight rows of 512 codes per compute unit take the staged kernel's 32 x 128 tile; the last tile is a ragged one
+    of x, and 33 rows stay where they were."""
+    before = rows_tests.RNG.bit_generator.state               # the stream that the files share goes on where it was
+    test_tiled_gemm_at_the_edges(Captured(hip) if captured else hip, "int8", rows, 49408, 512)
+    rows_tests.RNG.bit_generator.state = before
