@@ -77,6 +77,7 @@ struct AttnArgs {
   int *err = nullptr;   // optional: set to 1 when the merging block's bounded wait for the other chunks ran out
   float *partial;  // [n_kv_heads][nsplit][n_rep][HD + 2]
   int n_kv_heads, nsplit, max_context;
+  bool crowded = false;   // attention_stream.h: hardly more (sequence, kv head) pairs than compute units
   int kv_magic = 0;   // ceil(65536 / n_kv_heads): block id / n_kv_heads = (id * kv_magic) >> 16 for id * n_kv_heads < 65536 (attn_wo.hip)
   float scale;     // float(1 / sqrt(head_dim)) (tensor.ts:3923 `.div(Math.sqrt(d))` = mul by the folded reciprocal)
   // several sequences at the same position (grid z): distance between consecutive sequences, in bytes (q, out, caches)

@@ -40,6 +40,7 @@ def test_attn_decode_batch_at_the_chunk_lines(hip, hd, B, H, KV, positions):
     (64, 1, 8, 2, (1, 31, 32, 33, 127, 128, 129, 385, 2100, 4096, 9000)), (128, 1, 12, 4, (15, 16, 17, 64, 65, 257, 1025, 8200)),   # many blocks to a pair
     (64, 16, 16, 16, (128, 129, 400, 513, 5)), (128, 16, 16, 16, (64, 193, 256, 257, 500)),   # one
     (64, 41, 32, 8, (50, 900)), (128, 41, 24, 8, (50, 450)),   # more pairs than compute units
+    (64, 33, 32, 8, (50, 896, 897, 1500)), (128, 36, 24, 8, (448, 449, 1400)),   # a few more
     (64, 4, 16, 2, (40, 700)), (128, 4, 16, 2, (40, 700)), (64, 4, 6, 2, (40, 700)), (128, 3, 2, 1, (40, 700)),
 ])
 def test_attn_decode_batch_at_the_edges_of_tiles(hip, hd, B, H, KV, positions):
