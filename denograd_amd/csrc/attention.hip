@@ -61,7 +61,7 @@ __global__ __launch_bounds__(ATT_STREAM_NW * 64) void attn_decode_stream_kernel(
 static bool stream_crowded(int pairs) { return pairs > state().cu_count && pairs <= state().cu_count * 9 / 8; }
 static int stream_nsplit(int pairs) {
   const int cu = state().cu_count, n = stream_crowded(pairs) ? 6 : (pairs > cu ? 3 : 1) * cu / pairs;
-  return n < 1 ? 1 : (n > 64 ? 64 : n);
+  return n < 1 ? 1 : (n > ATT_STREAM_BLOCKS ? ATT_STREAM_BLOCKS : n);
 }
 
 template <typename AT, int HD, int NW> static int launch_attn(const AttnArgs &a, int n_rep) {
@@ -135,8 +135,8 @@ size_t jsgrad_hip_attn_workspace_bytes(int n_heads, int n_kv_heads, int head_dim
 }
 
 size_t jsgrad_hip_attn_batch_workspace_bytes(int batch, int n_heads, int n_kv_heads, int head_dim) {
-  // per sequence: n_kv_heads counters, then the partials as above
-  return (size_t)batch * (((size_t)n_kv_heads * sizeof(int) + 255) / 256 * 256 + (size_t)n_heads * 256 * (head_dim + 2) * sizeof(float));
+  // per sequence: n_kv_heads counters; the partial results of each one's most blocks
+  return (size_t)batch * (((size_t)n_kv_heads * sizeof(int) + 255) / 256 * 256 + (size_t)n_heads * ATT_STREAM_BLOCKS * (head_dim + 2) * sizeof(float));
 }
 
 int jsgrad_hip_attn_decode_batch(const void *q, const void *cache_k, const void *cache_v, const int32_t *st, void *out, void *workspace, int batch,
@@ -146,6 +146,7 @@ int jsgrad_hip_attn_decode_batch(const void *q, const void *cache_k, const void 
   JSG_REQUIRE(batch > 0 && batch <= 65535, "jsgrad_hip_attn_decode_batch: batch %d", batch);
   JSG_REQUIRE(n_heads > 0 && n_kv_heads > 0 && n_kv_heads <= 64 && n_heads % n_kv_heads == 0, "jsgrad_hip_attn_decode_batch: n_heads %d / n_kv_heads %d", n_heads, n_kv_heads);
   JSG_REQUIRE(head_dim == 64 || head_dim == 128, "jsgrad_hip_attn_decode_batch: head_dim %d (64 and 128 are built)", head_dim);
+  // the longest cache that one sequence alone could be decoded from (attn_decode_check)
   JSG_REQUIRE(max_context > 0 && max_context <= 256 * ATT_CHUNK_MAX, "jsgrad_hip_attn_decode_batch: max_context %d exceeds %d", max_context, 256 * ATT_CHUNK_MAX);
   const size_t counter_bytes = ((size_t)n_kv_heads * sizeof(int) + 255) / 256 * 256;
   AttnArgs a;
@@ -156,7 +157,7 @@ int jsgrad_hip_attn_decode_batch(const void *q, const void *cache_k, const void 
   a.scale = (float)(1.0 / sqrt((double)head_dim));
   a.q_bstride = (size_t)n_heads * head_dim * sizeof(_Float16);
   a.cache_bstride = (size_t)max_context * n_kv_heads * head_dim * sizeof(_Float16);
-  a.partial_bstride = (size_t)n_heads * 256 * (head_dim + 2);
+  a.partial_bstride = (size_t)n_heads * ATT_STREAM_BLOCKS * (head_dim + 2);
   const int n_rep = n_heads / n_kv_heads;
   return head_dim == 64 ? launch_attn_stream<64>(a, n_rep, batch) : launch_attn_stream<128>(a, n_rep, batch);
 }

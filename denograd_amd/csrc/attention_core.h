@@ -80,7 +80,7 @@ struct AttnArgs {
   bool crowded = false;   // attention_stream.h: hardly more (sequence, kv head) pairs than compute units
   int kv_magic = 0;   // ceil(65536 / n_kv_heads): block id / n_kv_heads = (id * kv_magic) >> 16 for id * n_kv_heads < 65536 (attn_wo.hip)
   float scale;     // float(1 / sqrt(head_dim)) (tensor.ts:3923 `.div(Math.sqrt(d))` = mul by the folded reciprocal)
-  // several sequences at the same position (grid z): distance between consecutive sequences, in bytes (q, out, caches)
+  // several sequences at the same position (grid y): distance between consecutive sequences, in bytes (q, out, caches)
   // and in elements (counters, partial); zero for a single sequence
   size_t q_bstride = 0, cache_bstride = 0, partial_bstride = 0;
   // when set, the merged output goes here as tagged words (value | out_tag << 16) for other blocks of the same launch

@@ -20,6 +20,8 @@
 
 namespace jsg {
 
+constexpr int ATT_STREAM_BLOCKS = 64;   // of a (sequence, kv head) pair: what the workspace has room for, and the merge a lane for each
+
 // Blocks for T visible positions of a (sequence, kv head) pair, of at most `most`.  One block takes the pair in `rounds` round trips of 0.8 us, n
 // blocks in an n-th of them, and a merge: 2 us, and more with n.  So n blocks are worth it where they save three rounds, and n^2 = 6 rounds is the most.
 // us, 1 | 2 | 3 | 4 | 6 | 8 | 12 | 16 blocks, head_dim 128: 2 sequences 2048 positions 30.4 | 19.2 | 15.4 | 13.1 | 11.3 | 10.5 | 10.4 | 11.5, 5 sequences
@@ -59,7 +61,7 @@ template <int HD, int NREP, int NW> struct AttnStream {
   static_assert(HD == 64 || HD == 128, "one or two V rows per 16 lanes");
   static_assert(HP == 1 || HP == 2 || HP == 4 || HP == 8, "heads divide the columns");
   struct Smem {
-    float sc[NREP][64];                        // the merge's weights
+    float sc[NREP][ATT_STREAM_BLOCKS];         // the merge's weights
     float o_part[NW][NREP * HD];
     float m[NREP][NW], l[NREP][NW], w[NREP][NW];
     float m_sh[NREP], l_sh[NREP];
@@ -266,7 +268,7 @@ template <int HD, int NREP, int NW> struct AttnStream {
     __syncthreads();
     if (!sm.is_last) return;
     // A value's partial results are asked for together with the (m, l) that their weights are made of, MB blocks at a time: one round trip.
-    // One wavefront per query head makes the weights; block lane < n_active <= 64.
+    // One wavefront per query head makes the weights; block lane < n_active <= ATT_STREAM_BLOCKS.
     auto part = [&](int i, int s) { return ld_coherent(base + (size_t)min(s, n_active - 1) * NREP * (HD + 2) + i); };
     constexpr int PER = (NREP * HD + nthreads - 1) / nthreads;
     auto merge = [&](auto I) {

@@ -64,3 +64,19 @@ def test_attn_decode_batch_at_the_edges_of_tiles(hip, hd, B, H, KV, positions):
             assert np.all(got[B] == 7.0)
             ref = attention_ref(q, ck, cv, B, 1, T - 1, H, KV, hd)
             assert np.max(np.abs(got[:B] - ref)) < 4e-3, T
+
+
+@pytest.mark.parametrize("hd,B,H,KV,T", [(64, 1, 8, 1, 20000), (128, 2, 4, 2, 12000), (128, 33, 8, 8, 1400)])
+def test_the_workspace_has_room_for_the_most_blocks(hip, hd, B, H, KV, T):
+    """Nothing behind the bytes that the library asks for is written; counters are zero again.  The last sequence's partial results end where they do."""
+    rng = np.random.default_rng(T)
+    q = rng.standard_normal((B, H * hd)).astype(np.float16)
+    ck, cv = (rng.standard_normal((B, T, KV, hd)).astype(np.float16) for _ in range(2))
+    nbytes = hip.jsgrad_hip_attn_batch_workspace_bytes(B, H, KV, hd)
+    assert nbytes == B * (256 + H * 64 * (hd + 2) * 4)
+    ws = Tensor(np.concatenate([np.zeros(nbytes, np.uint8), np.full(4096, 7, np.uint8)]))
+    tq, tk, tv, st, out = Tensor(q), Tensor(ck), Tensor(cv), Tensor(np.array([0, T - 1], np.int32)), Tensor.full((B, H * hd), 7.0, "float16")
+    check(hip.jsgrad_hip_attn_decode_batch(tq.ptr, tk.ptr, tv.ptr, st.ptr, out.ptr, ws.ptr, B, H, KV, hd, T))
+    words = ws.numpy()
+    assert np.all(words[nbytes:] == 7) and not words[:B * KV * 4].any()
+    assert np.max(np.abs(out.numpy().astype(np.float64) - attention_ref(q, ck, cv, B, 1, T - 1, H, KV, hd))) < 4e-3
