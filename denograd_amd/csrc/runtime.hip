@@ -297,7 +297,7 @@ int jsgrad_hip_read_step(const int32_t *st, const void *attn_wo_workspace, const
   static std::mutex lock;
   static uint64_t *slot = nullptr;
   static uint32_t calls = 0;
-  std::lock_guard<std::mutex> guard(lock);
+  std::lock_guard<std::mutex> guard(lock);                     // held while waiting: a second reader's kernel would be queued behind this one's anyway
   if (!slot) {
     JSG_HIP(hipHostMalloc((void **)&slot, 2 * sizeof(uint64_t), hipHostMallocCoherent | hipHostMallocMapped));
     slot[0] = slot[1] = 0;
@@ -309,7 +309,8 @@ int jsgrad_hip_read_step(const int32_t *st, const void *attn_wo_workspace, const
   for (uint32_t spin = 1;; spin++) {
     for (int i = 0; i < 2; i++) w[i] = __atomic_load_n(&slot[i], __ATOMIC_RELAXED);
     if ((uint32_t)(w[0] >> 32) == seq && (uint32_t)(w[1] >> 32) == seq) break;
-    if (spin % 4096) continue;
+    __builtin_ia32_pause();                                    // the core's other thread may have something to do
+    if (spin % 1024) continue;
     const hipError_t e = hipStreamQuery(state().stream);       // now and then: has the device given up
     if (e == hipErrorNotReady) { (void)hipGetLastError(); continue; }
     JSG_HIP(e);

@@ -57,12 +57,13 @@ def test_read_step_returns_the_token_and_the_error_word_in_stream_order(hip):
 
 def test_read_step_from_two_threads(hip):
     states = [Tensor(np.array([t * 1000 + 5, 0], np.int32)) for t in range(2)]
-    bad = []
+    bad, done = [], [0, 0]
 
     def loop(t):
         words = (C.c_int32 * 2)()
         for _ in range(200):
             check(hip.jsgrad_hip_read_step(states[t].ptr, None, None, words))
+            done[t] += 1                                      # a thread that an error has ended stays below 200
             if list(words) != [t * 1000 + 5, 0]:
                 bad.append((t, list(words)))
 
@@ -71,7 +72,7 @@ def test_read_step_from_two_threads(hip):
         t.start()
     for t in threads:
         t.join()
-    assert not bad
+    assert not bad and done == [200, 200]
 
 
 def test_an_error_of_the_attention_launches_is_raised_with_the_token(hip):
