@@ -88,7 +88,7 @@ __device__ __forceinline__ float square_sum(h8_t x, float s) {
 
 // What a test asks for, or null.  Looking a variable up costs a walk through the environment, so a call makes one walk for all of them.
 inline bool any_pins() {
-  for (char **e = environ; *e; e++)
+  for (char **e = environ; e && *e; e++)                     // null behind clearenv()
     if (!strncmp(*e, "JSG_", 4)) return true;
   return false;
 }

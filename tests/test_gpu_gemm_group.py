@@ -3,6 +3,9 @@ K parts, under every epilogue, at ragged row tiles and where turns of its ring r
 turns than the ring holds, a last turn with stages for some groups only.
 
 Tolerance: products and sums are those of the oracle's several-row Linear in another order (assert_close)."""
+import ctypes as C
+import os
+
 import numpy as np
 import pytest
 
@@ -123,3 +126,21 @@ def test_lines_to_the_kernel_for_short_rows_of_nf4_gates(hip, monkeypatch, rows,
         check(hip.jsgrad_hip_gemm_ffn_gate(ffi.W_NF4, w.ptr, s.ptr, w.ptr + hidden * dim // 2, s.ptr, x.ptr, rows, y.ptr, dim, hidden))
         out.append(y.numpy().view(np.uint16))
     assert np.array_equal(*out) == skinny
+
+
+def test_a_process_without_an_environment(hip):
+    """clearenv() leaves no list of variables at all: the calls that look for pins in it run as they do without any."""
+    x, w = Tensor.randn((4 * 512,), "float16", 1, 1.0), Tensor.randn((128 * 512,), "float16", 2, 0.05)
+    out = []
+    for clear in (False, True):
+        y = Tensor.empty((4, 128), "float16")
+        if clear:
+            C.CDLL(None).clearenv()
+        try:
+            status = hip.jsgrad_hip_gemm(ffi.W_F16, w.ptr, None, 128, 512, x.ptr, 4, y.ptr, None)
+        finally:
+            for name, value in os.environ.items():
+                os.putenv(name, value)
+        check(status)
+        out.append(y.numpy().view(np.uint16))
+    assert np.array_equal(*out)
