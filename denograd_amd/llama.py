@@ -132,13 +132,17 @@ class TransformerBlock:
 
     def call_rows(self, x: Tensor, bsz: int, seqlen: int, start_pos: int, state: Tensor, freqs_cis: Tensor, rows: "_RowScratch") -> Tensor:
         """TransformerBlock.call (llama.ts:124-127) on x [bsz*seqlen, dim]; the result is written back into x."""
-        lib, n = ffi.load(), bsz * seqlen
-        h = self.attention.call_rows(x, bsz, seqlen, start_pos, state, freqs_cis, rows, residual=x, out=rows.h2, norm=self.attention_norm)
-        if type(self.feed_forward).call_rows is FeedForward.call_rows:
-            return self.feed_forward.call_rows(h, n, rows, residual=h, out=x, norm=self.ffn_norm)
-        # a feed forward of the caller's own takes its rows normed
-        check(lib.jsgrad_hip_rmsnorm_rows(h.ptr, self.ffn_norm.weight.ptr, rows.xn.ptr, n, self.attention.dim, self.ffn_norm.eps))
-        return self.feed_forward.call_rows(rows.xn, n, rows, residual=h, out=x)
+        n = bsz * seqlen
+
+        def call(part, norm: RMSNorm, x: Tensor, *args, **kw) -> Tensor:
+            if getattr(part.call_rows, "__func__", None) in (Attention.call_rows, FeedForward.call_rows):
+                return part.call_rows(x, *args, **kw, norm=norm)
+            # one of the caller's own, of its class or set on the object, takes its rows normed
+            check(ffi.load().jsgrad_hip_rmsnorm_rows(x.ptr, norm.weight.ptr, rows.xn.ptr, n, self.attention.dim, norm.eps))
+            return part.call_rows(rows.xn, *args, **kw)
+
+        h = call(self.attention, self.attention_norm, x, bsz, seqlen, start_pos, state, freqs_cis, rows, residual=x, out=rows.h2)
+        return call(self.feed_forward, self.ffn_norm, h, n, rows, residual=h, out=x)
 
 
 def attn_wo_fits(n_heads: int, n_kv_heads: int, head_dim: int, max_context: int, kind: int, dim: int, capacity: int | None = None) -> bool:
