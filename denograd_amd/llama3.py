@@ -227,8 +227,13 @@ class Llama3:
     # ---- inference (token ids in, token ids out)
     def _call(self, tok: int) -> int:
         """llama3.ts:334-337: one model call and the per-token device->host read."""
-        self.model.call(np.array([[tok]], np.int32), self.start_pos, self.temperature, self.top_k, self.top_p, self.alpha_f, self.alpha_p)
-        return self.model.read_token()
+        model = self.model
+        res = model.call(np.array([[tok]], np.int32), self.start_pos, self.temperature, self.top_k, self.top_p, self.alpha_f, self.alpha_p)
+        if isinstance(model, Transformer) and isinstance(res, Tensor) and res.ptr == model.state.ptr:
+            return model.read_token()
+        tok = int(res.item())                  # a call of the user's own, with a token that it picked itself
+        model.check_errors()
+        return tok
 
     def _prefill(self, toks: list[int]) -> None:
         """llama3.ts:297-312: skip the shared prefix of the previous prompt when starting over, then feed tokens one at a time."""

@@ -83,3 +83,22 @@ def test_an_error_of_the_attention_launches_is_raised_with_the_token(hip):
     check(hip.jsgrad_hip_memset(llm.model._ctx.attn_wo_ws.ptr + 256, 1, 4))     # as a bounded wait that ran out would leave it
     with pytest.raises(ffi.HipError, match="gave up waiting"):
         llm._call(4)
+
+
+def test_the_token_is_the_one_that_the_models_call_returns(hip):
+    """A call of the user's own on top of the model's, which picks another token from the logits."""
+    cfg = synthetic.config("tiny16")
+    llm = Llama3.from_config(cfg).load_weights(synthetic.random_state_dict(cfg, seed=0), quantized=True)
+    plain = llm.model.call
+
+    def second_best(*args):
+        plain(*args)
+        return Tensor(np.argsort(llm.model.logits.numpy().astype(np.float32))[-2:-1].astype(np.int32))
+
+    llm.chat_tokens([1, 2, 3], 2)
+    llm.model.call = second_best
+    got = llm._call(4)
+    llm.model.call = plain
+    order = np.argsort(llm.model.logits.numpy().astype(np.float32))
+    assert got == order[-2] != order[-1]
+    assert llm._call(4) == llm.model.state.numpy()[0]

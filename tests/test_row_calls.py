@@ -1,10 +1,11 @@
-"""What the host side of a several-row call hands to whom: the library is replaced by one that writes its calls down."""
+"""What the host side of a model call hands to whom: the library, or the model, is replaced by one that writes its calls down."""
 import types
 
 import pytest
 
-from denograd_amd import ffi, llama
+from denograd_amd import ffi
 from denograd_amd.llama import Attention, FeedForward, TransformerBlock
+from denograd_amd.llama3 import Llama3
 
 buffer = lambda p: types.SimpleNamespace(ptr=p)
 X, XN, H2 = buffer(100), buffer(200), buffer(300)
@@ -84,3 +85,20 @@ def test_parts_of_the_callers_own_take_their_rows_normed(lib, own):
     assert run(b) is X
     assert b.attention.seen == (XN, X, H2) and b.feed_forward.seen == (XN, H2, X)
     assert lib.calls == [("jsgrad_hip_rmsnorm_rows", (X.ptr, 1, XN.ptr, 6, 64, 1e-5)), ("jsgrad_hip_rmsnorm_rows", (H2.ptr, 2, XN.ptr, 6, 64, 1e-5))]
+
+
+def test_a_model_of_the_callers_own_is_asked_for_its_token_and_its_errors():
+    llm, seen = Llama3.__new__(Llama3), []
+
+    class Model:
+        def call(self, tokens, start_pos, *sampling):
+            seen.append((tokens.tolist(), start_pos, sampling))
+            return types.SimpleNamespace(item=lambda: 42.0)
+
+        def check_errors(self):
+            seen.append("errors")
+
+    llm.model, llm.start_pos = Model(), 5
+    llm.temperature, llm.top_k, llm.top_p, llm.alpha_f, llm.alpha_p = 0.5, 1, 0.2, 0.3, 0.4
+    assert llm._call(7) == 42
+    assert seen == [([[7]], 5, (0.5, 1, 0.2, 0.3, 0.4)), "errors"]
