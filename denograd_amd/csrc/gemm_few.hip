@@ -278,7 +278,7 @@ int gemm_few(int epi, int kind, const GemmArgs &a, int prof_kind, bool *taken) {
   // The norm's weights are read here in 16-byte pieces; from any other address in memory first.
   if (a.norm_w && (a.K > 4096 || (uintptr_t)a.norm_w & 15)) return 0;
   if (kind == JSGRAD_W_I8 && (elements > (size_t)36 << 20 || (a.M > 8 && a.K > 3072))) return 0;
-  if (pin_env(a, "JSG_GEMM_NO_SKINNY") || pin_env(a, "JSG_GEMM_SKINNY_TILES") || pin_env(a, "JSG_SG_TPW")) return 0;   // tests that want one of the other kernels
+  if (pin_env(a, "JSG_GEMM_NO_SKINNY") || pin_env(a, "JSG_GEMM_SKINNY_TILES")) return 0;   // tests that want one of the other kernels
   if (epi == GEPI_STORE) return gemm_few_epi<GEPI_STORE>(kind, a, prof_kind, taken);
   if (epi == GEPI_ROPE_KV) return gemm_few_epi<GEPI_ROPE_KV>(kind, a, prof_kind, taken);
   return gemm_few_epi<GEPI_SWIGLU>(kind, a, prof_kind, taken);
