@@ -49,18 +49,25 @@ __global__ __launch_bounds__(ATT_STREAM_NW * 64) void attn_decode_stream_kernel(
     a.counters += z * a.n_kv_heads;
     a.partial += z * a.partial_bstride;
   }
-  A::item(a, sm, g, split, [&](int T) { return att_stream_blocks<HD, ATT_STREAM_NW>(T, a.nsplit, a.crowded); });
+  A::item(a, sm, g, split, [&](int T) { return att_stream_blocks<HD, ATT_STREAM_NW>(T, a.nsplit, a.split_from); });
 }
 
 // Blocks per (sequence, kv head) of the streaming launch: one block to a compute unit, whose rows on their way (32 KB) are enough, for every
 // block more is a longer merge.  us, head_dim 128, 2050 positions, 1 | 2 | 3 | 4 | 6 | 8 blocks: 16 sequences of 8 kv heads 34.4 | 29.0 | 33.1 | 30.6 | 30.1 |
 // 31.1, 8 sequences 32.5 | 21.9 | 18.1 | 18.0 | 19.8 | 17.9; 1000 positions, 24 sequences 21.8 | 24.8 | 25.7 | 23.4 | 24.8 | 24.8, 32 27.6 | 29.1 | 29.1 | 30.4 |
 // 30.9 | 32.1.  With more pairs than units some have two: three to a unit, 40 sequences 39.7 | 37.2 | 36.3 | 36.7 | 38.0 | 39.0.
-// Up to an eighth more pairs than units: six blocks.  us, 2 | 3 | 6 blocks, 33 sequences: head_dim 128, 4 query heads 1300 positions 43.1 | 41.5 | 39.7, 3000 93.9 |
-// 90.2 | 86.6, one 3000 91.2 | 87.1 | 83.1; head_dim 64, 4 query heads 3000 58.7 | 54.9 | 52.4; 36 sequences 3000 60.0 | 57.2 | 55.3, 40 62.2 | 60.0 | 61.5.
-static bool stream_crowded(int pairs) { return pairs > state().cu_count && pairs <= state().cu_count * 9 / 8; }
-static int stream_nsplit(int pairs) {
-  const int cu = state().cu_count, n = stream_crowded(pairs) ? 6 : (pairs > cu ? 3 : 1) * cu / pairs;
+// Where one or two blocks a pair leave many units idle, or some with twice the work of the others, long pairs are split further.  us, 4 query heads, 33
+// sequences, 2 | 3 | 6 blocks: head_dim 128 1300 positions 43.1 | 41.5 | 39.7, 3000 93.9 | 90.2 | 86.6, head_dim 64 3000 58.7 | 54.9 | 52.4; 40 sequences
+// 62.2 | 60.0 | 61.5; 1 | 3 | 5 blocks: 18 sequences, head_dim 128 550 14.4 | 14.1 | 14.7, 2050 38.4 | 34.2 | 33.7, 4000 66.7 | 53.9 | 51.5, head_dim 64
+// 4000 41.4 | 38.0 | 36.6; 20 sequences, head_dim 128 2050 39.0 | 35.8 | 40.7, 4000 71.8 | 59.0 | 67.2, head_dim 64 1300 17.1 | 17.8 | 17.7, 4000
+// 42.6 | 39.6 | 43.8; 22 sequences 4000 74.0 | 83.1 | 74.3.
+static int stream_nsplit(int pairs, int &split_from) {
+  const int cu = state().cu_count;
+  split_from = 0;
+  if (pairs > cu && pairs <= cu * 9 / 8) { split_from = 8; return 6; }
+  if (pairs > cu / 2 && pairs <= cu * 9 / 16) { split_from = 10; return 5; }
+  if (pairs > cu / 2 && pairs <= cu * 2 / 3) { split_from = 24; return 3; }
+  const int n = (pairs > cu ? 3 : 1) * cu / pairs;
   return n < 1 ? 1 : (n > ATT_STREAM_BLOCKS ? ATT_STREAM_BLOCKS : n);
 }
 
@@ -153,7 +160,7 @@ int jsgrad_hip_attn_decode_batch(const void *q, const void *cache_k, const void 
   a.q = q; a.cache_k = cache_k; a.cache_v = cache_v; a.st = st; a.out = out;
   a.counters = (int *)workspace;                                   // [batch][n_kv_heads], densely packed
   a.partial = (float *)((char *)workspace + (size_t)batch * counter_bytes);
-  a.n_kv_heads = n_kv_heads; a.nsplit = stream_nsplit(n_kv_heads * batch); a.crowded = stream_crowded(n_kv_heads * batch); a.max_context = max_context;
+  a.n_kv_heads = n_kv_heads; a.nsplit = stream_nsplit(n_kv_heads * batch, a.split_from); a.max_context = max_context;
   a.scale = (float)(1.0 / sqrt((double)head_dim));
   a.q_bstride = (size_t)n_heads * head_dim * sizeof(_Float16);
   a.cache_bstride = (size_t)max_context * n_kv_heads * head_dim * sizeof(_Float16);

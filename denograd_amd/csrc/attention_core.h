@@ -77,9 +77,9 @@ struct AttnArgs {
   int *err = nullptr;   // optional: set to 1 when the merging block's bounded wait for the other chunks ran out
   float *partial;  // [n_kv_heads][nsplit][n_rep][HD + 2]
   int n_kv_heads, nsplit, max_context;
-  bool crowded = false;   // attention_stream.h: hardly more (sequence, kv head) pairs than compute units
   int kv_magic = 0;   // ceil(65536 / n_kv_heads): block id / n_kv_heads = (id * kv_magic) >> 16 for id * n_kv_heads < 65536 (attn_wo.hip)
   float scale;     // float(1 / sqrt(head_dim)) (tensor.ts:3923 `.div(Math.sqrt(d))` = mul by the folded reciprocal)
+  int split_from = 0;     // attention_stream.h: rounds of loads from which a (sequence, kv head) pair that could have a compute unit of its own is split; 0: few pairs
   // several sequences at the same position (grid y): distance between consecutive sequences, in bytes (q, out, caches)
   // and in elements (counters, partial); zero for a single sequence
   size_t q_bstride = 0, cache_bstride = 0, partial_bstride = 0;

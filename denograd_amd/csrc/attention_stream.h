@@ -27,13 +27,13 @@ constexpr int ATT_STREAM_BLOCKS = 64;   // of a (sequence, kv head) pair: what t
 // us, 1 | 2 | 3 | 4 | 6 | 8 | 12 | 16 blocks, head_dim 128: 2 sequences 2048 positions 30.4 | 19.2 | 15.4 | 13.1 | 11.3 | 10.5 | 10.4 | 11.5, 5 sequences
 // 90 5.8 | 6.7 | 6.9 | 6.9 | 7.1 | 7.6 | 7.7 | 8.5, 300 8.4 | 8.3 | 7.9 | 7.8 | 7.6 | 7.9 | 8.3 | 8.7, 1000 17.8 | 12.8 | 11.5 | 10.2 | 9.7 | 10.9 | 11.1 | 11.9;
 // head_dim 64: 5 sequences 300 6.7 | 7.3 | 6.7 | 6.8 | 6.9 | 7.1 | 7.2 | 7.4, 600 8.2 | 8.3 | 7.6 | 7.6 | 7.3 | 7.3 | 7.4 | 7.6.
-// Crowded: there are a few more pairs than compute units, and a unit with two whole ones is twice as long at work as the others (a.crowded).  There
-// parts of a pair wait for each other's loads, not only for their own: n^2 = 3 rounds, from eight rounds on.
-template <int HD, int NW> __device__ __forceinline__ int att_stream_blocks(int T, int most, bool crowded) {
+// split_from: there are about as many pairs as compute units (attention.hip), so that parts of a pair wait for each other's loads, not only for their
+// own: only from that many rounds on, and n^2 = 3 rounds.
+template <int HD, int NW> __device__ __forceinline__ int att_stream_blocks(int T, int most, int split_from) {
   constexpr int ROUND = NW * (HD == 64 ? 32 : 16);
   const int rounds = (T + ROUND - 1) / ROUND;
-  if (crowded && rounds < 8) return 1;
-  const int n = min(min(most, rounds), (int)__builtin_amdgcn_sqrtf((crowded ? 3.0f : 6.0f) * (float)rounds));
+  if (rounds < split_from) return 1;
+  const int n = min(min(most, rounds), (int)__builtin_amdgcn_sqrtf((split_from ? 3.0f : 6.0f) * (float)rounds));
   return rounds - (rounds + n - 1) / n >= 3 ? n : 1;
 }
 template <int I, int N, typename F> __device__ __forceinline__ void static_for(F &&f) {
@@ -102,7 +102,7 @@ template <int HD, int NREP, int NW> struct AttnStream {
     };
     // the first one before the position has arrived: what lies behind it is masked.  Not where blocks that may have nothing to do come on top of a full
     // chip (33 sequences at 60 of 4000 positions, us: 9.5, without their loads 5.7; one block per pair 5.5)
-    if (a.crowded && split != 0 && split >= blocks(a.st[1] + 1)) return;
+    if (split != 0 && a.split_from && split >= blocks(a.st[1] + 1)) return;
     int tb = (split * NW + wave) * TILE;
     load_k(tb, a.max_context - 1);
     load_v(tb, a.max_context - 1);

@@ -41,6 +41,7 @@ def test_attn_decode_batch_at_the_chunk_lines(hip, hd, B, H, KV, positions):
     (64, 16, 16, 16, (128, 129, 400, 513, 5)), (128, 16, 16, 16, (64, 193, 256, 257, 500)),   # one
     (64, 41, 32, 8, (50, 900)), (128, 41, 24, 8, (50, 450)),   # more pairs than compute units
     (64, 33, 32, 8, (50, 896, 897, 1500)), (128, 36, 24, 8, (448, 449, 1400)),   # a few more
+    (64, 18, 32, 8, (1152, 1153, 2200)), (128, 20, 24, 8, (1472, 1473, 1700)),   # one unit a pair leaves many idle
     (64, 4, 16, 2, (40, 700)), (128, 4, 16, 2, (40, 700)), (64, 4, 6, 2, (40, 700)), (128, 3, 2, 1, (40, 700)),
 ])
 def test_attn_decode_batch_at_the_edges_of_tiles(hip, hd, B, H, KV, positions):
