@@ -257,8 +257,9 @@ int gemm_few(int epi, int kind, const GemmArgs &a, int prof_kind, bool *taken) {
   *taken = false;
   if (a.M > 16 || a.N % 16 || ((uintptr_t)a.s0 | (uintptr_t)a.s1 | (uintptr_t)a.s2) & 3) return 0;
   // int8: the codes of a tile are half the bytes behind the same x, and a tile is over in a step or two; gemm_group.hip keeps its ring full
-  // over wide matrices.  us, 8 / 16 rows, that one | this one: 5120 x 3072 9.2 / 9.3 | 7.7 / 8.5, 3072 x 8192 10.6 / 10.9 | 10.5 / 12.7, 16384 x 2048
-  // 10.9 / 10.5 | 10.7 / 11.1, 6144 x 4096 10.4 / 10.7 | 10.7 / 12.0, 16384 x 3072 13.3 / 13.2 | 14.1 / 15.0, 28672 x 4096 22.2 / 22.1 | 28.7 / 30.3.
+  // over wide matrices.  us, 8 / 16 rows, that one | this one: 5120 x 3072 8.6 / 8.7 | 7.6 / 8.3, 2048 x 8192 9.1 / 9.4 | 9.2 / 12.0, 3072 x 8192 9.9 / 10.1 |
+  // 10.4 / 12.5, 4096 x 6144 10.3 / 10.4 | 9.3 / 12.3, 6144 x 4096 9.6 / 9.8 | 10.6 / 12.0, 16384 x 3072 12.3 / 12.3 | 14.1 / 15.0, 28672 x 4096 21.9 / 21.9 |
+  // 28.7 / 30.3.  (Up to 36 M codes behind 8 rows the two are within a tenth of each other; the line is from before the group kernel's 16x64 tiles shared units.)
   // fp16, skinny_gemm_kernel | this one, 2 / 8 / 16 rows: 2048 x 2048 6.2 / 6.3 / 6.3 | 4.5 / 4.5 / 5.1, 2048 x 8192 14.1 / 14.9 / 15.9 |
   // 8.8 / 9.5 / 12.4, 16384 x 2048 23.6 / 23.7 / 24.4 | 16.3 / 17.2 / 18.2, 128256 x 2048 147 / 153 / 162 | 88 / 92 / 94 (6.0 TB/s).
   // fp16 rows of more than 4096 elements (6144 and 8192 come here): the more rows of x a block reads for its few tiles, the nearer gemm_group.hip, which reads x from LDS, comes.  us,

@@ -3,12 +3,12 @@
 //
 // The launch should be bound by reading W once.  With few rows a tile has little arithmetic, and what a compute unit can draw is the
 // bytes it has on their way over the time they take (2 us under load): so one block of eight wavefronts owns nearly all of a unit's
-// LDS as a ring of ST turns.  A turn is G neighbouring K stages of the tile (G x 64 elements, nf4 G x 128), one per K group; the WN
+// LDS (int8 in 16x64 tiles: two blocks half each) as a ring of ST turns.  A turn is G neighbouring K stages of the tile (G x 64 elements, nf4 G x 128), one per K group; the WN
 // wavefronts of a group split the tile's columns, so a weight is dequantised once per block and a piece of x is read by WN wavefronts.
 // Fragments are read a turn ahead of the matrix instructions that use them, one barrier per turn.  The groups' sums are
 // added in LDS in group order; K parts over blocks as in gemm_tile.hip, in part order.
-// Measured (weights from memory, us, the kernels it took the sizes from | this one): 16 rows, int8 28672 x 4096 27.0 | 22.1 (5.3 TB/s), 4096 x 14336 17.8 |
-// 15.8; 24 rows, int8 16384 x 3072 22.8 | 15.0, 128256 x 3072 213 | 77; fp16 16384 x 2048 23.8 | 14.7, 128256 x 3072 265 | 126 (6.2 TB/s), 4096 x 14336
+// Measured (weights from memory, us, the kernels it took the sizes from | this one): 16 rows, int8 28672 x 4096 27.0 | 21.9 (5.4 TB/s), 4096 x 14336 17.8 |
+// 15.1; 24 rows, int8 16384 x 3072 22.8 | 15.0, 128256 x 3072 213 | 77; fp16 16384 x 2048 23.8 | 14.7, 128256 x 3072 265 | 126 (6.2 TB/s), 4096 x 14336
 // 36 | 23; nf4 28672 x 4096 46 | 25, with 8 rows 36.7 | 21.7.  From 33 rows on LDS reads and matrix instructions of a turn take as long as its bytes to
 // arrive, and it is ahead by less: 57 rows, 16384 x 3072 int8 19.5 | 17.5, nf4 21.4 | 18.4, 128256 x 3072 int8 112 | 104.
 #include <type_traits>
@@ -68,7 +68,10 @@ template <int KIND, int EPI, int WB, int BM, int BN, int WN, int ST> __global__ 
   // Weight rows whose distance is a multiple of 4 KiB: blocks start their walk through K at different turns and wrap around, so that they
   // don't queue at the same offset of such rows for the same memory channels (28672 x 4096, us: int8, 8 rows 30.1 -> 26.4, 24 rows 33.9 ->
   // 32.2; fp16, 24 rows in 32x64 tiles 46.3 -> 41.9, but in 32x128 47 -> 55 and 57 rows 49.3 -> 56.7; other distances and K parts: 1 % slower).
-  const int first = BM <= 32 && (KIND != JSGRAD_W_F16 || BM * BN < 4096) && t.split == 1 && w_bytes % 4096 == 0 ? (int)((unsigned)(id.col / CW) % (unsigned)turns) : 0;
+  // int8 in 16x64 tiles: a turn is 256 bytes of a row, neighbours start two of them apart (14336 x 8192, one | two | four: 28.3 | 22.4 | 22.0, w1|w3 of
+  // 8192 x 8192 25.8 | 23.5 | 35.2).
+  constexpr unsigned APART = KIND == JSGRAD_W_I8 && BM == 16 && BN == 64 ? 2 : 1;
+  const int first = BM <= 32 && (KIND != JSGRAD_W_F16 || BM * BN < 4096) && t.split == 1 && w_bytes % 4096 == 0 ? (int)((unsigned)(id.col / CW) * APART % (unsigned)turns) : 0;
   auto turn_of = [&](int turn) { const int r = turn + first; return r >= turns ? r - turns : r; };
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)group_lds;
   const i4_t ra = dma_rsrc(a.x + (size_t)m0 * a.K);
@@ -322,10 +325,12 @@ template <int KIND, int EPI, int WB, int BM, int BN, int WN, int ST> static int 
 
 // Turns in LDS: as many as fit.  Stages have 128 bytes of a weight row, whole cache lines for eight rows per load: with 64 bytes of sixteen rows int8
 // codes came at three quarters of the rate (us, 64 | 128: 16384 x 3072, 16 rows 16.7 | 13.2, 28672 x 4096 27.4 | 22.1, 24 rows 32.7 | 26.6, 128256 x 3072 101 |
-// 77; nf4 28672 x 4096, 24 rows 29 | 25).  nf4 behind 64 rows of x, where that many K elements of x leave no room for a third turn, keeps 64.
+// 77; nf4 28672 x 4096, 24 rows 29 | 25).  int8 in 16x64 tiles: two K groups and 74 KB, so that two blocks share a unit and one's first loads and sums run
+// beside the other's turns (four groups and 146 KB | two: 41984 x 2560 31 | 21.7, 128256 x 1024 42.3 | 27.8, 28672 x 4096 26.5 | 22.5, 4096 x 14336 15.5 |
+// 14.7).  nf4 behind 64 rows of x, where that many K elements of x leave no room for a third turn, keeps 64.
 template <int KIND, int EPI> static int launch_group_kind(int bm, int bn, const TileArgs &t, int prof_kind) {
   constexpr bool NF4 = KIND == JSGRAD_W_NF4, F16 = KIND == JSGRAD_W_F16;
-  if (bm == 16 && bn == 64) return launch_group_as<KIND, EPI, 128, 16, 64, NF4 ? 4 : 2, 3>(t, prof_kind);
+  if (bm == 16 && bn == 64) return launch_group_as<KIND, EPI, 128, 16, 64, F16 ? 2 : 4, 3>(t, prof_kind);
   if (bm == 16 && bn == 128) return launch_group_as<KIND, EPI, 128, 16, 128, F16 ? 2 : 4, F16 || NF4 ? 2 : 3>(t, prof_kind);
   if (bm == 32 && bn == 64) return launch_group_as<KIND, EPI, 128, 32, 64, F16 ? 2 : 4, F16 ? 3 : (NF4 ? 2 : 4)>(t, prof_kind);
   if (bm == 32 && bn == 128) return launch_group_as<KIND, EPI, 128, 32, 128, 4, NF4 ? 2 : 3>(t, prof_kind);
@@ -349,12 +354,12 @@ static int launch_group(int epi, int kind, int bm, int bn, const TileArgs &t, in
 // The shapes with their K groups, and what a block's time is made of (us): a turn when every block has a compute unit to itself, what is
 // added to it when all units have one, a turn when there are several rounds of blocks, and a round's end.  Fitted to 8 to 57 rows over the matrices
 // of the 1B, 3B and 8B models in the three formats, weights from memory, each under every shape and number of K parts that could
-// matter; the choice is 2 % slower than the best shape on average.
+// matter; the choice is 2 % slower than the best shape on average.  (int8 16x64, two blocks to a unit: for the choice rather than for the single time.)
 struct GroupShape { int bm, bn, stage, groups; float step, fill, round_step, end; };   // stage: K elements
 constexpr int N_GROUP = 6;
 static const GroupShape GROUP_SHAPES[3][N_GROUP] = {   // fp16, int8, nf4
   {{16, 64, 64, 4, 0.44f, 0.43f, 0.91f, 1.3f}, {16, 128, 64, 4, 1.19f, 0.89f, 2.06f, 1.1f}, {32, 64, 64, 4, 0.52f, 0.51f, 1.07f, 1.5f}, {32, 128, 64, 2, 0.46f, 0.60f, 0.98f, 1.6f}, {64, 64, 64, 4, 1.06f, 0.54f, 1.64f, 1.6f}, {64, 128, 64, 2, 0.54f, 0.88f, 1.27f, 2.4f}},
-  {{16, 64, 128, 4, 0.62f, 0.37f, 1.21f, 1.7f}, {16, 128, 128, 2, 0.54f, 0.42f, 1.03f, 1.8f}, {32, 64, 128, 2, 0.39f, 0.29f, 0.77f, 1.7f}, {32, 128, 128, 2, 0.64f, 0.60f, 1.23f, 2.4f}, {64, 64, 128, 2, 0.53f, 0.45f, 1.03f, 2.4f}, {64, 128, 128, 2, 0.82f, 1.11f, 1.70f, 3.6f}},
+  {{16, 64, 128, 2, 0.325f, 0.168f, 0.456f, 0.91f}, {16, 128, 128, 2, 0.54f, 0.42f, 1.03f, 1.8f}, {32, 64, 128, 2, 0.39f, 0.29f, 0.77f, 1.7f}, {32, 128, 128, 2, 0.64f, 0.60f, 1.23f, 2.4f}, {64, 64, 128, 2, 0.53f, 0.45f, 1.03f, 2.4f}, {64, 128, 128, 2, 0.82f, 1.11f, 1.70f, 3.6f}},
   {{16, 64, 256, 2, 0.87f, 0.26f, 1.33f, 1.6f}, {16, 128, 256, 2, 1.69f, 0.45f, 2.27f, 1.9f}, {32, 64, 256, 2, 1.25f, 0.30f, 1.77f, 1.9f}, {32, 128, 256, 2, 1.94f, 0.63f, 2.56f, 2.5f}, {64, 64, 128, 2, 0.83f, 0.26f, 1.18f, 2.5f}, {64, 128, 128, 2, 1.06f, 0.81f, 1.70f, 3.8f}},
 };
 // The K parts' sums of a launch lie in memory that belongs to the library: they are also there in a graph capture and on a full device, and
@@ -390,8 +395,9 @@ GroupChoice choose_group(int epi, int kind, const GemmArgs &a) {
     for (int d = 1; d <= 16 && d <= stages; d++) {
       if (pin && d != (split < stages ? split : stages)) continue;
       const int blocks = tiles * d, turns = ((stages + d - 1) / d + s.groups - 1) / s.groups;
-      // parts of at least two turns, and not more than two blocks for every unit
-      if (d > 1 && (tiles > GROUP_COUNTERS || group_bytes(s, a.M, weight_rows, d) > GROUP_SUMS || (!pin && (turns < 2 || blocks > 2 * cus)))) break;
+      // parts of at least two turns (int8 behind 16 rows, whose turns are short: four; 16 x 1024 x 6144 in 12 parts of two 9.7 us, in six of four 8.5),
+      // and not more than two blocks for every unit
+      if (d > 1 && (tiles > GROUP_COUNTERS || group_bytes(s, a.M, weight_rows, d) > GROUP_SUMS || (!pin && (turns < (kind == JSGRAD_W_I8 && s.bm == 16 ? 4 : 2) || blocks > 2 * cus)))) break;
       const float fill = (float)blocks / cus;
       float us = 3.5f + (fill <= 1.0f ? (s.step + s.fill * fill) * turns + s.end : ((blocks + cus - 1) / cus) * (s.round_step * turns + s.end));
       if (d > 1) us += 1.7f + (float)d * s.bm * s.bn * 4 / 83e3f * (fill > 1.0f ? fill : 1.0f);
@@ -424,8 +430,9 @@ int gemm_group(int epi, int kind, const GemmArgs &a, int prof_kind, bool *taken)
     // One round of skinny_gemm_kernel's blocks over short rows: no K parts whose sums have to travel.  us, that | this one: 24 rows, fp16
     // 2048 x 2048 7.5 | 7.5, 3072 x 2048 8.1 | 8.1, 3072 x 3072 9.9 | 9.3, 4096 x 3072 9.9 | 10.5, 4096 x 3584 11.3 | 11.1, 2048 x 8192 18.7 | 11.5; int8
     // 1024 x 4096 8.7 | 8.2, 2048 x 4096 8.9 | 9.6, 4096 x 3584 9.2 | 10.2, 4096 x 4096 10.2 | 10.3, 4096 x 4608 11.0 | 10.8, 6144 x 4096 17.5 | 11.4, 28672 x 4096 50 | 27; nf4
-    // 4096 x 4096 9.3 | 10.9, 4096 x 5120 12.0 | 12.4, 4096 x 6144 12.8 | 12.6, 3072 x 8192 14.8 | 12.9, 28672 x 4096 46 | 25; 16 rows, int8 4096 x 4096
-    // 9.1 | 9.6, 2560 x 5120 9.9 | 9.0, 3840 x 5120 10.1 | 10.5 (w1|w3 of 2048 x 5120 14.2 | 12.0), 4096 x 5632 10.2 | 10.8, 6144 x 4096 13.5 | 10.7; nf4 4096 x 6144 10.3 | 10.9, 4096 x 8192
+    // 4096 x 4096 9.3 | 10.9, 4096 x 5120 12.0 | 12.4, 4096 x 6144 12.8 | 12.6, 3072 x 8192 14.8 | 12.9, 28672 x 4096 46 | 25; 16 / 2 rows, int8 4096 x 4096
+    // 8.9 / 8.4 | 9.0 / 8.8, 2560 x 5120 10.0 / 8.7 | 8.4 / 8.2, 3840 x 5120 10.0 / 8.9 | 9.8 / 9.5 (w1|w3 of 2048 x 5120 14.2 / 13.2 | 11.3 / 11.3), 4096 x 5632
+    // 10.3 / 9.0 | 10.2 / 9.8, 6144 x 4096 13.3 / 11.6 | 9.8 / 9.7; 16 rows, nf4 4096 x 6144 10.3 | 10.9, 4096 x 8192
     // 11.9 | 12.1, 4096 x 10240 14.8 | 13.4; 8 rows, nf4 4096 x 4096 7.8 | 9.4, 3072 x 8192 10.7 | 11.5, 6144 x 4096 11.3 | 10.7, 28672 x 4096 36.7 | 21.7.
     // Where this one finds four or five parts for a unit each (up to 3072 weight rows) the line lies lower.
     const int rows = a.N * (epi == GEPI_SWIGLU ? 2 : 1), round = 16 * state().cu_count;
