@@ -132,17 +132,19 @@ class TransformerBlock:
 
     def call_rows(self, x: Tensor, bsz: int, seqlen: int, start_pos: int, state: Tensor, freqs_cis: Tensor, rows: "_RowScratch") -> Tensor:
         """TransformerBlock.call (llama.ts:124-127) on x [bsz*seqlen, dim]; the result is written back into x."""
-        n = bsz * seqlen
+        n, attend, feed = bsz * seqlen, self.attention.call_rows, self.feed_forward.call_rows
+        # only the two classes' own methods norm on their way: one of the caller's own, of a class or set on the object, takes its rows normed
+        if getattr(attend, "__func__", None) is Attention.call_rows:
+            h = attend(x, bsz, seqlen, start_pos, state, freqs_cis, rows, x, rows.h2, self.attention_norm)
+        else:
+            h = attend(self._normed(x, self.attention_norm, rows, n), bsz, seqlen, start_pos, state, freqs_cis, rows, residual=x, out=rows.h2)
+        if getattr(feed, "__func__", None) is FeedForward.call_rows:
+            return feed(h, n, rows, h, x, self.ffn_norm)
+        return feed(self._normed(h, self.ffn_norm, rows, n), n, rows, residual=h, out=x)
 
-        def call(part, norm: RMSNorm, x: Tensor, *args, **kw) -> Tensor:
-            if getattr(part.call_rows, "__func__", None) in (Attention.call_rows, FeedForward.call_rows):
-                return part.call_rows(x, *args, **kw, norm=norm)
-            # one of the caller's own, of its class or set on the object, takes its rows normed
-            check(ffi.load().jsgrad_hip_rmsnorm_rows(x.ptr, norm.weight.ptr, rows.xn.ptr, n, self.attention.dim, norm.eps))
-            return part.call_rows(rows.xn, *args, **kw)
-
-        h = call(self.attention, self.attention_norm, x, bsz, seqlen, start_pos, state, freqs_cis, rows, residual=x, out=rows.h2)
-        return call(self.feed_forward, self.ffn_norm, h, n, rows, residual=h, out=x)
+    def _normed(self, x: Tensor, norm: RMSNorm, rows: "_RowScratch", n: int) -> Tensor:
+        check(ffi.load().jsgrad_hip_rmsnorm_rows(x.ptr, norm.weight.ptr, rows.xn.ptr, n, self.attention.dim, norm.eps))
+        return rows.xn
 
 
 def attn_wo_fits(n_heads: int, n_kv_heads: int, head_dim: int, max_context: int, kind: int, dim: int, capacity: int | None = None) -> bool:
