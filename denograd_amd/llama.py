@@ -119,6 +119,9 @@ class FeedForward:
         return out
 
 
+ATTENTION_ROWS, FEED_FORWARD_ROWS = Attention.call_rows, FeedForward.call_rows
+
+
 class TransformerBlock:
     def __init__(self, dim: int, hidden_dim: int, n_heads: int, n_kv_heads: int | None, norm_eps: float, max_context: int, linear=Linear, feed_forward=FeedForward):
         self.attention = Attention(dim, n_heads, n_kv_heads, max_context, linear)
@@ -134,11 +137,11 @@ class TransformerBlock:
         """TransformerBlock.call (llama.ts:124-127) on x [bsz*seqlen, dim]; the result is written back into x."""
         n, attend, feed = bsz * seqlen, self.attention.call_rows, self.feed_forward.call_rows
         # only the two classes' own methods norm on their way: one of the caller's own, of a class or set on the object, takes its rows normed
-        if getattr(attend, "__func__", None) is Attention.call_rows:
+        if getattr(attend, "__func__", None) is ATTENTION_ROWS:
             h = attend(x, bsz, seqlen, start_pos, state, freqs_cis, rows, x, rows.h2, self.attention_norm)
         else:
             h = attend(self._normed(x, self.attention_norm, rows, n), bsz, seqlen, start_pos, state, freqs_cis, rows, residual=x, out=rows.h2)
-        if getattr(feed, "__func__", None) is FeedForward.call_rows:
+        if getattr(feed, "__func__", None) is FEED_FORWARD_ROWS:
             return feed(h, n, rows, h, x, self.ffn_norm)
         return feed(self._normed(h, self.ffn_norm, rows, n), n, rows, residual=h, out=x)
 

@@ -73,15 +73,20 @@ def own_on_the_object(b):
     b.attention.call_rows, b.feed_forward.call_rows = attention, feed_forward
 
 
+def own_in_the_class(b, monkeypatch):
+    monkeypatch.setattr(Attention, "call_rows", OwnAttention.call_rows)
+    monkeypatch.setattr(FeedForward, "call_rows", OwnFeedForward.call_rows)
+
+
 def own_objects(b):
     b.attention, b.feed_forward = types.SimpleNamespace(dim=64), types.SimpleNamespace()
     own_on_the_object(b)
 
 
-@pytest.mark.parametrize("own", [own_of_the_class, own_on_the_object, own_objects])
-def test_parts_of_the_callers_own_take_their_rows_normed(lib, own):
+@pytest.mark.parametrize("own", [own_of_the_class, own_in_the_class, own_on_the_object, own_objects])
+def test_parts_of_the_callers_own_take_their_rows_normed(lib, own, monkeypatch):
     b = block()
-    own(b)
+    own(b, *[monkeypatch] * (own is own_in_the_class))
     assert run(b) is X
     assert b.attention.seen == (XN, X, H2) and b.feed_forward.seen == (XN, H2, X)
     assert lib.calls == [("jsgrad_hip_rmsnorm_rows", (X.ptr, 1, XN.ptr, 6, 64, 1e-5)), ("jsgrad_hip_rmsnorm_rows", (H2.ptr, 2, XN.ptr, 6, 64, 1e-5))]
