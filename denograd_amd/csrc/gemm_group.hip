@@ -401,6 +401,9 @@ GroupChoice choose_group(int epi, int kind, const GemmArgs &a) {
       const float fill = (float)blocks / cus;
       float us = 3.5f + (fill <= 1.0f ? (s.step + s.fill * fill) * turns + s.end : ((blocks + cus - 1) / cus) * (s.round_step * turns + s.end));
       if (d > 1) us += 1.7f + (float)d * s.bm * s.bn * 4 / 83e3f * (fill > 1.0f ? fill : 1.0f);
+      // int8 in two row tiles of 16, whole rows: the weights come twice, and half the bytes in tiles of 32 with K parts are the faster by what the estimates
+      // are apart (24 x 6144 x 4096: 11.1 us, 32x64 in two parts 10.8; in parts they are not, 24 x 2048 x 8192: 10.1 | 10.8)
+      else if (kind == JSGRAD_W_I8 && s.bm == 16 && a.M > 16 && a.M <= 32) us += 0.5f;
       if (best.shape < 0 || us < best.us) { best.us = us; best.shape = i; best.split = d; }
     }
   }
