@@ -310,8 +310,10 @@ int jsgrad_hip_read_step(const int32_t *st, const void *attn_wo_workspace, const
     for (int i = 0; i < 2; i++) w[i] = __atomic_load_n(&slot[i], __ATOMIC_RELAXED);
     if ((uint32_t)(w[0] >> 32) == seq && (uint32_t)(w[1] >> 32) == seq) break;
     __builtin_ia32_pause();                                    // the core's other thread may have something to do
-    if (spin % 1024) continue;
-    const hipError_t e = hipStreamQuery(state().stream);       // now and then: has the device given up
+    if (spin % 65536) continue;
+    // every few milliseconds: has the device given up.  A look takes microseconds in which the words may arrive: every 40 us, 11 tokens of a two-layer model
+    // behind 1684 868 us, 20 sampled ones behind 300 1500; every few ms 795 and 1365 (some 8 us apart, without the pause: 803 and 1394)
+    const hipError_t e = hipStreamQuery(state().stream);
     if (e == hipErrorNotReady) { (void)hipGetLastError(); continue; }
     JSG_HIP(e);
     for (int i = 0; i < 2; i++) w[i] = __atomic_load_n(&slot[i], __ATOMIC_RELAXED);
