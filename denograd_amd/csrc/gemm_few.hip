@@ -28,15 +28,16 @@ template <int KIND, int EPI, int SB> struct FwShape {
   static_assert(NS >= 2, "one step arrives while another is used");
 };
 
-// K = 8 wavefronts x PARTS steps x SB bytes of a weight row
-template <int KIND, int EPI, int SB, int PARTS, bool LONG> __global__ __launch_bounds__(FW_THREADS, 2) void few_rows_kernel(GemmArgs a, int tiles) {
+// K = 8 wavefronts x PARTS steps x SB bytes of a weight row.  NORM as a kernel of its own: with the question asked inside the one without a norm was slower as
+// well (us, w1|w3 of 2 / 12 rows x 8192 x 2048 15.9 / 16.5, without 15.3 / 15.3).
+template <int KIND, int EPI, int SB, int PARTS, bool LONG, bool NORM> __global__ __launch_bounds__(FW_THREADS, 2) void few_rows_kernel(GemmArgs a, int tiles) {
   typedef FwShape<KIND, EPI, SB> S;
   constexpr int NMAT = EPI == GEPI_SWIGLU ? 2 : 1, LOADS = S::LOADS, NS = S::NS;
   constexpr int KB = KIND == JSGRAD_W_F16 ? 2 : 1;            // bytes of a weight
   constexpr int NFR = SB / 64;                                // 16-byte fragment reads of a lane per step
   constexpr int MPR = KIND == JSGRAD_W_F16 ? 1 : 2;           // matrix instructions per fragment read
   constexpr int NF = PARTS * NFR * MPR;                       // x fragments
-  static_assert(NF <= 32, "x fits 128 registers");
+  static_assert(NF <= (NORM ? 16 : 32), "x fits 128 registers; with the norm's weights it takes twice as many");
   extern __shared__ __align__(16) unsigned char few_lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, lq = lane >> 4;
   const int G = gridDim.x;
@@ -102,35 +103,32 @@ template <int KIND, int EPI, int SB, int PARTS, bool LONG> __global__ __launch_b
 #pragma unroll
     for (int f = 0; f < NF; f++) xf[f] = *(const h8_t *)(xr + (f / MPR) * (64 / KB) + (f % MPR) * 8);
   }
-  constexpr bool NORM = NF <= 16;                             // with the norm's weights x takes twice the registers
-  const bool norm = NORM && a.norm_w;
-  if constexpr (NORM)
-    if (norm) {
-      // Normed in registers: sums over a wavefront's share, the eight shares through LDS in order.  Using x waits for all loads before it and behind
-      // it, so the first step goes out ahead of that and the others behind.
-      h8_t wf[NF];
-      const _Float16 *wr = a.norm_w + k_first / KB + lq * (16 / KB);
+  if constexpr (NORM) {
+    // Normed in registers: sums over a wavefront's share, the eight shares through LDS in order.  Using x waits for all loads before it and behind
+    // it, so the first step goes out ahead of that and the others behind.
+    h8_t wf[NF];
+    const _Float16 *wr = a.norm_w + k_first / KB + lq * (16 / KB);
 #pragma unroll
-      for (int f = 0; f < NF; f++) wf[f] = *(const h8_t *)(wr + (f / MPR) * (64 / KB) + (f % MPR) * 8);
-      if (n_steps > 0) issue(0);
-      float ss = 0.0f;
+    for (int f = 0; f < NF; f++) wf[f] = *(const h8_t *)(wr + (f / MPR) * (64 / KB) + (f % MPR) * 8);
+    if (n_steps > 0) issue(0);
+    float ss = 0.0f;
 #pragma unroll
-      for (int f = 0; f < NF; f++) ss = square_sum(xf[f], ss);
-      ss = add_xor32(add_xor16(ss));
-      float *const part = (float *)(few_lds + FW_WAVES * S::RING);
-      if (lq == 0) part[wave * 16 + l16] = ss;
-      lds_barrier();
-      float tot = part[l16];
+    for (int f = 0; f < NF; f++) ss = square_sum(xf[f], ss);
+    ss = add_xor32(add_xor16(ss));
+    float *const part = (float *)(few_lds + FW_WAVES * S::RING);
+    if (lq == 0) part[wave * 16 + l16] = ss;
+    lds_barrier();
+    float tot = part[l16];
 #pragma unroll
-      for (int w = 1; w < FW_WAVES; w++) tot += part[w * 16 + l16];
-      const float r = norm_factor(a, tot);
+    for (int w = 1; w < FW_WAVES; w++) tot += part[w * 16 + l16];
+    const float r = norm_factor(a, tot);
 #pragma unroll
-      for (int f = 0; f < NF; f++) xf[f] = norm_piece(xf[f], r, wf[f]);
-      lds_barrier();                                          // the sums have been read
-    }
+    for (int f = 0; f < NF; f++) xf[f] = norm_piece(xf[f], r, wf[f]);
+    lds_barrier();                                          // the sums have been read
+  }
 #pragma unroll
   for (int i = 0; i < NS; i++)
-    if (i < n_steps && !(i == 0 && norm)) issue(i);
+    if (i < n_steps && !(NORM && i == 0)) issue(i);
   // Waited for here, or the compiler, which does not count the direct loads, would wait for all of them at the first use of x in
   // every turn of the loop below.  Where there is hardly a second turn the steps behind the first need not have landed yet.
   if constexpr (LONG)
@@ -212,21 +210,23 @@ template <int KIND, int EPI, int SB, int PARTS, bool LONG> __global__ __launch_b
   }
 }
 
-template <int KIND, int EPI, int SB, int PARTS, bool LONG> static int launch_few_as(const GemmArgs &a, int tiles, int grid, int prof_kind) {
+template <int KIND, int EPI, int SB, int PARTS, bool LONG, bool NORM> static int launch_few_as(const GemmArgs &a, int tiles, int grid, int prof_kind) {
   constexpr int lds = FwShape<KIND, EPI, SB>::LDS;
   static bool raised = false;
   if (!raised) {
-    JSG_HIP(hipFuncSetAttribute((const void *)few_rows_kernel<KIND, EPI, SB, PARTS, LONG>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    JSG_HIP(hipFuncSetAttribute((const void *)few_rows_kernel<KIND, EPI, SB, PARTS, LONG, NORM>, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
     raised = true;
   }
-  JSG_LAUNCH(prof_kind, (few_rows_kernel<KIND, EPI, SB, PARTS, LONG>), dim3(grid), dim3(FW_THREADS), lds, a, tiles);
+  JSG_LAUNCH(prof_kind, (few_rows_kernel<KIND, EPI, SB, PARTS, LONG, NORM>), dim3(grid), dim3(FW_THREADS), lds, a, tiles);
   return 0;
 }
 // Two weight tiles or more per block: LONG (us, with and without: fp16 16384 x 2048 16.3 | 17.1, 2048 x 8192 9.2 | 8.7)
 template <int KIND, int EPI, int SB, int PARTS> static int launch_few(const GemmArgs &a, int prof_kind) {
   const int tiles = a.N / 16, cus = state().cu_count, grid = 2 * tiles < cus ? 2 * tiles : cus;
-  if (tiles * (EPI == GEPI_SWIGLU ? 2 : 1) >= 2 * grid) return launch_few_as<KIND, EPI, SB, PARTS, true>(a, tiles, grid, prof_kind);
-  return launch_few_as<KIND, EPI, SB, PARTS, false>(a, tiles, grid, prof_kind);
+  const bool is_long = tiles * (EPI == GEPI_SWIGLU ? 2 : 1) >= 2 * grid;
+  if constexpr (PARTS * SB * (KIND == JSGRAD_W_F16 ? 1 : 2) <= 1024)   // rows of at most 4096: what gemm_few takes with a norm
+    if (a.norm_w) return is_long ? launch_few_as<KIND, EPI, SB, PARTS, true, true>(a, tiles, grid, prof_kind) : launch_few_as<KIND, EPI, SB, PARTS, false, true>(a, tiles, grid, prof_kind);
+  return is_long ? launch_few_as<KIND, EPI, SB, PARTS, true, false>(a, tiles, grid, prof_kind) : launch_few_as<KIND, EPI, SB, PARTS, false, false>(a, tiles, grid, prof_kind);
 }
 
 // A wavefront's share of a weight row, in steps of 512, 384 or 256 bytes: long steps ask for long stretches of a row, the number
