@@ -450,6 +450,13 @@ int gemm_group(int epi, int kind, const GemmArgs &a, int prof_kind, bool *taken)
   }
   const GroupChoice c = choose_group(epi, kind, a);
   if (c.shape < 0) return pin ? fail("jsgrad_hip_gemm: no tile shape") : 0;
+  if (!pin && kind == JSGRAD_W_NF4 && a.N <= 16 * state().cu_count && epi != GEPI_SWIGLU) {
+    // nf4, one round of that kernel's blocks.  9 to 16 rows: its time is nearly a line in K, this one's has the steps of its turns; us, 12 / 16 rows, that | this
+    // one: 3072 x 5120 9.4 / 9.5 | 9.0 / 9.1, x 6144 9.7 / 10.1 | 10.2 / 10.3, x 7168 10.2 / 10.8 | 9.8 / 9.9, x 8192 10.6 /
+    // 11.2 | 11.3 / 11.4, 2560 x 8192 10.6 / 11.1 | 9.9 / 10.1.  At most 8 rows: 4096 x 10240 12.7 | 12.7, x 11264 12.7 | 13.4, x 12288 13.0 | 13.8, x 14336 15.2 | 14.9.
+    if (a.M > 8 && a.M <= 16 && a.K > 5120 && a.K <= 8192 && c.us > 7.05f + 0.00047f * a.K) return 0;
+    if (a.M <= 8 && a.N > 3072 && a.K > 10240 && a.K <= 12288) return 0;
+  }
   *taken = true;
   return run_group(epi, kind, a, c, prof_kind);
 }

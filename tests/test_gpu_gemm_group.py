@@ -97,6 +97,7 @@ def test_int8_scales_between_two_words_take_the_same_kernel(hip, monkeypatch, ro
     ("int8", 16, 4096, 5632, True), ("int8", 12, 4096, 6144, False), ("int8", 16, 3072, 4096, True), ("int8", 16, 3072, 4608, False),
     ("int8", 24, 2048, 4096, True), ("int8", 24, 1024, 4096, False), ("int8", 24, 4096, 4608, False),
     ("nf4", 16, 4096, 8192, True), ("nf4", 16, 4096, 8704, False), ("nf4", 16, 3072, 4608, False), ("nf4", 8, 3072, 8192, True),
+    ("nf4", 16, 3072, 8192, True), ("nf4", 12, 3072, 7168, False), ("nf4", 5, 4096, 11264, True), ("nf4", 8, 4096, 14336, False),
     ("nf4", 17, 4096, 5120, True), ("nf4", 17, 4096, 5632, False)])
 def test_lines_to_the_kernel_for_short_rows(hip, monkeypatch, kind, rows, out_f, in_f, skinny):
     """Which kernel a call comes to, by its bits: the K groups and parts of this one add the sums in another order."""
