@@ -723,12 +723,13 @@ template <int EPI> static int gemm_tiled_epi(int kind, const GemmArgs &a, int pr
   // At most 64 rows: the group kernel, where its estimate is the least.  The estimates of the tiled kernels are without the rate at which
   // they can draw weights with so few rows (57 rows, from 12 MB on: fp16 4.6 TB/s, codes 3.9, and for codes a seventh too low below that): us,
   // theirs measured | the group kernel: fp16 16384 x 3072 25.5 | 24.2, 28672 x 4096 52.5 | 49.4; int8 16384 x 2048 15.3 | 13.6, 16384 x 3072
-  // 18.8 | 17.5, 128256 x 3072 112 | 104; nf4 16384 x 3072 20.9 | 18.4, 28672 x 4096 34.5 | 31.6; with K parts level, 3072 x 8192 int8 14.9 | 15.4.
+  // 18.8 | 17.5, 128256 x 3072 112 | 104; nf4 16384 x 3072 20.9 | 18.4, 28672 x 4096 34.5 | 31.6; with K parts level, 3072 x 8192 int8 14.9 | 15.4;
+  // nf4 of 13 MB (10240 x 2560) 14.1 | 15.7, of 17 (w1|w3 of 8192 x 2048) 17.0 | 14.0.
   const GroupChoice g = pin.family ? GroupChoice() : choose_group(EPI, kind, a);
   auto group_first = [&](float us) {
     if (g.shape < 0) return false;
     const float mb = (float)((double)wrows * a.K * (kind == JSGRAD_W_F16 ? 2.0 : (kind == JSGRAD_W_I8 ? 1.0 : 0.5)) * 1e-6);
-    if (g.split == 1 && mb > 12.0f) us = kind == JSGRAD_W_F16 ? std::max(us, 3.8f + mb / 4.6f) : std::max(us * 1.15f, 3.8f + mb / 3.9f);
+    if (g.split == 1 && mb > (kind == JSGRAD_W_NF4 ? 14.0f : 12.0f)) us = kind == JSGRAD_W_F16 ? std::max(us, 3.8f + mb / 4.6f) : std::max(us * 1.15f, 3.8f + mb / 3.9f);
     return g.us < us;
   };
   if (kind == JSGRAD_W_F16) {
