@@ -29,7 +29,7 @@ template <int KIND, int EPI, int SB> struct FwShape {
 };
 
 // K = 8 wavefronts x PARTS steps x SB bytes of a weight row.  NORM as a kernel of its own: with the question asked inside the one without a norm was slower as
-// well (us, w1|w3 of 2 / 12 rows x 8192 x 2048 15.9 / 16.5, without 15.3 / 15.3).
+// well (us, w1|w3 of 2 / 12 rows x 8192 x 2048 15.9 / 16.5, now 15.0 / 15.1).
 template <int KIND, int EPI, int SB, int PARTS, bool LONG, bool NORM> __global__ __launch_bounds__(FW_THREADS, 2) void few_rows_kernel(GemmArgs a, int tiles) {
   typedef FwShape<KIND, EPI, SB> S;
   constexpr int NMAT = EPI == GEPI_SWIGLU ? 2 : 1, LOADS = S::LOADS, NS = S::NS;
