@@ -10,6 +10,8 @@
 // added through LDS in wavefront order.
 // Tiles that are left after whole rounds over the compute units are dealt as halves of eight rows where that is enough for
 // everybody (w1|w3 of 14336 rows: 896 tiles on 256 units are 3.5 rounds instead of 4).
+#include <type_traits>
+
 #include "gemm.h"
 
 namespace jsg {
@@ -84,58 +86,91 @@ template <int KIND, int EPI, int SB, int PARTS, bool LONG, bool NORM> __global__
     if constexpr (KIND == JSGRAD_W_I8) dma4(dma_rsrc(sc + row), (uint32_t)(lane & (half ? 3 : 7)) * 4, 0, to + S::SLOT);
   };
   constexpr int FULL = LOADS + (KIND == JSGRAD_W_I8 ? 1 : 0), HALF = LOADS / 2 + (KIND == JSGRAD_W_I8 ? 1 : 0);
-  // wait until step s has landed: what was issued behind it may stay in flight
-  auto landed = [&](int s) {
+  // Wait until what was issued in front of the `steps` steps from s on has landed; those may stay in flight, and so may a store that went out behind
+  // them (memory operations of a wavefront are counted in the order they were issued).
+  auto arrived = [&](int s, auto steps, bool store) {
+    constexpr int N = decltype(steps)::value;
     int behind = 0;
 #pragma unroll
-    for (int i = 1; i < NS; i++)
+    for (int i = 0; i < N; i++)
       if (s + i < n_steps) behind += is_half((s + i) / (NMAT * PARTS)) ? HALF : FULL;
-    if (behind >= (NS - 1) * FULL) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 1) * FULL) : "memory");
-    else if (NS > 2 && behind >= FULL) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(FULL) : "memory");
-    else if (behind >= HALF) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(HALF) : "memory");
+    if (N > 0 && behind >= N * FULL && store) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N * FULL + 1) : "memory");
+    else if (N > 0 && behind >= N * FULL) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N * FULL) : "memory");
+    else if (N > 1 && behind >= FULL) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(FULL) : "memory");
+    else if (N > 0 && behind >= HALF) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(HALF) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   };
 
   // x first: fragment f of read i holds the K elements that a lane finds in its 16 bytes of the weight row
+  float *const red = (float *)(few_lds + FW_WAVES * S::RING);  // [matrix][wavefront][16 x rows][16 weight rows]
   h8_t xf[NF];
-  {
+  constexpr int XS = PARTS * MPR;                              // slots that the wavefront's share of x would fill
+  if constexpr (XS <= NS) {
+    // Through the last slots of the ring, which are free until their steps are asked for.  The compiler does not count direct loads: a load of x
+    // to registers would be waited for with every step asked for behind it, and nothing would be on its way until they are used.
+    const i4_t rx = dma_rsrc(a.x);
+#pragma unroll
+    for (int i = 0; i < XS; i++)
+#pragma unroll
+      for (int j = 0; j < LOADS; j++) {
+        const int o = j * 1024 + lane * 16, r = o / SB, p = (o % SB) / 16;
+        if (j < LOADS / 2 || a.M > 8)                         // rows past the end: the last one again, or what the slot held, and never stored
+          dma16(rx, (uint32_t)min(r, a.M - 1) * (uint32_t)a.K * 2 + (uint32_t)(p ^ swizzle(r)) * 16, k_first * MPR + i * SB, ring0 + (NS - XS + i) * (S::SLOT + S::SCALE) + j * 1024);
+      }
+    // the norm's weights of the wavefront's share into its part of the sums' space: at most 1 KiB
+    unsigned char *const nw = (unsigned char *)red + wave * 1024;
+    if constexpr (NORM) dma16(dma_rsrc(a.norm_w), min((uint32_t)lane * 16, (uint32_t)(XS * SB) - 16), k_first * MPR, (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)nw);
+#pragma unroll
+    for (int i = 0; i < NS - XS; i++)
+      if (i < n_steps) issue(i);
+    arrived(0, std::integral_constant<int, NS - XS>(), false);
+#pragma unroll
+    for (int f = 0; f < NF; f++) {
+      const int at = f / MPR * (64 * MPR) + f % MPR * 16;     // byte of the wavefront's share of a row, without the lane quarter's
+      xf[f] = *(const h8_t *)(ring + (NS - XS + at / SB) * (S::SLOT + S::SCALE) + l16 * SB + ((at % SB / 16 + lq * MPR) ^ swizzle(l16)) * 16);
+    }
+    h8_t wf[NORM ? NF : 1];
+    if constexpr (NORM)
+#pragma unroll
+      for (int f = 0; f < NF; f++) wf[f] = *(const h8_t *)(nw + f / MPR * (64 * MPR) + f % MPR * 16 + lq * (MPR * 16));
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");        // x is in registers: its slots are filled
+#pragma unroll
+    for (int i = NS - XS; i < NS; i++)
+      if (i < n_steps) issue(i);
+    if constexpr (NORM) {
+      // normed in registers: sums over a wavefront's share, the eight shares through LDS in order
+      float ss = 0.0f;
+#pragma unroll
+      for (int f = 0; f < NF; f++) ss = square_sum(xf[f], ss);
+      ss = add_xor32(add_xor16(ss));
+      if (lq == 0) ((float *)nw)[l16] = ss;
+      lds_barrier();
+      float tot = red[l16];
+#pragma unroll
+      for (int w = 1; w < FW_WAVES; w++) tot += red[w * 256 + l16];
+      const float r = norm_factor(a, tot);
+#pragma unroll
+      for (int f = 0; f < NF; f++) xf[f] = norm_piece(xf[f], r, wf[f]);
+      lds_barrier();                                          // the sums have been read
+    }
+  } else {
+    static_assert(!NORM, "rows short enough for the norm have room in the ring");
     const _Float16 *xr = a.x + (size_t)min(l16, a.M - 1) * a.K + k_first / KB + lq * (16 / KB);   // rows past the end: never stored
 #pragma unroll
     for (int f = 0; f < NF; f++) xf[f] = *(const h8_t *)(xr + (f / MPR) * (64 / KB) + (f % MPR) * 8);
+#pragma unroll
+    for (int i = 0; i < NS; i++)
+      if (i < n_steps) issue(i);
+    // Waited for here, or the compiler, which does not count the direct loads, would wait for all of them at the first use of x in
+    // every turn of the loop below.  Where there is hardly a second turn the steps behind the first need not have landed yet.
+    if constexpr (LONG)
+#pragma unroll
+      for (int f = 0; f < NF; f++) asm volatile("" : "+v"(xf[f]));
   }
-  if constexpr (NORM) {
-    // Normed in registers: sums over a wavefront's share, the eight shares through LDS in order.  Using x waits for all loads before it and behind
-    // it, so the first step goes out ahead of that and the others behind.
-    h8_t wf[NF];
-    const _Float16 *wr = a.norm_w + k_first / KB + lq * (16 / KB);
-#pragma unroll
-    for (int f = 0; f < NF; f++) wf[f] = *(const h8_t *)(wr + (f / MPR) * (64 / KB) + (f % MPR) * 8);
-    if (n_steps > 0) issue(0);
-    float ss = 0.0f;
-#pragma unroll
-    for (int f = 0; f < NF; f++) ss = square_sum(xf[f], ss);
-    ss = add_xor32(add_xor16(ss));
-    float *const part = (float *)(few_lds + FW_WAVES * S::RING);
-    if (lq == 0) part[wave * 16 + l16] = ss;
-    lds_barrier();
-    float tot = part[l16];
-#pragma unroll
-    for (int w = 1; w < FW_WAVES; w++) tot += part[w * 16 + l16];
-    const float r = norm_factor(a, tot);
-#pragma unroll
-    for (int f = 0; f < NF; f++) xf[f] = norm_piece(xf[f], r, wf[f]);
-    lds_barrier();                                          // the sums have been read
-  }
-#pragma unroll
-  for (int i = 0; i < NS; i++)
-    if (i < n_steps && !(NORM && i == 0)) issue(i);
-  // Waited for here, or the compiler, which does not count the direct loads, would wait for all of them at the first use of x in
-  // every turn of the loop below.  Where there is hardly a second turn the steps behind the first need not have landed yet.
-  if constexpr (LONG)
-#pragma unroll
-    for (int f = 0; f < NF; f++) asm volatile("" : "+v"(xf[f]));
 
-  float *const red = (float *)(few_lds + FW_WAVES * S::RING);  // [matrix][wavefront][16 x rows][16 weight rows]
+  // whether this wavefront stores sums of a unit.  Not asked for one int8 matrix, whose units are over in a step or two: the longer code costs more than
+  // it saves (us, 5 rows, without | with: int8 4096 x 4096 6.1 | 6.3; fp16 w1|w3 of 8192 x 3072 16.8 | 16.4, 16 rows 17.7 | 16.9).
+  const bool stores = (KIND == JSGRAD_W_F16 || EPI == GEPI_SWIGLU) && wave * 4 < a.M;
   int s = 0;
   for (int u = 0; u < units; u++) {
 #pragma unroll
@@ -143,7 +178,7 @@ template <int KIND, int EPI, int SB, int PARTS, bool LONG, bool NORM> __global__
       f4_t acc = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
       for (int part = 0; part < PARTS; part++, s++) {
-        landed(s);
+        arrived(s + 1, std::integral_constant<int, NS - 1>(), stores && u > 0 && q * PARTS + part < NS);
         const unsigned char *const from = ring + (s % NS) * (S::SLOT + S::SCALE);
         u4_t raw[NFR];
 #pragma unroll
@@ -220,13 +255,15 @@ template <int KIND, int EPI, int SB, int PARTS, bool LONG, bool NORM> static int
   JSG_LAUNCH(prof_kind, (few_rows_kernel<KIND, EPI, SB, PARTS, LONG, NORM>), dim3(grid), dim3(FW_THREADS), lds, a, tiles);
   return 0;
 }
-// Two weight tiles or more per block: LONG (us, with and without: fp16 16384 x 2048 16.3 | 17.1, 2048 x 8192 9.2 | 8.7)
+// LONG, where x does not come through the ring: two weight tiles or more per block (us, with and without: fp16 16384 x 2048 16.3 | 17.1, 2048 x 8192 9.2 | 8.7)
 template <int KIND, int EPI, int SB, int PARTS> static int launch_few(const GemmArgs &a, int prof_kind) {
+  constexpr int MPR = KIND == JSGRAD_W_F16 ? 1 : 2;
   const int tiles = a.N / 16, cus = state().cu_count, grid = 2 * tiles < cus ? 2 * tiles : cus;
-  const bool is_long = tiles * (EPI == GEPI_SWIGLU ? 2 : 1) >= 2 * grid;
-  if constexpr (PARTS * SB * (KIND == JSGRAD_W_F16 ? 1 : 2) <= 1024)   // rows of at most 4096: what gemm_few takes with a norm
-    if (a.norm_w) return is_long ? launch_few_as<KIND, EPI, SB, PARTS, true, true>(a, tiles, grid, prof_kind) : launch_few_as<KIND, EPI, SB, PARTS, false, true>(a, tiles, grid, prof_kind);
-  return is_long ? launch_few_as<KIND, EPI, SB, PARTS, true, false>(a, tiles, grid, prof_kind) : launch_few_as<KIND, EPI, SB, PARTS, false, false>(a, tiles, grid, prof_kind);
+  if constexpr (PARTS * SB * MPR <= 1024)                     // rows of at most 4096: what gemm_few takes with a norm
+    if (a.norm_w) return launch_few_as<KIND, EPI, SB, PARTS, false, true>(a, tiles, grid, prof_kind);
+  if constexpr (PARTS * MPR > FwShape<KIND, EPI, SB>::NS)
+    if (tiles * (EPI == GEPI_SWIGLU ? 2 : 1) >= 2 * grid) return launch_few_as<KIND, EPI, SB, PARTS, true, false>(a, tiles, grid, prof_kind);
+  return launch_few_as<KIND, EPI, SB, PARTS, false, false>(a, tiles, grid, prof_kind);
 }
 
 // A wavefront's share of a weight row, in steps of 512, 384 or 256 bytes: long steps ask for long stretches of a row, the number
@@ -257,9 +294,11 @@ int gemm_few(int epi, int kind, const GemmArgs &a, int prof_kind, bool *taken) {
   *taken = false;
   if (a.M > 16 || a.N % 16 || ((uintptr_t)a.s0 | (uintptr_t)a.s1 | (uintptr_t)a.s2) & 3) return 0;
   // int8: the codes of a tile are half the bytes behind the same x, and a tile is over in a step or two; gemm_group.hip keeps its ring full
-  // over wide matrices.  us, 8 / 16 rows, that one | this one: 5120 x 3072 8.6 / 8.7 | 7.6 / 8.3, 2048 x 8192 9.1 / 9.4 | 9.2 / 12.0, 3072 x 8192 9.9 / 10.1 |
-  // 10.4 / 12.5, 4096 x 6144 10.3 / 10.4 | 9.3 / 12.3, 6144 x 4096 9.6 / 9.8 | 10.6 / 12.0, 16384 x 3072 12.3 / 12.3 | 14.1 / 15.0, 28672 x 4096 21.9 / 21.9 |
-  // 28.7 / 30.3.  (Up to 36 M codes behind 8 rows the two are within a tenth of each other; the line is from before the group kernel's 16x64 tiles shared units.)
+  // over wide matrices.  us, 8 / 16 rows, that one | this one: 2048 x 8192 9.1 / 9.4 | 9.2 / 12.0, 3072 x 8192 9.9 / 10.1 | 10.4 / 12.5, 4096 x 6144
+  // 10.3 / 10.4 | 9.3 / 12.3; with x through the ring 3072 x 4096 - / 8.0 | 5.6 / 5.9, 4096 x 4096 - / 8.6 | 6.1 / 6.7, 6144 x 4096 - / 9.6 | 9.2 / 9.8, 8192 x 4096
+  // - / 9.7 | 10.3 / 10.8, 16384 x 3072 11.7 / 11.7 | 11.6 / 12.1, 28672 x 4096 21.4 / 21.5 | 25.2 / 25.9, 128256 x 2048 45 / 47 | 53 / 59.  With a norm in
+  // front, which there is a launch of its own, w1|w3 of 8192 x 3072 13.6 / 13.7 | 12.3 / 12.7, of 14336 x 3072 19.8 / 20.1 | 18.2 / 18.7, of 6144 x 4096
+  // 14.7 / 15.0 | 15.1 / 15.5, one matrix of 16384 x 3072 13.3 / 13.5 | 13.3 / 14.2, of 24576 x 2048 13.6 / 14.0 | 13.6 / 14.3.
   // fp16, skinny_gemm_kernel | this one, 2 / 8 / 16 rows: 2048 x 2048 6.2 / 6.3 / 6.3 | 4.5 / 4.5 / 5.1, 2048 x 8192 14.1 / 14.9 / 15.9 |
   // 8.8 / 9.5 / 12.4, 16384 x 2048 23.6 / 23.7 / 24.4 | 16.3 / 17.2 / 18.2, 128256 x 2048 147 / 153 / 162 | 88 / 92 / 94 (6.0 TB/s).
   // fp16 rows of more than 4096 elements (6144 and 8192 come here): the more rows of x a block reads for its few tiles, the nearer gemm_group.hip, which reads x from LDS, comes.  us,
@@ -278,7 +317,8 @@ int gemm_few(int epi, int kind, const GemmArgs &a, int prof_kind, bool *taken) {
   // costs more than the launches: 8B int8 16 rows 3321 | 3403, 8B NF4 16 layers 8 rows 1403 | 1467.
   // The norm's weights are read here in 16-byte pieces; from any other address in memory first.
   if (a.norm_w && (a.K > 4096 || (uintptr_t)a.norm_w & 15)) return 0;
-  if (kind == JSGRAD_W_I8 && (elements > (size_t)36 << 20 || (a.M > 8 && a.K > 3072))) return 0;
+  const size_t most = (size_t)(a.norm_w && epi == GEPI_SWIGLU && a.K <= 3072 ? 88 : 36) << 20;
+  if (kind == JSGRAD_W_I8 && (elements > most || (a.M > 8 && (a.K > 4096 || (a.K > 3072 && rows > 4096))))) return 0;
   if (pin_env(a, "JSG_GEMM_NO_SKINNY") || pin_env(a, "JSG_GEMM_SKINNY_TILES")) return 0;   // tests that want one of the other kernels
   if (epi == GEPI_STORE) return gemm_few_epi<GEPI_STORE>(kind, a, prof_kind, taken);
   if (epi == GEPI_ROPE_KV) return gemm_few_epi<GEPI_ROPE_KV>(kind, a, prof_kind, taken);

@@ -101,6 +101,12 @@ def test_normed_ffn_gate(hip, kind, rows, dim, hidden):
     assert_close(got.numpy().astype(np.float32), ref.numpy().astype(np.float32), True, f"{kind} {rows}", composed=True)
 
 
+@pytest.mark.parametrize("rows,dim,hidden", [(1, 3072, 8192), (16, 3072, 14976), (3, 3072, 15104), (9, 2048, 9216)])
+def test_normed_ffn_gate_of_wide_int8_matrices(hip, rows, dim, hidden):
+    """From 36 M codes on the norm alone decides between two kernels (up to 88 M)."""
+    test_normed_ffn_gate(hip, "int8", rows, dim, hidden)
+
+
 @pytest.mark.parametrize("kind", ["float16", "int8", "nf4"])
 @pytest.mark.parametrize("batch,seq,dim", [(5, 1, 2048), (16, 1, 4096), (2, 7, 3072), (3, 9, 1024)])
 def test_normed_qkv_rope(hip, kind, batch, seq, dim):
