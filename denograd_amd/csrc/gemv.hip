@@ -78,10 +78,22 @@ template <int KIND, typename AT, int EPI, int ROWS, int UNROLL, int NW = 4> stat
 }
 // Two register buffers of UNROLL x NM x ROWS 16-byte loads each: (2 rows, 4 steps) for one matrix, (2 rows, 2 steps)
 // for the SwiGLU pair, i.e. 8 loads = 8 KiB per wavefront per buffer either way.
+// Rows of fewer k-steps than that take items of as many as they have (fp16 activations).  A step behind the end of a row asks for the row's
+// last vector again, and the launch is bound by how fast its requests go out: us, four steps | as many as there are: int8 32000 x 1024 12.7 | 9.0,
+// 8192 x 1024 5.0 | 4.2, wq|wk|wv of 2048 4.7 | 4.2; nf4 wq|wk|wv of 4096 7.5 | 6.6, 4096 x 4096 5.1 | 4.7, 128256 x 4096 55 | 50; fp16 32000 x 1024 14.9 | 12.5,
+// wq|wk|wv of 256 3.2 | 3.1; w1|w3, two steps | one: nf4 8192 x 2048 8.9 | 8.1, fp16 4096 x 512 4.4 | 3.8.  Three steps pay for int8 where every wavefront has a
+// group or none (wq|wk|wv of 3072 6.5 | 6.3), not where it walks many (128256 x 3072 62 | 63), and not for nf4 (5120 x 5120 7.6 | 8.5).
 template <int KIND, typename AT, int EPI> static int launch_rows(const GemvArgs &a, int total_rows) {
-  if constexpr (EPI == EPI_SWIGLU) return launch_cfg<KIND, AT, EPI, 2, 2>(a, total_rows);
-  else
-  return launch_cfg<KIND, AT, EPI, 2, 4>(a, total_rows);
+  constexpr int UNROLL = EPI == EPI_SWIGLU ? 2 : 4, STEP = Gemv<KIND, AT, EPI, 2, UNROLL, false>::STEP;
+  if constexpr (sizeof(AT) == 2) {
+    if (a.in_f <= STEP) return launch_cfg<KIND, AT, EPI, 2, 1>(a, total_rows);
+    if constexpr (EPI != EPI_SWIGLU) {
+      if (a.in_f <= 2 * STEP) return launch_cfg<KIND, AT, EPI, 2, 2>(a, total_rows);
+      if constexpr (KIND == JSGRAD_W_I8)
+        if (a.in_f <= 3 * STEP && total_rows <= 2 * 16 * state().cu_count) return launch_cfg<KIND, AT, EPI, 2, 3>(a, total_rows);
+    }
+  }
+  return launch_cfg<KIND, AT, EPI, 2, UNROLL>(a, total_rows);
 }
 template <int EPI> static int dispatch(int kind, int act, const GemvArgs &a, int total_rows) {
 #define JSG_CASE(K)                                                          \

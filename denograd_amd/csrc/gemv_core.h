@@ -430,8 +430,9 @@ template <typename AT> __device__ __forceinline__ void stage_x_finish(const Gemv
 
 // One item's registers: the weight vectors plus, on the item that finishes a row group, the operands its epilogue will
 // need (row scales, residual, rotary pair), fetched with the weights so that no load latency is left at the end.
-// Every configuration in use moves 8 x 16 bytes per lane and item (UNROLL x NM x ROWS = 8) and has ROWS = 2, so one
-// plain struct serves all of them; the whole-step kernel can then carry ONE prefetched buffer from phase to phase.
+// Every configuration in use moves up to 8 x 16 bytes per lane and item (UNROLL x NM x ROWS <= 8; fewer than 8 for rows of fewer k-steps
+// than an item has otherwise) and has ROWS = 2, so one plain struct serves all of them; the whole-step kernel can then carry ONE
+// prefetched buffer from phase to phase.
 struct GemvBuf {
   u4_t w[8];            // [u][j][r] flattened
   // Small per-row operands, kept exactly as the loads returned them (16-bit loads stay 16-bit values) and converted
@@ -461,7 +462,7 @@ template <int KIND, typename AT, int EPI, int ROWS, int UNROLL, bool COHERENT, i
   static constexpr int STEP = 64 * VEC;                 // elements one wavefront covers per k-step
   static constexpr int NM = EPI == EPI_SWIGLU ? 2 : 1;  // matrices a wavefront evaluates on the same rows
   typedef GemvBuf Buf;
-  static_assert(ROWS == 2 && UNROLL * NM * ROWS == 8, "GemvBuf holds 8 vectors for 2 rows");
+  static_assert(ROWS == 2 && UNROLL * NM * ROWS <= 8, "GemvBuf holds 8 vectors for 2 rows");
   __device__ static __forceinline__ constexpr int wi(int u, int j, int r) { return (u * NM + j) * ROWS + r; }
   __device__ static __forceinline__ constexpr int si(int j, int r) { return j * ROWS + r; }
 
