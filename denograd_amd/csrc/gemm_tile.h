@@ -14,6 +14,7 @@ struct TileArgs {
   const _Float16 *s[3];                // codes: their scales
   int b_end[2];                        // ends of the first two (SWIGLU: b[0] is w1, b[1] is w3, row for row)
   int split;                           // K parts
+  int whole = 0;                       // 256 x 256: tiles of whole K, in front of those that come in parts
   float *ws;                           // split > 1: [tile][part][BM * BN] floats
   int *counters;                       // split > 1: one per tile, zero, and zero again afterwards
 };
@@ -36,15 +37,18 @@ __device__ __forceinline__ void turn_barrier_lds() {
 // operand tiles in its L2.  (GROUP 2 / 4 / 8 / 16 at 32768 x 4096 x 14336: 1453 / 1451 / 1413 / 1334 TFLOP/s, at
 // 32768 x 28672 x 4096: 1392 / 1422 / 1440 / 1318.)
 struct TileId { int tile, part, m0, col; };
-template <int BM, int CW> __device__ __forceinline__ TileId tile_id(const TileArgs &t) {
+// The first `whole` tiles are a block each and come first.
+template <int BM, int CW> __device__ __forceinline__ TileId tile_id(const TileArgs &t, int whole = 0) {
   constexpr int GROUP = 4;
-  const int tiles_m = (t.g.M + BM - 1) / BM, tiles_n = t.g.N / CW, nblocks = tiles_m * tiles_n * t.split;
-  int bid = blockIdx.x;
+  const int tiles_m = (t.g.M + BM - 1) / BM, tiles_n = t.g.N / CW;
+  const bool in_parts = (int)blockIdx.x >= whole;
+  const int split = in_parts ? t.split : 1, nblocks = in_parts ? (tiles_m * tiles_n - whole) * split : whole;
+  int bid = (int)blockIdx.x - (in_parts ? whole : 0);
   const int per = nblocks / 8;
   if (bid < per * 8) bid = (bid & 7) * per + (bid >> 3);
   TileId r;
-  r.part = bid % t.split;
-  r.tile = bid / t.split;
+  r.part = bid % split;
+  r.tile = (in_parts ? whole : 0) + bid / split;
   const int in_group = GROUP * tiles_n, first_m = (r.tile / in_group) * GROUP, gsz = min(tiles_m - first_m, GROUP);
   r.m0 = (first_m + (r.tile % in_group) % gsz) * BM;
   r.col = ((r.tile % in_group) / gsz) * CW;

@@ -78,7 +78,8 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs &a, _Float16 *ep, i
 // count goes up once the block's stores are acknowledged.  The part is in the vector offset: behind a 16-byte store with its
 // offset in a scalar register the compiler overwrites the first data register too early (sums came out with every fourth
 // value zero).
-template <int TM, int TN, int SUMS> __device__ __forceinline__ bool sum_parts(const TileArgs &t, const TileId &id, int wave, f4_t (&acc)[TM][TN]) {
+// RB: rows of accumulators fetched at a time, where there are no registers for all of a part
+template <int TM, int TN, int SUMS, int RB = TM> __device__ __forceinline__ bool sum_parts(const TileArgs &t, const TileId &id, int wave, f4_t (&acc)[TM][TN]) {
   __shared__ int last;
   const __amdgpu_buffer_rsrc_t rw = wave_buffer(t.ws + (size_t)id.tile * t.split * SUMS, (uint32_t)t.split * SUMS * 4u);
   const uint32_t o0 = ((uint32_t)wave * TM * TN * 64 + (threadIdx.x & 63)) * 16;
@@ -101,16 +102,19 @@ template <int TM, int TN, int SUMS> __device__ __forceinline__ bool sum_parts(co
 #pragma unroll
     for (int j = 0; j < TN; j++) acc[i][j] = __builtin_bit_cast(f4_t, __builtin_amdgcn_raw_buffer_load_b128(rw, o0 + (i * TN + j) * 1024, 0, 16));
   for (int p = 1; p < t.split; p++) {
-    f4_t u[TM][TN];
 #pragma unroll
-    for (int i = 0; i < TM; i++)
+    for (int i0 = 0; i0 < TM; i0 += RB) {
+      f4_t u[RB][TN];
 #pragma unroll
-      for (int j = 0; j < TN; j++)
-        u[i][j] = __builtin_bit_cast(f4_t, __builtin_amdgcn_raw_buffer_load_b128(rw, o0 + (uint32_t)p * SUMS * 4u + (i * TN + j) * 1024, 0, 16));
+      for (int i = 0; i < RB; i++)
 #pragma unroll
-    for (int i = 0; i < TM; i++)
+        for (int j = 0; j < TN; j++)
+          u[i][j] = __builtin_bit_cast(f4_t, __builtin_amdgcn_raw_buffer_load_b128(rw, o0 + (uint32_t)p * SUMS * 4u + ((i0 + i) * TN + j) * 1024, 0, 16));
 #pragma unroll
-      for (int j = 0; j < TN; j++) acc[i][j] += u[i][j];
+      for (int i = 0; i < RB; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) acc[i0 + i][j] += u[i][j];
+    }
   }
   return true;
 }
@@ -124,6 +128,8 @@ template <int TM, int TN, int SUMS> __device__ __forceinline__ bool sum_parts(co
 // at once with the tile after next (A0 read in slots 0 and 1, refilled in slots 2 and 3; B0 in 4 and 5; B1, read in 2 and
 // 3, in 6 and 7; A1, read in 4 and 5, in 8 and 9), so every load has 11 slots (3000 cycles) to arrive and five pairs of a
 // wavefront's loads may be outstanding when a phase needs the sixth.
+// Tiles behind the last whole round of blocks may come in K parts (t.whole, t.split), so that the last round is a short one: us, as chosen without |
+// with, 1200 x 4096 x 14336 162 | 136, w1|w3 of 14336 x 4096 behind 1600 rows 388 | 354, 3300 x 6144 x 4096 164 | 149, 4096 x 6144 x 4096 177 | 172.
 // Measured (fp16): 32768 x 28672 x 4096 1420, 32768 x 4096 x 14336 1430-1450, 4096^3 1410 TFLOP/s (1050-1110 for the kernel
 // with 32x32 instructions and tiles through registers it replaces; the same loop without its epilogue 1500).
 constexpr int T256_OPERAND = 256 * 128;                       // bytes of one operand tile
@@ -133,7 +139,7 @@ template <int EPI> __global__ __launch_bounds__(TILE_THREADS, 2) void tile256_ke
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, lq = lane >> 4;
   const int g = wave >> 2, wn = wave & 3;
   constexpr int CW = EPI == GEPI_SWIGLU ? 128 : 256;
-  const TileId id = tile_id<256, CW>(t);
+  const TileId id = tile_id<256, CW>(t, t.whole);
   const int m0 = id.m0;
 
   // Loads: half h of an operand is 128 rows = 16 loads of eight rows, two per wavefront.  The tile's rows are ordered by
@@ -158,28 +164,24 @@ template <int EPI> __global__ __launch_bounds__(TILE_THREADS, 2) void tile256_ke
     }
   const uint32_t vb = (uint32_t)lr * row_bytes + piece;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)tile_lds;
-  const int nk = a.K / TILE_BK;
+  const int nkt = a.K / TILE_BK, parts = id.tile < t.whole ? 1 : t.split, k0 = id.part * nkt / parts, nk = (id.part + 1) * nkt / parts - k0;
   // past the last tile the last one is asked for again, into a buffer nobody computes from any more
   auto load_a = [&](int kt, int h) {
-    const uint32_t so = (uint32_t)min(kt, nk - 1) * 128, base = lds0 + (kt & 1) * 2 * T256_OPERAND;
+    const uint32_t so = (uint32_t)(k0 + min(kt, nk - 1)) * 128, base = lds0 + (kt & 1) * 2 * T256_OPERAND;
     dma16(ra, va[h][0], so, base + la[h][0]);
     dma16(ra, va[h][1], so, base + la[h][1]);
   };
   auto load_b = [&](int kt, int h) {
-    const uint32_t so = (uint32_t)min(kt, nk - 1) * 128, base = lds0 + (kt & 1) * 2 * T256_OPERAND;
+    const uint32_t so = (uint32_t)(k0 + min(kt, nk - 1)) * 128, base = lds0 + (kt & 1) * 2 * T256_OPERAND;
     dma16(rb[h][0], vb, so, base + lb[h][0]);
     dma16(rb[h][1], vb, so, base + lb[h][1]);
   };
 
-  f4_t acc[2][4][2][2];                                       // [x half][row tile][weight half][column tile]
+  f4_t acc[8][4];                                             // [x half, row tile][weight half, column tile]
 #pragma unroll
-  for (int p = 0; p < 2; p++)
+  for (int i = 0; i < 8; i++)
 #pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-      for (int q = 0; q < 2; q++)
-#pragma unroll
-        for (int j = 0; j < 2; j++) acc[p][i][q][j] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int j = 0; j < 4; j++) acc[i][j] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
   h8_t af[4][2], bf[2][2][2];
   const uint32_t sw0 = (uint32_t)(lq ^ (l16 & 7)) * 16, sw1 = sw0 ^ 64;   // position of K pieces lq and lq + 4 in rows congruent to l16
   auto read_a = [&](int cur, int h) {
@@ -205,7 +207,7 @@ template <int EPI> __global__ __launch_bounds__(TILE_THREADS, 2) void tile256_ke
 #pragma unroll
       for (int i = 0; i < 4; i++)
 #pragma unroll
-        for (int j = 0; j < 2; j++) acc[ah][i][bh][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bf[bh][j][k], af[i][k], acc[ah][i][bh][j], 0, 0, 0);
+        for (int j = 0; j < 2; j++) acc[ah * 4 + i][bh * 2 + j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bf[bh][j][k], af[i][k], acc[ah * 4 + i][bh * 2 + j], 0, 0, 0);
     __builtin_amdgcn_s_setprio(0);
   };
 
@@ -233,11 +235,17 @@ template <int EPI> __global__ __launch_bounds__(TILE_THREADS, 2) void tile256_ke
   wait_loads<0>();
   turn_barrier();                                             // nobody reads or fills the tiles any more
 
+  if (parts > 1) {
+    TileId in_parts = id;
+    in_parts.tile -= t.whole;
+    if (!sum_parts<8, 4, 65536, 2>(t, in_parts, wave, acc)) return;
+  }
+
   constexpr int C16 = EPI == GEPI_SWIGLU ? 2 : 4;
   _Float16 *ep = (_Float16 *)tile_lds + wave * 64 * (C16 * 16 + 8);
   tile_epilogue<EPI, 8, C16, 4>(a, ep, m0 + g * 128, id.col + wn * C16 * 16, [&](int i, int j, int c) {
-    if constexpr (EPI == GEPI_SWIGLU) return swiglu(acc[i >> 2][i & 3][0][j][c], acc[i >> 2][i & 3][1][j][c]);
-    else return acc[i >> 2][i & 3][j >> 1][j & 1][c];
+    if constexpr (EPI == GEPI_SWIGLU) return swiglu(acc[i][j][c], acc[i][2 + j][c]);
+    else return acc[i][j][c];
   });
 }
 
@@ -566,6 +574,8 @@ constexpr int TILE_COUNTERS = 4096;
 constexpr size_t SUMS_LIMIT = (size_t)256 << 20, REALISED_LIMIT = (size_t)2 << 30;
 static __device__ int tile_counters[TILE_COUNTERS];
 
+// 256 x 256 with K parts: only the tiles behind the last whole round of blocks come in parts
+static int whole_tiles(int tiles) { return tiles / state().cu_count * state().cu_count; }
 template <int EPI> static int launch_tile256(const TileArgs &t, int prof_kind) {
   constexpr int lds = 4 * T256_OPERAND;
   static bool raised = false;   // one process, one device, one thread: set once per instantiation
@@ -574,7 +584,9 @@ template <int EPI> static int launch_tile256(const TileArgs &t, int prof_kind) {
     raised = true;
   }
   const int tiles = ((t.g.M + 255) / 256) * (t.g.N / (EPI == GEPI_SWIGLU ? 128 : 256));
-  JSG_LAUNCH(prof_kind, (tile256_kernel<EPI>), dim3(tiles), dim3(TILE_THREADS), lds, t);
+  TileArgs u = t;
+  u.whole = t.split > 1 ? whole_tiles(tiles) : tiles;
+  JSG_LAUNCH(prof_kind, (tile256_kernel<EPI>), dim3(u.whole + (tiles - u.whole) * t.split), dim3(TILE_THREADS), lds, u);
   return 0;
 }
 template <int EPI, int BM, int BN, int ST, int WR = 1> static int launch_tile(const TileArgs &t, int prof_kind) {
@@ -624,7 +636,8 @@ static const TileShape STAGED_SHAPES_NF4[] = {{32, 128, 64, 0.53f, 0.17f, 0.29f,
 constexpr int N_SHAPES = sizeof(TILE_SHAPES) / sizeof(TILE_SHAPES[0]), N_QSHAPES = sizeof(QTILE_SHAPES_I8) / sizeof(QTILE_SHAPES_I8[0]), N_STAGED = sizeof(STAGED_SHAPES_I8) / sizeof(STAGED_SHAPES_I8[0]);
 
 // Which shape and how many K parts: the least of an estimate of the launch's time (4.5 us for start and first tiles; for K parts 1.7 us
-// and the sums' way through memory).  Over the measured sizes the choice is 0.9 % slower than the best shape on average.  Examples, us with weights from memory, this choice | others: 371 x 2048 x 8192 128x128 in 5 parts 26.3 | in 3 parts
+// and the sums' way through memory; 256 x 256, whose blocks wait for each other's 256 KB and share the chip's power, 20 us: with less it is taken where it
+// loses, 2048 x 4096 x 4096 64 | 72, 1200 x 6144 x 4096 61 | 68).  Over the measured sizes the choice is 0.9 % slower than the best shape on average.  Examples, us with weights from memory, this choice | others: 371 x 2048 x 8192 128x128 in 5 parts 26.3 | in 3 parts
 // 32.2, 64x128 in 2 32.9, 256x128 in 7 34.4; 371 x 2048 x 2048 64x64 12.7 | 64x128 in 2 parts 12.4, in one 15.5; 700 x 28672 x 4096
 // 256x128 185 | 256x256 188, 128x128 223; 2048 x 6144 x 4096 256x256 90 | 128x128 111, 256x128 112; int8 codes, 57 x 5120 x 3072 64x64 in
 // 3 parts 11.2 | 64x128 in 5 12.4, 64x64 in 6 12.9.
@@ -644,7 +657,9 @@ static Pin read_pin(int epi, const GemmArgs &a) {
   sscanf(e + (p.family != 't'), "%dx%d/%d", &p.bm, &p.bn, &p.split);
   return p;
 }
+// tail: 256 x 256 tiles may have K parts too (tile256_kernel)
 static Choice choose_tile(const TileShape *shapes, int n_shapes, int epi, int M, int weight_rows, int K, size_t ws_limit, const Pin &pin) {
+  const bool tail = shapes == TILE_SHAPES;
   const int cus = state().cu_count;
   Choice best = {0.0f, -1, 1};
   for (int s = 0; s < n_shapes; s++) {
@@ -652,12 +667,15 @@ static Choice choose_tile(const TileShape *shapes, int n_shapes, int epi, int M,
     if (weight_rows % c.bn || K % c.bk || (epi == GEPI_SWIGLU && !c.pairs)) continue;
     const int tiles = ((M + c.bm - 1) / c.bm) * (weight_rows / c.bn), nk = K / c.bk;
     for (int d = 1; d <= 16; d++) {
-      if (d > 1 && (c.bm * c.bn == 65536 || nk < d || tiles > TILE_COUNTERS || (size_t)tiles * d * c.bm * c.bn * 4 > ws_limit)) break;
-      if (d > 1 && (pin.family ? d > pin.split : nk / d * c.bk < 256 || tiles * d > 2 * cus)) break;
+      const bool big = c.bm * c.bn == 65536;
+      const int whole = big ? whole_tiles(tiles) : 0, in_parts = tiles - whole;
+      if (d > 1 && ((big && !tail) || in_parts == 0 || nk < d || in_parts > TILE_COUNTERS || (size_t)in_parts * d * c.bm * c.bn * 4 > ws_limit)) break;
+      if (d > 1 && (pin.family ? d > pin.split : nk / d * c.bk < (big ? 512 : 256) || in_parts * d > (big ? 1 : 2) * cus)) break;
       const int blocks = tiles * d, steps = (nk + d - 1) / d;
       const float fill = (float)blocks / cus;
       float us = 4.5f + (fill <= 1.0f ? (c.step + c.fill * fill) * steps + c.end : ((blocks + cus - 1) / cus) * (c.round_step * steps + c.end));
-      if (d > 1) us += 1.7f + (float)d * c.bm * c.bn * 4 / 83e3f * (fill > 1.0f ? fill : 1.0f);
+      if (d > 1 && big) us = 4.5f + (float)(whole / cus) * (c.round_step * nk + c.end) + c.round_step * steps + c.end;
+      if (d > 1) us += (big ? 20.0f : 1.7f) + (float)d * c.bm * c.bn * 4 / 83e3f * (fill > 1.0f && !big ? fill : 1.0f);
       if (pin.bm == c.bm && pin.bn == c.bn && d == pin.split) us = 0.0f;   // taken
       if (best.shape < 0 || us < best.us) best = {us, s, d};
     }
@@ -667,8 +685,8 @@ static Choice choose_tile(const TileShape *shapes, int n_shapes, int epi, int M,
 
 static size_t sums_bytes(const TileShape *shapes, const Choice &c, int M, int weight_rows) {
   if (c.split < 2) return 0;
-  const int bm = shapes[c.shape].bm, bn = shapes[c.shape].bn;
-  return (size_t)((M + bm - 1) / bm) * (weight_rows / bn) * c.split * bm * bn * 4;
+  const int bm = shapes[c.shape].bm, bn = shapes[c.shape].bn, tiles = ((M + bm - 1) / bm) * (weight_rows / bn);
+  return (size_t)(tiles - (bm * bn == 65536 ? whole_tiles(tiles) : 0)) * c.split * bm * bn * 4;
 }
 
 template <int KIND, int EPI> static int launch_qshape(int s, const TileArgs &t, int prof_kind) {

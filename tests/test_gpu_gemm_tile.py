@@ -178,3 +178,18 @@ def test_many_short_int8_rows(hip, rows, captured):
     before = rows_tests.RNG.bit_generator.state               # the stream that the files share goes on where it was
     test_tiled_gemm_at_the_edges(Captured(hip) if captured else hip, "int8", rows, 49408, 512)
     rows_tests.RNG.bit_generator.state = before
+
+
+@pytest.mark.parametrize("kind", ["float16", "int8"])
+@pytest.mark.parametrize("tile", ["256x256/2", "256x256/3"])
+def test_largest_tiles_in_parts(hip, monkeypatch, kind, tile):
+    """K parts of the largest tile: where all tiles of a launch come in parts, under every epilogue, and where only two behind a whole round do."""
+    before = rows_tests.RNG.bit_generator.state               # the stream that the files share goes on where it was
+    monkeypatch.setenv("JSG_GEMM_TILE", tile)
+    for rows in (57, 295):
+        test_tiled_gemm_at_the_edges(hip, kind, rows, 768, 640)
+        rows_tests.test_gemm_ffn_gate(hip, kind, rows, 640, 384)
+    rows_tests.test_gemm_qkv_rope_writes_queries_and_cache(hip, kind, 64, 3, 19, 640)
+    rows_tests.test_gemm_qkv_rope_writes_queries_and_cache(hip, kind, 128, 5, 59, 640)
+    test_tiled_gemm_at_the_edges(hip, kind, 295, 129 * 256, 320)
+    rows_tests.RNG.bit_generator.state = before
