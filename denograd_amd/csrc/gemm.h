@@ -72,8 +72,7 @@ __device__ __forceinline__ void dma4(i4_t rs, uint32_t voff, uint32_t soff, uint
 }
 
 // RMSNorm.call (nn/index.ts:586-588) with the rounding points of rmsnorm_rows_kernel: the factor of a row with this sum of squares, and
-// eight elements of it.  The product and its rounding as one instruction with -0 added, v_fma_mixlo / mixhi_f16, instead of a conversion, a product and
-// a conversion: sixteen rows of 4096 take a compute unit 1.2 us instead of 2.4.
+// eight elements of it
 __device__ __forceinline__ float norm_factor(const GemmArgs &a, float sum) { return __fsqrt_rn(__fdiv_rn(1.0f, __fadd_rn(__fmul_rn(sum, a.inv_k), a.eps))); }
 __device__ __forceinline__ h8_t norm_piece(h8_t x, float r, h8_t w) {
   h8_t n;
@@ -81,10 +80,12 @@ __device__ __forceinline__ h8_t norm_piece(h8_t x, float r, h8_t w) {
   for (int e = 0; e < 8; e++) n[e] = (_Float16)__fmul_rn((float)x[e], r);
   return n * w;
 }
-// plus the squares of eight elements, two a step: products of halves are exact (norm and 6144 x 4096, int8, 5 rows: 11.4 us, element by element 11.8)
+// Plus the squares of eight elements, one by one (products of halves are exact, so each costs one rounding).  v_dot2_f32_f16 adds two at once and its sums are
+// further off: of 85 M normed elements of rows of 1024 to 4096, 4472 were not the nearest half, one by one 4176.  What that costs, us, 5 rows, two | one:
+// norm and wq|wk|wv of 3072 x 2048 5.6 | 5.9, w1|w3 of 8192 x 2048 14.6 | 14.6, int8 w1|w3 of 8192 x 3072 12.2 | 12.4.
 __device__ __forceinline__ float square_sum(h8_t x, float s) {
 #pragma unroll
-  for (int e = 0; e < 4; e++) s = __builtin_amdgcn_fdot2(as_h2(__builtin_bit_cast(u4_t, x)[e]), as_h2(__builtin_bit_cast(u4_t, x)[e]), s, false);
+  for (int e = 0; e < 8; e++) s = fmaf((float)x[e], (float)x[e], s);
   return s;
 }
 

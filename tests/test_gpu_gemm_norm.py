@@ -79,6 +79,54 @@ def test_rows_too_long_to_norm_in_registers_take_the_kernel_of_normed_rows(hip, 
     assert np.array_equal(got.numpy().view(np.uint16), ref.numpy().view(np.uint16))
 
 
+def factor_of_the_few_row_kernel(x, eps, kind):
+    """A lane (a quarter of the 32 or 64 elements of a fragment read) adds its squares one by one, in float with one rounding each, the four quarters of a
+    wavefront's eighth of the row meet in pairs and the eighths in order."""
+    rows, dim = x.shape
+    piece = 8 if kind == "float16" else 16
+    lanes = x.astype(np.float64).reshape(rows, 8, -1, 4, piece).transpose(0, 1, 3, 2, 4).reshape(rows, 8, 4, -1)
+    s = np.zeros(lanes.shape[:3], np.float32)
+    for e in range(lanes.shape[3]):
+        s = (s + lanes[..., e] ** 2).astype(np.float32)
+    s = (s[..., 0] + s[..., 1]) + (s[..., 2] + s[..., 3])
+    tot = s[:, 0]
+    for w in range(1, 8):
+        tot = tot + s[:, w]
+    return np.sqrt(np.float32(1) / (tot * np.float32(1 / dim) + np.float32(eps)))
+
+
+@pytest.mark.parametrize("kind,dim", [("float16", k) for k in (1024, 1536, 2048, 3072, 4096)] + [("int8", k) for k in (2048, 3072, 4096)])
+@pytest.mark.parametrize("rows", [16, 5])
+def test_squares_are_added_one_by_one(hip, kind, dim, rows):
+    """Seen through an identity matrix: ordinary rows of three sizes, subnormal ones, rows where a lane begins with 2^24 and adds squares between one and two
+    (each is rounded to two; the other half of the row makes the factor visible), the largest halves, and infinities and NaN, which spread over their own row
+    and no further.  The device's square root may be one unit off, and it may round x times the factor to a half at once or to float first: every
+    element of a row has to be that of one of three factors."""
+    rng = np.random.default_rng(dim + rows)
+    nw = (1.0 + 0.3 * rng.standard_normal(dim)).astype(np.float16)
+    eye, one = np.eye(dim, dtype=np.float16 if kind == "float16" else np.int8), np.ones(dim, np.float16)
+    w, s, tn = Tensor(eye), Tensor(one), Tensor(nw)
+    scratch, y = Tensor.full((rows, dim), 9.0, "float16"), Tensor.full((rows, dim), 7.0, "float16")
+    for turn in range(4):
+        x = (rng.standard_normal((rows, dim)) * np.array([1.0, 3e-3, 30.0, 2e-6, 1.0])[np.arange(rows) % 5, None]).astype(np.float16)
+        eighths = x[4::5].reshape(-1, 8, dim // 8)            # a view
+        eighths[:, :4] = 1.0 + 0.2 * rng.random(eighths[:, :4].shape)
+        eighths[:, :4, :64 if kind == "int8" else 32:16 if kind == "int8" else 8] = 4096.0
+        if turn % 2:
+            x[0] = 60000.0
+            x[1, dim // 3], x[2, 7], x[3, dim - 1] = np.inf, np.nan, -np.inf
+        tx, eps = Tensor(x), (EPS, 1e-16)[turn // 2]
+        check(hip.jsgrad_hip_gemm_norm(KINDS[kind], w.ptr, s.ptr, dim, dim, tx.ptr, tn.ptr, eps, scratch.ptr, rows, y.ptr))
+        got, whole = y.numpy(), np.isfinite(x).all(axis=1)
+        assert np.isnan(got[~whole]).all()                    # 0 * NaN in every product of such a row
+        r = factor_of_the_few_row_kernel(x[whole], eps, kind)
+        fits = np.zeros(r.shape, bool)
+        for f in (np.nextafter(r, np.float32(0)), r, np.nextafter(r, np.float32(np.inf))):
+            a, b = (p.astype(np.float16) * nw for p in (x[whole].astype(np.float32) * f[:, None], x[whole].astype(np.float64) * f[:, None].astype(np.float64)))
+            fits |= ((got[whole] == a) | (got[whole] == b)).all(axis=1)
+        assert fits.all(), (kind, dim, rows, turn, np.nonzero(whole)[0][~fits])
+
+
 @pytest.mark.parametrize("kind", ["float16", "int8", "nf4"])
 @pytest.mark.parametrize("tile", ["g16x64", "g32x64/3"])
 def test_normed_in_front_of_the_group_kernel(hip, monkeypatch, kind, tile):
