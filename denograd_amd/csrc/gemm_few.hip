@@ -318,9 +318,10 @@ int gemm_few(int epi, int kind, const GemmArgs &a, int prof_kind, bool *taken) {
   // The norm's weights are read here in 16-byte pieces; from any other address in memory first.
   if (a.norm_w && (a.K > 4096 || (uintptr_t)a.norm_w & 15)) return 0;
   const size_t most = (size_t)(a.norm_w && epi == GEPI_SWIGLU && a.K <= 3072 ? 88 : 36) << 20;
-  // 9 to 16 rows, K above 3072: only the weight rows of a model that wide (3073 to 4096 of them).  Narrower ones, 5.9 here against 8.0, keep the order of
-  // sums that such calls have had.
-  if (kind == JSGRAD_W_I8 && (elements > most || (a.M > 8 && (a.K > 4096 || (a.K > 3072 && (rows > 4096 || rows <= 3072)))))) return 0;
+  // int8 rows of 4096 behind 9 to 16 rows: up to 4096 weight rows.  us, 9 / 16 rows, the kernels below | this one: 512 weight rows 6.5 / 6.9 | 4.6 / 4.7, 1024 6.7 /
+  // 7.0 | 4.8 / 4.8, 2048 7.0 / 7.3 | 5.1 / 5.2, 3072 7.3 / 7.6 | 5.8 / 5.8, 4096 7.8 / 8.1 | 6.6 / 6.6; behind the line 5120 8.8 / 8.8 | 8.5 / 8.5, 6144 9.2 / 9.3 |
+  // 9.1 / 9.2, 8192 9.7 / 9.7 | 10.7 / 10.6; w1|w3 of 1024 9.8 / 10.0 | 6.3 / 6.3, of 2048 10.5 / 10.7 | 6.9 / 7.1.
+  if (kind == JSGRAD_W_I8 && (elements > most || (a.M > 8 && (a.K > 4096 || (a.K > 3072 && rows > 4096))))) return 0;
   if (pin_env(a, "JSG_GEMM_NO_SKINNY") || pin_env(a, "JSG_GEMM_SKINNY_TILES")) return 0;   // tests that want one of the other kernels
   if (epi == GEPI_STORE) return gemm_few_epi<GEPI_STORE>(kind, a, prof_kind, taken);
   if (epi == GEPI_ROPE_KV) return gemm_few_epi<GEPI_ROPE_KV>(kind, a, prof_kind, taken);
