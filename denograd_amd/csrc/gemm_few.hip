@@ -105,7 +105,22 @@ template <int KIND, int EPI, int SB, int PARTS, bool LONG, bool NORM> __global__
   float *const red = (float *)(few_lds + FW_WAVES * S::RING);  // [matrix][wavefront][16 x rows][16 weight rows]
   h8_t xf[NF];
   constexpr int XS = PARTS * MPR;                              // slots that the wavefront's share of x would fill
-  if constexpr (XS <= NS) {
+  auto norm_x = [&](const h8_t (&wf)[NORM ? NF : 1]) {         // in registers: sums over a wavefront's share, the eight shares through LDS in order
+    float ss = 0.0f;
+#pragma unroll
+    for (int f = 0; f < NF; f++) ss = square_sum(xf[f], ss);
+    ss = add_xor32(add_xor16(ss));
+    if (lq == 0) red[wave * 256 + l16] = ss;
+    lds_barrier();
+    float tot = red[l16];
+#pragma unroll
+    for (int w = 1; w < FW_WAVES; w++) tot += red[w * 256 + l16];
+    const float r = norm_factor(a, tot);
+#pragma unroll
+    for (int f = 0; f < NF; f++) xf[f] = norm_piece(xf[f], r, wf[f]);
+    lds_barrier();                                            // the sums have been read
+  };
+  if constexpr (XS <= NS && !(LONG && NORM)) {
     // Through the last slots of the ring, which are free until their steps are asked for.  The compiler does not count direct loads: a load of x
     // to registers would be waited for with every step asked for behind it, and nothing would be on its way until they are used.
     const i4_t rx = dma_rsrc(a.x);
@@ -137,29 +152,22 @@ template <int KIND, int EPI, int SB, int PARTS, bool LONG, bool NORM> __global__
 #pragma unroll
     for (int i = NS - XS; i < NS; i++)
       if (i < n_steps) issue(i);
-    if constexpr (NORM) {
-      // normed in registers: sums over a wavefront's share, the eight shares through LDS in order
-      float ss = 0.0f;
-#pragma unroll
-      for (int f = 0; f < NF; f++) ss = square_sum(xf[f], ss);
-      ss = add_xor32(add_xor16(ss));
-      if (lq == 0) ((float *)nw)[l16] = ss;
-      lds_barrier();
-      float tot = red[l16];
-#pragma unroll
-      for (int w = 1; w < FW_WAVES; w++) tot += red[w * 256 + l16];
-      const float r = norm_factor(a, tot);
-#pragma unroll
-      for (int f = 0; f < NF; f++) xf[f] = norm_piece(xf[f], r, wf[f]);
-      lds_barrier();                                          // the sums have been read
-    }
+    if constexpr (NORM) norm_x(wf);
   } else {
-    static_assert(!NORM, "rows short enough for the norm have room in the ring");
     const _Float16 *xr = a.x + (size_t)min(l16, a.M - 1) * a.K + k_first / KB + lq * (16 / KB);   // rows past the end: never stored
 #pragma unroll
     for (int f = 0; f < NF; f++) xf[f] = *(const h8_t *)(xr + (f / MPR) * (64 / KB) + (f % MPR) * 8);
+    if constexpr (NORM) {
+      // using x waits for all loads before it and behind it: the first step goes out ahead of that and the others behind
+      h8_t wf[NF];
+      const _Float16 *wr = a.norm_w + k_first / KB + lq * (16 / KB);
 #pragma unroll
-    for (int i = 0; i < NS; i++)
+      for (int f = 0; f < NF; f++) wf[f] = *(const h8_t *)(wr + (f / MPR) * (64 / KB) + (f % MPR) * 8);
+      if (n_steps > 0) issue(0);
+      norm_x(wf);
+    }
+#pragma unroll
+    for (int i = NORM ? 1 : 0; i < NS; i++)
       if (i < n_steps) issue(i);
     // Waited for here, or the compiler, which does not count the direct loads, would wait for all of them at the first use of x in
     // every turn of the loop below.  Where there is hardly a second turn the steps behind the first need not have landed yet.
@@ -255,12 +263,20 @@ template <int KIND, int EPI, int SB, int PARTS, bool LONG, bool NORM> static int
   JSG_LAUNCH(prof_kind, (few_rows_kernel<KIND, EPI, SB, PARTS, LONG, NORM>), dim3(grid), dim3(FW_THREADS), lds, a, tiles);
   return 0;
 }
-// LONG, where x does not come through the ring: two weight tiles or more per block (us, with and without: fp16 16384 x 2048 16.3 | 17.1, 2048 x 8192 9.2 | 8.7)
+// LONG, where x does not come through the ring: two weight tiles or more per block (us, with and without: fp16 16384 x 2048 16.3 | 17.1, 2048 x 8192 9.2 | 8.7).
+// With a norm: int8 rows of 4096, whose x fills the ring, so that no weights are asked for until it is in registers.  Up to seven rows, and from seven quarters of a
+// step per block on (w1|w3 six), x goes to registers straight, the first step of weights beside it.  us, 1 / 5 / 8 rows, ring | registers: 6656 x 4096 11.2 / 11.4 / 11.5
+// | 10.8 / 11.2 / 11.7, 7168 11.6 / 11.8 / 11.8 | 11.1 / 11.6 / 12.1, 8192 12.5 / 12.7 / 12.7 | 11.6 / 12.2 / 12.7, w1|w3 of 2560 10.1 / 10.2 / 10.2 | 9.7 / 10.1 / 10.6,
+// 3072 10.8 / 10.9 / 11.0 | 10.2 / 10.6 / 11.2, 4096 12.4 / 12.4 / 12.5 | 11.5 / 12.0 / 12.6; less per block: 4096 8.1 / 8.0 / 8.0 | 8.6 / 8.7 / 9.2.
 template <int KIND, int EPI, int SB, int PARTS> static int launch_few(const GemmArgs &a, int prof_kind) {
   constexpr int MPR = KIND == JSGRAD_W_F16 ? 1 : 2;
   const int tiles = a.N / 16, cus = state().cu_count, grid = 2 * tiles < cus ? 2 * tiles : cus;
   if constexpr (PARTS * SB * MPR <= 1024)                     // rows of at most 4096: what gemm_few takes with a norm
-    if (a.norm_w) return launch_few_as<KIND, EPI, SB, PARTS, false, true>(a, tiles, grid, prof_kind);
+    if (a.norm_w) {
+      if constexpr (KIND == JSGRAD_W_I8 && SB == 512)
+        if (a.M <= 7 && (EPI == GEPI_SWIGLU ? 2 * tiles >= grid + grid / 2 : tiles >= grid + grid * 3 / 4)) return launch_few_as<KIND, EPI, SB, PARTS, true, true>(a, tiles, grid, prof_kind);
+      return launch_few_as<KIND, EPI, SB, PARTS, false, true>(a, tiles, grid, prof_kind);
+    }
   if constexpr (PARTS * MPR > FwShape<KIND, EPI, SB>::NS)
     if (tiles * (EPI == GEPI_SWIGLU ? 2 : 1) >= 2 * grid) return launch_few_as<KIND, EPI, SB, PARTS, true, false>(a, tiles, grid, prof_kind);
   return launch_few_as<KIND, EPI, SB, PARTS, false, false>(a, tiles, grid, prof_kind);

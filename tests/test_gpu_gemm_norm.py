@@ -127,6 +127,43 @@ def test_squares_are_added_one_by_one(hip, kind, dim, rows):
         assert fits.all(), (kind, dim, rows, turn, np.nonzero(whole)[0][~fits])
 
 
+@pytest.mark.parametrize("out_f,hidden", [(7040, 2944), (7168, 3072), (8192, 4096), (9216, 4608)])
+def test_int8_rows_of_4096_have_the_same_bits_by_either_way_of_x(hip, out_f, hidden):
+    """Up to seven rows in front of wide matrices x comes to registers straight, otherwise through the ring: the rows of calls of 1, 5 and 7 are those of
+    a call of 8, under every epilogue, an infinite and a NaN row among them."""
+    dim, hd, rng = 4096, 128, np.random.default_rng(out_f)
+    x = (rng.standard_normal((8, dim)) * 3).astype(np.float16)
+    x[2, 5], x[3, dim - 1], x[4] = np.inf, np.nan, 0.0
+    tx, tn = Tensor(x), Tensor((1.0 + 0.3 * rng.standard_normal(dim)).astype(np.float16))
+    w, s = dev(*make_weight("int8", out_f, dim))
+    kv = 128
+    q_rows = out_f - 2 * kv
+    table, scratch = Tensor.zeros((64, hd // 2, 2), "float16"), Tensor.empty((8, dim), "float16")
+    check(hip.jsgrad_hip_rope_table(table.ptr, hd, 64, 500000.0, ffi.F16))
+    at = lambda row: (w.ptr + row * dim, s.ptr + row * 2)
+    calls = []
+    for rows in (8, 1, 5, 7):
+        y, g, q = (Tensor.full((rows + 1, n), 7.0, "float16") for n in (out_f, hidden, q_rows))
+        caches = [Tensor.full((rows, 32, kv), 7.0, "float16") for _ in range(2)]
+        check(hip.jsgrad_hip_gemm_norm(ffi.W_I8, *at(0), out_f, dim, tx.ptr, tn.ptr, EPS, scratch.ptr, rows, y.ptr))
+        check(hip.jsgrad_hip_gemm_ffn_gate_norm(ffi.W_I8, *at(0), *at(hidden), tx.ptr, tn.ptr, EPS, scratch.ptr, rows, g.ptr, dim, hidden))
+        check(hip.jsgrad_hip_gemm_qkv_rope_norm(ffi.W_I8, *at(0), *at(q_rows), *at(q_rows + kv), tx.ptr, tn.ptr, EPS, scratch.ptr, rows, 1, 3, table.ptr, q.ptr,
+                                                caches[0].ptr, caches[1].ptr, dim, q_rows // hd, kv // hd, hd, 32))
+        for t in (y, g, q):
+            assert np.all(t.numpy()[rows] == 7.0)
+        calls.append([t.numpy()[:rows].view(np.uint16) for t in (y, g, q, *caches)])
+    for got in calls[1:]:
+        for a, b in zip(got, calls[0]):
+            nan = np.isnan(a.view(np.float16)) & np.isnan(b[:len(a)].view(np.float16))
+            assert np.array_equal(np.where(nan, 0, a), np.where(nan, 0, b[:len(a)]))
+
+
+@pytest.mark.parametrize("rows,out_f,hidden", [(1, 7040, 2944), (1, 7168, 3072), (7, 7168, 3072), (8, 7168, 3072), (5, 9216, 4608)])
+def test_normed_int8_rows_of_4096(hip, rows, out_f, hidden):
+    check_plain(hip, "int8", rows, out_f, 4096)
+    test_normed_ffn_gate(hip, "int8", rows, 4096, hidden)
+
+
 @pytest.mark.parametrize("kind", ["float16", "int8", "nf4"])
 @pytest.mark.parametrize("tile", ["g16x64", "g32x64/3"])
 def test_normed_in_front_of_the_group_kernel(hip, monkeypatch, kind, tile):
