@@ -129,7 +129,9 @@ template <int KIND, int EPI, int SB, int PARTS, bool LONG, bool NORM> __global__
 #pragma unroll
       for (int j = 0; j < LOADS; j++) {
         const int o = j * 1024 + lane * 16, r = o / SB, p = (o % SB) / 16;
-        if (j < LOADS / 2 || a.M > 8)                         // rows past the end: the last one again, or what the slot held, and never stored
+        // Rows past the end: the last one again, or what the slot held, and never stored.  Steps of 256 bytes: a load is four rows, the last one of nobody's up
+        // to 12 (us, 9 / 12 rows, with it | without: int8 4096 x 2048 4.6 / 4.6 | 4.4 / 4.4, wq|wk|wv of 3072 x 2048 4.4 / 4.5 | 4.2 / 4.3)
+        if (j < LOADS / 2 || a.M > (SB == 256 && j == LOADS - 1 ? 12 : 8))
           dma16(rx, (uint32_t)min(r, a.M - 1) * (uint32_t)a.K * 2 + (uint32_t)(p ^ swizzle(r)) * 16, k_first * MPR + i * SB, ring0 + (NS - XS + i) * (S::SLOT + S::SCALE) + j * 1024);
       }
     // the norm's weights of the wavefront's share into its part of the sums' space: at most 1 KiB

@@ -79,3 +79,19 @@ def test_int8_rows_of_4096_behind_up_to_16_rows(hip, rows, out_f, in_f):
         check(hip.jsgrad_hip_gemm(KINDS["int8"], w.ptr, s.ptr, out_f, in_f, x.ptr, n, y.ptr, None))
         out.append(y.numpy().view(np.uint16)[:8])
     assert np.array_equal(*out) == (out_f <= 4096)
+
+
+@pytest.mark.parametrize("kind,in_f", [("float16", 1024), ("int8", 2048)])
+@pytest.mark.parametrize("rows", [9, 12, 13])
+@pytest.mark.parametrize("out_f", [256, 6400])
+def test_steps_of_256_bytes_ask_for_twelve_or_sixteen_rows(hip, kind, in_f, rows, out_f):
+    """The fourth load of x is left out where nobody has its rows: the oracle's values, and the bits of the first rows of a call of 16."""
+    test_few_rows_against_oracle(hip, kind, in_f, rows, out_f)
+    w, s = dev(*make_weight(kind, out_f, in_f))
+    x = Tensor.randn((16 * in_f,), "float16", 2, 1.0)
+    out = []
+    for n in (16, rows):
+        y = Tensor.empty((n, out_f), "float16")
+        check(hip.jsgrad_hip_gemm(KINDS[kind], w.ptr, sp(s), out_f, in_f, x.ptr, n, y.ptr, None))
+        out.append(y.numpy().view(np.uint16)[:rows])
+    assert np.array_equal(*out)
