@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 import oracle as orc
+from denograd_amd import ffi
 from denograd_amd.ffi import check
 from denograd_amd.tensor import Tensor
 from tests.helpers import assert_close
@@ -95,3 +96,39 @@ def test_steps_of_256_bytes_ask_for_twelve_or_sixteen_rows(hip, kind, in_f, rows
         check(hip.jsgrad_hip_gemm(KINDS[kind], w.ptr, sp(s), out_f, in_f, x.ptr, n, y.ptr, None))
         out.append(y.numpy().view(np.uint16)[:rows])
     assert np.array_equal(*out)
+
+
+# A wavefront that stores a part of a unit's outputs leaves that store in flight behind the steps that it waits for; one to four of the eight do.  Several whole
+# rounds of units, a last one of halves (8320 columns) or a ragged one (11392):
+
+@pytest.mark.parametrize("rows,hidden", [(1, 11392), (4, 8320), (5, 11392), (13, 8320), (16, 8320)])
+@pytest.mark.parametrize("dim", [1024, 2048, 3072])
+def test_fp16_gates_with_several_rounds_of_tiles(hip, rows, hidden, dim):
+    ffn_gate(hip, "float16", rows, dim, hidden)
+
+
+@pytest.mark.parametrize("kind,dim", [("float16", 1024), ("float16", 2048), ("float16", 4096), ("int8", 2048)])
+@pytest.mark.parametrize("rows,heads", [(1, 174), (4, 126), (5, 174), (13, 126), (16, 126)])
+def test_qkv_rope_with_several_rounds_of_tiles(hip, kind, dim, rows, heads):
+    """Against the plain product of the stacked matrices, which adds in the same order, and the oracle's rotary step."""
+    hd, kv, ctx, start, rng = 64, 2, 16, 5, np.random.default_rng(rows + dim)
+    n = (heads + 2 * kv) * hd
+    w, s = dev(*make_weight(kind, n, dim))
+    x = Tensor(rng.standard_normal((rows, dim)).astype(np.float16))
+    y = Tensor.empty((rows, n), "float16")
+    check(hip.jsgrad_hip_gemm(KINDS[kind], w.ptr, sp(s), n, dim, x.ptr, rows, y.ptr, None))
+    raw = y.numpy().astype(np.float32)
+    table = Tensor.empty((2 * ctx, hd // 2, 2), "float16")
+    check(hip.jsgrad_hip_rope_table(table.ptr, hd, 2 * ctx, 500000.0, ffi.F16))
+    fc = table.numpy().astype(np.float32)
+    at = lambda row: (w.ptr + row * dim * (2 if kind == "float16" else 1), s.ptr + row * 2 if s is not None else None)
+    q, ck, cv = Tensor.full((rows + 1, heads * hd), 7.0, "float16"), Tensor.zeros((rows, ctx, kv * hd), "float16"), Tensor.zeros((rows, ctx, kv * hd), "float16")
+    check(hip.jsgrad_hip_gemm_qkv_rope(KINDS[kind], *at(0), *at(heads * hd), *at((heads + kv) * hd), x.ptr, rows, 1, start, table.ptr, q.ptr, ck.ptr, cv.ptr,
+                                       dim, heads, kv, hd, ctx))
+    assert np.all(q.numpy()[rows] == 7.0)
+    q_raw, k_raw, v_raw = np.split(raw, [heads * hd, (heads + kv) * hd], axis=1)
+    assert_close(q.numpy()[:rows].astype(np.float32), np.stack([orc.rope(r, heads, hd, fc[start], True) for r in q_raw]), True, "q", composed=True)
+    assert_close(ck.numpy()[:, start].astype(np.float32), np.stack([orc.rope(r, kv, hd, fc[start], True) for r in k_raw]), True, "k", composed=True)
+    assert np.array_equal(cv.numpy()[:, start].astype(np.float32), v_raw)
+    rest = np.arange(ctx) != start
+    assert not ck.numpy()[:, rest].any() and not cv.numpy()[:, rest].any()

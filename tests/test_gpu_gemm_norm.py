@@ -186,6 +186,11 @@ def test_normed_ffn_gate(hip, kind, rows, dim, hidden):
     assert_close(got.numpy().astype(np.float32), ref.numpy().astype(np.float32), True, f"{kind} {rows}", composed=True)
 
 
+@pytest.mark.parametrize("rows,dim,hidden", [(1, 2048, 11392), (4, 2048, 8320), (5, 3072, 11392), (13, 2048, 8320), (16, 3072, 8320)])
+def test_normed_fp16_gates_with_several_rounds_of_tiles(hip, rows, dim, hidden):
+    test_normed_ffn_gate(hip, "float16", rows, dim, hidden)
+
+
 @pytest.mark.parametrize("rows,dim,hidden", [(1, 3072, 8192), (16, 3072, 14976), (3, 3072, 15104), (9, 2048, 9216)])
 def test_normed_ffn_gate_of_wide_int8_matrices(hip, rows, dim, hidden):
     """From 36 M codes on the norm alone decides between two kernels (up to 88 M)."""
