@@ -3,11 +3,11 @@
 //
 // The launch is bound by reading W once.  A block of eight wavefronts stays on its compute unit and walks tiles of 16 weight rows;
 // the wavefronts split K, and a wavefront's share of x (16 rows of K / 8 elements, at most 128 registers) is in operand layout in
-// its registers for the whole launch, so x costs one read per block and no LDS traffic, and no barrier stands between a
-// wavefront and its weights.  Those come by direct global-to-LDS loads into a ring that belongs to the wavefront (16 KiB:
-// 128 KiB of every compute unit's LDS are on their way), 256 to 512 contiguous bytes of a row at a time: asked for in operand
-// layout (64 bytes of each of 16 rows per load) the same bytes take a quarter longer.  Per tile the eight partial sums are
-// added through LDS in wavefront order.
+// its registers for the whole launch, so x costs one read per block, and no barrier stands between a wavefront and its weights.
+// Those come by direct global-to-LDS loads into a ring that belongs to the wavefront (16 KiB: 128 KiB of every compute unit's LDS
+// are on their way), 256 to 512 contiguous bytes of a row at a time: asked for in operand layout (64 bytes of each of 16 rows per
+// load) the same bytes take a quarter longer.  Where the ring has room for it, x comes through its last slots.  Per tile the eight
+// partial sums are added through LDS in wavefront order.
 // Tiles that are left after whole rounds over the compute units are dealt as halves of eight rows where that is enough for
 // everybody (w1|w3 of 14336 rows: 896 tiles on 256 units are 3.5 rounds instead of 4).
 #include <type_traits>
@@ -315,8 +315,10 @@ int gemm_few(int epi, int kind, const GemmArgs &a, int prof_kind, bool *taken) {
   // over wide matrices.  us, 8 / 16 rows, that one | this one: 2048 x 8192 9.1 / 9.4 | 9.2 / 12.0, 3072 x 8192 9.9 / 10.1 | 10.4 / 12.5, 4096 x 6144
   // 10.3 / 10.4 | 9.3 / 12.3; with x through the ring 3072 x 4096 - / 8.0 | 5.6 / 5.9, 4096 x 4096 - / 8.6 | 6.1 / 6.7, 6144 x 4096 - / 9.6 | 9.2 / 9.8, 8192 x 4096
   // - / 9.7 | 10.3 / 10.8, 16384 x 3072 11.7 / 11.7 | 11.6 / 12.1, 28672 x 4096 21.4 / 21.5 | 25.2 / 25.9, 128256 x 2048 45 / 47 | 53 / 59.  With a norm in
-  // front, which there is a launch of its own, w1|w3 of 8192 x 3072 13.6 / 13.7 | 12.3 / 12.7, of 14336 x 3072 19.8 / 20.1 | 18.2 / 18.7, of 6144 x 4096
-  // 14.7 / 15.0 | 15.1 / 15.5, one matrix of 16384 x 3072 13.3 / 13.5 | 13.3 / 14.2, of 24576 x 2048 13.6 / 14.0 | 13.6 / 14.3.
+  // front, which there is a launch of its own: one matrix level (16384 x 3072 13.5 / 13.6 | 13.6 / 14.4, 24576 x 2048 13.9 / 14.2 | 13.8 / 14.3), w1|w3 of
+  // rows of 2048 and 3072 faster here at any number (9216 x 2048 13.5 / 13.8 | 12.6 / 13.1, 14336 15.6 / 15.8 | 15.1 / 15.8, 20480 21.6 / 21.9 | 18.1 / 18.9, 28672
+  // 27.2 / 27.6 | 22.5 / 23.4; 8192 x 3072 14.2 / 14.3 | 12.7 / 13.4, 14336 20.8 / 21.1 | 19.2 / 19.8, 20480 28.0 / 28.7 | 23.6 / 24.2, 28672 36.4 / 37.0 | 30.5 / 31.5),
+  // of rows of 4096 slower (6144 x 4096 15.0 / 15.5 | 15.7 / 16.4).
   // fp16, skinny_gemm_kernel | this one, 2 / 8 / 16 rows: 2048 x 2048 6.2 / 6.3 / 6.3 | 4.5 / 4.5 / 5.1, 2048 x 8192 14.1 / 14.9 / 15.9 |
   // 8.8 / 9.5 / 12.4, 16384 x 2048 23.6 / 23.7 / 24.4 | 16.3 / 17.2 / 18.2, 128256 x 2048 147 / 153 / 162 | 88 / 92 / 94 (6.0 TB/s).
   // fp16 rows of more than 4096 elements (6144 and 8192 come here): the more rows of x a block reads for its few tiles, the nearer gemm_group.hip, which reads x from LDS, comes.  us,
@@ -335,7 +337,7 @@ int gemm_few(int epi, int kind, const GemmArgs &a, int prof_kind, bool *taken) {
   // costs more than the launches: 8B int8 16 rows 3321 | 3403, 8B NF4 16 layers 8 rows 1403 | 1467.
   // The norm's weights are read here in 16-byte pieces; from any other address in memory first.
   if (a.norm_w && (a.K > 4096 || (uintptr_t)a.norm_w & 15)) return 0;
-  const size_t most = (size_t)(a.norm_w && epi == GEPI_SWIGLU && a.K <= 3072 ? 88 : 36) << 20;
+  const size_t most = a.norm_w && epi == GEPI_SWIGLU && a.K <= 3072 ? SIZE_MAX : (size_t)36 << 20;
   // int8 rows of 4096 behind 9 to 16 rows: up to 4096 weight rows.  us, 9 / 16 rows, the kernels below | this one: 512 weight rows 6.5 / 6.9 | 4.6 / 4.7, 1024 6.7 /
   // 7.0 | 4.8 / 4.8, 2048 7.0 / 7.3 | 5.1 / 5.2, 3072 7.3 / 7.6 | 5.8 / 5.8, 4096 7.8 / 8.1 | 6.6 / 6.6; behind the line 5120 8.8 / 8.8 | 8.5 / 8.5, 6144 9.2 / 9.3 |
   // 9.1 / 9.2, 8192 9.7 / 9.7 | 10.7 / 10.6; w1|w3 of 1024 9.8 / 10.0 | 6.3 / 6.3, of 2048 10.5 / 10.7 | 6.9 / 7.1.

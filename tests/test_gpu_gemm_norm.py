@@ -193,7 +193,7 @@ def test_normed_fp16_gates_with_several_rounds_of_tiles(hip, rows, dim, hidden):
 
 @pytest.mark.parametrize("rows,dim,hidden", [(1, 3072, 8192), (16, 3072, 14976), (3, 3072, 15104), (9, 2048, 9216)])
 def test_normed_ffn_gate_of_wide_int8_matrices(hip, rows, dim, hidden):
-    """From 36 M codes on the norm alone decides between two kernels (up to 88 M)."""
+    """From 36 M codes on the norm decides between two kernels."""
     test_normed_ffn_gate(hip, "int8", rows, dim, hidden)
 
 
