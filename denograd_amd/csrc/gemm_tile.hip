@@ -129,7 +129,10 @@ template <int TM, int TN, int SUMS, int RB = TM> __device__ __forceinline__ bool
 // 3, in 6 and 7; A1, read in 4 and 5, in 8 and 9), so every load has 11 slots (3000 cycles) to arrive and five pairs of a
 // wavefront's loads may be outstanding when a phase needs the sixth.
 // Tiles behind the last whole round of blocks may come in K parts (t.whole, t.split), so that the last round is a short one: us, as chosen without |
-// with, 1200 x 4096 x 14336 162 | 136, w1|w3 of 14336 x 4096 behind 1600 rows 388 | 354, 3300 x 6144 x 4096 164 | 149, 4096 x 6144 x 4096 177 | 172.
+// with, launches one after the other, 1200 x 4096 x 14336 162 | 135, w1|w3 of 14336 x 4096 behind 1600 rows 390 | 358, 3300 x 6144 x 4096 160 | 148, 4099 x 4096 x
+// 14336 449 | 391, 8192 x 3072 x 8192 332 | 314, 4096 x 6144 x 4096 176 | 168; the last one between the other launches of a prompt, where the chip is at its
+// power limit and half of it idle runs faster, 184 | 189.  ms of prompts, 8 layers of the 8B shape, nf4: 1200 6.06 | 5.51, 1600 7.26 | 6.84, 4099 15.4 | 14.7, 6000
+// 21.6 | 20.8, 4096 13.50 | 13.53 (two runs differ by 0.5 %).
 // Measured (fp16): 32768 x 28672 x 4096 1420, 32768 x 4096 x 14336 1430-1450, 4096^3 1410 TFLOP/s (1050-1110 for the kernel
 // with 32x32 instructions and tiles through registers it replaces; the same loop without its epilogue 1500).
 constexpr int T256_OPERAND = 256 * 128;                       // bytes of one operand tile
