@@ -130,9 +130,8 @@ template <int TM, int TN, int SUMS, int RB = TM> __device__ __forceinline__ bool
 // wavefront's loads may be outstanding when a phase needs the sixth.
 // Tiles behind the last whole round of blocks may come in K parts (t.whole, t.split), so that the last round is a short one: us, as chosen without |
 // with, launches one after the other, 1200 x 4096 x 14336 162 | 135, w1|w3 of 14336 x 4096 behind 1600 rows 390 | 358, 3300 x 6144 x 4096 160 | 148, 4099 x 4096 x
-// 14336 449 | 391, 8192 x 3072 x 8192 332 | 314, 4096 x 6144 x 4096 176 | 168; the last one between the other launches of a prompt, where the chip is at its
-// power limit and half of it idle runs faster, 184 | 189.  ms of prompts, 8 layers of the 8B shape, nf4: 1200 6.06 | 5.51, 1600 7.26 | 6.84, 4099 15.4 | 14.7, 6000
-// 21.6 | 20.8, 4096 13.50 | 13.53 (two runs differ by 0.5 %).
+// 14336 449 | 391, 8192 x 3072 x 8192 332 | 314.  ms of prompts, 8 layers of the 8B shape, nf4: 1200 6.06 | 5.51, 1600 7.26 | 6.84, 4099 15.4 | 14.7, 6000
+// 21.6 | 20.8 (two runs differ by 0.5 %).
 // Measured (fp16): 32768 x 28672 x 4096 1420, 32768 x 4096 x 14336 1430-1450, 4096^3 1410 TFLOP/s (1050-1110 for the kernel
 // with 32x32 instructions and tiles through registers it replaces; the same loop without its epilogue 1500).
 constexpr int T256_OPERAND = 256 * 128;                       // bytes of one operand tile
@@ -680,7 +679,12 @@ static Choice choose_tile(const TileShape *shapes, int n_shapes, int epi, int M,
       if (d > 1 && big) us = 4.5f + (float)(whole / cus) * (c.round_step * nk + c.end) + c.round_step * steps + c.end;
       if (d > 1) us += (big ? 20.0f : 1.7f) + (float)d * c.bm * c.bn * 4 / 83e3f * (fill > 1.0f && !big ? fill : 1.0f);
       if (pin.bm == c.bm && pin.bn == c.bn && d == pin.split) us = 0.0f;   // taken
-      if (best.shape < 0 || us < best.us) best = {us, s, d};
+      // Parts behind whole rounds instead of a smaller tile: only where the estimate is 6 % lower.  Alone they keep what it says (4096 x 6144 x 4096 176 | 168), but
+      // between the other launches of a prompt, where the chip is at its power limit, a last round that leaves units idle runs faster.  us there, smaller tile | parts, with
+      // estimates that are 2 to 5.6 % lower: 3000 x 6144 x 4096 147 | 155, 4096 182 | 184 (189 | 196 on another card), 4200 x 5120 x 3072 138 | 147, 7000 x 3072 x 3072 127 |
+      // 130; 7 % int8 6400 x 3072 x 3072 135 | 121, 16 % 3300 x 6144 x 4096 175 | 165, 5000 x 4096 x 4096 166 | 157.
+      const bool sure = d == 1 || whole == 0 || (best.shape >= 0 && shapes[best.shape].bm == c.bm && shapes[best.shape].bn == c.bn);
+      if (best.shape < 0 || us * (sure ? 1.0f : 1.06f) < best.us) best = {us, s, d};
     }
   }
   return best;

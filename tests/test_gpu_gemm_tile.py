@@ -193,3 +193,19 @@ def test_largest_tiles_in_parts(hip, monkeypatch, kind, tile):
     rows_tests.test_gemm_qkv_rope_writes_queries_and_cache(hip, kind, 128, 5, 59, 640)
     test_tiled_gemm_at_the_edges(hip, kind, 295, 129 * 256, 320)
     rows_tests.RNG.bit_generator.state = before
+
+
+@pytest.mark.parametrize("rows,out_f,in_f,tile,other", [
+    (4096, 6144, 4096, "256x128", "256x256/2"), (3000, 6144, 4096, "192x128", "256x256/5"), (4200, 5120, 3072, "256x128", "256x256/3"),
+    (3300, 6144, 4096, "256x256/4", "256x128"), (1200, 4096, 14336, "256x256/3", "256x128")])
+def test_lines_to_largest_tiles_in_parts(hip, monkeypatch, rows, out_f, in_f, tile, other):
+    """Which tile a call comes to, by its bits: parts add the sums in another order."""
+    x, w = Tensor.randn((rows * in_f,), "float16", 1, 1.0), Tensor.randn((out_f * in_f,), "float16", 2, 0.02)
+    out = []
+    for pin in ("", tile, other):
+        if pin:
+            monkeypatch.setenv("JSG_GEMM_TILE", pin)
+        y = Tensor.empty((rows, out_f), "float16")
+        check(hip.jsgrad_hip_gemm(ffi.W_F16, w.ptr, None, out_f, in_f, x.ptr, rows, y.ptr, None))
+        out.append(y.numpy().view(np.uint16))
+    assert np.array_equal(out[0], out[1]) and not np.array_equal(out[0], out[2])
